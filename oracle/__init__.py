@@ -30,7 +30,7 @@ def build(reference=None):
     """make -C oracle (and oracle/_ref when the reference tree is present)."""
     subprocess.run(["make", "-s", "-C", HERE], check=True)
     ref = reference or "/root/reference"
-    if os.path.isdir(ref):
+    if os.path.isfile(os.path.join(ref, "quadrature.cpp")):
         subprocess.run(["make", "-s", "-C", HERE, "ref", "REF=" + ref], check=True)
 
 
