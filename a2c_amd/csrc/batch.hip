@@ -1422,9 +1422,10 @@ int fused_eval(a2c_batch* b, const std::vector<int>& ids_in, bool fp64, StateOf 
     lats[k] = L;
     const int nb = site_blocks(s.N());
     map.insert(map.end(), nb, (int32_t)k);
-    omap.insert(omap.end(), (size_t)nb * kl, (int32_t)k);
+    const int no = owner_units(L.npd, L.nh, kl);
+    omap.insert(omap.end(), (size_t)no, (int32_t)k);
     cum += nb;
-    ocum += nb * kl;
+    ocum += no;
   }
   size_t need = ((lats.size() * sizeof(LatDev) + 255) & ~(size_t)255) + ((map.size() * 4 + 255) & ~(size_t)255) +
                 ((omap.size() * 4 + 255) & ~(size_t)255);

@@ -46,6 +46,10 @@ int upload_state(a2c_fe_ctx* c, const double* X) {
   return A2C_OK;
 }
 
+// entries of the block -> lattice map: site blocks or the units of a
+// pair-owner pass at any lanes per site
+int map_units(int N) { return owner_units(N, MAX_LANES_PER_SITE) + 1; }
+
 bool aligned32(const void* p) { return ((uintptr_t)p & 31u) == 0; }
 
 }  // namespace
@@ -114,7 +118,9 @@ int a2c::fe_create(const a2c_fe_desc* desc, hipStream_t shared, a2c_fe_ctx** out
             dmalloc(&c->dFp, 8 * N) == hipSuccess && dmalloc(&c->demb, 8 * N) == hipSuccess &&
             dmalloc(&c->dpart, 8 * (size_t)c->nblk_red) == hipSuccess && dmalloc(&c->dF, 64) == hipSuccess &&
             dmalloc(&c->dlat, sizeof(LatDev)) == hipSuccess &&
-            dmalloc(&c->db2l, 4 * (size_t)c->nblk_red * MAX_LANES_PER_SITE) == hipSuccess;
+            dmalloc(&c->dqxy, 16 * N) == hipSuccess && dmalloc(&c->dqzs, 16 * N) == hipSuccess &&
+            dmalloc(&c->dxrow, 8 * nh) == hipSuccess && dmalloc(&c->dgown, 32 * N) == hipSuccess &&
+            dmalloc(&c->db2l, 4 * (size_t)map_units(c->N)) == hipSuccess;
   if (!ok) return fail(A2C_ENOMEM);
   {
     DeviceTables t;
@@ -122,7 +128,7 @@ int a2c::fe_create(const a2c_fe_desc* desc, hipStream_t shared, a2c_fe_ctx** out
     c->dtab64 = t.t64;  // shared, not freed with the context
   }
   // all-zero block -> lattice map, long enough for the pair-owner launches too
-  if (hipMemset(c->db2l, 0, 4 * (size_t)c->nblk_red * MAX_LANES_PER_SITE) != hipSuccess) return fail(A2C_EHIP);
+  if (hipMemset(c->db2l, 0, 4 * (size_t)map_units(c->N)) != hipSuccess) return fail(A2C_EHIP);
   c->lat_dirty = true;
   if (desc->precision == A2C_PREC_MIXED && build_tables(c) != A2C_OK) return fail(A2C_EHIP);
   *out = c;
@@ -135,7 +141,8 @@ void a2c_fe_destroy(a2c_fe_ctx* c) {
   if (!c) return;
   if (c->stream) hipStreamSynchronize(c->stream);
   dfree(c->dX); dfree(c->dG); dfree(c->dx); dfree(c->drho); dfree(c->dFp);
-  dfree(c->demb); dfree(c->dpart); dfree(c->dF); dfree(c->dpdpdnum); dfree(c->daux);  // dtab, dtab64: shared
+  dfree(c->demb); dfree(c->dpart); dfree(c->dF); dfree(c->dpdpdnum); dfree(c->daux);
+  dfree(c->dqxy); dfree(c->dqzs); dfree(c->dxrow); dfree(c->dgown);  // dtab, dtab64: shared
   gen_free(c);
   for (int w = 0; w < 5; ++w) {
     dfree(c->ell[w].idx); dfree(c->ell[w].cnt);

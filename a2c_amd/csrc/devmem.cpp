@@ -183,6 +183,7 @@ hipError_t device_tables(int device, DeviceTables* out) {
     std::vector<float4> t32;
     std::vector<double> t64;
     host_tables(t32);
+    host_tables_s(t32);
     host_tables64(t64);
     DeviceTables d;
     hipError_t e = hipMalloc(&d.t32, sizeof(float4) * t32.size());

@@ -7,19 +7,18 @@
 //         per-site accumulation of the per-pair sums, rho, F(rho), F'(rho),
 //         the per-site objective share and the global reduction.
 //   FP32: the 12 quadrature points of a pair: |r|^2 = |d|^2 + a^2 +- 2 a d_c
-//         (each point displaces d along one axis by a = sqrt(6) sigma), 1/|r|
-//         by v_rsq_f32, and the EAM functions.  Under the Gauss-Hermite rule
-//         the 27 nodes r_k = d + s sqrt(3) a_k (a_k in {-1,0,1}^3) have
+//         (each point displaces d along one axis by a = sqrt(6) sigma), and the
+//         EAM functions there.  Under the Gauss-Hermite rule the 27 nodes
+//         r_k = d + s sqrt(3) a_k (a_k in {-1,0,1}^3) have
 //         |r_k|^2 = |d|^2 + 3 s^2 |a_k|^2 + 2 sqrt(3) s (a_k . d).
 //
-// The EAM functions are piecewise cubic Hermite polynomials on a uniform grid
-// in r (h = 0.01 A over [1, 6] A, switch radii 5.0, 5.05, 5.35 on grid
-// nodes), built on the host in 80-bit long double from the closed forms and
-// their analytic derivatives, stored as FP32 coefficients in the local
-// coordinate u in [0,1), and staged in LDS (5 tables x 500 intervals x 16 B =
-// 40 KB per workgroup).  Beyond 6 A every function is the exponential tail
-// of potential.cpp, evaluated directly.  Interpolation error is below the FP32
-// rounding of the table values (~1e-7 relative, mean bias ~1e-10).
+// The EAM functions are piecewise cubics built on the host in 80-bit long
+// double, stored as FP32 coefficients in the local coordinate u in [0, 1) and
+// staged in LDS.  The pair-once passes take them on a uniform grid in |r|^2
+// (see "pair-once"), the full-list passes on one in |r|: cubic Hermite pieces
+// of h = 0.01 A over [1, 6] A, switch radii 5.0, 5.05, 5.35 on grid nodes, 1/|r|
+// by v_rsq_f32.  Beyond 6 A every function is the exponential tail of
+// potential.cpp, evaluated directly.
 #include <cmath>
 #include <cstdlib>
 #include <cstring>
@@ -42,7 +41,11 @@ constexpr double SQ6 = 2.449489742783178098;
 constexpr float SQ6F = 2.449489742783178098f;
 constexpr int GH3 = A2C_QUAD_GH3;
 constexpr float GHZF = 1.7320508075688772935f;  // Gauss-Hermite node sqrt(3)
-__device__ constexpr float ghwf(int a) { return a == 0 ? 2.0f / 3.0f : 1.0f / 6.0f; }
+// Gauss-Hermite weights times 6 per axis: 4, 1 and their products are exact in
+// FP32, where 2/3 and 1/6 are not and leave the sum of the 27 weights 1e-7 off
+// one (a bias of every density and pair energy); the receive passes divide by 216.
+__device__ constexpr float ghwf(int a) { return a == 0 ? 4.0f : 1.0f; }
+constexpr double GHQW = 1.0 / 216.0;
 enum { T_FPD = 0, T_FH = 1, T_PHPD = 2, T_PHPDH = 3, T_PHH = 4, NTAB = 5 };
 
 // Exponential tails beyond the switch radii: funRc * exp(k (r - rs)).
@@ -99,17 +102,6 @@ __device__ __forceinline__ float tab_v(const float4* __restrict__ tab, int w, fl
   if (!p.far) return cubic(tab[w * NT + p.k], p.u);
   return tail(w, r);
 }
-// The same without the branch: the row of the clamped interval, with far set
-// when r lies outside the table.  A per-point branch makes every point its own
-// basic block, so a wave waits out each point's LDS read before the next one
-// can issue; the pair passes evaluate all points of a pair this way and redo
-// the (rare) pair with a point outside [1, 6) A through the branching form.
-__device__ __forceinline__ float tab_vf(const float4* __restrict__ tab, int w, float r, bool& far) {
-  const Pos p = tab_pos(r);
-  far |= p.far;
-  return cubic(tab[w * NT + p.k], p.u);
-}
-
 // f_H(r) = 11.0025 exp(-1.30927 r) (potential.cpp:105-119; the exponential
 // tail past 5.35 A continues the same function to 1e-13), evaluated without a
 // table as 11.0025 * 2^(K r), K = -1.30927 log2(e) split into FP32 hi and lo
@@ -130,14 +122,6 @@ __device__ __forceinline__ float fH_exp(float r) {
   const float v = FH_C * __builtin_amdgcn_exp2f(e) * fmaf(el, LN2F, 1.0f);
   return r >= R0 ? v : __builtin_nanf("");
 }
-// density of a species at r: f_H directly, f_Pd from the value table in LDS
-// rows [0, NT) of the pair-owner density pass
-template <bool H, bool FAST>
-__device__ __forceinline__ float dens(const float4* __restrict__ tab, float r, bool& far) {
-  if (H) return fH_exp(r);
-  return FAST ? tab_vf(tab, T_FPD, r, far) : tab_v(tab, T_FPD, r);
-}
-
 struct Site {
   double q[3];
   double s;
@@ -146,18 +130,17 @@ __device__ __forceinline__ Site load_site(const double* __restrict__ X, int s) {
   const double4 v = *reinterpret_cast<const double4*>(X + 4 * (size_t)s);
   return {{v.x, v.y, v.z}, v.w};
 }
-__device__ __forceinline__ Site load_site(const A2C_GLOBAL double4* __restrict__ X, int s) {
-  const double4 v = X[s];
-  return {{v.x, v.y, v.z}, v.w};
+__device__ __forceinline__ Site load_row(const A2C_GLOBAL double2* __restrict__ qxy,
+                                         const A2C_GLOBAL double2* __restrict__ qzs, int p) {
+  const double2 a = qxy[p], b = qzs[p];
+  return {{a.x, a.y, b.x}, b.y};
 }
 // d = q_i - image(q_j) in FP64, rounded to FP32 (geometry held in registers)
 __device__ __forceinline__ void pair_vec32(const Image& g, const Site& a, const Site& b, float d[3]) {
+  double dd[3];
+  image_vec(g, a.q, b.q, dd);
 #pragma unroll
-  for (int c = 0; c < 3; ++c) {
-    double qj = b.q[c];
-    if (g.per[c]) qj = qj - g.box[c] * rint((qj - a.q[c]) * g.ibox[c]);
-    d[c] = (float)(a.q[c] - qj);
-  }
+  for (int c = 0; c < 3; ++c) d[c] = (float)dd[c];
 }
 // d = q_i - image(q_j) in FP64, rounded to FP32
 __device__ __forceinline__ void pair_vec32(const LatDev& S, const Site& a, const Site& b, float d[3]) {
@@ -256,9 +239,8 @@ __global__ __launch_bounds__(TB) void k_density32(const LatDev* __restrict__ lat
 // of the objective, dE/dr = F'_i f_j'(r) + F'_j f_i'(r) + phi'(r) (f_k: the
 // density function of site k's species).  One table position serves all
 // three functions.
-template <int KIND, bool FAST = false>
-__device__ __forceinline__ void point_coef(const float4* tab, float r, float Fi, float Fj, float& phi, float& cu,
-                                           bool& far) {
+template <int KIND>
+__device__ __forceinline__ void point_coef(const float4* tab, float r, float Fi, float Fj, float& phi, float& cu) {
   constexpr int WP = KIND == 0 ? G_PHPD : (KIND == 3 ? G_PHH : G_PHPDH);    // LDS table of phi
   constexpr int TP = KIND == 0 ? T_PHPD : (KIND == 3 ? T_PHH : T_PHPDH);    // its tail
   const Pos p = tab_pos(r);
@@ -275,9 +257,7 @@ __device__ __forceinline__ void point_coef(const float4* tab, float r, float Fi,
     const float Fh = KIND == 1 ? Fj : Fi;   // F' of the H site multiplies f_Pd'
     cu = fmaf(Fpd, hdfh, fmaf(Fh, quad(tab[G_FPD * NT + p.k], p.u), dphi));
   }
-  if (FAST) {
-    far |= p.far;
-  } else if (p.far) {
+  if (p.far) {
     phi = tail(TP, r);
     const float dp = TAIL[TP][1] * phi;
     float c;
@@ -317,8 +297,7 @@ __device__ __forceinline__ PairSums pair_grad(const float4* tab, const float d[3
       const float x = fmaxf(r2[q], 1e-12f);
       const float rinv = rsq(x);
       float phi, cc;
-      bool far = false;
-      point_coef<KIND>(tab, x * rinv, Fi, Fj, phi, cc, far);
+      point_coef<KIND>(tab, x * rinv, Fi, Fj, phi, cc);
       pe += phi;
       u[q] = cc * rinv;
     }
@@ -414,154 +393,330 @@ __global__ __launch_bounds__(TB) void k_grad32(const LatDev* __restrict__ lats, 
 // received slot; a gather kernel adds the received shares in FP64.  Each
 // buffer entry is written by exactly one lane, so results are deterministic.
 
-// 12-point sums of two densities at the same points: the density of the
-// neighbor's species (for this site) and of this site's species (for the
-// neighbor); one sum when the species are the same.  NB_H / ME_H: neighbor /
-// this site is an H site.  FAST: no per-point branch (see tab_vf).
-template <bool NB_H, bool ME_H, bool FAST>
-__device__ __forceinline__ void pair_density2(const float4* tab, const float d[3], float ai, float aj, float& sa,
-                                              float& sb, bool& far) {
-  const float D2 = d[0] * d[0] + d[1] * d[1] + d[2] * d[2];
-  const float bi = D2 + ai * ai, bj = D2 + aj * aj;
-  sa = 0.0f;
-  sb = 0.0f;
+// The owner passes read the EAM functions from cubic tables on a uniform
+// grid in s = |r|^2: a node's s is D2 + a^2 +- 2 a d_c (linear in what
+// differs between the nodes of a pair), so the table coordinate of a node is
+// one addition, and dE/ds = (dE/dr) / (2 |r|) is the factor every gradient term needs --
+// no square root and no division per node.  h = 0.5025 / 14 puts the switch
+// radii 5.0 and 5.05 A on grid nodes (25 and 25.5025 A^2; 5.35 A joins two
+// forms of the same function); SNT intervals from S0 reach past 36 A^2.
+// Rows: values (S_FPD, the density pass) and slopes (S_DFPD) interpolate at
+// the Chebyshev points; the pair functions (S_PH*) integrate the quadratic
+// interpolating their slope, so value and slope come from one row.
+// f_H = 11.0025 exp(-1.30927 |r|) is evaluated directly: |r| and the
+// exponential cost fewer clocks (8 for each transcendental) than one more
+// 16-byte row gathered from LDS (~12 clocks of the whole CU's LDS, which the
+// two other rows of a Pd-H node already keep busy).
+// Error against FP64 at 40^3 cells, tables in |r| (h = 0.01 A) and these: gradient
+// 6.8e-6 and 4.7e-7, objective 6.8e-9 and 7.8e-9 (12-point rule).
+constexpr double SH64 = 0.5025 / 14.0, S064 = 25.5025 - 683 * SH64;
+constexpr float SH = (float)SH64, S0 = (float)S064, SINV = (float)(1.0 / SH64), SB = (float)(-S064 / SH64);
+constexpr float SLO = 1.0f, SHI = 36.0f;  // nodes the tables serve: [1, 6) A
+constexpr int SNT = 977;
+enum { S_FPD = 0, S_DFPD = 1, S_PHPD = 2, S_PHPDH = 3, S_PHH = 4, NSTAB = 5 };  // S_DFPD.. are G_FPD.. of the gradient pass
+constexpr int S_BASE = NTAB * NT;  // first row of these tables after those in r
+static_assert(683 * SH64 < 24.515 && S064 < 1.0 && S064 + (SNT - 1) * SH64 > 36.0, "the grid covers [1, 36] A^2");
+
+// Table coordinates and displacement squares of one pair.  12-point rule: the
+// nodes of site i have s = bi +- 2 ai d_c, of site j bj -+ 2 aj d_c.
+// inside(): every node lies in [1, 6) A; the largest |2 a d_c| bounds them.
+struct Nodes12 {
+  float xi, xj, gi, gj, lo, hi;  // ti = gi d_c, tj = gj d_c
+  __device__ __forceinline__ Nodes12(const float d[3], float ai, float aj) {
+    const float D2 = d[0] * d[0] + d[1] * d[1] + d[2] * d[2];
+    const float bi = fmaf(ai, ai, D2), bj = fmaf(aj, aj, D2);
+    const float ei = 2.0f * ai, ej = 2.0f * aj;
+    const float m = fmaxf(fmaxf(fabsf(d[0]), fabsf(d[1])), fabsf(d[2]));
+    lo = fminf(fmaf(-fabsf(ei), m, bi), fmaf(-fabsf(ej), m, bj));
+    hi = fmaxf(fmaf(fabsf(ei), m, bi), fmaf(fabsf(ej), m, bj));
+    xi = fmaf(bi, SINV, SB);
+    xj = fmaf(bj, SINV, SB);
+    gi = ei * SINV;
+    gj = ej * SINV;
+  }
+};
+// Gauss-Hermite rule: s = D2 + 3 s^2 |a|^2 + 2 sqrt(3) s (a . d).
+struct Nodes27 {
+  float x0, n1, t[3], lo, hi;
+  __device__ __forceinline__ Nodes27(const float d[3], float sd) {
+    const float D2 = d[0] * d[0] + d[1] * d[1] + d[2] * d[2];
+    const float s3 = 3.0f * sd * sd, tt = 2.0f * GHZF * sd;
+    lo = hi = D2;
 #pragma unroll
-  for (int c = 0; c < 3; ++c) {
-    const float ti = 2.0f * ai * d[c], tj = 2.0f * aj * d[c];
-    const float r2[4] = {bi + ti, bi - ti, bj - tj, bj + tj};
+    for (int c = 0; c < 3; ++c) {
+      const float e = tt * fabsf(d[c]);
+      lo += fminf(s3 - e, 0.0f);
+      hi += s3 + e;
+      t[c] = tt * SINV * d[c];
+    }
+    x0 = fmaf(D2, SINV, SB);
+    n1 = s3 * SINV;
+  }
+};
+__device__ __forceinline__ bool inside(float lo, float hi) { return lo >= SLO && hi < SHI; }
+
+// The nodes of a pair one at a time, for the pairs with a node outside.
+// x(k): table coordinate of node k; w, off: its weight and displacement.
+template <int RULE>
+struct Edge {
+  static constexpr int N = RULE == GH3 ? 27 : 12;
+  float d[3], ai, aj, sd, off[3], w;
+  int end;  // 12-point rule: the site that moves (0: i, 1: j)
+  __device__ __forceinline__ Edge(const float* dd, float si, float sj)
+      : d{dd[0], dd[1], dd[2]}, ai(SQ6F * si), aj(SQ6F * sj), sd(sqrtf(si * si + sj * sj)), w(1.0f), end(0) {}
+  __device__ __forceinline__ float x(int k) {
+    if (RULE == GH3) {
+      const int a0 = k % 3 - 1, a1 = (k / 3) % 3 - 1, a2 = k / 9 - 1;
+      w = ghwf(a0) * ghwf(a1) * ghwf(a2);
+      off[0] = GHZF * sd * (float)a0;
+      off[1] = GHZF * sd * (float)a1;
+      off[2] = GHZF * sd * (float)a2;
+    } else {
+      end = k >= 6;
+      const float a = (k & 1 ? -1.0f : 1.0f) * (end ? aj : ai);
+      const int c = (k >> 1) % 3;
+      off[0] = c == 0 ? a : 0.0f;
+      off[1] = c == 1 ? a : 0.0f;
+      off[2] = c == 2 ? a : 0.0f;
+    }
+    float s = d[0] * d[0] + d[1] * d[1] + d[2] * d[2];
 #pragma unroll
-    for (int q = 0; q < 4; ++q) {
-      const float x = fmaxf(r2[q], 1e-12f);
-      const float r = x * rsq(x);
-      sa += dens<NB_H, FAST>(tab, r, far);
-      if (NB_H != ME_H) sb += dens<ME_H, FAST>(tab, r, far);
+    for (int c = 0; c < 3; ++c) s = fmaf(off[c], fmaf(2.0f, d[c], off[c]), s);
+    return fmaf(s, SINV, SB);
+  }
+};
+
+// f_H / 11.0025 at s, and 1/|r|: 2^(K r), K = -1.30927 log2(e) split into
+// FP32 hi and lo parts, with the rounding of K r carried into a first-order
+// correction (within about an ulp of FP32).  Callers scale their sums.
+__device__ __forceinline__ float fH_s(float s, float& rinv) {
+  rinv = rsq(s);
+  const float r = s * rinv;
+  const float e = FH_KHI * r;
+  const float el = fmaf(FH_KLO, r, fmaf(FH_KHI, r, -e));
+  return __builtin_amdgcn_exp2f(e) * fmaf(el, LN2F, 1.0f);
+}
+// Row position of table coordinate x: interval k and u in [0, 1).
+struct SPos {
+  int k;
+  float u;
+};
+__device__ __forceinline__ SPos s_pos(float x) { return {(int)x, __builtin_amdgcn_fractf(x)}; }
+// s of a table coordinate, and whether the tables serve it (a pair with a
+// node outside is evaluated node by node: the exponential tails from 6 A on,
+// NaN below 1 A -- no physical configuration comes that close, and the
+// non-finite objective makes the caller fall back to the FP64 path).
+__device__ __forceinline__ float s_of(float x) { return fmaf(x, SH, S0); }
+__device__ __forceinline__ bool s_in(float s) { return s >= SLO && s < SHI; }
+__device__ __forceinline__ float s_tail(int w, float s) { return tail(w, s * rsq(s)); }
+
+// Densities at one node: f_Pd (tab: its value rows) and f_H / 11.0025, as wanted.
+template <bool WANT_PD, bool WANT_H, bool IN>
+__device__ __forceinline__ void node_dens(const float4* tab, float x, float& fpd, float& fh) {
+  const float s = s_of(x);
+  const bool in = IN || s_in(s);
+  if (WANT_PD) {
+    if (in) {
+      const SPos p = s_pos(x);
+      fpd = cubic(tab[p.k], p.u);
+    } else {
+      fpd = s_tail(T_FPD, s);
     }
   }
-  if (NB_H == ME_H) sb = sa;
+  if (WANT_H) {
+    float ri;
+    fh = in || s >= SHI ? fH_s(s, ri) : __builtin_nanf("");
+  }
 }
 
-// Weighted Gauss-Hermite sums of the two densities at the 27 nodes of a pair
-// (s = sqrt(sigma_i^2 + sigma_j^2)): a rolled loop over the z offset a2, the
-// 9 nodes of each plane unrolled (a fully unrolled 27 spills at 64 VGPRs).
-template <bool NB_H, bool ME_H, bool FAST>
-__device__ __forceinline__ void pair_density2_gh(const float4* tab, const float d[3], float sd, float& sa,
-                                                 float& sb, bool& far) {
-  const float D2 = d[0] * d[0] + d[1] * d[1] + d[2] * d[2];
-  const float s3 = 3.0f * sd * sd, tt = 2.0f * GHZF * sd;
-  const float t0 = tt * d[0], t1 = tt * d[1], t2 = tt * d[2];
-  sa = 0.0f;
-  sb = 0.0f;
+// Sums over a pair's nodes of two densities: the density of the neighbor's
+// species (for this site) and of this site's species (for the neighbor); one
+// sum when the species are the same.  NB_H / ME_H: neighbor / this site is an
+// H site.  IN: every node is inside the tables.
+template <bool NB_H, bool ME_H, bool IN>
+__device__ __forceinline__ void pair_density2(const float4* tab, const Nodes12& q, const float d[3], float& sa, float& sb) {
+  constexpr bool WP = !NB_H || !ME_H, WH = NB_H || ME_H;
+  float sp = 0.0f, sh = 0.0f;
+#pragma unroll
+  for (int c = 0; c < 3; ++c) {
+    const float ti = q.gi * d[c], tj = q.gj * d[c];
+    const float x[4] = {q.xi + ti, q.xi - ti, q.xj - tj, q.xj + tj};
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      float fp = 0.0f, fh = 0.0f;
+      node_dens<WP, WH, IN>(tab, x[k], fp, fh);
+      if (WP) sp += fp;
+      if (WH) sh += fh;
+    }
+  }
+  sa = NB_H ? FH_C * sh : sp;
+  sb = ME_H ? FH_C * sh : sp;
+}
+// The Gauss-Hermite sums: a rolled loop over the z offset a2, the 9 nodes of
+// each plane unrolled (a fully unrolled 27 spills).
+template <bool NB_H, bool ME_H, bool IN>
+__device__ __forceinline__ void pair_density2_gh(const float4* tab, const Nodes27& q, float& sa, float& sb) {
+  constexpr bool WP = !NB_H || !ME_H, WH = NB_H || ME_H;
+  float sp = 0.0f, sh = 0.0f;
 #pragma unroll 1
   for (int a2 = -1; a2 <= 1; ++a2) {
-    const float base = D2 + s3 * (float)(a2 * a2) + (float)a2 * t2;
-    float pa = 0.0f, pb = 0.0f;
+    const float base = q.x0 + q.n1 * (float)(a2 * a2) + (float)a2 * q.t[2];
+    float pp = 0.0f, ph = 0.0f;
 #pragma unroll
     for (int a1 = -1; a1 <= 1; ++a1) {
 #pragma unroll
       for (int a0 = -1; a0 <= 1; ++a0) {
         const float w = ghwf(a0) * ghwf(a1);
-        const float x = fmaxf(base + s3 * (float)(a0 * a0 + a1 * a1) + (a0 * t0 + a1 * t1), 1e-12f);
-        const float r = x * rsq(x);
-        pa += w * dens<NB_H, FAST>(tab, r, far);
-        if (NB_H != ME_H) pb += w * dens<ME_H, FAST>(tab, r, far);
+        float fp = 0.0f, fh = 0.0f;
+        node_dens<WP, WH, IN>(tab, base + q.n1 * (float)(a0 * a0 + a1 * a1) + (a0 * q.t[0] + a1 * q.t[1]), fp, fh);
+        if (WP) pp += w * fp;
+        if (WH) ph += w * fh;
       }
     }
-    const float w2 = a2 ? 1.0f / 6.0f : 2.0f / 3.0f;
-    sa += w2 * pa;
-    sb += w2 * pb;
+    const float w2 = a2 ? 1.0f : 4.0f;
+    if (WP) sp += w2 * pp;
+    if (WH) sh += w2 * ph;
   }
-  if (NB_H == ME_H) sb = sa;
-}
-
-template <int RULE, bool NB_H, bool ME_H, bool FAST>
-__device__ __forceinline__ void pair_dens_rule(const float4* tab, const float d[3], float as, float bs, float& mine,
-                                               float& theirs, bool& far) {
-  if (RULE == GH3) pair_density2_gh<NB_H, ME_H, FAST>(tab, d, sqrtf(as * as + bs * bs), mine, theirs, far);
-  else pair_density2<NB_H, ME_H, FAST>(tab, d, SQ6F * as, SQ6F * bs, mine, theirs, far);
-}
-// all points without a branch; the pair again with the tails if a point fell
-// outside the table
-template <int RULE, bool NB_H, bool ME_H>
-__device__ __attribute__((noinline)) float2 pair_dens_tails(const float4* tab, float d0, float d1, float d2, float as,
-                                                            float bs) {
-  const float d[3] = {d0, d1, d2};
-  bool far = false;
-  float mine, theirs;
-  pair_dens_rule<RULE, NB_H, ME_H, false>(tab, d, as, bs, mine, theirs, far);
-  return make_float2(mine, theirs);
+  sa = NB_H ? FH_C * sh : sp;
+  sb = ME_H ? FH_C * sh : sp;
 }
 template <int RULE, bool NB_H, bool ME_H>
 __device__ __forceinline__ void pair_dens(const float4* tab, const float d[3], float as, float bs, float& mine,
                                           float& theirs) {
-  bool far = false;
-  pair_dens_rule<RULE, NB_H, ME_H, true>(tab, d, as, bs, mine, theirs, far);
-  if (far) {
-    const float2 v = pair_dens_tails<RULE, NB_H, ME_H>(tab, d[0], d[1], d[2], as, bs);
-    mine = v.x;
-    theirs = v.y;
+  bool in;
+  if (RULE == GH3) {
+    const Nodes27 q(d, sqrtf(as * as + bs * bs));
+    in = inside(q.lo, q.hi);
+    if (in) pair_density2_gh<NB_H, ME_H, true>(tab, q, mine, theirs);
+  } else {
+    const Nodes12 q(d, SQ6F * as, SQ6F * bs);
+    in = inside(q.lo, q.hi);
+    if (in) pair_density2<NB_H, ME_H, true>(tab, q, d, mine, theirs);
+  }
+  if (!in) {  // node by node, rolled (rare: a call would cost every pair the registers it keeps across it)
+    constexpr bool WP = !NB_H || !ME_H, WH = NB_H || ME_H;
+    Edge<RULE> q(d, as, bs);
+    float sp = 0.0f, sh = 0.0f;
+#pragma unroll 1
+    for (int k = 0; k < Edge<RULE>::N; ++k) {
+      float fp = 0.0f, fh = 0.0f;
+      node_dens<WP, WH, false>(tab, q.x(k), fp, fh);
+      sp += q.w * fp;
+      sh += q.w * fh;
+    }
+    mine = NB_H ? FH_C * sh : sp;
+    theirs = ME_H ? FH_C * sh : sp;
   }
 }
 
-// Partner list of each list: PdPd<->PdPd, PdH<->HPd, HH<->HH.
-__device__ __forceinline__ const Ell& partner_of(const LatDev& S, int list) {
-  return list == 0 ? S.pdpd : (list == 1 ? S.hpd : (list == 2 ? S.pdh : S.hh));
+// Owned pairs of one list of one row, K lanes per row.  Software pipeline: at
+// a pair's turn the state of the next one and the index and slot of the one
+// after it are requested, then the pair is evaluated and its share stored.
+// Loads and stores complete in order on one counter, so a load requested
+// after a store cannot be waited for without waiting for the store to reach
+// memory; requested one pair earlier, every load is older than the stores
+// still in flight.  (Requested in the pair's own turn, the waits for the
+// stores added 100 us to k_grad_own at 40^3 cells.)  geom(b) returns the pair's
+// geometry; eval(geometry, F'_j, w_j, neighbor row, received slot) the rest;
+// w_j: the occupancy of an H neighbor.
+template <bool NB_H, bool WITH_F, class Geom, class Eval>
+__device__ __forceinline__ void owned_pairs(const Ell& L, const OwnerLane& ln, int K, int off,
+                                            const A2C_GLOBAL double2* qxy, const A2C_GLOBAL double2* qzs,
+                                            const A2C_GLOBAL float2* aux, const A2C_GLOBAL double* w, Geom geom,
+                                            Eval eval) {
+  const size_t rows = L.rows, first = (size_t)ln.ph * rows + ln.row, step = (size_t)K * rows;
+  const A2C_GLOBAL int32_t* __restrict__ oj = gmem((const int32_t*)L.oj) + first;
+  const A2C_GLOBAL int32_t* __restrict__ orv = gmem((const int32_t*)L.orv) + first;
+  qxy += off;
+  qzs += off;
+  aux += off;
+  const int n = gmem((const int32_t*)L.ocnt)[ln.row];
+  int t = ln.ph;
+  if (t >= n) return;
+  size_t e = t + K < n ? step : 0;  // past the row's end its last entry is requested again: no branch around
+                                    // a load, or the waits behind it cover everything outstanding
+  int j1 = oj[0], r1 = orv[0], j2 = oj[e], r2 = orv[e];
+  Site b = load_row(qxy, qzs, j1);
+  float F = WITH_F ? aux[j1].x : 0.0f;
+  double wj = NB_H ? w[j1] : 1.0;
+  __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0): the loop's own waits then count only what the loop requests
+  do {
+    const auto g = geom(b);
+    const int jc = j1, rc = r1;
+    const float Fc = F;
+    const double wc = wj;
+    j1 = j2;
+    r1 = r2;
+    b = load_row(qxy, qzs, j1);
+    if (WITH_F) F = aux[j1].x;
+    if (NB_H) wj = w[j1];
+    e += t + 2 * K < n ? step : 0;
+    j2 = oj[e];
+    r2 = orv[e];
+    eval(g, Fc, wc, jc, rc);
+    t += K;
+  } while (t < n);
+}
+struct Pair32 {
+  float d[3], bs;
+};
+
+template <int RULE, bool NB_H, bool ME_H>
+__device__ __forceinline__ void dens_list(const float4* tab, const LatDev& S, const OwnerLane& ln, const Site& a,
+                                          const Image& img, double wme, double& rho) {
+  const Ell& L = ME_H ? (NB_H ? S.hh : S.hpd) : (NB_H ? S.pdh : S.pdpd);
+  const Ell& P = ME_H ? (NB_H ? S.hh : S.pdh) : (NB_H ? S.hpd : S.pdpd);  // partner rows
+  A2C_GLOBAL float* __restrict__ prb = gmem(reinterpret_cast<float*>(P.rbuf));
+  const size_t prows = P.rows;
+  const float as = (float)a.s;
+  owned_pairs<NB_H, false>(
+      L, ln, S.kl32, NB_H ? S.npd : 0, gmem((const double2*)S.qxy), gmem((const double2*)S.qzs),
+      gmem((const float2*)S.aux), gmem((const double*)S.xrow),
+      [&](const Site& b) {
+        Pair32 p;
+        pair_vec32(img, a, b, p.d);
+        p.bs = (float)b.s;
+        return p;
+      },
+      [&](const Pair32& p, float, double wj, int jl, int rv) {
+        float mine, theirs;  // neighbor-species density (for me), my-species density (for the neighbor)
+        pair_dens<RULE, NB_H, ME_H>(tab, p.d, as, p.bs, mine, theirs);
+        rho += wj * (double)mine;
+        // shares leave weighted by the sender's occupancy
+        prb[(size_t)rv * prows + jl] = ME_H ? (float)(wme * (double)theirs) : theirs;
+      });
 }
 
-// At least 6 waves per SIMD (at most 80 VGPRs): the 12-point pass takes 71
-// without spills (7 waves), the Gauss-Hermite planes 80
+// Bound by the vector ALUs and, as much, by the gathers' path through L1 (40^3
+// cells: 70% and 88% of the time busy).  6 waves per SIMD: 80 VGPRs hold both
+// rules' node blocks without spills.  40^3 cells, 12-point / Gauss-Hermite rule:
+// 214 / 340 us with tables in |r|, sites in lattice order and the loads of a
+// pair in its own turn, 147 / 255 us as it is.
 template <int RULE>
 __global__ __launch_bounds__(TB) __attribute__((amdgpu_waves_per_eu(6))) void k_dens_own(
     const LatDev* __restrict__ lats, const int32_t* __restrict__ ob2l, const float4* __restrict__ gtab) {
-  __shared__ float4 tab[NT];  // f_Pd (f_H is evaluated directly)
+  __shared__ float4 tab[SNT];  // f_Pd (f_H is evaluated directly)
   const int w = xcd_block();
   const LatDev& S = lats[ob2l[w]];
   if (S.rule != RULE) return;  // whole workgroup: the other rule's instance serves this lattice
-  stage_tables(tab, gtab, NT);
-  const int K = S.kl32;  // lanes per site: lane ph takes owned slots ph, ph + K, ...
-  const int s = (w - S.owg0_32) * (TB / K) + (int)threadIdx.x / K;
-  const int ph = (int)threadIdx.x % K;
-  const int npd = S.npd;
-  const int N = npd + S.nh;
-  if (s >= N) return;  // whole lane groups
-  // everything the pair loops use, out of the descriptor and into registers
-  const A2C_GLOBAL double4* __restrict__ X = gmem(reinterpret_cast<const double4*>(S.X));
-  const A2C_GLOBAL double* __restrict__ xo = gmem(S.x);
+  stage_tables(tab, gtab + S_BASE + S_FPD * SNT, SNT);
+  const int K = S.kl32;
+  const OwnerLane ln(S, w - S.owg0_32, K);
+  if (ln.row >= ln.rows) return;  // whole lane groups
   const Image img = image_of(S);
-  const bool pd = s < npd;
-  const int row = pd ? s : s - npd;
-  const Site a = load_site(X, s);
-  const double wme = pd ? 1.0 : xo[row];  // shares leave weighted by the sender's occupancy
+  const int s = ln.pd ? ln.row : S.npd + ln.row;
+  const Site a = load_row(gmem((const double2*)S.qxy), gmem((const double2*)S.qzs), s);
   double rho = 0.0;
-#pragma unroll
-  for (int side = 0; side < 2; ++side) {  // Pd neighbors, then H neighbors
-    const int list = pd ? side : 2 + side;
-    const Ell& L = list == 0 ? S.pdpd : (list == 1 ? S.pdh : (list == 2 ? S.hpd : S.hh));
-    const Ell& P = partner_of(S, list);
-    const A2C_GLOBAL int32_t* __restrict__ oj = gmem(L.oj);
-    const A2C_GLOBAL int32_t* __restrict__ orv = gmem(L.orv);
-    A2C_GLOBAL float* __restrict__ prb = gmem(reinterpret_cast<float*>(P.rbuf));
-    const size_t rows = L.rows, prows = P.rows;
-    const int n = gmem(L.ocnt)[row];
-    for (int t = ph; t < n; t += K) {
-      const size_t e = (size_t)t * rows + row;
-      const int jl = oj[e];
-      const int rv = orv[e];
-      const Site b = load_site(X, side == 0 ? jl : npd + jl);
-      const double wj = side == 0 ? 1.0 : xo[jl];
-      float d[3];
-      pair_vec32(img, a, b, d);
-      float mine, theirs;  // neighbor-type density (for me), my-type density (for the neighbor)
-      const float as = (float)a.s, bs = (float)b.s;
-      if (list == 0) pair_dens<RULE, false, false>(tab, d, as, bs, mine, theirs);
-      else if (list == 1) pair_dens<RULE, true, false>(tab, d, as, bs, mine, theirs);
-      else if (list == 2) pair_dens<RULE, false, true>(tab, d, as, bs, mine, theirs);
-      else pair_dens<RULE, true, true>(tab, d, as, bs, mine, theirs);
-      rho += wj * (double)mine;
-      if (rv >= 0) prb[(size_t)rv * prows + jl] = (float)(wme * (double)theirs);
-    }
+  if (ln.pd) {
+    dens_list<RULE, false, false>(tab, S, ln, a, img, 1.0, rho);
+    dens_list<RULE, true, false>(tab, S, ln, a, img, 1.0, rho);
+  } else {
+    const double wme = gmem((const double*)S.xrow)[ln.row];
+    dens_list<RULE, false, true>(tab, S, ln, a, img, wme, rho);
+    dens_list<RULE, true, true>(tab, S, ln, a, img, wme, rho);
   }
   rho = site_sum(rho, K);
-  if (ph == 0) gmem(S.rho)[s] = rho;
+  if (ln.ph == 0) gmem(S.rho)[s] = rho;
 }
 
 __global__ __launch_bounds__(TB) void k_dens_recv(const LatDev* __restrict__ lats, const int32_t* __restrict__ b2l) {
@@ -570,7 +725,7 @@ __global__ __launch_bounds__(TB) void k_dens_recv(const LatDev* __restrict__ lat
   const int s = (blk - S.blk0) * TB + threadIdx.x;
   const int N = S.npd + S.nh;
   if (s >= N) return;
-  const double* __restrict__ xo = S.x;
+  const double* __restrict__ xo = S.xrow;
   const bool pd = s < S.npd;
   const int row = pd ? s : s - S.npd;
   double rho = S.rho[s];
@@ -582,7 +737,7 @@ __global__ __launch_bounds__(TB) void k_dens_recv(const LatDev* __restrict__ lat
     // shares arrive weighted by their senders
     for_row_shares<RECV_RU_SCALAR>(gmem(reinterpret_cast<const float*>(L.rbuf)), L.rows, row, n, [&](float v) { rho += (double)v; });
   }
-  rho *= S.rule == GH3 ? 1.0 : QW;
+  rho *= S.rule == GH3 ? GHQW : QW;
   S.rho[s] = rho;
   const double xs = pd ? 1.0 : xo[row];
   const eam::VD F = pd ? eam::F_Pd_vd(rho) : eam::F_H_vd(rho);
@@ -597,118 +752,100 @@ struct PairSums2 {
   float gsj;   // partner sigma term
 };
 
-template <int KIND, bool FAST>
-__device__ __forceinline__ PairSums2 pair_grad2(const float4* tab, const float d[3], float ai, float aj, float Fi,
-                                                float Fj, bool& far) {
-  const float D2 = d[0] * d[0] + d[1] * d[1] + d[2] * d[2];
-  const float bi = D2 + ai * ai, bj = D2 + aj * aj;
-  float su = 0.0f, ui = 0.0f, uj = 0.0f, pe = 0.0f, ti[3], tj[3];
-#pragma unroll
-  for (int c = 0; c < 3; ++c) {
-    const float t1 = 2.0f * ai * d[c], t2 = 2.0f * aj * d[c];
-    const float r2[4] = {bi + t1, bi - t1, bj - t2, bj + t2};
-    float u[4];
-#pragma unroll
-    for (int q = 0; q < 4; ++q) {
-      const float x = fmaxf(r2[q], 1e-12f);
-      const float rinv = rsq(x);
-      float phi, cc;
-      point_coef<KIND, FAST>(tab, x * rinv, Fi, Fj, phi, cc, far);
-      pe += phi;
-      u[q] = cc * rinv;
+// One node: the pair energy phi and cu = SH dE/ds, E = F'_i f_j + F'_j f_i + phi
+// (f_k: the density function of site k's species; KIND as in point_coef).
+// FP multiplies f_Pd', FH f_H' / |r| (it carries FH_D).  tab: LDS rows of the
+// gradient pass (G_*).
+constexpr float FH_D = (float)(0.5 * SH64 * FH_K * 11.0025);
+template <int KIND, bool IN>
+__device__ __forceinline__ void node_coef(const float4* tab, float x, float FP, float FH, float& phi, float& cu) {
+  constexpr int WP = KIND == 0 ? G_PHPD : (KIND == 3 ? G_PHH : G_PHPDH);
+  constexpr int TP = KIND == 0 ? T_PHPD : (KIND == 3 ? T_PHH : T_PHPDH);
+  const float s = s_of(x);
+  if (IN || s_in(s)) {
+    const SPos p = s_pos(x);
+    float dphi;
+    cubic_vd(tab[WP * SNT + p.k], p.u, phi, dphi);
+    cu = dphi;
+    if (KIND != 3) cu = fmaf(FP, quad(tab[G_FPD * SNT + p.k], p.u), cu);
+    if (KIND != 0) {
+      float ri;
+      const float fh = fH_s(s, ri);
+      cu = fmaf(FH, fh * ri, cu);
     }
-    ti[c] = u[0] - u[1];
-    tj[c] = u[2] - u[3];
-    ui += u[0] + u[1];
-    uj += u[2] + u[3];
+  } else {
+    const float ri = rsq(s);
+    phi = s_tail(TP, s);
+    float c = TAIL[TP][1] * phi;
+    if (KIND != 3) c = fmaf(FP, TAIL[T_FPD][1] * s_tail(T_FPD, s), c);
+    cu = 0.5f * SH * c * ri;
+    if (KIND != 0) {
+      float r2;
+      cu = fmaf(FH, s >= SHI ? fH_s(s, r2) * ri : __builtin_nanf(""), cu);
+    }
   }
-  su = ui + uj;
-  PairSums2 p;
-  p.pe = pe;
-#pragma unroll
-  for (int c = 0; c < 3; ++c) p.g[c] = INVH * fmaf(d[c], su, ai * ti[c] - aj * tj[c]);
-  p.gsi = INVH * fmaf(d[0], ti[0], fmaf(d[1], ti[1], fmaf(d[2], ti[2], ai * ui)));
-  p.gsj = INVH * fmaf(aj, uj, -fmaf(d[0], tj[0], fmaf(d[1], tj[1], d[2] * tj[2])));
-  return p;
 }
 
-// pair_grad2 for the points inside the table, with the table rows of one
-// axis's four points read before any of them is used (their LDS latencies
-// overlap); far is set when a point lies outside [1, 6) A.
-template <int KIND>
-__device__ __forceinline__ PairSums2 pair_grad2_rows(const float4* tab, const float d[3], float ai, float aj,
-                                                     float Fi, float Fj, bool& far) {
-  constexpr int WP = KIND == 0 ? G_PHPD : (KIND == 3 ? G_PHH : G_PHPDH);
-  constexpr bool NEED_F = KIND != 3;  // f_Pd' row
-  const float D2 = d[0] * d[0] + d[1] * d[1] + d[2] * d[2];
-  const float bi = D2 + ai * ai, bj = D2 + aj * aj;
-  float ui = 0.0f, uj = 0.0f, pe = 0.0f, ti[3], tj[3];
-#pragma unroll
-  for (int c = 0; c < 3; ++c) {
-    const float t1 = 2.0f * ai * d[c], t2 = 2.0f * aj * d[c];
-    const float r2[4] = {bi + t1, bi - t1, bj - t2, bj + t2};
-    float rinv[4], r[4], u[4];
-    Pos p[4];
-    float4 rp[4], rf[4];
-#pragma unroll
-    for (int q = 0; q < 4; ++q) {
-      const float x = fmaxf(r2[q], 1e-12f);
-      rinv[q] = rsq(x);
-      r[q] = x * rinv[q];
-      p[q] = tab_pos(r[q]);
-      far |= p[q].far;
-      rp[q] = tab[WP * NT + p[q].k];
-      if (NEED_F) rf[q] = tab[G_FPD * NT + p[q].k];
+// 12-point sums.  Site e's points are r = d +- a e_c with a = ai for the
+// site and -aj for its partner.  With u = 2 SINV cu = (dE/dr) / |r| per node,
+// T_c the difference of u between the two points of an axis, U_e their sum:
+//   q-gradient  sum u r = d (U_i + U_j) + sum_e a T,
+//   sigma terms d . T + a U (site i), its negative (partner).
+// One axis of one site (2 nodes) per trip, the components rotating through
+// d0 and h2: unrolled, the table rows of all nodes are in flight and their
+// registers leave 4 waves per SIMD.
+template <int KIND, bool IN>
+__device__ __forceinline__ PairSums2 pair_grad2(const float4* tab, const Nodes12& n, const float d[3], float ai,
+                                                float aj, float FP, float FH) {
+  float pe = 0.0f, su = 0.0f, d0 = d[0], d1 = d[1], d2 = d[2], h0 = 0.0f, h1 = 0.0f, h2 = 0.0f;
+  float a = ai, xb = n.xi, g = n.gi;
+  PairSums2 p;
+#pragma unroll 1
+  for (int e = 0; e < 2; ++e) {
+    float ue = 0.0f, se = 0.0f;
+#pragma unroll 1
+    for (int c = 0; c < 3; ++c) {
+      const float t = g * d0;
+      float phi0, phi1, u0, u1;
+      node_coef<KIND, IN>(tab, xb + t, FP, FH, phi0, u0);
+      node_coef<KIND, IN>(tab, xb - t, FP, FH, phi1, u1);
+      pe += phi0 + phi1;
+      const float T = u0 - u1;
+      ue += u0 + u1;
+      se = fmaf(d0, T, se);
+      const float h = fmaf(a, T, h0), dt = d0;
+      h0 = h1;
+      h1 = h2;
+      h2 = h;
+      d0 = d1;
+      d1 = d2;
+      d2 = dt;
     }
-#pragma unroll
-    for (int q = 0; q < 4; ++q) {
-      float phi, dphi, cu;
-      cubic_vd(rp[q], p[q].u, phi, dphi);
-      if (KIND == 0) {
-        cu = fmaf(Fi + Fj, quad(rf[q], p[q].u), dphi);
-      } else {
-        const float hdfh = (FH_KF / INVH) * fH_exp(r[q]);
-        if (KIND == 3) {
-          cu = fmaf(Fi + Fj, hdfh, dphi);
-        } else {
-          const float Fpd = KIND == 1 ? Fi : Fj;
-          const float Fh = KIND == 1 ? Fj : Fi;
-          cu = fmaf(Fpd, hdfh, fmaf(Fh, quad(rf[q], p[q].u), dphi));
-        }
-      }
-      pe += phi;
-      u[q] = cu * rinv[q];
-    }
-    ti[c] = u[0] - u[1];
-    tj[c] = u[2] - u[3];
-    ui += u[0] + u[1];
-    uj += u[2] + u[3];
+    su += ue;
+    p.gsj = -(2.0f * SINV) * fmaf(a, ue, se);
+    if (e == 0) p.gsi = -p.gsj;
+    a = -aj;
+    xb = n.xj;
+    g = -n.gj;
   }
-  const float su = ui + uj;
-  PairSums2 pr;
-  pr.pe = pe;
-#pragma unroll
-  for (int c = 0; c < 3; ++c) pr.g[c] = INVH * fmaf(d[c], su, ai * ti[c] - aj * tj[c]);
-  pr.gsi = INVH * fmaf(d[0], ti[0], fmaf(d[1], ti[1], fmaf(d[2], ti[2], ai * ui)));
-  pr.gsj = INVH * fmaf(aj, uj, -fmaf(d[0], tj[0], fmaf(d[1], tj[1], d[2] * tj[2])));
-  return pr;
+  p.pe = pe;
+  p.g[0] = (2.0f * SINV) * fmaf(d[0], su, h0);
+  p.g[1] = (2.0f * SINV) * fmaf(d[1], su, h1);
+  p.g[2] = (2.0f * SINV) * fmaf(d[2], su, h2);
+  return p;
 }
 
 // Gauss-Hermite pair sums.  With u_k = w_k (c/|r_k|) and the node offsets
 // a_k, n_k = |a_k|^2:  U = sum u, Va = sum u a, Wn = sum u n;
 //   q-gradient  sum u r = d U + sqrt(3) s Va,
 //   Sz = sum u (r . z) = sqrt(3) d . Va + 3 s Wn,  d/dsigma_k = Sz sigma_k / s.
-template <int KIND, bool FAST>
-__device__ __forceinline__ PairSums2 pair_grad2_gh(const float4* tab, const float d[3], float si, float sj, float Fi,
-                                                   float Fj, bool& far) {
-  const float sd = sqrtf(si * si + sj * sj);
-  const float D2 = d[0] * d[0] + d[1] * d[1] + d[2] * d[2];
-  const float s3 = 3.0f * sd * sd, tt = 2.0f * GHZF * sd;
-  const float t0 = tt * d[0], t1 = tt * d[1], t2 = tt * d[2];
+template <int KIND, bool IN>
+__device__ __forceinline__ PairSums2 pair_grad2_gh(const float4* tab, const Nodes27& q, const float d[3], float sd,
+                                                   float si, float sj, float FP, float FH) {
   float pe = 0.0f, U = 0.0f, V0 = 0.0f, V1 = 0.0f, V2 = 0.0f, Wn = 0.0f;
 #pragma unroll 1  // one z plane (9 nodes, unrolled) per trip, as in pair_density2_gh
   for (int a2 = -1; a2 <= 1; ++a2) {
-    const float base = D2 + s3 * (float)(a2 * a2) + (float)a2 * t2;
+    const float base = q.x0 + q.n1 * (float)(a2 * a2) + (float)a2 * q.t[2];
     float p9 = 0.0f, u9 = 0.0f, v0 = 0.0f, v1 = 0.0f, n9 = 0.0f;
 #pragma unroll
     for (int a1 = -1; a1 <= 1; ++a1) {
@@ -716,19 +853,17 @@ __device__ __forceinline__ PairSums2 pair_grad2_gh(const float4* tab, const floa
       for (int a0 = -1; a0 <= 1; ++a0) {
         const int n = a0 * a0 + a1 * a1;
         const float w = ghwf(a0) * ghwf(a1);
-        const float x = fmaxf(base + s3 * (float)n + (a0 * t0 + a1 * t1), 1e-12f);
-        const float rinv = rsq(x);
         float phi, cc;
-        point_coef<KIND, FAST>(tab, x * rinv, Fi, Fj, phi, cc, far);
+        node_coef<KIND, IN>(tab, base + q.n1 * (float)n + (a0 * q.t[0] + a1 * q.t[1]), FP, FH, phi, cc);
         p9 += w * phi;
-        const float u = w * cc * rinv;
+        const float u = w * cc;
         u9 += u;
         if (a0) v0 += a0 * u;
         if (a1) v1 += a1 * u;
         if (n) n9 += n * u;
       }
     }
-    const float w2 = a2 ? 1.0f / 6.0f : 2.0f / 3.0f;
+    const float w2 = a2 ? 1.0f : 4.0f;
     pe += w2 * p9;
     U += w2 * u9;
     V0 += w2 * v0;
@@ -739,121 +874,138 @@ __device__ __forceinline__ PairSums2 pair_grad2_gh(const float4* tab, const floa
   PairSums2 p;
   p.pe = pe;
   const float sv = GHZF * sd;
-  p.g[0] = INVH * fmaf(d[0], U, sv * V0);
-  p.g[1] = INVH * fmaf(d[1], U, sv * V1);
-  p.g[2] = INVH * fmaf(d[2], U, sv * V2);
-  const float sz = INVH * fmaf(GHZF, fmaf(d[0], V0, fmaf(d[1], V1, d[2] * V2)), 3.0f * sd * Wn);
+  p.g[0] = (2.0f * SINV) * fmaf(d[0], U, sv * V0);
+  p.g[1] = (2.0f * SINV) * fmaf(d[1], U, sv * V1);
+  p.g[2] = (2.0f * SINV) * fmaf(d[2], U, sv * V2);
+  const float sz = (2.0f * SINV) * fmaf(GHZF, fmaf(d[0], V0, fmaf(d[1], V1, d[2] * V2)), 3.0f * sd * Wn);
   p.gsi = sz * (si / sd);
   p.gsj = sz * (sj / sd);
   return p;
 }
 
-// all points without a branch; the pair again with the tails if a point fell
-// outside the table
-template <int RULE, int KIND>
-__device__ __attribute__((noinline)) PairSums2 pair_grad_tails(const float4* tab, float d0, float d1, float d2,
-                                                               float as, float bs, float Fi, float Fj) {
-  const float d[3] = {d0, d1, d2};
-  bool far = false;
-  return RULE == GH3 ? pair_grad2_gh<KIND, false>(tab, d, as, bs, Fi, Fj, far)
-                     : pair_grad2<KIND, false>(tab, d, SQ6F * as, SQ6F * bs, Fi, Fj, far);
-}
 template <int RULE, int KIND>
 __device__ __forceinline__ PairSums2 pair_grad(const float4* tab, const float d[3], float as, float bs, float Fi,
                                                float Fj) {
-  bool far = false;
-  PairSums2 p = RULE == GH3 ? pair_grad2_gh<KIND, true>(tab, d, as, bs, Fi, Fj, far)
-                            : pair_grad2_rows<KIND>(tab, d, SQ6F * as, SQ6F * bs, Fi, Fj, far);
-  if (far) p = pair_grad_tails<RULE, KIND>(tab, d[0], d[1], d[2], as, bs, Fi, Fj);
+  const float FP = KIND == 0 ? Fi + Fj : (KIND == 1 ? Fj : Fi);           // F' of the H site multiplies f_Pd'
+  const float FH = FH_D * (KIND == 3 ? Fi + Fj : (KIND == 1 ? Fi : Fj));  // F' of the Pd site f_H'
+  PairSums2 p;
+  bool in;
+  if (RULE == GH3) {
+    const float sd = sqrtf(as * as + bs * bs);
+    const Nodes27 n(d, sd);
+    in = inside(n.lo, n.hi);
+    if (in) p = pair_grad2_gh<KIND, true>(tab, n, d, sd, as, bs, FP, FH);
+  } else {
+    const float ai = SQ6F * as, aj = SQ6F * bs;
+    const Nodes12 n(d, ai, aj);
+    in = inside(n.lo, n.hi);
+    if (in) p = pair_grad2<KIND, true>(tab, n, d, ai, aj, FP, FH);
+  }
+  if (!in) {  // node by node, rolled, as in pair_dens
+    Edge<RULE> q(d, as, bs);
+    p = PairSums2{};
+    float sz = 0.0f;
+#pragma unroll 1
+    for (int k = 0; k < Edge<RULE>::N; ++k) {
+      float phi, u;
+      node_coef<KIND, false>(tab, q.x(k), FP, FH, phi, u);
+      p.pe = fmaf(q.w, phi, p.pe);
+      u *= 2.0f * SINV * q.w;
+      float ro = 0.0f;  // r . off
+#pragma unroll
+      for (int c = 0; c < 3; ++c) {
+        const float r = d[c] + q.off[c];
+        p.g[c] = fmaf(u, r, p.g[c]);
+        ro = fmaf(r, q.off[c], ro);
+      }
+      if (RULE == GH3) sz = fmaf(u, ro, sz);
+      else if (q.end) p.gsj = fmaf(u, ro / q.aj, p.gsj);
+      else p.gsi = fmaf(u, ro / q.ai, p.gsi);
+    }
+    if (RULE == GH3) {  // off = s z: d/dsigma_k = (sum u r . z) sigma_k / s
+      p.gsi = sz * as / (q.sd * q.sd);
+      p.gsj = sz * bs / (q.sd * q.sd);
+    }
+  }
   return p;
 }
 
-template <int RULE>
-__global__ __launch_bounds__(TB) void k_grad_own(const LatDev* __restrict__ lats, const int32_t* __restrict__ ob2l,
-                                                 const float4* __restrict__ gtab) {
-  __shared__ float4 tab[NGTAB * NT];
-  const int w = xcd_block();
-  const LatDev& S = lats[ob2l[w]];
-  if (S.rule != RULE) return;  // whole workgroup: the other rule's instance serves this lattice
-  stage_grad_tables(tab, gtab);
-  const int K = S.kl32;  // lanes per site: lane ph takes owned slots ph, ph + K, ...
-  const int s = (w - S.owg0_32) * (TB / K) + (int)threadIdx.x / K;
-  const int ph = (int)threadIdx.x % K;
-  const int npd = S.npd;
-  const int N = npd + S.nh;
-  if (s >= N) return;  // whole lane groups
-  // everything the pair loops use, out of the descriptor and into registers
-  const A2C_GLOBAL double4* __restrict__ X = gmem(reinterpret_cast<const double4*>(S.X));
-  const A2C_GLOBAL double* __restrict__ xo = gmem(S.x);
-  const A2C_GLOBAL float2* __restrict__ aux = gmem(S.aux);
-  const Image img = image_of(S);
-  const bool pd = s < npd;
-  const int row = pd ? s : s - npd;
-  const Site a = load_site(X, s);
-  const float Fi = aux[s].x;
-  const double wme = pd ? 1.0 : xo[row];  // shares leave weighted by the sender's occupancy
+// Sums of one row's owned pairs.
+struct Own {
   double e = 0.0, g0 = 0.0, g1 = 0.0, g2 = 0.0, gs = 0.0;
-#pragma unroll
-  for (int side = 0; side < 2; ++side) {
-    const int list = pd ? side : 2 + side;
-    const Ell& L = list == 0 ? S.pdpd : (list == 1 ? S.pdh : (list == 2 ? S.hpd : S.hh));
-    const Ell& P = partner_of(S, list);
-    const A2C_GLOBAL int32_t* __restrict__ oj = gmem(L.oj);
-    const A2C_GLOBAL int32_t* __restrict__ orv = gmem(L.orv);
-    A2C_GLOBAL float4* __restrict__ prb = gmem(reinterpret_cast<float4*>(P.rbuf));
-    const size_t rows = L.rows, prows = P.rows;
-    const int n = gmem(L.ocnt)[row];
-    const int off = side == 0 ? 0 : npd;  // site index of neighbor 0 of this list
-    // the next pair's neighbor, slot, state, F' and weight (loaded one pair ahead)
-    int jl_n = 0, rv_n = -1;
-    Site b_n{};
-    float Fj_n = 0.0f;
-    double w_n = 1.0;
-    if (ph < n) {
-      const size_t e0 = (size_t)ph * rows + row;
-      jl_n = oj[e0];
-      rv_n = orv[e0];
-      b_n = load_site(X, off + jl_n);
-      Fj_n = aux[off + jl_n].x;
-      if (side) w_n = xo[jl_n];
-    }
-    for (int t = ph; t < n; t += K) {
-      const int jl = jl_n, rv = rv_n;
-      const Site b = b_n;
-      const float Fj = Fj_n;
-      const double wj = w_n;
-      if (t + K < n) {  // the next pair's gathers overlap this pair's points
-        const size_t en = (size_t)(t + K) * rows + row;
-        jl_n = oj[en];
-        rv_n = orv[en];
-        b_n = load_site(X, off + jl_n);
-        Fj_n = aux[off + jl_n].x;
-        if (side) w_n = xo[jl_n];
-      }
-      float d[3];
-      pair_vec32(img, a, b, d);
-      const float as = (float)a.s, bs = (float)b.s;
-      PairSums2 p;
-      if (list == 0) p = pair_grad<RULE, 0>(tab, d, as, bs, Fi, Fj);
-      else if (list == 1) p = pair_grad<RULE, 1>(tab, d, as, bs, Fi, Fj);
-      else if (list == 2) p = pair_grad<RULE, 2>(tab, d, as, bs, Fi, Fj);
-      else p = pair_grad<RULE, 3>(tab, d, as, bs, Fi, Fj);
-      e += wj * p.pe;
-      g0 += wj * p.g[0]; g1 += wj * p.g[1]; g2 += wj * p.g[2];
-      gs += wj * p.gsi;
-      if (rv >= 0)
-        prb[(size_t)rv * prows + jl] =
-            make_float4((float)(-wme * p.g[0]), (float)(-wme * p.g[1]), (float)(-wme * p.g[2]), (float)(wme * p.gsj));
-    }
+};
+template <int RULE, int KIND>
+__device__ __forceinline__ void grad_list(const float4* tab, const LatDev& S, const OwnerLane& ln, const Site& a,
+                                          float Fi, const Image& img, double wme, Own& o) {
+  constexpr bool ME_H = KIND >= 2, NB_H = KIND & 1;
+  const Ell& L = ME_H ? (NB_H ? S.hh : S.hpd) : (NB_H ? S.pdh : S.pdpd);
+  const Ell& P = ME_H ? (NB_H ? S.hh : S.pdh) : (NB_H ? S.hpd : S.pdpd);  // partner rows
+  A2C_GLOBAL float4* __restrict__ prb = gmem(reinterpret_cast<float4*>(P.rbuf));
+  const size_t prows = P.rows;
+  const float as = (float)a.s;
+  owned_pairs<NB_H, true>(
+      L, ln, S.kl32, NB_H ? S.npd : 0, gmem((const double2*)S.qxy), gmem((const double2*)S.qzs),
+      gmem((const float2*)S.aux), gmem((const double*)S.xrow),
+      [&](const Site& b) {
+        Pair32 p;
+        pair_vec32(img, a, b, p.d);
+        p.bs = (float)b.s;
+        return p;
+      },
+      [&](const Pair32& q, float Fj, double wj, int jl, int rv) {
+        const PairSums2 p = pair_grad<RULE, KIND>(tab, q.d, as, q.bs, Fi, Fj);
+        o.e += wj * p.pe;
+        o.g0 += wj * p.g[0];
+        o.g1 += wj * p.g[1];
+        o.g2 += wj * p.g[2];
+        o.gs += wj * p.gsi;
+        // the partner's share leaves weighted by the sender's occupancy
+        float4 v = make_float4(-p.g[0], -p.g[1], -p.g[2], p.gsj);
+        if (ME_H)
+          v = make_float4((float)(wme * (double)v.x), (float)(wme * (double)v.y), (float)(wme * (double)v.z),
+                          (float)(wme * (double)v.w));
+        prb[(size_t)rv * prows + jl] = v;
+      });
+}
+
+// Bound by what a pair moves: 8 B of list, ~50 B gathered through L1 and 16 B of
+// share written (0.33 GB at 40^3 cells) keep the kernel at 246 us with its
+// nodes taken out; with them 261 us (12-point rule; 364 us before the tables
+// in |r|^2, the row order and the pipelined loads) and 508 us (Gauss-Hermite;
+// 651 us).
+template <int RULE, int TBO>
+__global__ __launch_bounds__(TBO) __attribute__((amdgpu_waves_per_eu(TBO / 128))) void k_grad_own(
+    const LatDev* __restrict__ lats, const int32_t* __restrict__ ob2l, int nblk, const float4* __restrict__ gtab) {
+  __shared__ float4 tab[NGTAB * SNT];
+  stage_tables(tab, gtab + S_BASE + S_DFPD * SNT, NGTAB * SNT);
+  const int w = xcd_block() * (TBO / TB) + __builtin_amdgcn_readfirstlane(threadIdx.x / TB);
+  if (w >= nblk) return;
+  const LatDev& S = lats[ob2l[w]];
+  if (S.rule != RULE) return;  // the other rule's instance serves this lattice
+  const int K = S.kl32;
+  const OwnerLane ln(S, w - S.owg0_32, K);
+  if (ln.row >= ln.rows) return;  // whole lane groups
+  const Image img = image_of(S);
+  const int s = ln.pd ? ln.row : S.npd + ln.row;
+  const Site a = load_row(gmem((const double2*)S.qxy), gmem((const double2*)S.qzs), s);
+  const float Fi = gmem((const float2*)S.aux)[s].x;
+  Own o;
+  if (ln.pd) {
+    grad_list<RULE, 0>(tab, S, ln, a, Fi, img, 1.0, o);
+    grad_list<RULE, 1>(tab, S, ln, a, Fi, img, 1.0, o);
+  } else {
+    const double wme = gmem((const double*)S.xrow)[ln.row];
+    grad_list<RULE, 2>(tab, S, ln, a, Fi, img, wme, o);
+    grad_list<RULE, 3>(tab, S, ln, a, Fi, img, wme, o);
   }
-  e = site_sum(e, K);
-  g0 = site_sum(g0, K);
-  g1 = site_sum(g1, K);
-  g2 = site_sum(g2, K);
-  gs = site_sum(gs, K);
-  if (ph != 0) return;
-  gmem(reinterpret_cast<double4*>(S.G))[s] = make_double4(g0, g1, g2, gs);
-  gmem(S.epair)[s] = e;
+  o.e = site_sum(o.e, K);
+  o.g0 = site_sum(o.g0, K);
+  o.g1 = site_sum(o.g1, K);
+  o.g2 = site_sum(o.g2, K);
+  o.gs = site_sum(o.gs, K);
+  if (ln.ph != 0) return;
+  gmem(S.gown)[s] = make_double4(o.g0, o.g1, o.g2, o.gs);
+  gmem(S.epair)[s] = o.e;
 }
 
 __global__ __launch_bounds__(TB) void k_grad_recv(const LatDev* __restrict__ lats, const int32_t* __restrict__ b2l) {
@@ -865,11 +1017,13 @@ __global__ __launch_bounds__(TB) void k_grad_recv(const LatDev* __restrict__ lat
   const int N = S.npd + S.nh;
   double fs = 0.0;
   if (s < N) {
-    const double* __restrict__ xo = S.x;
+    const double* __restrict__ xo = S.xrow;
     const bool pd = s < S.npd;
     const int row = pd ? s : s - S.npd;
     double* __restrict__ G = S.G;
-    double g0 = G[4 * (size_t)s], g1 = G[4 * (size_t)s + 1], g2 = G[4 * (size_t)s + 2], gs = G[4 * (size_t)s + 3];
+    const size_t site = pd ? site_of_row(row, S.npd) : S.npd + site_of_row(row, S.nh);
+    const double4 own = S.gown[s];
+    double g0 = own.x, g1 = own.y, g2 = own.z, gs = own.w;
 #pragma unroll
     for (int side = 0; side < 2; ++side) {
       const int list = pd ? side : 2 + side;
@@ -882,16 +1036,16 @@ __global__ __launch_bounds__(TB) void k_grad_recv(const LatDev* __restrict__ lat
       });
     }
     const double xi = pd ? 1.0 : xo[row];
-    const double sg = S.X[4 * (size_t)s + 3];
+    const double sg = S.qzs[s].y;
     const double T = S.T;
     const bool gh = S.rule == GH3;
-    const double qw = gh ? 1.0 : QW, sq = gh ? 1.0 : SQ6;
+    const double qw = gh ? GHQW : QW, sq = gh ? 1.0 : SQ6;
     const double V = S.emb[s] + qw * xi * S.epair[s];  // owned pairs carry their full energy
     const double sc = qw * xi / T;
-    G[4 * (size_t)s + 0] = sc * g0;
-    G[4 * (size_t)s + 1] = sc * g1;
-    G[4 * (size_t)s + 2] = sc * g2;
-    G[4 * (size_t)s + 3] = sq * sc * gs - 3.0 * KB * xi / sg;
+    G[4 * site + 0] = sc * g0;
+    G[4 * site + 1] = sc * g1;
+    G[4 * site + 2] = sc * g2;
+    G[4 * site + 3] = sq * sc * gs - 3.0 * KB * xi / sg;
     fs = V / T - 3.0 * KB * xi * log(sg);
   }
   red[threadIdx.x] = fs;
@@ -921,7 +1075,69 @@ void fill_table(float4* out, Fn g) {
   }
 }
 
+// Rows of the tables in s: g gives a function's value and slope in |r|.  In
+// the local coordinate u of an interval, the slope d/du is dg/dr h / (2 |r|).
+struct Row {
+  long double c[4] = {0, 0, 0, 0};
+};
+// polynomial through (u[i], y[i]), i < n, as monomials
+Row through(const long double* u, const long double* y, int n) {
+  long double c[4];
+  for (int i = 0; i < n; ++i) c[i] = y[i];
+  for (int j = 1; j < n; ++j)
+    for (int i = n - 1; i >= j; --i) c[i] = (c[i] - c[i - 1]) / (u[i] - u[i - j]);
+  Row m;
+  for (int i = n - 1; i >= 0; --i) {
+    for (int q = 3; q > 0; --q) m.c[q] = m.c[q - 1] - u[i] * m.c[q];
+    m.c[0] = c[i] - u[i] * m.c[0];
+  }
+  return m;
+}
+enum { FIT_VALUE, FIT_SLOPE, FIT_BOTH };
+template <class Fn>
+void fill_table_s(float4* out, int fit, Fn g) {
+  const long double PI = 3.14159265358979323846264338327950288L, h = 0.5025L / 14, s0 = 25.5025L - 683 * h;
+  auto node = [&](int i, int n) { return 0.5L - 0.5L * cosl((2 * i + 1) * PI / (2.0L * n)); };
+  for (int k = 0; k < SNT; ++k) {
+    auto at = [&](long double u) {
+      const long double r = sqrtl(s0 + (k + u) * h);
+      const eam::VDT<long double> v = g(r);
+      return eam::VDT<long double>{v.v, v.d * h / (2 * r)};
+    };
+    const int n = fit == FIT_VALUE ? 4 : 3;
+    long double u[4], y[4];
+    for (int i = 0; i < n; ++i) {
+      u[i] = node(i, n);
+      y[i] = fit == FIT_VALUE ? at(u[i]).v : at(u[i]).d;
+    }
+    Row m = through(u, y, n);
+    if (fit == FIT_BOTH) {  // the slope's integral, with the value's mean over four points
+      m = Row{{0, m.c[0], m.c[1] / 2, m.c[2] / 3}};
+      for (int i = 0; i < 4; ++i) {
+        const long double w = node(i, 4);
+        y[i] = at(w).v - w * (m.c[1] + w * (m.c[2] + w * m.c[3]));
+      }
+      m.c[0] = (y[0] + y[1] + y[2] + y[3]) / 4;
+    }
+    out[k] = make_float4((float)m.c[0], (float)m.c[1], (float)m.c[2], (float)m.c[3]);
+  }
+}
+
 }  // namespace
+
+void host_tables_s(std::vector<float4>& t) {
+  static const std::vector<float4> built = [] {  // once per process
+    using LD = long double;
+    std::vector<float4> u((size_t)NSTAB * SNT);
+    fill_table_s(&u[S_FPD * SNT], FIT_VALUE, [](LD r) { return eam::f_Pd_vd<LD>(r); });
+    fill_table_s(&u[S_DFPD * SNT], FIT_SLOPE, [](LD r) { return eam::f_Pd_vd<LD>(r); });
+    fill_table_s(&u[S_PHPD * SNT], FIT_BOTH, [](LD r) { return eam::phi_Pd_vd<LD>(r, eam::f_Pd_vd<LD>(r)); });
+    fill_table_s(&u[S_PHPDH * SNT], FIT_BOTH, [](LD r) { return eam::phi_morse_vd<0, LD>(r); });
+    fill_table_s(&u[S_PHH * SNT], FIT_BOTH, [](LD r) { return eam::phi_morse_vd<1, LD>(r); });
+    return u;
+  }();
+  t.insert(t.end(), built.begin(), built.end());
+}
 
 void host_tables(std::vector<float4>& t) {
   static const std::vector<float4> built = [] {  // once per process (~0.4 ms of long-double work)
@@ -945,6 +1161,24 @@ int build_tables(a2c_fe_ctx* c) {
   return A2C_OK;
 }
 
+namespace {
+// The tables of k_grad_own allow two workgroups per CU whatever their size: 512
+// lanes give every SIMD 4 waves (40^3 cells: 264 us against 416 us with 256
+// lanes and 2 waves).  With fewer units than two per CU the smaller
+// workgroups spread over more CUs (14^3 cells, Gauss-Hermite rule: 53 against
+// 56 us; 12-point rule 34 against 33 us).
+constexpr int GRAD_WIDE_UNITS = 512;
+template <int RULE>
+void launch_grad_own(const Launch& L) {
+  if (L.onblk >= GRAD_WIDE_UNITS)
+    hipLaunchKernelGGL((k_grad_own<RULE, 512>), dim3((L.onblk + 1) / 2), dim3(512), 0, L.stream, L.lats, L.ob2l,
+                       L.onblk, L.tab);
+  else
+    hipLaunchKernelGGL((k_grad_own<RULE, 256>), dim3(L.onblk), dim3(256), 0, L.stream, L.lats, L.ob2l, L.onblk,
+                       L.tab);
+}
+}  // namespace
+
 int run_eval32(const Launch& L, Timing* tm) {
   if (L.mixed_full && L.rules == (1 << A2C_QUAD_R12)) {  // every pair from both ends (12-point rule only)
     if (tm) tm->mark(L.stream, "density32");
@@ -958,6 +1192,8 @@ int run_eval32(const Launch& L, Timing* tm) {
       if (hipGetLastError() != hipSuccess) return A2C_EHIP;
     }
   } else if (L.nblk > 0) {
+    if (tm) tm->mark(L.stream, "rows");
+    if (run_rows(L)) return A2C_EHIP;
     if (tm) tm->mark(L.stream, "dens_own");
     if (L.rules & (1 << A2C_QUAD_R12))
       hipLaunchKernelGGL(k_dens_own<A2C_QUAD_R12>, dim3(L.onblk), dim3(TB), 0, L.stream, L.lats, L.ob2l, L.tab);
@@ -969,9 +1205,8 @@ int run_eval32(const Launch& L, Timing* tm) {
     if (hipGetLastError() != hipSuccess) return A2C_EHIP;
     if (tm) tm->mark(L.stream, "grad_own");
     if (L.rules & (1 << A2C_QUAD_R12))
-      hipLaunchKernelGGL(k_grad_own<A2C_QUAD_R12>, dim3(L.onblk), dim3(TB), 0, L.stream, L.lats, L.ob2l, L.tab);
-    if (L.rules & (1 << GH3))
-      hipLaunchKernelGGL(k_grad_own<GH3>, dim3(L.onblk), dim3(TB), 0, L.stream, L.lats, L.ob2l, L.tab);
+      launch_grad_own<A2C_QUAD_R12>(L);
+    if (L.rules & (1 << GH3)) launch_grad_own<GH3>(L);
     if (hipGetLastError() != hipSuccess) return A2C_EHIP;
     if (tm) tm->mark(L.stream, "grad_recv");
     hipLaunchKernelGGL(k_grad_recv, dim3(L.nblk), dim3(TB), 0, L.stream, L.lats, L.b2l);

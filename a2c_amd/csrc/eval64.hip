@@ -79,16 +79,12 @@ __device__ __forceinline__ void pair_vec(const LatDev& S, const Site& a, const S
 }
 // the same with the geometry held in registers (pair-owner loops)
 __device__ __forceinline__ void pair_vec(const Image& g, const Site& a, const Site& b, double d[3]) {
-#pragma unroll
-  for (int c = 0; c < 3; ++c) {
-    double qj = b.q[c];
-    if (g.per[c]) qj = qj - g.box[c] * rint((qj - a.q[c]) * g.ibox[c]);
-    d[c] = a.q[c] - qj;
-  }
+  image_vec(g, a.q, b.q, d);
 }
-__device__ __forceinline__ Site load_site(const A2C_GLOBAL double4* __restrict__ X, int s) {
-  const double4 v = X[s];
-  return {{v.x, v.y, v.z}, v.w};
+__device__ __forceinline__ Site load_row(const A2C_GLOBAL double2* __restrict__ qxy,
+                                         const A2C_GLOBAL double2* __restrict__ qzs, int p) {
+  const double2 a = qxy[p], b = qzs[p];
+  return {{a.x, a.y, b.x}, b.y};
 }
 
 // ---------------------------------------------------------------- FP64 tables
@@ -469,18 +465,17 @@ __global__ __launch_bounds__(TB) void k_dens_own64(const LatDev* __restrict__ la
   for (int i = threadIdx.x; i < T64_N * T64_P; i += blockDim.x) t64[i] = gtab64[(size_t)T64_FH * T64_N * T64_P + i];
   stage64(t64 + T64_PART1, gtab64 + T64_PART1 + (size_t)T64Q_FPD * T64_N * T64Q_P, T64_N * T64Q_P);
   const int K = S.kl64;  // lanes per site: lane ph takes owned slots ph, ph + K, ...
-  const int s = (w - S.owg0_64) * (TB / K) + (int)threadIdx.x / K;
-  const int ph = (int)threadIdx.x % K;
-  const int npd = S.npd;
-  const int N = npd + S.nh;
-  if (s >= N) return;  // whole lane groups
+  const OwnerLane ln(S, w - S.owg0_64, K);
+  if (ln.row >= ln.rows) return;  // whole lane groups
+  const int npd = S.npd, ph = ln.ph, row = ln.row;
+  const bool pd = ln.pd;
+  const int s = pd ? row : npd + row;
   // everything the pair loops use, out of the descriptor and into registers
-  const A2C_GLOBAL double4* __restrict__ X = gmem(reinterpret_cast<const double4*>(S.X));
-  const A2C_GLOBAL double* __restrict__ xo = gmem(S.x);
+  const A2C_GLOBAL double2* __restrict__ qxy = gmem((const double2*)S.qxy);
+  const A2C_GLOBAL double2* __restrict__ qzs = gmem((const double2*)S.qzs);
+  const A2C_GLOBAL double* __restrict__ xo = gmem((const double*)S.xrow);
   const Image img = image_of(S);
-  const bool pd = s < npd;
-  const int row = pd ? s : s - npd;
-  const Site a = load_site(X, s);
+  const Site a = load_row(qxy, qzs, s);
   const double ai = SQ6 * a.s;
   const double wme = pd ? 1.0 : xo[row];  // shares leave weighted by the sender's occupancy
   double rho = 0.0;
@@ -498,7 +493,7 @@ __global__ __launch_bounds__(TB) void k_dens_own64(const LatDev* __restrict__ la
       const size_t e = (size_t)t * rows + row;
       const int jl = oj[e];
       const int rv = orv[e];
-      const Site b = load_site(X, side == 0 ? jl : npd + jl);
+      const Site b = load_row(qxy, qzs, side == 0 ? jl : npd + jl);
       const double wj = side == 0 ? 1.0 : xo[jl];
       double d[3];
       pair_vec(img, a, b, d);
@@ -532,7 +527,7 @@ __global__ __launch_bounds__(TB) void k_dens_own64(const LatDev* __restrict__ la
         }
       }
       rho += wj * mine;
-      if (rv >= 0) share[(size_t)rv * prows + jl] = wme * theirs;
+      share[(size_t)rv * prows + jl] = wme * theirs;
     }
   }
   rho = site_sum(rho, K);
@@ -545,7 +540,7 @@ __global__ __launch_bounds__(TB) void k_dens_recv64(const LatDev* __restrict__ l
   const int s = (blk - S.blk0) * TB + threadIdx.x;
   const int N = S.npd + S.nh;
   if (s >= N) return;
-  const double* __restrict__ xo = S.x;
+  const double* __restrict__ xo = S.xrow;
   const bool pd = s < S.npd;
   const int row = pd ? s : s - S.npd;
   double rho = S.rho[s];
@@ -680,19 +675,18 @@ __global__ __launch_bounds__(TB) __attribute__((amdgpu_waves_per_eu(3))) void k_
   if (S.rule != RULE) return;
   stage64(t64, gtab64, T64_SIZE);
   const int K = S.kl64;  // lanes per site: lane ph takes owned slots ph, ph + K, ...
-  const int s = (w - S.owg0_64) * (TB / K) + (int)threadIdx.x / K;
-  const int ph = (int)threadIdx.x % K;
-  const int npd = S.npd;
-  const int N = npd + S.nh;
-  if (s >= N) return;  // whole lane groups
+  const OwnerLane ln(S, w - S.owg0_64, K);
+  if (ln.row >= ln.rows) return;  // whole lane groups
+  const int npd = S.npd, ph = ln.ph, row = ln.row;
+  const bool pd = ln.pd;
+  const int s = pd ? row : npd + row;
   // everything the pair loops use, out of the descriptor and into registers
-  const A2C_GLOBAL double4* __restrict__ X = gmem(reinterpret_cast<const double4*>(S.X));
-  const A2C_GLOBAL double* __restrict__ xo = gmem(S.x);
+  const A2C_GLOBAL double2* __restrict__ qxy = gmem((const double2*)S.qxy);
+  const A2C_GLOBAL double2* __restrict__ qzs = gmem((const double2*)S.qzs);
+  const A2C_GLOBAL double* __restrict__ xo = gmem((const double*)S.xrow);
   const A2C_GLOBAL double* __restrict__ Fp = gmem(S.Fp);
   const Image img = image_of(S);
-  const bool pd = s < npd;
-  const int row = pd ? s : s - npd;
-  const Site a = load_site(X, s);
+  const Site a = load_row(qxy, qzs, s);
   const double Fi = Fp[s];
   const double wme = pd ? 1.0 : xo[row];  // shares leave weighted by the sender's occupancy
   double e = 0.0, g0 = 0.0, g1 = 0.0, g2 = 0.0, gs = 0.0;
@@ -713,7 +707,7 @@ __global__ __launch_bounds__(TB) __attribute__((amdgpu_waves_per_eu(3))) void k_
       const size_t ei = (size_t)t * rows + row;
       const int jl = oj[ei];
       const int rv = orv[ei];
-      const Site b = load_site(X, off + jl);
+      const Site b = load_row(qxy, qzs, off + jl);
       const double Fj = Fp[off + jl];
       const double wj = side == 0 ? 1.0 : xo[jl];
       double d[3];
@@ -726,7 +720,7 @@ __global__ __launch_bounds__(TB) __attribute__((amdgpu_waves_per_eu(3))) void k_
       e += wj * pe;
       g0 += wj * pg[0]; g1 += wj * pg[1]; g2 += wj * pg[2];
       gs += wj * psi;
-      if (rv >= 0) share[(size_t)rv * prows + jl] = make_double4(-wme * pg[0], -wme * pg[1], -wme * pg[2], wme * psj);
+      share[(size_t)rv * prows + jl] = make_double4(-wme * pg[0], -wme * pg[1], -wme * pg[2], wme * psj);
     }
   }
   e = site_sum(e, K);
@@ -735,7 +729,7 @@ __global__ __launch_bounds__(TB) __attribute__((amdgpu_waves_per_eu(3))) void k_
   g2 = site_sum(g2, K);
   gs = site_sum(gs, K);
   if (ph != 0) return;
-  gmem(reinterpret_cast<double4*>(S.G))[s] = make_double4(g0, g1, g2, gs);
+  gmem(S.gown)[s] = make_double4(g0, g1, g2, gs);
   gmem(S.epair)[s] = e;
 }
 
@@ -748,11 +742,13 @@ __global__ __launch_bounds__(TB) void k_grad_recv64(const LatDev* __restrict__ l
   const int N = S.npd + S.nh;
   double fs = 0.0;
   if (s < N) {
-    const double* __restrict__ xo = S.x;
+    const double* __restrict__ xo = S.xrow;
     const bool pd = s < S.npd;
     const int row = pd ? s : s - S.npd;
     double* __restrict__ G = S.G;
-    double g0 = G[4 * (size_t)s], g1 = G[4 * (size_t)s + 1], g2 = G[4 * (size_t)s + 2], gs = G[4 * (size_t)s + 3];
+    const size_t site = pd ? site_of_row(row, S.npd) : S.npd + site_of_row(row, S.nh);
+    const double4 own = S.gown[s];
+    double g0 = own.x, g1 = own.y, g2 = own.z, gs = own.w;
 #pragma unroll
     for (int side = 0; side < 2; ++side) {
       const Ell& L = list_of(S, pd ? side : 2 + side);
@@ -764,16 +760,16 @@ __global__ __launch_bounds__(TB) void k_grad_recv64(const LatDev* __restrict__ l
       });
     }
     const double xi = pd ? 1.0 : xo[row];
-    const double sg = S.X[4 * (size_t)s + 3];
+    const double sg = S.qzs[s].y;
     const double T = S.T;
     const bool gh = S.rule == GH3;
     const double qw = gh ? 1.0 : QW, sq = gh ? 1.0 : SQ6;
     const double V = S.emb[s] + qw * xi * S.epair[s];  // owned pairs carry their full energy
     const double sc = qw * xi / T;
-    G[4 * (size_t)s + 0] = sc * g0;
-    G[4 * (size_t)s + 1] = sc * g1;
-    G[4 * (size_t)s + 2] = sc * g2;
-    G[4 * (size_t)s + 3] = sq * sc * gs - 3.0 * KB * xi / sg;
+    G[4 * site + 0] = sc * g0;
+    G[4 * site + 1] = sc * g1;
+    G[4 * site + 2] = sc * g2;
+    G[4 * site + 3] = sq * sc * gs - 3.0 * KB * xi / sg;
     fs = V / T - 3.0 * KB * xi * log(sg);
   }
   red[threadIdx.x] = fs;
@@ -784,6 +780,21 @@ __global__ __launch_bounds__(TB) void k_grad_recv64(const LatDev* __restrict__ l
     __syncthreads();
   }
   if (threadIdx.x == 0) S.part[lb] = red[0];
+}
+
+// Row-order copies of the state and the occupancy for the pair passes.
+__global__ __launch_bounds__(TB) void k_rows(const LatDev* __restrict__ lats, const int32_t* __restrict__ b2l) {
+  const int blk = xcd_block();
+  const LatDev& S = lats[b2l[blk]];
+  const int s = (blk - S.blk0) * TB + threadIdx.x;
+  if (s >= S.npd + S.nh) return;
+  const double4 v = reinterpret_cast<const double4*>(S.X)[s];
+  const bool pd = s < S.npd;
+  const int row = pd ? row_of_site(s, S.npd) : row_of_site(s - S.npd, S.nh);
+  const int p = pd ? row : S.npd + row;
+  S.qxy[p] = make_double2(v.x, v.y);
+  S.qzs[p] = make_double2(v.z, v.w);
+  if (!pd) S.xrow[row] = S.x[s - S.npd];
 }
 
 }  // namespace
@@ -830,6 +841,8 @@ int run_density64(const Launch& L) {
 int run_eval64(const Launch& L, Timing* tm) {
   if (L.deriv_mode == A2C_DERIV_ANALYTIC && !L.full_pairs64) {
     if (L.nblk > 0) {
+      if (tm) tm->mark(L.stream, "rows");
+      if (run_rows(L)) return A2C_EHIP;
       if (tm) tm->mark(L.stream, "dens_own64");
       if (per_rule<DensOwn>(L, L.onblk, L.lats, L.ob2l, L.tab64)) return A2C_EHIP;
       if (tm) tm->mark(L.stream, "dens_recv64");
@@ -858,6 +871,11 @@ int run_eval64(const Launch& L, Timing* tm) {
   if (int rc = run_final_sum(L)) return rc;
   if (tm) tm->mark(L.stream, nullptr);
   return A2C_OK;
+}
+
+int run_rows(const Launch& L) {
+  hipLaunchKernelGGL(k_rows, dim3(L.nblk), dim3(TB), 0, L.stream, L.lats, L.b2l);
+  return hipGetLastError() == hipSuccess ? A2C_OK : A2C_EHIP;
 }
 
 int run_final_sum(const Launch& L) {
@@ -933,7 +951,7 @@ static Launch single_launch(a2c_fe_ctx* c, bool fp64) {
   L.lats = c->dlat;
   L.b2l = c->db2l;
   L.ob2l = c->db2l;
-  L.onblk = site_blocks(c->N) * lanes_per_site(c->N, fp64);
+  L.onblk = owner_units(c->desc.n_pd, c->desc.n_h, lanes_per_site(c->N, fp64));
   L.nblk = site_blocks(c->N);
   L.nlat = 1;
   L.rules = 1 << c->desc.quad_rule;

@@ -28,6 +28,29 @@ hipError_t hfree(const void* ptr);
 constexpr double KB = 8.6173324e-5;  // Boltzmann constant, eV/K (minimizer.cpp:92)
 constexpr int NBR_CAP = 256;          // per-site neighbor cap of the build kernel
 
+// Row order of the pair-once evaluation.  An FCC crystal lists its sites cell
+// by cell, four to a cell, and the four see their neighbors in different
+// directions: 64 consecutive sites at the same list slot gather from 64
+// scattered places.  The split lists, the shares and the per-site arrays the
+// pair passes read are therefore kept with every fourth site together -- the
+// first site of all cells, then the second, ... (rows past the last whole
+// group of four keep their place) -- so a wave's 64 rows are the same site of
+// 64 consecutive cells: slot t of all of them is the same neighbor vector, the
+// neighbors are consecutive rows too, and gathers and share stores touch 8 to
+// 16 cache lines instead of 64, and shares fill whole lines.  (40^3 cells, mixed:
+// k_dens_own 211 -> 170 us, k_grad_own 355 -> 280 us; k_rows costs 14 us.)  Any
+// other site order only loses that: this is a permutation of each species' rows.
+__host__ __device__ inline int row_of_site(int r, int rows) {
+  const int q = rows >> 2;
+  return r < 4 * q ? (r & 3) * q + (r >> 2) : r;
+}
+__host__ __device__ inline int site_of_row(int p, int rows) {
+  const int q = rows >> 2;
+  if (p >= 4 * q) return p;
+  const int b = (p >= q) + (p >= 2 * q) + (p >= 3 * q);
+  return (p - b * q) * 4 + b;
+}
+
 // One neighbor list in ELL layout: entry t of row r is idx[t * rows + r], so
 // lane r of a wave reading slot t touches consecutive words (coalesced).
 // Indices are species-local (Pd index or H index), rows sorted ascending.
@@ -37,6 +60,7 @@ struct Ell {
   int32_t* idx = nullptr;  // width * rows
   int32_t* cnt = nullptr;  // rows
   // Pair-once evaluation (each unordered pair evaluated once, by its owner).
+  // Rows and neighbor indices of this part are in row order (row_of_site).
   // Every row is split, keeping its order, into the entries this row owns
   // and the entries it receives; both halves are compact (slot-major, no
   // gaps), so a wave's lanes step through their halves without masking each
@@ -84,6 +108,12 @@ struct LatDev {
   double* epair = nullptr;    // N pair-energy partial (mixed path)
   double* part = nullptr;     // ceil(N/256) block partial sums of f
   double* f = nullptr;        // objective
+  // pair-once evaluation, per species in row order (Pd rows, then H rows; rho,
+  // Fp, aux, emb and epair are in this order too while it runs):
+  double2* qxy = nullptr;     // N {x, y} and
+  double2* qzs = nullptr;     // N {z, sigma}: two 16-byte arrays, each gathered whole lines at a time
+  double* xrow = nullptr;     // nh occupancy
+  double4* gown = nullptr;    // N gradient sums of the owned pairs
 };
 using DevSys = LatDev;
 constexpr int SITE_BLOCK = 256;  // sites per block of every site-parallel kernel
@@ -141,6 +171,14 @@ constexpr int RECV_RU_SCALAR = 8, RECV_RU_WIDE = 2;
 // lattice: its results are the same in any batch.
 int lanes_per_site(int n_sites, bool fp64);
 constexpr int MAX_LANES_PER_SITE = 16;
+// Workgroup units of a pair-owner pass: 256 lanes each, the rows of one species
+// per unit (Pd units first), so that everything that depends on the species --
+// list pointers, pair kind, weights -- is uniform and stays in scalar
+// registers.
+__host__ __device__ inline int owner_units(int rows, int K) {
+  return (int)(((int64_t)rows * K + SITE_BLOCK - 1) / SITE_BLOCK);
+}
+__host__ __device__ inline int owner_units(int npd, int nh, int K) { return owner_units(npd, K) + owner_units(nh, K); }
 
 // Fixed-order sum over the K lanes of a site (K a power of two <= 64, lanes
 // contiguous within a wave); the total lands in the group's first lane.
@@ -197,7 +235,7 @@ struct GenDev {
 // descriptor, and its fields would be reloaded for every pair).
 struct Image {
   double box[3], ibox[3];
-  bool per[3];
+  double half[3];  // L / 2 on a periodic axis, else infinity
 };
 __device__ __forceinline__ Image image_of(const LatDev& S) {
   Image g;
@@ -205,10 +243,43 @@ __device__ __forceinline__ Image image_of(const LatDev& S) {
   for (int c = 0; c < 3; ++c) {
     g.box[c] = S.box[c];
     g.ibox[c] = S.ibox[c];
-    g.per[c] = S.periodic[c] != 0;
+    g.half[c] = S.periodic[c] ? 0.5 * S.box[c] : __builtin_huge_val();
   }
   return g;
 }
+// d = q_i - image(q_j): a periodic axis shifts q_j by L rint((q_j - q_i) / L).
+// A listed pair is within rc <= L/2 of an image, so the shift is zero unless
+// |q_i - q_j| > L/2 -- no pair of most waves, which then skip it.
+__device__ __forceinline__ void image_vec(const Image& g, const double qi[3], const double qj[3], double d[3]) {
+  bool far = false;
+#pragma unroll
+  for (int c = 0; c < 3; ++c) {
+    d[c] = qi[c] - qj[c];
+    far |= fabs(d[c]) > g.half[c];
+  }
+  if (far) {
+#pragma unroll
+    for (int c = 0; c < 3; ++c)
+      if (fabs(d[c]) > g.half[c]) d[c] = qi[c] - (qj[c] - g.box[c] * rint((qj[c] - qi[c]) * g.ibox[c]));
+  }
+}
+
+// Place of a lane in a pair-owner pass: its row (row order) and its phase ph
+// among the row's K lanes, which take owned slots ph, ph + K, ...  u: the
+// wave's unit within the lattice (uniform).
+struct OwnerLane {
+  bool pd;   // uniform
+  int rows;  // of the species
+  int row, ph;
+  __device__ __forceinline__ OwnerLane(const LatDev& S, int u, int K) {
+    const int up = owner_units(S.npd, K), sh = 31 - __builtin_clz(K);
+    pd = u < up;
+    rows = pd ? S.npd : S.nh;
+    const int lane = (int)threadIdx.x % SITE_BLOCK;
+    ph = lane & (K - 1);
+    row = (pd ? u : u - up) * (SITE_BLOCK >> sh) + (lane >> sh);
+  }
+};
 
 // Logical site block of a workgroup.  Workgroups are dealt to the 8 XCDs
 // round-robin by index; this bijection gives XCD k one contiguous range of
@@ -275,6 +346,10 @@ struct a2c_fe_ctx {
   float4* dtab = nullptr;    // cubic coefficient tables (5 x 500 intervals)
   double* dtab64 = nullptr;  // FP64 polynomial tables of the exponential functions
   float2* daux = nullptr;    // per site {F'(rho), x} in FP32
+  double2* dqxy = nullptr;   // row-order copies of the state and occupancy, and the
+  double2* dqzs = nullptr;   // owned pairs' gradient sums (pair-once evaluation)
+  double* dxrow = nullptr;
+  double4* dgown = nullptr;
 
   // launch descriptors: this context is a batch of one lattice
   a2c::LatDev* hlat = nullptr;   // pinned host copy
@@ -319,6 +394,7 @@ struct a2c_fe_ctx {
     s.rule = desc.quad_rule;
     s.pdpd = ell[0]; s.pdh = ell[1]; s.hpd = ell[2]; s.hh = ell[3]; s.hh1 = ell[4];
     s.x = dx; s.rho = drho; s.Fp = dFp; s.aux = daux; s.emb = demb; s.part = dpart; s.epair = depair;
+    s.qxy = dqxy; s.qzs = dqzs; s.xrow = dxrow; s.gown = dgown;
     return s;
   }
 };
@@ -361,13 +437,15 @@ int run_density64(const Launch& L);
 int run_eval64(const Launch& L, Timing* tm);
 int run_eval32(const Launch& L, Timing* tm);
 int run_final_sum(const Launch& L);
+int run_rows(const Launch& L);  // row-order copies of state and occupancy (pair-once evaluation)
 int sync_lattice(a2c_fe_ctx* c, const double* dX, double* dG, double* dF);  // refresh the one-lattice descriptor
 int launch_eval64(a2c_fe_ctx* c, const double* dX, double* dG, double* dF, bool timed, Timing* tm);
 int launch_density64(a2c_fe_ctx* c, const double* dX);  // fills drho, dFp, demb
 int launch_eval32(a2c_fe_ctx* c, const double* dX, double* dG, double* dF, bool timed, Timing* tm);
 int build_tables(a2c_fe_ctx* c);                        // eval32.hip
 int tables_download(a2c_fe_ctx* c, float* out);         // 5*500 float4
-void host_tables(std::vector<float4>& t);              // FP32 cubic tables (host)
+void host_tables(std::vector<float4>& t);              // FP32 cubic tables in r (host)
+void host_tables_s(std::vector<float4>& t);            // appends the FP32 cubic tables in |r|^2
 // FP64 tables of the EAM functions: per function T64_N intervals of 0.05 A
 // over [1, 6) A, each a polynomial in the local coordinate u in [0, 1).  Part
 // one: the exponential functions (f_H, phi_PdH, phi_H), degree T64_D, T64_P

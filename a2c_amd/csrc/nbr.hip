@@ -304,10 +304,11 @@ __global__ __launch_bounds__(NT) void k_site(NbrArgs a, int nblk_pd) {
     if (live) {
       a.cnt[lp][row] = npn;
       a.cnt[lh][row] = nhn;
-      a.ocnt[lp][row] = op;
-      a.rcnt[lp][row] = npn - op;
-      a.ocnt[lh][row] = oh;
-      a.rcnt[lh][row] = nhn - oh;
+      const int p = row_of_site(row, nrows);
+      a.ocnt[lp][p] = op;
+      a.rcnt[lp][p] = npn - op;
+      a.ocnt[lh][p] = oh;
+      a.rcnt[lh][p] = nhn - oh;
       if (!pdb) a.cnt[4][row] = nh1;
     }
     // maxima over the wave, then one atomic per quantity
@@ -378,18 +379,18 @@ __global__ __launch_bounds__(NT) void k_site(NbrArgs a, int nblk_pd) {
 // loads of a pair slot coalesce.  (Ordering the owned half by distance, to
 // align table rows across lanes, measured 40% slower: it scatters those
 // gathers.)
-__global__ void k_split(Ell L, int s_off, int j_off) {
+__global__ void k_split(Ell L, int s_off, int j_off, int jrows) {
   const int r = blockIdx.x * blockDim.x + threadIdx.x;
   if (r >= L.rows) return;
   int32_t* rpos = reinterpret_cast<int32_t*>(L.rbuf);  // full-row slot -> received slot (-1 if owned)
   const int n = L.cnt[r];
-  const int s = s_off + r;
+  const int s = s_off + r, p = row_of_site(r, L.rows);
   int no = 0, nr = 0;
   for (int t = 0; t < n; ++t) {
     const size_t e = (size_t)t * L.rows + r;
     const int j = L.idx[e];
     if (pair_owner(s, j_off + j)) {
-      L.oj[(size_t)no * L.rows + r] = j;
+      L.oj[(size_t)no * L.rows + p] = row_of_site(j, jrows);
       rpos[e] = -1;
       ++no;
     } else {
@@ -400,16 +401,18 @@ __global__ void k_split(Ell L, int s_off, int j_off) {
 }
 
 // For every owned entry (r, j): the received slot of r in the partner row j,
-// found by binary search of r in that sorted row (-1 if absent, which the
-// symmetric lists never produce).
+// found by binary search of r in that sorted row (if absent, which the
+// symmetric lists never produce, a slot past the received half that nothing
+// reads: the owner passes store every share without a test).
 __global__ void k_orv(Ell L, Ell P) {
-  const int r = blockIdx.x * blockDim.x + threadIdx.x;
-  if (r >= L.rows) return;
+  const int p = blockIdx.x * blockDim.x + threadIdx.x;
+  if (p >= L.rows) return;
+  const int r = site_of_row(p, L.rows);
   const int32_t* prpos = reinterpret_cast<const int32_t*>(P.rbuf);
-  const int n = L.ocnt[r];
+  const int n = L.ocnt[p];
   for (int t = 0; t < n; ++t) {
-    const size_t e = (size_t)t * L.rows + r;
-    const int j = L.oj[e];
+    const size_t e = (size_t)t * L.rows + p;
+    const int j = site_of_row(L.oj[e], P.rows);
     int lo = 0, hi = P.cnt[j] - 1, k = -1;
     while (lo <= hi) {
       const int mid = (lo + hi) >> 1;
@@ -418,7 +421,7 @@ __global__ void k_orv(Ell L, Ell P) {
       if (v < r) lo = mid + 1;
       else hi = mid - 1;
     }
-    L.orv[e] = k >= 0 ? prpos[(size_t)k * P.rows + j] : -1;
+    L.orv[e] = k >= 0 ? prpos[(size_t)k * P.rows + j] : P.rwidth;
   }
 }
 
@@ -529,6 +532,8 @@ __global__ __launch_bounds__(NT) void k_refresh(RefreshArgs a, int4 blk0) {
   const int nrows = pdr ? a.npd : a.N - a.npd;
   const int lane = (int)threadIdx.x;
   const int row = (b - b0) * NT + lane;
+  const int prow = row_of_site(row, nrows);              // of the split lists
+  const int jrows = (w == 0 || w == 2) ? a.npd : a.N - a.npd;
   const bool live = row < nrows;
   const int s = (pdr ? 0 : a.npd) + (live ? row : 0);
   const int joff = (w == 0 || w == 2) ? 0 : a.npd;       // neighbors: Pd for PdPd and HPd
@@ -608,7 +613,7 @@ __global__ __launch_bounds__(NT) void k_refresh(RefreshArgs a, int4 blk0) {
   for (int u = 0, q = 0; u < mo; ++u) {
     if (u >= no) continue;
     while (!(col[q * CS + lane] & 2u)) ++q;
-    ooj[(size_t)u * orows + row] = (int)(col[q * CS + lane] >> 2);
+    ooj[(size_t)u * orows + prow] = row_of_site((int)(col[q * CS + lane] >> 2), jrows);
     ++q;
   }
   if (first) {
@@ -623,8 +628,8 @@ __global__ __launch_bounds__(NT) void k_refresh(RefreshArgs a, int4 blk0) {
   }
   if (live) {
     gmem(L.cnt)[row] = nk;
-    gmem(L.ocnt)[row] = no;
-    gmem(L.rcnt)[row] = nr;
+    gmem(L.ocnt)[prow] = no;
+    gmem(L.rcnt)[prow] = nr;
     if (first) gmem(a.out[4].cnt)[row] = nf;
     if (shells) {
       A2C_GLOBAL int32_t* pn = gmem(a.pdpdnum);
@@ -708,8 +713,9 @@ __global__ void k_srev(Ell L, Ell P) {
 // Reverse slots after a refresh, one thread per skin entry (slot t =
 // blockIdx.y): a kept, owned entry (fate -3 - k) takes the fate of its twin
 // in the partner's skin row -- the slot of this pair in the partner's
-// received half -- as the reverse slot of the row's k-th owned entry.
-__global__ void k_orv_skin(Ell S, Ell SP, Ell L) {
+// received half -- as the reverse slot of the row's k-th owned entry (spare:
+// the slot past every received half, as in k_orv).
+__global__ void k_orv_skin(Ell S, Ell SP, Ell L, int spare) {
   const int r = blockIdx.x * blockDim.x + threadIdx.x;
   const int t = blockIdx.y;
   if (r >= S.rows || t >= gmem(S.cnt)[r]) return;
@@ -718,8 +724,8 @@ __global__ void k_orv_skin(Ell S, Ell SP, Ell L) {
   if (f > -3) return;
   const int j = gmem(S.idx)[e];
   const int u = gmem(S.orv)[e];
-  gmem(L.orv)[(size_t)(-3 - f) * L.rows + r] =
-      u >= 0 ? gmem(reinterpret_cast<const int32_t*>(SP.rbuf))[(size_t)u * SP.rows + j] : -1;
+  gmem(L.orv)[(size_t)(-3 - f) * L.rows + row_of_site(r, L.rows)] =
+      u >= 0 ? gmem(reinterpret_cast<const int32_t*>(SP.rbuf))[(size_t)u * SP.rows + j] : spare;
 }
 
 }  // namespace
@@ -766,7 +772,8 @@ int size_lists(a2c_fe_ctx* c, Ell* L5, const int* w, const int* ow, const int* r
       A2C_HIP(c, dmalloc(&L.idx, sizeof(int32_t) * L.cap));
     }
     if (k == 4 || !ow) continue;
-    const int64_t on = (int64_t)std::max(ow[k], 1) * rows, rn = (int64_t)std::max(rw[k], 1) * rows;
+    const int64_t on = (int64_t)std::max(ow[k], 1) * rows;
+    const int64_t rn = (int64_t)(std::max(rw[k], 1) + 1) * rows;  // one slot to spare (k_orv)
     const int64_t bn = std::max<int64_t>(32 * rn, 4 * (int64_t)std::max(w[k], 1) * rows);
     if (on > L.ocap) {
       (void)dfree(L.oj); (void)dfree(L.orv);
@@ -926,7 +933,7 @@ int walk_cells(a2c_fe_ctx* c, double rc, Ell* L5, bool halves, int hm[16], unsig
       const Ell& L = L5[w];
       if (L.rows == 0) continue;
       hipLaunchKernelGGL(k_split, dim3((L.rows + TB - 1) / TB), dim3(TB), 0, c->stream, L, s_sp[w] * npd,
-                         j_sp[w] * npd);
+                         j_sp[w] * npd, j_sp[w] ? nh : npd);
       A2C_HIP(c, hipGetLastError());
     }
     if (int rc2 = reverse_slots(c, L5)) return rc2;
@@ -1048,7 +1055,7 @@ int refresh(a2c_fe_ctx* c, bool check, int hm[16], unsigned long long ht[5], dou
     if (S.rows == 0) continue;
     if (S.width == 0) continue;
     hipLaunchKernelGGL(k_orv_skin, dim3((S.rows + 255) / 256, S.width), dim3(256), 0, c->stream, S,
-                       c->nb_sup[partner[k]], c->ell[k]);
+                       c->nb_sup[partner[k]], c->ell[k], c->nb_sup[partner[k]].width);
     A2C_HIP(c, hipGetLastError());
   }
   std::vector<unsigned char> hb(MISC_BBOX);
