@@ -303,8 +303,7 @@ def lattice(n, a=3.89, seed=1, lattice_id=0, disp_std=0.02, sigma=(0.10, 0.10),
 
 
 def eam_tables64():
-    """FP64 polynomial tables of the FP64 pair-owner passes: (exp, pd) with
-    exp an array (3, 100, 10) for f_H, phi_PdH, phi_H (degree 8, one pad) and
+    """The EAM functions as FP64 polynomial tables in r: (exp, pd) with exp an array (3, 100, 10) for f_H, phi_PdH, phi_H (degree 8, one pad) and
     pd an array (2, 100, 12) for f_Pd, phi_Pd (degree 11); interval k is
     [1 + 0.05 k, 1 + 0.05 (k+1)), value sum_j c_j u^j, u = (r - 1)/0.05 - k."""
     n = lib.a2c_eam_tables64(None, 0)
@@ -314,7 +313,7 @@ def eam_tables64():
 
 
 def eam_tables():
-    """FP32 cubic tables of the mixed path: array (5, NT, 4); table order
+    """The EAM functions as FP32 cubic tables in r: array (5, NT, 4); table order
     f_Pd, f_H, phi_Pd, phi_PdH, phi_H; NT intervals of h = 5/NT A cover
     [1, 6) A, interval k being [1 + h k, 1 + h (k+1))."""
     n = lib.a2c_eam_tables(None, 0)

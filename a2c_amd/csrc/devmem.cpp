@@ -184,7 +184,7 @@ hipError_t device_tables(int device, DeviceTables* out) {
     std::vector<double> t64;
     host_tables(t32);
     host_tables_s(t32);
-    host_tables64(t64);
+    host_tables64_s(t64);
     DeviceTables d;
     hipError_t e = hipMalloc(&d.t32, sizeof(float4) * t32.size());
     if (e == hipSuccess) e = hipMalloc(&d.t64, sizeof(double) * t64.size());

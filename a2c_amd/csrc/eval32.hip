@@ -27,6 +27,7 @@
 
 #include "eam64.hpp"
 #include "fe_internal.hpp"
+#include "pair_rows.hpp"
 
 namespace a2c {
 namespace {
@@ -122,18 +123,9 @@ __device__ __forceinline__ float fH_exp(float r) {
   const float v = FH_C * __builtin_amdgcn_exp2f(e) * fmaf(el, LN2F, 1.0f);
   return r >= R0 ? v : __builtin_nanf("");
 }
-struct Site {
-  double q[3];
-  double s;
-};
 __device__ __forceinline__ Site load_site(const double* __restrict__ X, int s) {
   const double4 v = *reinterpret_cast<const double4*>(X + 4 * (size_t)s);
   return {{v.x, v.y, v.z}, v.w};
-}
-__device__ __forceinline__ Site load_row(const A2C_GLOBAL double2* __restrict__ qxy,
-                                         const A2C_GLOBAL double2* __restrict__ qzs, int p) {
-  const double2 a = qxy[p], b = qzs[p];
-  return {{a.x, a.y, b.x}, b.y};
 }
 // d = q_i - image(q_j) in FP64, rounded to FP32 (geometry held in registers)
 __device__ __forceinline__ void pair_vec32(const Image& g, const Site& a, const Site& b, float d[3]) {
@@ -609,54 +601,6 @@ __device__ __forceinline__ void pair_dens(const float4* tab, const float d[3], f
   }
 }
 
-// Owned pairs of one list of one row, K lanes per row.  Software pipeline: at
-// a pair's turn the state of the next one and the index and slot of the one
-// after it are requested, then the pair is evaluated and its share stored.
-// Loads and stores complete in order on one counter, so a load requested
-// after a store cannot be waited for without waiting for the store to reach
-// memory; requested one pair earlier, every load is older than the stores
-// still in flight.  (Requested in the pair's own turn, the waits for the
-// stores added 100 us to k_grad_own at 40^3 cells.)  geom(b) returns the pair's
-// geometry; eval(geometry, F'_j, w_j, neighbor row, received slot) the rest;
-// w_j: the occupancy of an H neighbor.
-template <bool NB_H, bool WITH_F, class Geom, class Eval>
-__device__ __forceinline__ void owned_pairs(const Ell& L, const OwnerLane& ln, int K, int off,
-                                            const A2C_GLOBAL double2* qxy, const A2C_GLOBAL double2* qzs,
-                                            const A2C_GLOBAL float2* aux, const A2C_GLOBAL double* w, Geom geom,
-                                            Eval eval) {
-  const size_t rows = L.rows, first = (size_t)ln.ph * rows + ln.row, step = (size_t)K * rows;
-  const A2C_GLOBAL int32_t* __restrict__ oj = gmem((const int32_t*)L.oj) + first;
-  const A2C_GLOBAL int32_t* __restrict__ orv = gmem((const int32_t*)L.orv) + first;
-  qxy += off;
-  qzs += off;
-  aux += off;
-  const int n = gmem((const int32_t*)L.ocnt)[ln.row];
-  int t = ln.ph;
-  if (t >= n) return;
-  size_t e = t + K < n ? step : 0;  // past the row's end its last entry is requested again: no branch around
-                                    // a load, or the waits behind it cover everything outstanding
-  int j1 = oj[0], r1 = orv[0], j2 = oj[e], r2 = orv[e];
-  Site b = load_row(qxy, qzs, j1);
-  float F = WITH_F ? aux[j1].x : 0.0f;
-  double wj = NB_H ? w[j1] : 1.0;
-  __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0): the loop's own waits then count only what the loop requests
-  do {
-    const auto g = geom(b);
-    const int jc = j1, rc = r1;
-    const float Fc = F;
-    const double wc = wj;
-    j1 = j2;
-    r1 = r2;
-    b = load_row(qxy, qzs, j1);
-    if (WITH_F) F = aux[j1].x;
-    if (NB_H) wj = w[j1];
-    e += t + 2 * K < n ? step : 0;
-    j2 = oj[e];
-    r2 = orv[e];
-    eval(g, Fc, wc, jc, rc);
-    t += K;
-  } while (t < n);
-}
 struct Pair32 {
   float d[3], bs;
 };
@@ -669,9 +613,8 @@ __device__ __forceinline__ void dens_list(const float4* tab, const LatDev& S, co
   A2C_GLOBAL float* __restrict__ prb = gmem(reinterpret_cast<float*>(P.rbuf));
   const size_t prows = P.rows;
   const float as = (float)a.s;
-  owned_pairs<NB_H, false>(
-      L, ln, S.kl32, NB_H ? S.npd : 0, gmem((const double2*)S.qxy), gmem((const double2*)S.qzs),
-      gmem((const float2*)S.aux), gmem((const double*)S.xrow),
+  owned_pairs<NB_H>(
+      L, ln, S.kl32, S, [](int) { return 0.0f; },
       [&](const Site& b) {
         Pair32 p;
         pair_vec32(img, a, b, p.d);
@@ -699,7 +642,8 @@ __global__ __launch_bounds__(TB) __attribute__((amdgpu_waves_per_eu(6))) void k_
   const int w = xcd_block();
   const LatDev& S = lats[ob2l[w]];
   if (S.rule != RULE) return;  // whole workgroup: the other rule's instance serves this lattice
-  stage_tables(tab, gtab + S_BASE + S_FPD * SNT, SNT);
+  stage16(tab, gtab + S_BASE + S_FPD * SNT, SNT);
+  __syncthreads();
   const int K = S.kl32;
   const OwnerLane ln(S, w - S.owg0_32, K);
   if (ln.row >= ln.rows) return;  // whole lane groups
@@ -943,9 +887,9 @@ __device__ __forceinline__ void grad_list(const float4* tab, const LatDev& S, co
   A2C_GLOBAL float4* __restrict__ prb = gmem(reinterpret_cast<float4*>(P.rbuf));
   const size_t prows = P.rows;
   const float as = (float)a.s;
-  owned_pairs<NB_H, true>(
-      L, ln, S.kl32, NB_H ? S.npd : 0, gmem((const double2*)S.qxy), gmem((const double2*)S.qzs),
-      gmem((const float2*)S.aux), gmem((const double*)S.xrow),
+  const A2C_GLOBAL float2* aux = gmem((const float2*)S.aux) + (NB_H ? S.npd : 0);
+  owned_pairs<NB_H>(
+      L, ln, S.kl32, S, [=](int j) { return aux[j].x; },
       [&](const Site& b) {
         Pair32 p;
         pair_vec32(img, a, b, p.d);
@@ -977,7 +921,8 @@ template <int RULE, int TBO>
 __global__ __launch_bounds__(TBO) __attribute__((amdgpu_waves_per_eu(TBO / 128))) void k_grad_own(
     const LatDev* __restrict__ lats, const int32_t* __restrict__ ob2l, int nblk, const float4* __restrict__ gtab) {
   __shared__ float4 tab[NGTAB * SNT];
-  stage_tables(tab, gtab + S_BASE + S_DFPD * SNT, NGTAB * SNT);
+  stage16(tab, gtab + S_BASE + S_DFPD * SNT, NGTAB * SNT);
+  __syncthreads();
   const int w = xcd_block() * (TBO / TB) + __builtin_amdgcn_readfirstlane(threadIdx.x / TB);
   if (w >= nblk) return;
   const LatDev& S = lats[ob2l[w]];

@@ -10,15 +10,9 @@
 // Analytic mode evaluates each unordered pair once (k_dens_own64 ->
 // k_dens_recv64 -> k_grad_own64 -> k_grad_recv64): the pair's owner computes
 // both ends' shares and writes the partner's share into the partner's
-// received slot, as the mixed path does.  These two owner kernels take EAM
-// functions from FP64 polynomial tables in LDS (on 0.05 A intervals,
-// interpolating the long-double closed forms): the exponential functions
-// (f_H, phi_PdH, phi_H) at degree 8, within 1e-13 of the closed forms in
-// value and slope, instead of three FP64 exp per quadrature point; the Pd
-// product polynomials f_Pd (density pass) and phi_Pd (gradient pass) at
-// degree 11, within the ~2e-11 rounding noise of the FP64 evaluation of
-// those polynomials themselves.  f_Pd' keeps its closed form.  1/|r| comes
-// from the hardware estimate refined by two Newton steps.  FD mode keeps the per-site
+// received slot, as the mixed path does.  These two owner kernels take the EAM
+// functions from FP64 polynomial tables in LDS, built from the long-double closed
+// forms (see "pair-once").  FD mode keeps the per-site
 // full-list loop nest of the reference (every pair from both ends), since
 // its derivatives are the reference's central differences per site.
 //
@@ -41,6 +35,7 @@
 
 #include "eam64.hpp"
 #include "fe_internal.hpp"
+#include "pair_rows.hpp"
 
 namespace a2c {
 namespace {
@@ -54,11 +49,6 @@ constexpr int GH3 = A2C_QUAD_GH3;
 // sqrt(6) short of d/dsigma; the Gauss-Hermite sums are complete.
 template <int RULE> constexpr double rule_qw() { return RULE == GH3 ? 1.0 : QW; }
 template <int RULE> constexpr double rule_sq() { return RULE == GH3 ? 1.0 : SQ6; }
-
-struct Site {
-  double q[3];
-  double s;
-};
 
 __device__ __forceinline__ Site load_site(const double* __restrict__ X, int s) {
   const double4 v = *reinterpret_cast<const double4*>(X + 4 * (size_t)s);
@@ -81,82 +71,6 @@ __device__ __forceinline__ void pair_vec(const LatDev& S, const Site& a, const S
 __device__ __forceinline__ void pair_vec(const Image& g, const Site& a, const Site& b, double d[3]) {
   image_vec(g, a.q, b.q, d);
 }
-__device__ __forceinline__ Site load_row(const A2C_GLOBAL double2* __restrict__ qxy,
-                                         const A2C_GLOBAL double2* __restrict__ qzs, int p) {
-  const double2 a = qxy[p], b = qzs[p];
-  return {{a.x, a.y, b.x}, b.y};
-}
-
-// ---------------------------------------------------------------- FP64 tables
-// Position of r in the tables: interval k, local coordinate u = (r - 1)/0.05 - k;
-// `in` is false outside [1, 6) A, where the closed forms are evaluated.
-struct Tpos {
-  int k;
-  double u;
-  bool in;
-};
-__device__ __forceinline__ Tpos tpos64(double r) {
-  const double x = fma(r, 20.0, -20.0);
-  Tpos p;
-  p.in = x >= 0.0 && x < (double)T64_N;
-  p.k = p.in ? (int)x : 0;
-  p.u = x - (double)p.k;
-  return p;
-}
-__device__ __forceinline__ double tab64_v(const double* c, double u) {
-  double v = c[T64_D];
-#pragma unroll
-  for (int j = T64_D - 1; j >= 0; --j) v = fma(v, u, c[j]);
-  return v;
-}
-__device__ __forceinline__ eam::VD tab64_vd(const double* c, double u) {
-  double v = c[T64_D], d = 0.0;
-#pragma unroll
-  for (int j = T64_D - 1; j >= 0; --j) {
-    d = fma(d, u, v);
-    v = fma(v, u, c[j]);
-  }
-  return {v, 20.0 * d};  // d/dr = 20 d/du
-}
-__device__ __forceinline__ const double* trow(const double* t, int f, int k) {
-  return t + ((size_t)f * T64_N + k) * T64_P;
-}
-// rows of the Pd polynomials (second part of the tables)
-__device__ __forceinline__ const double* qrow(const double* t, int f, int k) {
-  return t + T64_PART1 + ((size_t)f * T64_N + k) * T64Q_P;
-}
-template <int D>
-__device__ __forceinline__ double tabq_v(const double* c, double u) {
-  double v = c[D];
-#pragma unroll
-  for (int j = D - 1; j >= 0; --j) v = fma(v, u, c[j]);
-  return v;
-}
-template <int D>
-__device__ __forceinline__ eam::VD tabq_vd(const double* c, double u) {
-  double v = c[D], d = 0.0;
-#pragma unroll
-  for (int j = D - 1; j >= 0; --j) {
-    d = fma(d, u, v);
-    v = fma(v, u, c[j]);
-  }
-  return {v, 20.0 * d};
-}
-__device__ __forceinline__ void stage64(double* lds, const double* __restrict__ g, int n) {
-  for (int i = threadIdx.x; i < n; i += blockDim.x) lds[i] = g[i];
-  __syncthreads();
-}
-// 1/sqrt(x) for x in the normal range: the hardware estimate, then two steps
-// of Newton's iteration y <- y (3 - x y^2) / 2 (quadratic convergence; the
-// result is within a few ulp).
-__device__ __forceinline__ double rsqrt_nr(double x) {
-  double y = __builtin_amdgcn_rsq(x);
-  const double h = 0.5 * x;
-  y = y * fma(-h * y, y, 1.5);
-  y = y * fma(-h * y, y, 1.5);
-  return y;
-}
-
 template <int DM>
 __device__ __forceinline__ double dF(bool pd, double rho, double eps) {
   if (DM == A2C_DERIV_FD) {
@@ -284,46 +198,6 @@ __device__ __forceinline__ void pair_point(double r, double Fi, double Fj, doubl
   }
 }
 
-// pair_point (analytic) with the exponential functions from the tables t64;
-// `out` is set when r lies outside them (the caller then redoes the pair with
-// the closed forms; the values returned here are discarded)
-template <int KIND>
-__device__ __forceinline__ void pair_point_tab(double r, double Fi, double Fj, const double* t64, double& phi,
-                                               double& c, bool& out) {
-  const Tpos p = tpos64(r);
-  out |= !p.in;
-  // f_Pd' stays a closed form here: a second 96-byte row per point makes the
-  // pass LDS-bound (measured: 1.83 ms instead of 1.45 ms at 512,000 sites),
-  // while phi_Pd from the table keeps the pair energy free of the FP64
-  // rounding noise of the product polynomial (the relaxation endgame then
-  // needs ~20% fewer FP64 evaluations).
-  if (KIND == 0) {
-    const eam::VD f = eam::f_Pd_vd(r);
-    const eam::VD ph = tabq_vd<T64Q_D>(qrow(t64, T64Q_PHPD, p.k), p.u);
-    phi = ph.v;
-    c = (Fi + Fj) * f.d + ph.d;
-    return;
-  }
-  const eam::VD h = tab64_vd(trow(t64, T64_FH, p.k), p.u);
-  const eam::VD ph = tab64_vd(trow(t64, KIND == 3 ? T64_PHH : T64_PHPDH, p.k), p.u);
-  phi = ph.v;
-  if (KIND == 3) {
-    c = (Fi + Fj) * h.d + ph.d;
-  } else {
-    const eam::VD f = eam::f_Pd_vd(r);
-    c = (KIND == 1) ? Fi * h.d + Fj * f.d + ph.d : Fi * f.d + Fj * h.d + ph.d;
-  }
-}
-// f_H and f_Pd from the tables (values); closed forms outside [1, 6) A
-__device__ __forceinline__ double f_H_tab(double r, const double* t64) {
-  const Tpos p = tpos64(r);
-  return p.in ? tab64_v(trow(t64, T64_FH, p.k), p.u) : eam::f_H(r);
-}
-__device__ __forceinline__ double f_Pd_tab(double r, const double* t64) {
-  const Tpos p = tpos64(r);
-  return p.in ? tabq_v<T64Q_D>(qrow(t64, T64Q_FPD, p.k), p.u) : eam::f_Pd(r);
-}
-
 // Accumulate one neighbor pair: energy (phi summed over points), q-gradient
 // and sigma-gradient (12-point rule: r . xi1 is nonzero only on the six
 // points of site i; Gauss-Hermite rule: sum of w (c/|r|) (r . z) sigma_i/s).
@@ -445,93 +319,342 @@ __global__ __launch_bounds__(TB) void k_grad64(const LatDev* __restrict__ lats, 
 }
 
 // ================================================================ pair-once
-__device__ __forceinline__ const Ell& list_of(const LatDev& S, int list) {
-  return list == 0 ? S.pdpd : (list == 1 ? S.pdh : (list == 2 ? S.hpd : S.hh));
+// The nodes of a pair one at a time, for the pairs that leave the tables:
+// |r| of node k, its displacement z and its weight w (1 in the 12-point rule).
+template <int RULE>
+struct Closed {
+  static constexpr int N = RULE == GH3 ? 27 : 12;
+  double d[3], ai, aj, sd;
+  __device__ __forceinline__ Closed(const double* dd, double si, double sj)
+      : d{dd[0], dd[1], dd[2]}, ai(SQ6 * si), aj(SQ6 * sj), sd(sqrt(fma(si, si, sj * sj))) {}
+  __device__ __forceinline__ double node(int k, double z[3], double& w) const {
+    if (RULE == GH3) {
+      gh_node(k, z, w);
+#pragma unroll
+      for (int c = 0; c < 3; ++c) z[c] *= sd;
+    } else {
+      w = 1.0;
+      const int ax = (k >> 1) % 3;
+      const double a = (k & 1 ? -1.0 : 1.0) * (k < 6 ? ai : -aj);
+#pragma unroll
+      for (int c = 0; c < 3; ++c) z[c] = c == ax ? a : 0.0;
+    }
+    const double r0 = d[0] + z[0], r1 = d[1] + z[1], r2 = d[2] + z[2];
+    return sqrt(r0 * r0 + r1 * r1 + r2 * r2);
+  }
+};
+
+// The owner passes read the EAM functions from polynomial tables on a uniform
+// grid in s = |r|^2 (a node's coordinate is one addition, and dE/ds = (dE/dr) /
+// (2 |r|) is what the gradient needs: no square root per node).  h = 0.5025 / 12
+// puts the switch radii 5.0 and 5.05 A on grid nodes (25 and 25.5025 A^2; 5.35 A
+// joins two forms of the same function); the rows reach past 36 A^2.  Each row is
+// a polynomial in u in [0, 1) of six doubles: f_Pd and its slope interpolated at
+// the Chebyshev points, the pair functions as the integral of the interpolant of
+// their slope, so that value and slope belong together.  Slopes are within
+// 1e-12 of the closed forms at every distance that occurs.  That takes degree 5
+// for the slope of phi_Pd, whose part 2 0.251546 f_Pd falls as e^{-51.6 (r - 5)}
+// between 5.0 and 5.05 A: its two highest coefficients, at most 1e-4 of the
+// slope, share the sixth double as FP32 (rounding 1e-12).  Four functions on
+// this grid fill the 160 KB of LDS (one workgroup per CU); every row gathered
+// costs the CU's LDS ~30 clocks per wave.  f_H =
+// 11.0025 exp(-1.30927 |r|) is computed instead (exp2 by a 256-entry table and a
+// degree-4 polynomial): ~25 FP64 instructions on four SIMDs cost no more than a
+// row, and the two pipes work side by side.
+constexpr double SH = 0.5025 / 12.0, S0 = 25.5025 - 587 * SH, SINV = 1.0 / SH, SB = -S0 / SH;
+constexpr double SLO = 1.0, SHI = 36.0;  // nodes the tables serve: [1, 6) A
+constexpr int SNT = 839, SP = 6;         // rows, doubles per row
+static_assert(587 * SH < 24.5815 && S0 < 1.0 && S0 + (SNT - 1) * SH > 36.0, "the grid covers [1, 36] A^2");
+enum { S_FPD = 0, S_DFPD = 1, S_PHPD = 2, S_PHPDH = 3, S_PHH = 4, NSTAB = 5 };
+// phi_PdH has its rows in r instead, RH apart from R0 on: e^{-4.8 r} is steepest
+// at the Pd-H distances, where steps in s are the longest in r (slope 1e-10 off
+// at 1.6 A), and a Pd-H node has r at hand from f_H.
+constexpr double RH = 1.0 / 160.0, RINV = 160.0, R0 = 156.0 / 160.0;
+static_assert(R0 + (SNT - 1) * RH > 6.0, "the grid covers [1, 6] A");
+constexpr int S_ROWS = SNT * SP;                 // doubles per function
+constexpr int EXPN = 256;                        // 2^(i / 256)
+constexpr int S_EXP = NSTAB * S_ROWS, S_SIZE = S_EXP + EXPN;
+enum { G_DFPD = 0, G_PHPD = 1, G_PHPDH = 2, G_PHH = 3, NGTAB = 4 };  // the gradient pass's order in LDS
+
+struct SPos {
+  int k;
+  double u;
+};
+__device__ __forceinline__ SPos s_pos(double x) { return {(int)x, __builtin_amdgcn_fract(x)}; }
+__device__ __forceinline__ double s_of(double x) { return fma(x, SH, S0); }
+__device__ __forceinline__ const double* s_row(const double* tab, int f, int k) {
+  return tab + f * S_ROWS + __umul24(k, SP);
 }
-// partner list: PdPd<->PdPd, PdH<->HPd, HH<->HH
-__device__ __forceinline__ const Ell& partner_list(const LatDev& S, int list) {
-  return list == 0 ? S.pdpd : (list == 1 ? S.hpd : (list == 2 ? S.pdh : S.hh));
+template <int D>
+__device__ __forceinline__ double poly(const double* c, double u) {
+  double v = c[D];
+#pragma unroll
+  for (int j = D - 1; j >= 0; --j) v = fma(v, u, c[j]);
+  return v;
+}
+// value and d/du
+__device__ __forceinline__ void poly_vd(const double* c, double u, double& v, double& d) {
+  v = fma(c[5], u, c[4]);
+  d = fma(c[5], u, v);
+#pragma unroll
+  for (int j = 3; j >= 1; --j) {
+    v = fma(v, u, c[j]);
+    d = fma(d, u, v);
+  }
+  v = fma(v, u, c[0]);
+}
+// the same for a degree-6 row whose last two coefficients share a double (phi_Pd)
+__device__ __forceinline__ void poly6_vd(const double* c, double u, double& v, double& d) {
+  const double2 c45 = *reinterpret_cast<const double2*>(c + 4);  // one 16-byte read
+  const double hy = __int_as_float(__double2hiint(c45.y));
+  v = fma(hy, u, (double)__int_as_float(__double2loint(c45.y)));
+  d = fma(hy, u, v);
+  v = fma(v, u, c45.x);
+  d = fma(d, u, v);
+#pragma unroll
+  for (int j = 3; j >= 1; --j) {
+    v = fma(v, u, c[j]);
+    d = fma(d, u, v);
+  }
+  v = fma(v, u, c[0]);
+}
+// 1/sqrt(x): the hardware estimate y (relative error below 2^-20), then one
+// step of y <- y (1 + e/2 + 3 e^2 / 8), e = 1 - x y^2 (third order).
+__device__ __forceinline__ double rsqrt3(double x) {
+  const double y = __builtin_amdgcn_rsq(x);
+  const double e = fma(-(x * y), y, 1.0);
+  return fma(y * e, fma(e, 0.375, 0.5), y);
+}
+// f_H / 11.0025 = 2^(K r) at s = r^2, r and 1/r: n = rint(256 K r) picks 2^(n/256)
+// from the table, the remainder f in [-1/2, 1/2] goes through the series of
+// 2^(f/256) (next term 4e-17).
+__device__ __forceinline__ double fH_s(const double* exptab, double s, double& r, double& ri) {
+  constexpr double K = -1.30927 * 1.4426950408889634074 * EXPN, MAGIC = 6755399441055744.0;
+  constexpr double L1 = 0.69314718055994530942 / EXPN;
+  ri = rsqrt3(s);
+  r = s * ri;
+  const double t = fma(r, K, MAGIC);
+  const int n = (int)(unsigned)__double_as_longlong(t);
+  const double f = fma(r, K, -(t - MAGIC));
+  const double p = f * fma(f, fma(f, fma(f, L1 * L1 * L1 * L1 / 24.0, L1 * L1 * L1 / 6.0), L1 * L1 / 2.0), L1);
+  const double T = ldexp(exptab[n & (EXPN - 1)], n >> 8);
+  return fma(T, p, T);
 }
 
-template <int RULE>
-__global__ __launch_bounds__(TB) void k_dens_own64(const LatDev* __restrict__ lats, const int32_t* __restrict__ ob2l,
-                                                   const double* __restrict__ gtab64) {
-  // the table layout with only the rows this pass reads staged: f_H (part
-  // one, first function) and f_Pd (part two, first function)
-  __shared__ __align__(16) double t64[T64_PART1 + T64_N * T64Q_P];
-  const int w = xcd_block();
-  const LatDev& S = lats[ob2l[w]];
-  if (S.rule != RULE) return;
-  for (int i = threadIdx.x; i < T64_N * T64_P; i += blockDim.x) t64[i] = gtab64[(size_t)T64_FH * T64_N * T64_P + i];
-  stage64(t64 + T64_PART1, gtab64 + T64_PART1 + (size_t)T64Q_FPD * T64_N * T64Q_P, T64_N * T64Q_P);
-  const int K = S.kl64;  // lanes per site: lane ph takes owned slots ph, ph + K, ...
-  const OwnerLane ln(S, w - S.owg0_64, K);
-  if (ln.row >= ln.rows) return;  // whole lane groups
-  const int npd = S.npd, ph = ln.ph, row = ln.row;
-  const bool pd = ln.pd;
-  const int s = pd ? row : npd + row;
-  // everything the pair loops use, out of the descriptor and into registers
-  const A2C_GLOBAL double2* __restrict__ qxy = gmem((const double2*)S.qxy);
-  const A2C_GLOBAL double2* __restrict__ qzs = gmem((const double2*)S.qzs);
-  const A2C_GLOBAL double* __restrict__ xo = gmem((const double*)S.xrow);
-  const Image img = image_of(S);
-  const Site a = load_row(qxy, qzs, s);
-  const double ai = SQ6 * a.s;
-  const double wme = pd ? 1.0 : xo[row];  // shares leave weighted by the sender's occupancy
-  double rho = 0.0;
+// Table coordinates of one pair: 12-point rule (site e's nodes have
+// x = xb +- g d_c with g = 2 a / h, see pair_both) and Gauss-Hermite rule
+// (x = x0 + n1 |a|^2 + a . t).  inside(): every node lies in [1, 6) A; written in
+// explicit fma, so that the passes that ask get the same answer.
+struct Nodes12 {
+  double xi, xj, gi, gj, lo, hi;
+  __device__ __forceinline__ Nodes12(const double d[3], double ai, double aj) {
+    const double D2 = fma(d[0], d[0], fma(d[1], d[1], d[2] * d[2]));
+    const double bi = fma(ai, ai, D2), bj = fma(aj, aj, D2);
+    const double ei = 2.0 * ai, ej = 2.0 * aj;
+    const double m = fmax(fmax(fabs(d[0]), fabs(d[1])), fabs(d[2]));
+    lo = fmin(fma(-fabs(ei), m, bi), fma(-fabs(ej), m, bj));
+    hi = fmax(fma(fabs(ei), m, bi), fma(fabs(ej), m, bj));
+    xi = fma(bi, SINV, SB);
+    xj = fma(bj, SINV, SB);
+    gi = ei * SINV;
+    gj = ej * SINV;
+  }
+};
+struct Nodes27 {
+  double x0, n1, t[3], lo, hi;
+  __device__ __forceinline__ Nodes27(const double d[3], double sd) {
+    const double D2 = fma(d[0], d[0], fma(d[1], d[1], d[2] * d[2]));
+    const double s3 = 3.0 * sd * sd, tt = 2.0 * GH_Z * sd;
+    lo = hi = D2;
 #pragma unroll
-  for (int side = 0; side < 2; ++side) {  // Pd neighbors, then H neighbors
-    const int list = pd ? side : 2 + side;
-    const Ell& L = list_of(S, list);
-    const Ell& P = partner_list(S, list);
-    const A2C_GLOBAL int32_t* __restrict__ oj = gmem(L.oj);
-    const A2C_GLOBAL int32_t* __restrict__ orv = gmem(L.orv);
-    A2C_GLOBAL double* __restrict__ share = gmem(reinterpret_cast<double*>(P.rbuf));
-    const size_t rows = L.rows, prows = P.rows;
-    const int n = gmem(L.ocnt)[row];
-    for (int t = ph; t < n; t += K) {
-      const size_t e = (size_t)t * rows + row;
-      const int jl = oj[e];
-      const int rv = orv[e];
-      const Site b = load_row(qxy, qzs, side == 0 ? jl : npd + jl);
-      const double wj = side == 0 ? 1.0 : xo[jl];
-      double d[3];
-      pair_vec(img, a, b, d);
-      double mine = 0.0, theirs = 0.0;  // neighbor-species density at s, s-species density at the neighbor
-      if (RULE == GH3) {
-        const double sd = sqrt(a.s * a.s + b.s * b.s);
+    for (int c = 0; c < 3; ++c) {
+      lo += fmin(fma(-tt, fabs(d[c]), s3), 0.0);
+      hi += fma(tt, fabs(d[c]), s3);
+      t[c] = tt * SINV * d[c];
+    }
+    x0 = fma(D2, SINV, SB);
+    n1 = s3 * SINV;
+  }
+};
+__device__ __forceinline__ bool inside(double lo, double hi) { return lo >= SLO && hi < SHI; }
+
+// densities at one node inside the tables
+template <bool WANT_PD, bool WANT_H>
+__device__ __forceinline__ void node_dens(const double* tab, const double* exptab, double x, double& fpd, double& fh) {
+  if (WANT_PD) {
+    const SPos p = s_pos(x);
+    fpd = poly<5>(s_row(tab, 0, p.k), p.u);
+  }
+  if (WANT_H) {
+    double r, ri;
+    fh = fH_s(exptab, s_of(x), r, ri);
+  }
+}
+
+// Sums of f_Pd and f_H over the nodes of one pair in closed form.
+template <int RULE>
+__device__ __forceinline__ double2 closed_dens(const double d[3], double si, double sj) {
+  const Closed<RULE> q(d, si, sj);
+  double sp = 0.0, sh = 0.0;
 #pragma unroll 1
-        for (int k = 0; k < 27; ++k) {
-          double z[3], wk;
-          gh_node(k, z, wk);
-          const double r0 = d[0] + sd * z[0], r1 = d[1] + sd * z[1], r2 = d[2] + sd * z[2];
-          const double q2 = r0 * r0 + r1 * r1 + r2 * r2;
-          const double rn = q2 * rsqrt_nr(q2);
-          const double fpd = (side == 0 || pd) ? f_Pd_tab(rn, t64) : 0.0;
-          const double fh = (side == 1 || !pd) ? f_H_tab(rn, t64) : 0.0;
-          mine += wk * (side == 0 ? fpd : fh);
-          theirs += wk * (pd ? fpd : fh);
-        }
-      } else {
-        const double aj = SQ6 * b.s;
+  for (int k = 0; k < Closed<RULE>::N; ++k) {
+    double z[3], w;
+    const double r = q.node(k, z, w);
+    sp += w * eam::f_Pd(r);
+    sh += w * eam::f_H(r);
+  }
+  return make_double2(sp, sh);
+}
+
+// Sums over a pair's nodes of the density of the neighbor's species (mine) and
+// of this site's species (theirs); NB_H / ME_H: neighbor / this site is an H
+// site.  False, and zeros, if a node lies outside the tables.
+template <int RULE, bool NB_H, bool ME_H>
+__device__ __forceinline__ bool pair_dens(const double* tab, const double* exptab, const double d[3], double si,
+                                          double sj, double& mine, double& theirs) {
+  constexpr bool WP = !NB_H || !ME_H, WH = NB_H || ME_H;
+  double sp = 0.0, sh = 0.0;
+  bool in;
+  if (RULE == GH3) {
+    const double sd = sqrt(fma(si, si, sj * sj));
+    const Nodes27 q(d, sd);
+    in = inside(q.lo, q.hi);
+    if (in) {
 #pragma unroll 1
-        for (int p = 0; p < 12; ++p) {
-          double r[3];
-          point_r(p, d, ai, aj, r);
-          const double q2 = r[0] * r[0] + r[1] * r[1] + r[2] * r[2];
-          const double rn = q2 * rsqrt_nr(q2);
-          const double fpd = (side == 0 || pd) ? f_Pd_tab(rn, t64) : 0.0;
-          const double fh = (side == 1 || !pd) ? f_H_tab(rn, t64) : 0.0;
-          mine += side == 0 ? fpd : fh;
-          theirs += pd ? fpd : fh;
+      for (int a2 = -1; a2 <= 1; ++a2) {
+#pragma unroll 1
+        for (int a1 = -1; a1 <= 1; ++a1) {
+          const double xb = q.x0 + q.n1 * (double)(a2 * a2 + a1 * a1) + ((double)a2 * q.t[2] + (double)a1 * q.t[1]);
+          const double w = (a2 ? 1.0 : 4.0) * (a1 ? 1.0 : 4.0);
+          double pp = 0.0, ph = 0.0;
+#pragma unroll
+          for (int a0 = -1; a0 <= 1; ++a0) {
+            double fp = 0.0, fh = 0.0;
+            node_dens<WP, WH>(tab, exptab, a0 ? xb + q.n1 + a0 * q.t[0] : xb, fp, fh);
+            pp += a0 ? fp : 4.0 * fp;
+            ph += a0 ? fh : 4.0 * fh;
+          }
+          sp = fma(w, pp, sp);
+          sh = fma(w, ph, sh);
         }
       }
-      rho += wj * mine;
-      share[(size_t)rv * prows + jl] = wme * theirs;
+      sp *= 1.0 / 216.0;
+      sh *= 1.0 / 216.0;
+    }
+  } else {
+    const Nodes12 q(d, SQ6 * si, SQ6 * sj);
+    in = inside(q.lo, q.hi);
+    if (in) {
+#pragma unroll
+      for (int c = 0; c < 3; ++c) {
+        const double ti = q.gi * d[c], tj = q.gj * d[c];
+        const double x[4] = {q.xi + ti, q.xi - ti, q.xj - tj, q.xj + tj};
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+          double fp = 0.0, fh = 0.0;
+          node_dens<WP, WH>(tab, exptab, x[k], fp, fh);
+          if (WP) sp += fp;
+          if (WH) sh += fh;
+        }
+      }
     }
   }
+  sh *= 11.0025;
+  mine = NB_H ? sh : sp;
+  theirs = ME_H ? sh : sp;
+  return in;
+}
+
+// The pairs of a row that leave the tables, after its other pairs: the closed
+// forms hold ~190 registers and would cost every pair its waves if they stood
+// in its loop.
+template <bool NB_H, class Fn>
+__device__ __forceinline__ void far_pairs(const Ell& L, const OwnerLane& ln, int K, const LatDev& S, Fn fn) {
+  const int n = L.ocnt[ln.row];
+  for (int t = ln.ph; t < n; t += K) {
+    const size_t e = (size_t)t * L.rows + ln.row;
+    fn(L.oj[e], L.orv[e], (NB_H ? S.npd : 0) + L.oj[e]);
+  }
+}
+template <int RULE>
+__device__ __forceinline__ bool pair_inside(const double d[3], double si, double sj) {
+  if (RULE == GH3) {
+    const Nodes27 n(d, sqrt(fma(si, si, sj * sj)));
+    return inside(n.lo, n.hi);
+  }
+  const Nodes12 n(d, SQ6 * si, SQ6 * sj);
+  return inside(n.lo, n.hi);
+}
+
+struct Pair64 {
+  double d[3], s;
+};
+template <int RULE, bool NB_H, bool ME_H>
+__device__ __forceinline__ void dens_list(const double* tab, const double* exptab, const LatDev& S,
+                                          const OwnerLane& ln, const Site& a, const Image& img, double wme,
+                                          double& rho) {
+  const Ell& L = ME_H ? (NB_H ? S.hh : S.hpd) : (NB_H ? S.pdh : S.pdpd);
+  const Ell& P = ME_H ? (NB_H ? S.hh : S.pdh) : (NB_H ? S.hpd : S.pdpd);  // partner rows
+  A2C_GLOBAL double* __restrict__ share = gmem(reinterpret_cast<double*>(P.rbuf));
+  const size_t prows = P.rows;
+  bool far = false;
+  owned_pairs<NB_H>(
+      L, ln, S.kl64, S, [](int) { return 0.0f; },
+      [&](const Site& b) {
+        Pair64 p;
+        pair_vec(img, a, b, p.d);
+        p.s = b.s;
+        return p;
+      },
+      [&](const Pair64& p, float, double wj, int jl, int rv) {
+        double mine, theirs;
+        far |= !pair_dens<RULE, NB_H, ME_H>(tab, exptab, p.d, a.s, p.s, mine, theirs);
+        rho += wj * mine;
+        // shares leave weighted by the sender's occupancy
+        share[(size_t)rv * prows + jl] = ME_H ? wme * theirs : theirs;
+      });
+  if (far)
+    far_pairs<NB_H>(L, ln, S.kl64, S, [&](int jl, int rv, int j) {
+      const Site b = load_row(gmem((const double2*)S.qxy), gmem((const double2*)S.qzs), j);
+      double d[3];
+      pair_vec(img, a, b, d);
+      if (pair_inside<RULE>(d, a.s, b.s)) return;
+      const double2 v = closed_dens<RULE>(d, a.s, b.s);
+      rho += (NB_H ? S.xrow[jl] : 1.0) * (NB_H ? v.y : v.x);
+      share[(size_t)rv * prows + jl] = wme * (ME_H ? v.y : v.x);
+    });
+}
+
+// Bound by the LDS and the vector ALUs (40^3 cells: 60% and 75% busy): 654 us
+// with the tables in |r|, 276 us; Gauss-Hermite rule 1386 and 604 us.
+template <int RULE, int TBO>
+__global__ __launch_bounds__(TBO) __attribute__((amdgpu_waves_per_eu(4))) void k_dens_own64(
+    const LatDev* __restrict__ lats, const int32_t* __restrict__ ob2l, int nblk, const double* __restrict__ gtab) {
+  __shared__ __align__(16) double tab[S_ROWS + EXPN];  // f_Pd, 2^(i/256)
+  stage16(tab, gtab + S_FPD * S_ROWS, S_ROWS / 2);
+  stage16(tab + S_ROWS, gtab + S_EXP, EXPN / 2);
+  __syncthreads();
+  const int w = xcd_block() * (TBO / TB) + __builtin_amdgcn_readfirstlane(threadIdx.x / TB);
+  if (w >= nblk) return;
+  const LatDev& S = lats[ob2l[w]];
+  if (S.rule != RULE) return;  // the other rule's instance serves this lattice
+  const int K = S.kl64;
+  const OwnerLane ln(S, w - S.owg0_64, K);
+  if (ln.row >= ln.rows) return;  // whole lane groups
+  const Image img = image_of(S);
+  const int s = ln.pd ? ln.row : S.npd + ln.row;
+  const Site a = load_row(gmem((const double2*)S.qxy), gmem((const double2*)S.qzs), s);
+  double rho = 0.0;
+  if (ln.pd) {
+    dens_list<RULE, false, false>(tab, tab + S_ROWS, S, ln, a, img, 1.0, rho);
+    dens_list<RULE, true, false>(tab, tab + S_ROWS, S, ln, a, img, 1.0, rho);
+  } else {
+    const double wme = gmem((const double*)S.xrow)[ln.row];
+    dens_list<RULE, false, true>(tab, tab + S_ROWS, S, ln, a, img, wme, rho);
+    dens_list<RULE, true, true>(tab, tab + S_ROWS, S, ln, a, img, wme, rho);
+  }
   rho = site_sum(rho, K);
-  if (ph == 0) gmem(S.rho)[s] = rho;
+  if (ln.ph == 0) gmem(S.rho)[s] = rho;
 }
 
 __global__ __launch_bounds__(TB) void k_dens_recv64(const LatDev* __restrict__ lats, const int32_t* __restrict__ b2l) {
@@ -546,7 +669,7 @@ __global__ __launch_bounds__(TB) void k_dens_recv64(const LatDev* __restrict__ l
   double rho = S.rho[s];
 #pragma unroll
   for (int side = 0; side < 2; ++side) {
-    const Ell& L = list_of(S, pd ? side : 2 + side);
+    const Ell& L = pd ? (side ? S.pdh : S.pdpd) : (side ? S.hh : S.hpd);
     const int n = L.rcnt[row];
     // shares arrive weighted by their senders
     for_row_shares<RECV_RU_SCALAR>(gmem(reinterpret_cast<const double*>(L.rbuf)), L.rows, row, n, [&](double v) { rho += v; });
@@ -559,178 +682,269 @@ __global__ __launch_bounds__(TB) void k_dens_recv64(const LatDev* __restrict__ l
   S.emb[s] = xs * F.v;
 }
 
-// One owned pair: phi summed over the 12 points, the q-gradient g of site s
-// (the partner's is -g), and the sigma terms of both ends (site s: its own
-// six points; the partner: the six points that displace it, seen from its
-// side with r -> -r).
-template <int KIND, int RULE>
-__device__ __forceinline__ void pair_both_closed(const double d[3], double si, double sj, double Fi, double Fj,
-                                          double& pe, double g[3], double& gsi, double& gsj) {
-  pe = 0.0;
-  g[0] = g[1] = g[2] = 0.0;
-  gsi = gsj = 0.0;
-  if (RULE == GH3) {  // both ends move every node: dr/dsigma_k = z sigma_k / s
-    const double sd = sqrt(si * si + sj * sj);
-    double sz = 0.0;
-#pragma unroll 1
-    for (int k = 0; k < 27; ++k) {
-      double z[3], w;
-      gh_node(k, z, w);
-      const double r[3] = {d[0] + sd * z[0], d[1] + sd * z[1], d[2] + sd * z[2]};
-      const double q2 = r[0] * r[0] + r[1] * r[1] + r[2] * r[2];
-      const double ri = rsqrt_nr(q2);
-      double phi, c;
-      pair_point<A2C_DERIV_ANALYTIC, KIND>(q2 * ri, Fi, Fj, 0.0, phi, c);
-      pe += w * phi;
-      const double u = w * c * ri;
-      g[0] += u * r[0];
-      g[1] += u * r[1];
-      g[2] += u * r[2];
-      sz += u * (r[0] * z[0] + r[1] * z[1] + r[2] * z[2]);
+// One node inside the tables: the pair energy phi and cu = SH dE/ds, E = F'_i f_j
+// + F'_j f_i + phi.  FP multiplies f_Pd', FH f_H' / |r| (it carries FH_D).
+constexpr double FH_D = 0.5 * SH * -1.30927 * 11.0025;
+template <int KIND>
+__device__ __forceinline__ void node_coef(const double* tab, const double* exptab, double x, double FP, double FH,
+                                          double& phi, double& cu) {
+  const SPos p = s_pos(x);
+  if (KIND == 0) poly6_vd(s_row(tab, G_PHPD, p.k), p.u, phi, cu);
+  if (KIND == 3) poly_vd(s_row(tab, G_PHH, p.k), p.u, phi, cu);
+  if (KIND == 0) cu = fma(FP, poly<5>(s_row(tab, G_DFPD, p.k), p.u), cu);
+  if (KIND != 0) {
+    double r, ri;
+    const double fh = fH_s(exptab, s_of(x), r, ri);
+    if (KIND == 3) {
+      cu = fma(FH, fh * ri, cu);
+    } else {  // phi_PdH from its rows in r
+      const double y = fma(r, RINV, -156.0);
+      double d;
+      poly_vd(s_row(tab, G_PHPDH, (int)y), __builtin_amdgcn_fract(y), phi, d);
+      cu = fma(fma(FH, fh, (0.5 * SH * RINV) * d), ri, FP * poly<5>(s_row(tab, G_DFPD, p.k), p.u));
     }
-    gsi = sz * (si / sd);
-    gsj = sz * (sj / sd);
-    return;
-  }
-  const double ai = SQ6 * si, aj = SQ6 * sj;
-#pragma unroll 1  // rolled: the FP64 closed forms keep ~140 VGPRs live (3 waves per SIMD) instead of ~260 (1)
-  for (int p = 0; p < 12; ++p) {
-    double r[3];
-    point_r(p, d, ai, aj, r);
-    const double q2 = r[0] * r[0] + r[1] * r[1] + r[2] * r[2];
-    const double ri = rsqrt_nr(q2);
-    double phi, c;
-    pair_point<A2C_DERIV_ANALYTIC, KIND>(q2 * ri, Fi, Fj, 0.0, phi, c);
-    pe += phi;
-    const double u = c * ri;
-    g[0] += u * r[0];
-    g[1] += u * r[1];
-    g[2] += u * r[2];
-    const int ax = (p >> 1) % 3;
-    if (p < 6) gsi += ((p & 1) ? -u : u) * r[ax];
-    else gsj += ((p & 1) ? u : -u) * r[ax];
   }
 }
 
-template <int KIND, int RULE>
-__device__ __forceinline__ void pair_both(const double d[3], double si, double sj, double Fi, double Fj,
-                                          const double* t64, double& pe, double g[3], double& gsi, double& gsj) {
-  pe = 0.0;
-  g[0] = g[1] = g[2] = 0.0;
-  gsi = gsj = 0.0;
-  bool out = false;  // some point outside the tables' [1, 6) A
-  if (RULE == GH3) {  // both ends move every node: dr/dsigma_k = z sigma_k / s
-    const double sd = sqrt(si * si + sj * sj);
-    double sz = 0.0;
+struct PairSums {
+  double pe;        // sum of phi
+  double g[3];      // q-gradient of this site (the partner's is -g)
+  double gsi, gsj;  // sigma terms of both ends
+};
+// 12-point sums.  Site e's points are r = d +- a e_c with a = ai for the site
+// and -aj for its partner.  With u = 2 SINV cu = (dE/dr) / |r| per node, T_c the
+// difference of u between the two points of an axis, U_e their sum:
+//   q-gradient  sum u r = d (U_i + U_j) + sum_e a T,
+//   sigma terms d . T + a U (site i), its negative (partner).
+// One axis of one site (2 nodes) per trip, the components rotating through d0
+// and h2: more rows in flight would not fit the registers of 4 waves per SIMD.
+template <int KIND>
+__device__ __forceinline__ PairSums pair_sums12(const double* tab, const double* exptab, const Nodes12& n,
+                                                const double d[3], double ai, double aj, double FP, double FH) {
+  double pe = 0.0, su = 0.0, d0 = d[0], d1 = d[1], d2 = d[2], h0 = 0.0, h1 = 0.0, h2 = 0.0;
+  double a = ai, xb = n.xi, g = n.gi;
+  PairSums p;
 #pragma unroll 1
-    for (int k = 0; k < 27; ++k) {
-      double z[3], w;
-      gh_node(k, z, w);
-      const double r[3] = {d[0] + sd * z[0], d[1] + sd * z[1], d[2] + sd * z[2]};
-      const double q2 = r[0] * r[0] + r[1] * r[1] + r[2] * r[2];
-      const double ri = rsqrt_nr(q2);
-      double phi, c;
-      pair_point_tab<KIND>(q2 * ri, Fi, Fj, t64, phi, c, out);
-      pe += w * phi;
-      const double u = w * c * ri;
-      g[0] += u * r[0];
-      g[1] += u * r[1];
-      g[2] += u * r[2];
-      sz += u * (r[0] * z[0] + r[1] * z[1] + r[2] * z[2]);
+  for (int e = 0; e < 2; ++e) {
+    double ue = 0.0, se = 0.0;
+#pragma unroll 1
+    for (int c = 0; c < 3; ++c) {
+      const double t = g * d0;
+      double phi0, phi1, u0, u1;
+      node_coef<KIND>(tab, exptab, xb + t, FP, FH, phi0, u0);
+      node_coef<KIND>(tab, exptab, xb - t, FP, FH, phi1, u1);
+      pe += phi0 + phi1;
+      const double T = u0 - u1;
+      ue += u0 + u1;
+      se = fma(d0, T, se);
+      const double h = fma(a, T, h0), dt = d0;
+      h0 = h1;
+      h1 = h2;
+      h2 = h;
+      d0 = d1;
+      d1 = d2;
+      d2 = dt;
     }
-    gsi = sz * (si / sd);
-    gsj = sz * (sj / sd);
-    if (out) pair_both_closed<KIND, RULE>(d, si, sj, Fi, Fj, pe, g, gsi, gsj);
-    return;
+    su += ue;
+    p.gsj = -(2.0 * SINV) * fma(a, ue, se);
+    if (e == 0) p.gsi = -p.gsj;
+    a = -aj;
+    xb = n.xj;
+    g = -n.gj;
   }
-  const double ai = SQ6 * si, aj = SQ6 * sj;
-#pragma unroll 1  // rolled: the FP64 closed forms keep ~140 VGPRs live (3 waves per SIMD) instead of ~260 (1)
-  for (int p = 0; p < 12; ++p) {
-    double r[3];
-    point_r(p, d, ai, aj, r);
-    const double q2 = r[0] * r[0] + r[1] * r[1] + r[2] * r[2];
-    const double ri = rsqrt_nr(q2);
-    double phi, c;
-    pair_point_tab<KIND>(q2 * ri, Fi, Fj, t64, phi, c, out);
-    pe += phi;
-    const double u = c * ri;
-    g[0] += u * r[0];
-    g[1] += u * r[1];
-    g[2] += u * r[2];
-    const int ax = (p >> 1) % 3;
-    if (p < 6) gsi += ((p & 1) ? -u : u) * r[ax];
-    else gsj += ((p & 1) ? u : -u) * r[ax];
+  p.pe = pe;
+  p.g[0] = (2.0 * SINV) * fma(d[0], su, h0);
+  p.g[1] = (2.0 * SINV) * fma(d[1], su, h1);
+  p.g[2] = (2.0 * SINV) * fma(d[2], su, h2);
+  return p;
+}
+// Gauss-Hermite sums.  With u_k = w_k (dE/dr) / |r_k| and the node offsets a_k:
+// U = sum u, V = sum u a, Wn = sum u |a|^2;
+//   q-gradient  sum u r = d U + sqrt(3) s V,
+//   Sz = sum u (r . z) = sqrt(3) d . V + 3 s Wn,  d/dsigma_k = Sz sigma_k / s.
+// Weights 4 and 1 per axis, divided by 216 at the end; three nodes per trip.
+template <int KIND>
+__device__ __forceinline__ PairSums pair_sums27(const double* tab, const double* exptab, const Nodes27& q,
+                                                const double d[3], double sd, double si, double sj, double FP,
+                                                double FH) {
+  double pe = 0.0, U = 0.0, V0 = 0.0, V1 = 0.0, V2 = 0.0, Wn = 0.0;
+#pragma unroll 1
+  for (int a2 = -1; a2 <= 1; ++a2) {
+#pragma unroll 1
+    for (int a1 = -1; a1 <= 1; ++a1) {
+      const double n2 = (double)(a2 * a2 + a1 * a1);
+      const double xb = q.x0 + q.n1 * n2 + ((double)a2 * q.t[2] + (double)a1 * q.t[1]);
+      const double w = (a2 ? 1.0 : 4.0) * (a1 ? 1.0 : 4.0);
+      double f0, fm, fp, c0, cm, cp;
+      node_coef<KIND>(tab, exptab, xb, FP, FH, f0, c0);
+      node_coef<KIND>(tab, exptab, xb + q.n1 - q.t[0], FP, FH, fm, cm);
+      node_coef<KIND>(tab, exptab, xb + q.n1 + q.t[0], FP, FH, fp, cp);
+      pe = fma(w, fma(4.0, f0, fm + fp), pe);
+      const double e = cm + cp, u = w * fma(4.0, c0, e);
+      U += u;
+      V0 = fma(w, cp - cm, V0);
+      V1 = fma((double)a1, u, V1);
+      V2 = fma((double)a2, u, V2);
+      Wn = fma(w, e, fma(n2, u, Wn));
+    }
   }
-  if (out) pair_both_closed<KIND, RULE>(d, si, sj, Fi, Fj, pe, g, gsi, gsj);
+  constexpr double Q = 2.0 * SINV / 216.0;
+  const double sv = GH_Z * sd;
+  PairSums p;
+  p.pe = pe * (1.0 / 216.0);
+  p.g[0] = Q * fma(d[0], U, sv * V0);
+  p.g[1] = Q * fma(d[1], U, sv * V1);
+  p.g[2] = Q * fma(d[2], U, sv * V2);
+  const double sz = Q * fma(GH_Z, fma(d[0], V0, fma(d[1], V1, d[2] * V2)), 3.0 * sd * Wn);
+  p.gsi = sz * (si / sd);
+  p.gsj = sz * (sj / sd);
+  return p;
+}
+// One pair in closed form, node by node.
+template <int RULE, int KIND>
+__device__ __forceinline__ PairSums closed_sums(const double d[3], double si, double sj, double Fi, double Fj) {
+      const Closed<RULE> q(d, si, sj);
+      PairSums p{};
+      double sz = 0.0;
+  #pragma unroll 1
+      for (int k = 0; k < Closed<RULE>::N; ++k) {
+        double z[3], w, phi, c;
+        const double r = q.node(k, z, w);
+        pair_point<A2C_DERIV_ANALYTIC, KIND>(r, Fi, Fj, 0.0, phi, c);
+        p.pe += w * phi;
+        const double u = w * c / r;
+        double ro = 0.0;  // r . z
+  #pragma unroll
+        for (int x = 0; x < 3; ++x) {
+          const double rx = d[x] + z[x];
+          p.g[x] += u * rx;
+          ro += rx * z[x];
+        }
+        if (RULE == GH3) sz += u * ro;
+        else if (k < 6) p.gsi += u * ro / q.ai;
+        else p.gsj += u * ro / q.aj;
+      }
+      if (RULE == GH3) {  // z = s (node): d/dsigma_k = (sum u r . node) sigma_k / s
+        p.gsi = sz * si / (q.sd * q.sd);
+        p.gsj = sz * sj / (q.sd * q.sd);
+      }
+  return p;
+}
+// false, and zeros, if a node lies outside the tables
+template <int RULE, int KIND>
+__device__ __forceinline__ bool pair_both(const double* tab, const double* exptab, const double d[3], double si,
+                                          double sj, double Fi, double Fj, PairSums& p) {
+  const double FP = KIND == 0 ? Fi + Fj : (KIND == 1 ? Fj : Fi);           // F' of the H site multiplies f_Pd'
+  const double FH = FH_D * (KIND == 3 ? Fi + Fj : (KIND == 1 ? Fi : Fj));  // F' of the Pd site f_H'
+  bool in;
+  p = PairSums{};
+  if (RULE == GH3) {
+    const double sd = sqrt(fma(si, si, sj * sj));
+    const Nodes27 n(d, sd);
+    in = inside(n.lo, n.hi);
+    if (in) p = pair_sums27<KIND>(tab, exptab, n, d, sd, si, sj, FP, FH);
+  } else {
+    const double ai = SQ6 * si, aj = SQ6 * sj;
+    const Nodes12 n(d, ai, aj);
+    in = inside(n.lo, n.hi);
+    if (in) p = pair_sums12<KIND>(tab, exptab, n, d, ai, aj, FP, FH);
+  }
+  return in;
 }
 
-
-// 3 waves per SIMD (at most 168 VGPRs per lane)
-template <int RULE>
-__global__ __launch_bounds__(TB) __attribute__((amdgpu_waves_per_eu(3))) void k_grad_own64(
-    const LatDev* __restrict__ lats, const int32_t* __restrict__ ob2l, const double* __restrict__ gtab64) {
-  __shared__ __align__(16) double t64[T64_SIZE];
-  const int w = xcd_block();
-  const LatDev& S = lats[ob2l[w]];
-  if (S.rule != RULE) return;
-  stage64(t64, gtab64, T64_SIZE);
-  const int K = S.kl64;  // lanes per site: lane ph takes owned slots ph, ph + K, ...
-  const OwnerLane ln(S, w - S.owg0_64, K);
-  if (ln.row >= ln.rows) return;  // whole lane groups
-  const int npd = S.npd, ph = ln.ph, row = ln.row;
-  const bool pd = ln.pd;
-  const int s = pd ? row : npd + row;
-  // everything the pair loops use, out of the descriptor and into registers
-  const A2C_GLOBAL double2* __restrict__ qxy = gmem((const double2*)S.qxy);
-  const A2C_GLOBAL double2* __restrict__ qzs = gmem((const double2*)S.qzs);
-  const A2C_GLOBAL double* __restrict__ xo = gmem((const double*)S.xrow);
-  const A2C_GLOBAL double* __restrict__ Fp = gmem(S.Fp);
-  const Image img = image_of(S);
-  const Site a = load_row(qxy, qzs, s);
-  const double Fi = Fp[s];
-  const double wme = pd ? 1.0 : xo[row];  // shares leave weighted by the sender's occupancy
+struct Own {
   double e = 0.0, g0 = 0.0, g1 = 0.0, g2 = 0.0, gs = 0.0;
-#pragma unroll
-  for (int side = 0; side < 2; ++side) {
-    const int list = pd ? side : 2 + side;
-    const Ell& L = list_of(S, list);
-    const Ell& P = partner_list(S, list);
-    const A2C_GLOBAL int32_t* __restrict__ oj = gmem(L.oj);
-    const A2C_GLOBAL int32_t* __restrict__ orv = gmem(L.orv);
-    A2C_GLOBAL double4* __restrict__ share = gmem(reinterpret_cast<double4*>(P.rbuf));
-    const size_t rows = L.rows, prows = P.rows;
-    const int n = gmem(L.ocnt)[row];
-    const int off = side == 0 ? 0 : npd;  // site index of neighbor 0 of this list
-    for (int t = ph; t < n; t += K) {
-      // (no one-pair-ahead prefetch: an FP64 pair is long enough to cover its
-      // gathers, and the registers would push the kernel into spills)
-      const size_t ei = (size_t)t * rows + row;
-      const int jl = oj[ei];
-      const int rv = orv[ei];
-      const Site b = load_row(qxy, qzs, off + jl);
-      const double Fj = Fp[off + jl];
-      const double wj = side == 0 ? 1.0 : xo[jl];
+};
+template <int RULE, int KIND>
+__device__ __forceinline__ void grad_list(const double* tab, const double* exptab, const LatDev& S,
+                                          const OwnerLane& ln, const Site& a, double Fi, const Image& img, double wme,
+                                          Own& o) {
+  constexpr bool ME_H = KIND >= 2, NB_H = KIND & 1;
+  const Ell& L = ME_H ? (NB_H ? S.hh : S.hpd) : (NB_H ? S.pdh : S.pdpd);
+  const Ell& P = ME_H ? (NB_H ? S.hh : S.pdh) : (NB_H ? S.hpd : S.pdpd);  // partner rows
+  A2C_GLOBAL double4* __restrict__ share = gmem(reinterpret_cast<double4*>(P.rbuf));
+  const size_t prows = P.rows;
+  const A2C_GLOBAL double* Fp = gmem((const double*)S.Fp) + (NB_H ? S.npd : 0);
+  bool far = false;
+  owned_pairs<NB_H>(
+      L, ln, S.kl64, S, [=](int j) { return Fp[j]; },
+      [&](const Site& b) {
+        Pair64 p;
+        pair_vec(img, a, b, p.d);
+        p.s = b.s;
+        return p;
+      },
+      [&](const Pair64& q, double Fj, double wj, int jl, int rv) {
+        PairSums p;
+        far |= !pair_both<RULE, KIND>(tab, exptab, q.d, a.s, q.s, Fi, Fj, p);
+        o.e += wj * p.pe;
+        o.g0 += wj * p.g[0];
+        o.g1 += wj * p.g[1];
+        o.g2 += wj * p.g[2];
+        o.gs += wj * p.gsi;
+        // the partner's share leaves weighted by the sender's occupancy
+        const double w = ME_H ? wme : 1.0;
+        share[(size_t)rv * prows + jl] = make_double4(-w * p.g[0], -w * p.g[1], -w * p.g[2], w * p.gsj);
+      });
+  if (far)
+    far_pairs<NB_H>(L, ln, S.kl64, S, [&](int jl, int rv, int j) {
+      const Site b = load_row(gmem((const double2*)S.qxy), gmem((const double2*)S.qzs), j);
       double d[3];
       pair_vec(img, a, b, d);
-      double pe, pg[3], psi, psj;
-      if (list == 0) pair_both<0, RULE>(d, a.s, b.s, Fi, Fj, t64, pe, pg, psi, psj);
-      else if (list == 1) pair_both<1, RULE>(d, a.s, b.s, Fi, Fj, t64, pe, pg, psi, psj);
-      else if (list == 2) pair_both<2, RULE>(d, a.s, b.s, Fi, Fj, t64, pe, pg, psi, psj);
-      else pair_both<3, RULE>(d, a.s, b.s, Fi, Fj, t64, pe, pg, psi, psj);
-      e += wj * pe;
-      g0 += wj * pg[0]; g1 += wj * pg[1]; g2 += wj * pg[2];
-      gs += wj * psi;
-      share[(size_t)rv * prows + jl] = make_double4(-wme * pg[0], -wme * pg[1], -wme * pg[2], wme * psj);
-    }
+      if (pair_inside<RULE>(d, a.s, b.s)) return;
+      const PairSums p = closed_sums<RULE, KIND>(d, a.s, b.s, Fi, S.Fp[j]);
+      const double wj = NB_H ? S.xrow[jl] : 1.0;
+      o.e += wj * p.pe;
+      o.g0 += wj * p.g[0];
+      o.g1 += wj * p.g[1];
+      o.g2 += wj * p.g[2];
+      o.gs += wj * p.gsi;
+      share[(size_t)rv * prows + jl] = make_double4(-wme * p.g[0], -wme * p.g[1], -wme * p.g[2], wme * p.gsj);
+    });
+}
+
+// Bound by the LDS and the vector ALUs together (each busy 57% of the time at 2
+// waves per SIMD; 163 KB of tables leave one workgroup per CU, and 1024 lanes, 4
+// waves per SIMD, spill: 645 against 625 us).  40^3 cells: 1384 us before (degree
+// 8 / 11 tables in |r|, f_Pd' in closed form, two Newton steps per node, 153
+// instructions per node), 625 us; Gauss-Hermite rule 2920 and 1200 us.  f_H' from a
+// table, too, took 691 us.  Gradient error against 80-bit arithmetic (3^3 and 4^3
+// cells): 4e-12 to 1e-11 before, 3e-13 to 8e-13.
+template <int RULE, int TBO>
+__global__ __launch_bounds__(TBO) __attribute__((amdgpu_waves_per_eu(TBO / 256))) void k_grad_own64(
+    const LatDev* __restrict__ lats, const int32_t* __restrict__ ob2l, int nblk, const double* __restrict__ gtab) {
+  __shared__ __align__(16) double tab[NGTAB * S_ROWS + EXPN];
+  stage16(tab, gtab + S_DFPD * S_ROWS, (NGTAB * S_ROWS + EXPN) / 2);  // the exp2 table follows the functions
+  __syncthreads();
+  const int w = xcd_block() * (TBO / TB) + __builtin_amdgcn_readfirstlane(threadIdx.x / TB);
+  if (w >= nblk) return;
+  const LatDev& S = lats[ob2l[w]];
+  if (S.rule != RULE) return;  // the other rule's instance serves this lattice
+  const int K = S.kl64;
+  const OwnerLane ln(S, w - S.owg0_64, K);
+  if (ln.row >= ln.rows) return;  // whole lane groups
+  const double* exptab = tab + NGTAB * S_ROWS;
+  const Image img = image_of(S);
+  const int s = ln.pd ? ln.row : S.npd + ln.row;
+  const Site a = load_row(gmem((const double2*)S.qxy), gmem((const double2*)S.qzs), s);
+  const double Fi = gmem((const double*)S.Fp)[s];
+  Own o;
+  if (ln.pd) {
+    grad_list<RULE, 0>(tab, exptab, S, ln, a, Fi, img, 1.0, o);
+    grad_list<RULE, 1>(tab, exptab, S, ln, a, Fi, img, 1.0, o);
+  } else {
+    const double wme = gmem((const double*)S.xrow)[ln.row];
+    grad_list<RULE, 2>(tab, exptab, S, ln, a, Fi, img, wme, o);
+    grad_list<RULE, 3>(tab, exptab, S, ln, a, Fi, img, wme, o);
   }
-  e = site_sum(e, K);
-  g0 = site_sum(g0, K);
-  g1 = site_sum(g1, K);
-  g2 = site_sum(g2, K);
-  gs = site_sum(gs, K);
-  if (ph != 0) return;
-  gmem(S.gown)[s] = make_double4(g0, g1, g2, gs);
-  gmem(S.epair)[s] = e;
+  o.e = site_sum(o.e, K);
+  o.g0 = site_sum(o.g0, K);
+  o.g1 = site_sum(o.g1, K);
+  o.g2 = site_sum(o.g2, K);
+  o.gs = site_sum(o.gs, K);
+  if (ln.ph != 0) return;
+  gmem(S.gown)[s] = make_double4(o.g0, o.g1, o.g2, o.gs);
+  gmem(S.epair)[s] = o.e;
 }
 
 __global__ __launch_bounds__(TB) void k_grad_recv64(const LatDev* __restrict__ lats, const int32_t* __restrict__ b2l) {
@@ -751,7 +965,7 @@ __global__ __launch_bounds__(TB) void k_grad_recv64(const LatDev* __restrict__ l
     double g0 = own.x, g1 = own.y, g2 = own.z, gs = own.w;
 #pragma unroll
     for (int side = 0; side < 2; ++side) {
-      const Ell& L = list_of(S, pd ? side : 2 + side);
+      const Ell& L = pd ? (side ? S.pdh : S.pdpd) : (side ? S.hh : S.hpd);
       const int n = L.rcnt[row];
       // shares arrive weighted by their senders
       for_row_shares<RECV_RU_WIDE>(gmem(reinterpret_cast<const double4*>(L.rbuf)), L.rows, row, n, [&](const double4& v) {
@@ -829,8 +1043,22 @@ template <int R> struct DensFd { static constexpr auto fn = k_density64<A2C_DERI
 template <int R> struct DensAn { static constexpr auto fn = k_density64<A2C_DERIV_ANALYTIC, R>; };
 template <int R> struct GradFd { static constexpr auto fn = k_grad64<A2C_DERIV_FD, R>; };
 template <int R> struct GradAn { static constexpr auto fn = k_grad64<A2C_DERIV_ANALYTIC, R>; };
-template <int R> struct DensOwn { static constexpr auto fn = k_dens_own64<R>; };
-template <int R> struct GradOwn { static constexpr auto fn = k_grad_own64<R>; };
+// Owner launches: workgroups of TBO lanes, TBO / 256 units each.
+template <template <int, int> class K, int TBO>
+int owners(const Launch& L) {
+  const dim3 grid((L.onblk + TBO / TB - 1) / (TBO / TB));
+  if (L.rules & (1 << A2C_QUAD_R12))
+    hipLaunchKernelGGL((K<A2C_QUAD_R12, TBO>::fn), grid, dim3(TBO), 0, L.stream, L.lats, L.ob2l, L.onblk, L.tab64);
+  if (L.rules & (1 << GH3))
+    hipLaunchKernelGGL((K<GH3, TBO>::fn), grid, dim3(TBO), 0, L.stream, L.lats, L.ob2l, L.onblk, L.tab64);
+  return hipGetLastError() == hipSuccess ? A2C_OK : A2C_EHIP;
+}
+// Up to a unit per CU (gradient pass, one workgroup per CU) or two (density
+// pass) the units go to workgroups of their own; beyond, two to a workgroup, so
+// that a CU holds 8 waves on one copy of the tables.
+constexpr int GRAD_WIDE_UNITS = 256, DENS_WIDE_UNITS = 512;
+template <int R, int T> struct DensOwn { static constexpr auto fn = k_dens_own64<R, T>; };
+template <int R, int T> struct GradOwn { static constexpr auto fn = k_grad_own64<R, T>; };
 }  // namespace
 
 int run_density64(const Launch& L) {
@@ -844,12 +1072,12 @@ int run_eval64(const Launch& L, Timing* tm) {
       if (tm) tm->mark(L.stream, "rows");
       if (run_rows(L)) return A2C_EHIP;
       if (tm) tm->mark(L.stream, "dens_own64");
-      if (per_rule<DensOwn>(L, L.onblk, L.lats, L.ob2l, L.tab64)) return A2C_EHIP;
+      if (L.onblk > DENS_WIDE_UNITS ? owners<DensOwn, 512>(L) : owners<DensOwn, 256>(L)) return A2C_EHIP;
       if (tm) tm->mark(L.stream, "dens_recv64");
       hipLaunchKernelGGL(k_dens_recv64, dim3(L.nblk), dim3(TB), 0, L.stream, L.lats, L.b2l);
       if (hipGetLastError() != hipSuccess) return A2C_EHIP;
       if (tm) tm->mark(L.stream, "grad_own64");
-      if (per_rule<GradOwn>(L, L.onblk, L.lats, L.ob2l, L.tab64)) return A2C_EHIP;
+      if (L.onblk > GRAD_WIDE_UNITS ? owners<GradOwn, 512>(L) : owners<GradOwn, 256>(L)) return A2C_EHIP;
       if (tm) tm->mark(L.stream, "grad_recv64");
       hipLaunchKernelGGL(k_grad_recv64, dim3(L.nblk), dim3(TB), 0, L.stream, L.lats, L.b2l);
       if (hipGetLastError() != hipSuccess) return A2C_EHIP;
@@ -884,7 +1112,75 @@ int run_final_sum(const Launch& L) {
   return hipGetLastError() == hipSuccess ? A2C_OK : A2C_EHIP;
 }
 
-// FP64 tables: on each 0.05 A interval the polynomial (degree 8 for the
+// The tables of the owner passes (see "pair-once"), from the closed forms in
+// long double.
+void host_tables64_s(std::vector<double>& t) {
+  static const std::vector<double> built = [] {
+    using LD = long double;
+    std::vector<double> out((size_t)S_SIZE, 0.0);
+    const LD PI = 3.14159265358979323846264338327950288L, h = 0.5025L / 12, s0 = 25.5025L - 587 * h;
+    auto node = [&](int i, int n) { return 0.5L - 0.5L * cosl((2 * i + 1) * PI / (2.0L * n)); };
+    // polynomial through (u[i], y[i]), i < n, as monomials
+    auto through = [](const LD* u, const LD* y, int n, LD* m) {
+      LD c[SP];
+      for (int i = 0; i < n; ++i) c[i] = y[i];
+      for (int j = 1; j < n; ++j)
+        for (int i = n - 1; i >= j; --i) c[i] = (c[i] - c[i - 1]) / (u[i] - u[i - j]);
+      for (int q = 0; q < SP; ++q) m[q] = 0;
+      for (int i = n - 1; i >= 0; --i) {
+        for (int q = SP - 1; q > 0; --q) m[q] = m[q - 1] - u[i] * m[q];
+        m[0] = c[i] - u[i] * m[0];
+      }
+    };
+    enum { VALUE, SLOPE, BOTH };
+    auto fill = [&](int f, int fit, auto g) {  // g: value and slope in r
+      for (int k = 0; k < SNT; ++k) {
+        auto at = [&](LD u) {
+          const LD r = f == S_PHPDH ? (156 + k + u) / 160.0L : sqrtl(s0 + (k + u) * h);
+          const eam::VDT<LD> v = g(r);
+          return eam::VDT<LD>{v.v, v.d * (f == S_PHPDH ? 1 / 160.0L : h / (2 * r))};  // d/du
+        };
+        const bool split = f == S_PHPD;  // degree 6, the last two coefficients as floats
+        const int n = fit == BOTH && !split ? SP - 1 : SP;
+        LD u[SP], y[SP], m[SP + 1];
+        for (int i = 0; i < n; ++i) {
+          u[i] = node(i, n);
+          y[i] = fit == VALUE ? at(u[i]).v : at(u[i]).d;
+        }
+        through(u, y, n, m);
+        if (fit == BOTH) {  // the slope's integral, with the value's mean over the Chebyshev points
+          for (int q = SP; q > 0; --q) m[q] = m[q - 1] / q;  // the slope's degree is n - 1
+          if (!split) m[SP] = 0;
+          m[0] = 0;
+          LD c = 0;
+          for (int i = 0; i < SP; ++i) {
+            const LD w = node(i, SP);
+            LD v = 0;
+            for (int q = SP; q >= 0; --q) v = v * w + m[q];
+            c += at(w).v - v;
+          }
+          m[0] = c / SP;
+        }
+        double* row = &out[(size_t)f * S_ROWS + (size_t)k * SP];
+        for (int q = 0; q < SP; ++q) row[q] = (double)m[q];
+        if (split) {
+          const float hi[2] = {(float)m[5], (float)m[6]};
+          std::memcpy(row + 5, hi, sizeof hi);
+        }
+      }
+    };
+    fill(S_FPD, VALUE, [](LD r) { return eam::f_Pd_vd<LD>(r); });
+    fill(S_DFPD, SLOPE, [](LD r) { return eam::f_Pd_vd<LD>(r); });
+    fill(S_PHPD, BOTH, [](LD r) { return eam::phi_Pd_vd<LD>(r, eam::f_Pd_vd<LD>(r)); });
+    fill(S_PHPDH, BOTH, [](LD r) { return eam::phi_morse_vd<0, LD>(r); });
+    fill(S_PHH, BOTH, [](LD r) { return eam::phi_morse_vd<1, LD>(r); });
+    for (int i = 0; i < EXPN; ++i) out[S_EXP + i] = (double)exp2l((LD)i / EXPN);
+    return out;
+  }();
+  t = built;
+}
+
+// FP64 tables in r (exported, a2c_eam_tables64): on each 0.05 A interval the polynomial (degree 8 for the
 // exponential functions, 11 for the Pd polynomials) interpolating the
 // long-double closed form at the Chebyshev points, in Newton form, expanded
 // to monomials in u (all in long double); the switch radii 5.0, 5.05 and
@@ -1010,7 +1306,7 @@ int sync_lattice(a2c_fe_ctx* c, const double* dX, double* dG, double* dF) {
 
 }  // namespace a2c
 
-// Host-only: the FP64 tables of the FP64 pair-owner passes (layout in a2c_fe.h).
+// Host-only: the FP64 tables in r (layout in a2c_fe.h).
 extern "C" int a2c_eam_tables64(double* out, int32_t cap) {
   std::vector<double> t;
   a2c::host_tables64(t);

@@ -260,7 +260,7 @@ __device__ __forceinline__ void image_vec(const Image& g, const double qi[3], co
   if (far) {
 #pragma unroll
     for (int c = 0; c < 3; ++c)
-      if (fabs(d[c]) > g.half[c]) d[c] = qi[c] - (qj[c] - g.box[c] * rint((qj[c] - qi[c]) * g.ibox[c]));
+      if (fabs(d[c]) > g.half[c]) d[c] = qi[c] - fma(-g.box[c], rint((qj[c] - qi[c]) * g.ibox[c]), qj[c]);
   }
 }
 
@@ -446,7 +446,7 @@ int build_tables(a2c_fe_ctx* c);                        // eval32.hip
 int tables_download(a2c_fe_ctx* c, float* out);         // 5*500 float4
 void host_tables(std::vector<float4>& t);              // FP32 cubic tables in r (host)
 void host_tables_s(std::vector<float4>& t);            // appends the FP32 cubic tables in |r|^2
-// FP64 tables of the EAM functions: per function T64_N intervals of 0.05 A
+// FP64 tables of the EAM functions in r (exported; no kernel reads them): per function T64_N intervals of 0.05 A
 // over [1, 6) A, each a polynomial in the local coordinate u in [0, 1).  Part
 // one: the exponential functions (f_H, phi_PdH, phi_H), degree T64_D, T64_P
 // doubles per row (c0..c8, one pad); part two, after it: the Pd polynomials
@@ -458,6 +458,7 @@ enum { T64Q_FPD = 0, T64Q_PHPD = 1 };
 constexpr int T64_PART1 = T64_NF * T64_N * T64_P;                // doubles
 constexpr int T64_SIZE = T64_PART1 + T64Q_NF * T64_N * T64Q_P;  // doubles
 void host_tables64(std::vector<double>& t);
+void host_tables64_s(std::vector<double>& t);  // those of the FP64 owner passes, in |r|^2 (eval64.hip)
 // The FP32 and FP64 EAM tables on one device, uploaded at the first call for
 // that device and shared by every context and batch of the process until it
 // ends (they depend on nothing but the compiled-in potential); never freed.

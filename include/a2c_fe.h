@@ -313,13 +313,14 @@ int a2c_fe_time_diffuse(a2c_fe_ctx* ctx, double dt, double nu, double Qm, double
                         const double* d_gamma, const int32_t* d_full_h, double* d_x, int32_t iters,
                         a2c_timing* out);
 
-/* Host-only (no GPU): the FP32 EAM tables of the mixed path, 5 tables
+/* Host-only (no GPU): the EAM functions as FP32 tables in r, 5 tables
  * (f_Pd, f_H, phi_Pd, phi_PdH, phi_H) x 500 intervals x 4 cubic coefficients;
  * interval k covers r in [1 + 0.01k, 1 + 0.01(k+1)) A.  Returns the float count
  * (10000); fills out when cap is large enough. */
 int a2c_eam_tables(float* out, int32_t cap);
 
-/* Host-only (no GPU): the FP64 tables of the FP64 pair-owner passes.  Part
+/* Host-only (no GPU): the EAM functions as FP64 tables in r, to the rounding
+ * of the closed forms (the FP64 pair-owner passes read tables in r^2).  Part
  * one: 3 functions (f_H, phi_PdH, phi_H) x 100 intervals x 10 doubles
  * (polynomial coefficients c0..c8 and one pad); part two, after it: 2
  * functions (f_Pd, phi_Pd) x 100 intervals x 12 doubles (c0..c11).  Interval
