@@ -1002,13 +1002,7 @@ __global__ __launch_bounds__(TB) void k_rows(const LatDev* __restrict__ lats, co
   const LatDev& S = lats[b2l[blk]];
   const int s = (blk - S.blk0) * TB + threadIdx.x;
   if (s >= S.npd + S.nh) return;
-  const double4 v = reinterpret_cast<const double4*>(S.X)[s];
-  const bool pd = s < S.npd;
-  const int row = pd ? row_of_site(s, S.npd) : row_of_site(s - S.npd, S.nh);
-  const int p = pd ? row : S.npd + row;
-  S.qxy[p] = make_double2(v.x, v.y);
-  S.qzs[p] = make_double2(v.z, v.w);
-  if (!pd) S.xrow[row] = S.x[s - S.npd];
+  copy_row(S, s);
 }
 
 }  // namespace

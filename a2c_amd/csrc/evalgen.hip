@@ -3,15 +3,20 @@
 // node table (a2c_fe_set_quadrature).  The reference's loop nests
 // (minimizer.cpp:140-157 and :162-351 for the objective and gradient,
 // :588-802 for the chemical potential, electrondensity.cpp:12-56 for the
-// density) with the EAM functions and the rule as data:
+// density) with the EAM functions and the rule as data.  Density and gradient
+// take each pair once, at its owner, like the passes of the built-in rules
+// (row order and shares: Ell and LatDev):
 //
-//   k_gen_density  one lane per site over its full lists: rho, F(rho),
-//                  F'(rho), the embedding energy
-//   k_gen_grad     one lane per site over its full lists: every pair's energy
-//                  and coefficient c = F'_i f_j' + F'_j f_i' + phi' at each
-//                  node, q- and sigma-gradient, the site's share of f, and a
-//                  fixed-shape block sum (k_final_sum completes f)
-//   k_gen_chem     per H site: dV/dx_a + the correction terms, gamma, cap
+//   k_gen_rows       row-order copies of the state and the occupancy
+//   k_gen_dens_own   owned pairs' density: own sums, shares to the partners
+//   k_gen_dens_recv  rho, F(rho), F'(rho), the embedding energy
+//   k_gen_grad_own   owned pairs' energy and coefficient c = F'_i f_j' +
+//                    F'_j f_i' + phi' at each node, both ends' q- and
+//                    sigma-gradient
+//   k_gen_grad_recv  gradient, the site's share of f, and a fixed-shape block
+//                    sum (k_final_sum completes f)
+//   k_gen_chem       per H site over its full lists: dV/dx_a + the correction
+//                    terms, gamma, cap
 //
 // A node k of a 6-D table puts the pair vector at r_k = d + a_i xi1_k -
 // a_j xi2_k with a = sqrt(2) sigma, so dr_k/dsigma_i = sqrt(2) xi1_k; a
@@ -24,130 +29,196 @@
 // FP32 from FP32 pieces of the r-functions, summed per pair in FP32 and per
 // site in FP64.  F(rho) and F'(rho) are FP64 in both.
 #include <cmath>
+#include <type_traits>
 
 #include "eam64.hpp"
 #include "fe_internal.hpp"
+#include "pair_rows.hpp"
 
 namespace a2c {
 namespace {
 
 constexpr int TB = SITE_BLOCK;
-constexpr double KB = 8.6173324e-5;  // minimizer.cpp:92
 constexpr double SQ2 = 1.4142135623730950488;
 
-struct Site {
-  double q[3];
-  double s;
-};
 __device__ __forceinline__ Site load_site(const double* __restrict__ X, int s) {
   const double4 v = *reinterpret_cast<const double4*>(X + 4 * (size_t)s);
   return {{v.x, v.y, v.z}, v.w};
 }
-__device__ __forceinline__ void pair_vec(const LatDev& S, const Site& a, const Site& b, double d[3]) {
-#pragma unroll
-  for (int c = 0; c < 3; ++c) {
-    double qj = b.q[c];
-    if (S.periodic[c]) qj = qj - S.box[c] * rint((qj - a.q[c]) * S.ibox[c]);
-    d[c] = a.q[c] - qj;
-  }
+__device__ __forceinline__ void pair_vec(const Image& g, const Site& a, const Site& b, double d[3]) {
+  image_vec(g, a.q, b.q, d);
 }
 
-// ------------------------------------------------------------ pieces
-// Value and slope of a piecewise cubic at x (coefficients c0..c3 in the
-// local coordinate u of piece k).  Past the last node: 0 for the r-functions,
-// the end tangent for the embedding functions (emb).
-template <class R, class C>
-__device__ __forceinline__ eam::VDT<R> piece_vd(const GenFn& F, const C* __restrict__ tab, R x, bool emb) {
-  const R p = x * (R)F.ih;
+// ------------------------------------------------------------ functions
+// Embedding functions in FP64: closed forms or pieces (the cubic in the local
+// coordinate u of piece k; past the last node the end tangent).
+__device__ __forceinline__ eam::VD emb_vd(const GenFn& F, const double4* __restrict__ tab, double x) {
+  const double p = x * F.ih;
   int k = (int)p;
   if (k < 0) k = 0;
-  if (k >= F.n - 1) {
-    if (emb) return {(R)F.yend + (R)F.dend * (x - (R)(F.n - 1) / (R)F.ih), (R)F.dend};
-    return {R(0), R(0)};
-  }
-  const R u = p - (R)k;
-  const C c = tab[F.off + k];
-  const R v = (R)c.x + u * ((R)c.y + u * ((R)c.z + u * (R)c.w));
-  const R d = (R)c.y + u * (R(2) * (R)c.z + u * R(3) * (R)c.w);
-  return {v, d * (R)F.ih};
+  if (k >= F.n - 1) return {F.yend + F.dend * (x - (double)(F.n - 1) / F.ih), F.dend};
+  const double u = p - (double)k;
+  const double4 c = tab[F.off + k];
+  return {c.x + u * (c.y + u * (c.z + u * c.w)), (c.y + u * (2.0 * c.z + u * 3.0 * c.w)) * F.ih};
 }
-
-// Embedding functions in FP64: closed forms or pieces.
 template <int POT>
 __device__ __forceinline__ double F_val(const GenDev& g, bool pd, double rho) {
   if (POT == 0) return pd ? eam::F_Pd(rho) : eam::F_H(rho);
-  return piece_vd<double>(g.fn[pd ? GEN_F_PD : GEN_F_H], g.tab, rho, true).v;
+  return emb_vd(g.fn[pd ? GEN_F_PD : GEN_F_H], g.tab, rho).v;
 }
 template <int POT, int DM>
 __device__ __forceinline__ double F_der(const GenDev& g, bool pd, double rho, double eps) {
   if (DM == A2C_DERIV_FD) return (F_val<POT>(g, pd, rho + eps) - F_val<POT>(g, pd, rho - eps)) / (2.0 * eps);
   if (POT == 0) return pd ? eam::F_Pd_vd(rho).d : eam::F_H_vd(rho).d;
-  return piece_vd<double>(g.fn[pd ? GEN_F_PD : GEN_F_H], g.tab, rho, true).d;
+  return emb_vd(g.fn[pd ? GEN_F_PD : GEN_F_H], g.tab, rho).d;
 }
 
-// r-functions: density f (fn GEN_RHO_*) and pair phi (fn GEN_RPHI_*, stored
-// as r phi).  POT 0 in FP64: the closed forms; otherwise the pieces (FP64, or
-// FP32 for R = float).
-template <int POT, class R>
-struct RFun {
-  const GenDev& g;
-  __device__ __forceinline__ R val(int fn, R r) const {
-    if (POT == 0 && sizeof(R) == 8) {
-      const double x = (double)r;
-      switch (fn) {
-        case GEN_RHO_PD: return (R)eam::f_Pd(x);
-        case GEN_RHO_H: return (R)eam::f_H(x);
-        case GEN_RPHI_PD: return (R)eam::phi_Pd(x);
-        case GEN_RPHI_PDH: return (R)eam::phi_morse<0>(x);
-        default: return (R)eam::phi_morse<1>(x);
-      }
-    }
-    const eam::VDT<R> z = look(fn, r);
-    return fn >= GEN_RPHI_PD ? z.v / r : z.v;
+// |r| and 1/|r| from |r|^2, to the last place or so: the hardware estimate of
+// 1/sqrt and Newton steps; at 0, infinity and NaN the limits (r = x, and the
+// estimate itself).
+__device__ __forceinline__ void root(double x, double& r, double& ri) {
+  const double y = __builtin_amdgcn_rsq(x);
+  const double e = fma(-(x * y), y, 1.0);
+  ri = fma(y * e, fma(e, 0.375, 0.5), y);
+  r = x * ri;
+  r = fma(0.5 * ri, fma(-r, r, x), r);
+  if (!(x > 0.0 && x < __builtin_huge_val())) r = x, ri = y;
+}
+__device__ __forceinline__ void root(float x, float& r, float& ri) {
+  const float y = __builtin_amdgcn_rsqf(x);
+  r = x * y;
+  r = fmaf(0.5f * y, fmaf(-r, r, x), r);
+  ri = fmaf(y, fmaf(-r, y, 1.0f), y);
+  if (!(x > 0.0f && x < __builtin_huge_valf())) r = x, ri = y;
+}
+
+// A radius located in the r-functions' table: the row of its interval, the
+// coordinate u in it, and whether it lies inside (past the table's end the
+// functions are 0).
+template <class R>
+struct At;
+template <>
+struct At<double> {
+  const A2C_GLOBAL double2* row;
+  double r, ri, u, ih;
+  bool in;
+  // the Hermite piece of two nodes: c0, c1 from the first, c3 = s0 + s1 - 2 (y1
+  // - y0), c2 = (y1 - y0) - s0 - c3
+  template <int SLOT>
+  __device__ __forceinline__ eam::VD vd() const {
+    const double2 a = row[SLOT], b = row[GEN_NS + SLOT];
+    const double dy = b.x - a.x, c3 = fma(-2.0, dy, a.y + b.y), c2 = (dy - a.y) - c3;
+    return {fma(u, fma(u, fma(u, c3, c2), a.y), a.x), fma(u, fma(u, 3.0 * c3, c2 + c2), a.y) * ih};
   }
-  __device__ __forceinline__ eam::VDT<R> vd(int fn, R r) const {
-    if (POT == 0 && sizeof(R) == 8) {
-      const double x = (double)r;
-      eam::VD o;
-      switch (fn) {
-        case GEN_RHO_PD: o = eam::f_Pd_vd(x); break;
-        case GEN_RHO_H: o = eam::f_H_vd(x); break;
-        case GEN_RPHI_PD: o = eam::phi_Pd_vd(x, eam::f_Pd_vd(x)); break;
-        case GEN_RPHI_PDH: o = eam::phi_morse_vd<0>(x); break;
-        default: o = eam::phi_morse_vd<1>(x); break;
-      }
-      return {(R)o.v, (R)o.d};
-    }
-    const eam::VDT<R> z = look(fn, r);
-    if (fn < GEN_RPHI_PD) return z;
-    const R phi = z.v / r;
-    return {phi, (z.d - phi) / r};  // (r phi)' = phi + r phi'
-  }
-  __device__ __forceinline__ eam::VDT<R> look(int fn, R r) const {
-    if (sizeof(R) == 8) return piece_vd<R>(g.fn[fn], g.tab, r, false);
-    return piece_vd<R>(g.fn32[fn], g.tab32, r, false);
-  }
-  // slope by the reference's central difference (DM = FD) or analytically
-  template <int DM>
-  __device__ __forceinline__ eam::VDT<R> vd_dm(int fn, R r, R eps) const {
-    if (DM == A2C_DERIV_FD) return {val(fn, r), (val(fn, r + eps) - val(fn, r - eps)) / (R(2) * eps)};
-    return vd(fn, r);
+};
+template <>
+struct At<float> {
+  const A2C_GLOBAL float4* row;
+  float r, ri, u, ih;
+  bool in;
+  template <int SLOT>
+  __device__ __forceinline__ eam::VDT<float> vd() const {
+    const float4 c = row[SLOT];
+    return {fmaf(u, fmaf(u, fmaf(u, c.w, c.z), c.y), c.x), fmaf(u, fmaf(u, 3.0f * c.w, c.z + c.z), c.y) * ih};
   }
 };
 
-// The rule's nodes staged in LDS: xi1 (or z), xi2, w as R.
+// r-functions by slot: density f and pair phi (stored as r phi).  POT 0 in
+// FP64: the closed forms; otherwise the table.
+template <int POT, class R>
+struct RFun {
+  using E = std::conditional_t<sizeof(R) == 8, double2, float4>;
+  static constexpr bool CLOSED = POT == 0 && sizeof(R) == 8;
+  const A2C_GLOBAL E* row;
+  int last;  // the last interval
+  R ih;
+  __device__ __forceinline__ explicit RFun(const GenDev& g) {
+    if constexpr (sizeof(R) == 8) row = gmem((const E*)g.r64.row), last = g.r64.n - 2, ih = g.r64.ih;
+    else row = gmem((const E*)g.r32.row), last = g.r32.n - 2, ih = (R)g.r32.ih;
+  }
+  __device__ __forceinline__ At<R> at(R r, R ri) const {
+    At<R> a;
+    a.r = r;
+    a.ri = ri;
+    if (CLOSED) return a;
+    const R p = r * ih;
+    const int k = max((int)p, 0);
+    a.u = p - (R)k;
+    a.ih = ih;
+    a.in = k <= last;
+    a.row = row + (size_t)GEN_NS * min(k, last);  // no branch around the loads: several nodes' are in flight together
+    return a;
+  }
+  template <int SLOT>
+  __device__ __forceinline__ eam::VDT<R> vd(const At<R>& a) const {
+    if constexpr (CLOSED) {
+      if constexpr (SLOT == GEN_S_RHO_PD) return eam::f_Pd_vd(a.r);
+      else if constexpr (SLOT == GEN_S_RHO_H) return eam::f_H_vd(a.r);
+      else if constexpr (SLOT == GEN_S_RPHI_PD) return eam::phi_Pd_vd(a.r, eam::f_Pd_vd(a.r));
+      else return eam::phi_morse_vd<SLOT == GEN_S_RPHI_PDH ? 0 : 1>(a.r);
+    } else {
+      eam::VDT<R> z = a.template vd<SLOT>();
+      if (!a.in) z = {R(0), R(0)};
+      if constexpr (SLOT == GEN_S_RHO_PD || SLOT == GEN_S_RHO_H) return z;
+      const R phi = z.v * a.ri;
+      return {phi, (z.d - phi) * a.ri};  // (r phi)' = phi + r phi'
+    }
+  }
+  template <int SLOT>
+  __device__ __forceinline__ R val(const At<R>& a) const {
+    if constexpr (CLOSED) {
+      if constexpr (SLOT == GEN_S_RHO_PD) return eam::f_Pd(a.r);
+      else if constexpr (SLOT == GEN_S_RHO_H) return eam::f_H(a.r);
+      else if constexpr (SLOT == GEN_S_RPHI_PD) return eam::phi_Pd(a.r);
+      else return eam::phi_morse<SLOT == GEN_S_RPHI_PDH ? 0 : 1>(a.r);
+    } else {
+      return vd<SLOT>(a).v;
+    }
+  }
+};
+
+// One node of a pair as the derivative mode wants it: the radius, and for the
+// reference's central differences the radii eps to either side.
+template <int POT, int DM, class R>
+struct NodeR {
+  RFun<POT, R> fun;
+  At<R> c, hi, lo;
+  R h;  // 1 / (2 eps)
+  __device__ __forceinline__ NodeR(const RFun<POT, R>& f, R r, R ri, R eps) : fun(f), c(f.at(r, ri)) {
+    if (DM == A2C_DERIV_FD) {
+      hi = f.at(r + eps, R(1) / (r + eps));
+      lo = f.at(r - eps, R(1) / (r - eps));
+      h = R(2) * eps;
+    }
+  }
+  template <int SLOT>
+  __device__ __forceinline__ eam::VDT<R> vd() const {
+    if (DM == A2C_DERIV_FD)
+      return {fun.template val<SLOT>(c), (fun.template val<SLOT>(hi) - fun.template val<SLOT>(lo)) / h};
+    return fun.template vd<SLOT>(c);
+  }
+};
+
+// The rule's nodes staged in LDS as R, 8 to a node: xi1 (or z), xi2, w, 0.
+extern __shared__ __align__(16) unsigned char gen_lds[];
 template <class R>
-__device__ __forceinline__ void stage_nodes(R* nd, const GenDev& g) {
-  for (int i = threadIdx.x; i < g.K * 7; i += blockDim.x) nd[i] = (R)g.nodes[(i / 7) * 8 + i % 7];
+__device__ __forceinline__ const R* stage_nodes(const GenDev& g) {
+  R* nd = reinterpret_cast<R*>(gen_lds);
+  for (int i = threadIdx.x; i < g.K * 8; i += blockDim.x) nd[i] = (R)g.nodes[i];
   __syncthreads();
+  return nd;
+}
+template <class R>
+size_t node_bytes(const GenDev& g) {
+  return sizeof(R) * 8 * (size_t)g.K;
 }
 
-// Node k of a pair: r_k (in R) and the factor that turns r . xi1 into
-// r . dr/dsigma_i.
+// Nodes of a pair: r_k = d + a xi1_k - b xi2_k; dr_k/dsigma of the first site
+// is fi xi1_k, of the second -fj xi2_k (6-D nodes) or fj z_k (relative ones).
 template <class R>
 struct PairFrame {
-  R d[3], a, b;  // r_k = d + a xi1_k - b xi2_k
-  R fac;         // dr/dsigma_i = fac * xi1_k
+  R d[3], a, b;
+  R fi, fj;
 };
 template <class R>
 __device__ __forceinline__ PairFrame<R> frame(const GenDev& g, const double d[3], double si, double sj) {
@@ -159,155 +230,242 @@ __device__ __forceinline__ PairFrame<R> frame(const GenDev& g, const double d[3]
     const double s = sqrt(si * si + sj * sj);
     f.a = (R)s;
     f.b = R(0);
-    f.fac = (R)(si / s);
+    f.fi = (R)(si / s);
+    f.fj = (R)(sj / s);
   } else {
     f.a = (R)(SQ2 * si);
     f.b = (R)(SQ2 * sj);
-    f.fac = (R)SQ2;
+    f.fi = f.fj = (R)SQ2;
   }
   return f;
 }
 template <class R>
-__device__ __forceinline__ void node_r(const PairFrame<R>& f, const R* nd, int k, R r[3]) {
-  const R* n = nd + 7 * k;
+__device__ __forceinline__ R node_r2(const PairFrame<R>& f, const R* n, R r[3]) {
 #pragma unroll
   for (int c = 0; c < 3; ++c) r[c] = f.d[c] + f.a * n[c] - f.b * n[3 + c];
+  return r[0] * r[0] + r[1] * r[1] + r[2] * r[2];
+}
+
+struct GenPair {
+  double d[3], s;
+};
+__device__ __forceinline__ GenPair gen_pair(const Image& img, const Site& a, const Site& b) {
+  GenPair p;
+  pair_vec(img, a, b, p.d);
+  p.s = b.s;
+  return p;
+}
+
+__global__ __launch_bounds__(TB) void k_gen_rows(const LatDev* __restrict__ lat) {
+  const LatDev& S = *lat;
+  const int s = xcd_block() * TB + threadIdx.x;
+  if (s >= S.npd + S.nh) return;
+  copy_row(S, s);
 }
 
 // ------------------------------------------------------------ density
-template <int POT, int DM, class R>
-__global__ __launch_bounds__(TB) void k_gen_density(const LatDev* __restrict__ lat, GenDev g, double eps) {
-  __shared__ R nd[A2C_QUAD_MAX_NODES * 7];
-  stage_nodes(nd, g);
+template <int POT, class R, bool NB_H, bool ME_H>
+__device__ __forceinline__ void dens_list(const LatDev& S, const GenDev& g, const RFun<POT, R>& fun, const R* nd,
+                                          const OwnerLane& ln, int KL, const Site& a, const Image& img, double wme,
+                                          double& rho) {
+  constexpr int NB = NB_H ? GEN_S_RHO_H : GEN_S_RHO_PD, ME = ME_H ? GEN_S_RHO_H : GEN_S_RHO_PD;
+  const Ell& L = ME_H ? (NB_H ? S.hh : S.hpd) : (NB_H ? S.pdh : S.pdpd);
+  const Ell& P = ME_H ? (NB_H ? S.hh : S.pdh) : (NB_H ? S.hpd : S.pdpd);  // partner rows
+  A2C_GLOBAL double* __restrict__ share = gmem(reinterpret_cast<double*>(P.rbuf));
+  const size_t prows = P.rows;
+  owned_pairs<NB_H>(
+      L, ln, KL, S, [](int) { return 0.0f; }, [&](const Site& b) { return gen_pair(img, a, b); },
+      [&](const GenPair& p, float, double wj, int jl, int rv) {
+        const PairFrame<R> f = frame<R>(g, p.d, a.s, p.s);
+        R mine = R(0), theirs = R(0);
+#pragma unroll 2  // two nodes' gathers in flight
+        for (int k = 0; k < g.K; ++k) {
+          const R* n = nd + 8 * k;
+          R r[3], rn, ri;
+          root(node_r2(f, n, r), rn, ri);
+          const At<R> at = fun.at(rn, ri);
+          mine += n[6] * fun.template val<NB>(at);
+          if (NB != ME) theirs += n[6] * fun.template val<ME>(at);
+        }
+        if (NB == ME) theirs = mine;
+        rho += wj * (double)mine;
+        share[(size_t)rv * prows + jl] = wme * (double)theirs;
+      });
+}
+
+// 16^3 cells, tabulated potential, 12 nodes, FP64: full lists, one lane per site
+// 306 us, this 77 us; the gradient pass 727 and 118 us.  Bound by the L1: a node's
+// gathers (two 16-byte words per function) touch a line per lane.  5^3 cells (memory
+// latency): 62 us with a branch around the table's end, 52 without, 41 with two
+// nodes in flight; more nodes only take registers.
+template <int POT, class R>
+__global__ __launch_bounds__(TB) void k_gen_dens_own(const LatDev* __restrict__ lat, GenDev g, int KL) {
+  const R* nd = stage_nodes<R>(g);
+  const LatDev& S = *lat;
+  const OwnerLane ln(S, __builtin_amdgcn_readfirstlane(xcd_block()), KL);
+  if (ln.row >= ln.rows) return;  // whole lane groups
+  const RFun<POT, R> fun(g);
+  const Image img = image_of(S);
+  const int s = ln.pd ? ln.row : S.npd + ln.row;
+  const Site a = load_row(gmem((const double2*)S.qxy), gmem((const double2*)S.qzs), s);
+  double rho = 0.0;
+  if (ln.pd) {
+    dens_list<POT, R, false, false>(S, g, fun, nd, ln, KL, a, img, 1.0, rho);
+    dens_list<POT, R, true, false>(S, g, fun, nd, ln, KL, a, img, 1.0, rho);
+  } else {
+    const double wme = gmem((const double*)S.xrow)[ln.row];
+    dens_list<POT, R, false, true>(S, g, fun, nd, ln, KL, a, img, wme, rho);
+    dens_list<POT, R, true, true>(S, g, fun, nd, ln, KL, a, img, wme, rho);
+  }
+  rho = site_sum(rho, KL);
+  if (ln.ph == 0) gmem(S.epair)[s] = rho;
+}
+
+// by_site: rho, F' and the embedding energy in site order (the chemical
+// potential and a caller's density), else in row order (the gradient pass).
+template <int POT, int DM>
+__global__ __launch_bounds__(TB) void k_gen_dens_recv(const LatDev* __restrict__ lat, GenDev g, double eps,
+                                                      int by_site) {
   const LatDev& S = *lat;
   const int s = xcd_block() * TB + threadIdx.x;
-  const int N = S.npd + S.nh;
-  if (s >= N) return;
-  const RFun<POT, R> fun{g};
-  const double* __restrict__ X = S.X;
-  const double* __restrict__ xo = S.x;
+  if (s >= S.npd + S.nh) return;
   const bool pd = s < S.npd;
   const int row = pd ? s : s - S.npd;
-  const Site a = load_site(X, s);
-  const int K = g.K;
-  double rho = 0.0;
-  for (int side = 0; side < 2; ++side) {  // Pd neighbors, then H neighbors (electrondensity.cpp:20-48)
-    const Ell L = side == 0 ? (pd ? S.pdpd : S.hpd) : (pd ? S.pdh : S.hh);
-    const int fn = side == 0 ? GEN_RHO_PD : GEN_RHO_H;
-    const int n = L.cnt[row];
-    for (int t = 0; t < n; ++t) {
-      const int jl = L.idx[(size_t)t * L.rows + row];
-      const int j = side == 0 ? jl : S.npd + jl;
-      const Site b = load_site(X, j);
-      double d[3];
-      pair_vec(S, a, b, d);
-      const PairFrame<R> f = frame<R>(g, d, a.s, b.s);
-      R acc = R(0);
-      for (int k = 0; k < K; ++k) {
-        R r[3];
-        node_r(f, nd, k, r);
-        acc += nd[7 * k + 6] * fun.val(fn, sqrt(r[0] * r[0] + r[1] * r[1] + r[2] * r[2]));
-      }
-      rho += (side == 0 ? 1.0 : xo[jl]) * (double)acc;
-    }
+  double rho = S.epair[s];
+#pragma unroll
+  for (int side = 0; side < 2; ++side) {
+    const Ell& L = pd ? (side ? S.pdh : S.pdpd) : (side ? S.hh : S.hpd);
+    for_row_shares<RECV_RU_SCALAR>(gmem(reinterpret_cast<const double*>(L.rbuf)), L.rows, row, L.rcnt[row],
+                                   [&](double v) { rho += v; });
   }
-  S.rho[s] = rho;
   const double F = F_val<POT>(g, pd, rho);
-  S.Fp[s] = F_der<POT, DM>(g, pd, rho, eps);
-  S.emb[s] = pd ? F : xo[row] * F;
+  const int o = !by_site ? s : pd ? site_of_row(row, S.npd) : S.npd + site_of_row(row, S.nh);
+  S.rho[o] = rho;
+  S.Fp[o] = F_der<POT, DM>(g, pd, rho, eps);
+  S.emb[o] = pd ? F : S.xrow[row] * F;
 }
 
 // ------------------------------------------------------------ gradient
 // Kinds: 0 Pd-Pd, 1 Pd site / H neighbor, 2 H site / Pd neighbor, 3 H-H.
-template <int POT, int DM, class R>
-__device__ __forceinline__ void node_terms(const RFun<POT, R>& fun, int kind, R rn, R Fi, R Fj, R eps, R& phi,
-                                           R& c) {
-  if (kind == 0) {
-    const eam::VDT<R> f = fun.template vd_dm<DM>(GEN_RHO_PD, rn, eps);
-    const eam::VDT<R> p = fun.template vd_dm<DM>(GEN_RPHI_PD, rn, eps);
-    phi = p.v;
-    c = (Fi + Fj) * f.d + p.d;
-  } else if (kind == 3) {
-    const eam::VDT<R> h = fun.template vd_dm<DM>(GEN_RHO_H, rn, eps);
-    const eam::VDT<R> p = fun.template vd_dm<DM>(GEN_RPHI_H, rn, eps);
-    phi = p.v;
-    c = (Fi + Fj) * h.d + p.d;
-  } else {
-    const eam::VDT<R> f = fun.template vd_dm<DM>(GEN_RHO_PD, rn, eps);
-    const eam::VDT<R> h = fun.template vd_dm<DM>(GEN_RHO_H, rn, eps);
-    const eam::VDT<R> p = fun.template vd_dm<DM>(GEN_RPHI_PDH, rn, eps);
-    phi = p.v;
-    // site i's density takes the neighbor's f, the neighbor's takes i's
-    c = kind == 1 ? Fi * h.d + Fj * f.d + p.d : Fi * f.d + Fj * h.d + p.d;
-  }
+// phi and c = dE/dr of one node; FP multiplies f_Pd', FH f_H'.
+template <int POT, int DM, class R, int KIND>
+__device__ __forceinline__ void node_terms(const NodeR<POT, DM, R>& n, R FP, R FH, R& phi, R& c) {
+  constexpr int PHI = KIND == 0 ? GEN_S_RPHI_PD : KIND == 3 ? GEN_S_RPHI_H : GEN_S_RPHI_PDH;
+  const eam::VDT<R> p = n.template vd<PHI>();
+  phi = p.v;
+  c = p.d;
+  if (KIND != 3) c += FP * n.template vd<GEN_S_RHO_PD>().d;
+  if (KIND != 0) c += FH * n.template vd<GEN_S_RHO_H>().d;
 }
 
-template <int POT, int DM, class R>
-__global__ __launch_bounds__(TB) void k_gen_grad(const LatDev* __restrict__ lat, GenDev g, double eps) {
-  __shared__ R nd[A2C_QUAD_MAX_NODES * 7];
-  __shared__ double red[TB];
-  stage_nodes(nd, g);
-  const LatDev& S = *lat;
-  const int lb = xcd_block();
-  const int s = lb * TB + threadIdx.x;
-  const int N = S.npd + S.nh;
-  double fs = 0.0;
-  if (s < N) {
-    const RFun<POT, R> fun{g};
-    const double* __restrict__ X = S.X;
-    const double* __restrict__ xo = S.x;
-    const double* __restrict__ Fp = S.Fp;
-    const bool pd = s < S.npd;
-    const int row = pd ? s : s - S.npd;
-    const Site a = load_site(X, s);
-    const double Fi = Fp[s];
-    const double xi = pd ? 1.0 : xo[row];
-    const int K = g.K;
-    double e = 0.0, gq[3] = {0.0, 0.0, 0.0}, gs = 0.0;
-    for (int side = 0; side < 2; ++side) {
-      const Ell L = side == 0 ? (pd ? S.pdpd : S.hpd) : (pd ? S.pdh : S.hh);
-      const int kind = side == 0 ? (pd ? 0 : 2) : (pd ? 1 : 3);
-      const int n = L.cnt[row];
-      for (int t = 0; t < n; ++t) {
-        const int jl = L.idx[(size_t)t * L.rows + row];
-        const int j = side == 0 ? jl : S.npd + jl;
-        const Site b = load_site(X, j);
-        double d[3];
-        pair_vec(S, a, b, d);
-        const PairFrame<R> f = frame<R>(g, d, a.s, b.s);
-        R pe = R(0), px = R(0), py = R(0), pz = R(0), ps = R(0);
-        for (int k = 0; k < K; ++k) {
-          R r[3];
-          node_r(f, nd, k, r);
-          const R rn = sqrt(r[0] * r[0] + r[1] * r[1] + r[2] * r[2]);
-          R phi, c;
-          node_terms<POT, DM, R>(fun, kind, rn, (R)Fi, (R)Fp[j], (R)eps, phi, c);
-          const R w = nd[7 * k + 6];
+struct Own {
+  double e = 0.0, g0 = 0.0, g1 = 0.0, g2 = 0.0, gs = 0.0;
+};
+template <int POT, int DM, class R, int KIND>
+__device__ __forceinline__ void grad_list(const LatDev& S, const GenDev& g, const RFun<POT, R>& fun, const R* nd,
+                                          const OwnerLane& ln, int KL, const Site& a, double Fi, const Image& img,
+                                          double wme, R eps, Own& o) {
+  constexpr bool ME_H = KIND >= 2, NB_H = KIND & 1;
+  const Ell& L = ME_H ? (NB_H ? S.hh : S.hpd) : (NB_H ? S.pdh : S.pdpd);
+  const Ell& P = ME_H ? (NB_H ? S.hh : S.pdh) : (NB_H ? S.hpd : S.pdpd);  // partner rows
+  A2C_GLOBAL double4* __restrict__ share = gmem(reinterpret_cast<double4*>(P.rbuf));
+  const size_t prows = P.rows;
+  const A2C_GLOBAL double* Fp = gmem((const double*)S.Fp) + (NB_H ? S.npd : 0);
+  owned_pairs<NB_H>(
+      L, ln, KL, S, [=](int j) { return Fp[j]; }, [&](const Site& b) { return gen_pair(img, a, b); },
+      [&](const GenPair& q, double Fj, double wj, int jl, int rv) {
+        const PairFrame<R> f = frame<R>(g, q.d, a.s, q.s);
+        // a site's density takes the partner's f
+        const R FP = KIND == 0 ? (R)Fi + (R)Fj : KIND == 1 ? (R)Fj : (R)Fi;
+        const R FH = KIND == 3 ? (R)Fi + (R)Fj : KIND == 1 ? (R)Fi : (R)Fj;
+        R pe = R(0), px = R(0), py = R(0), pz = R(0), ps = R(0), pt = R(0);
+#pragma unroll 1
+        for (int k = 0; k < g.K; ++k) {
+          const R* n = nd + 8 * k;
+          R r[3], rn, ri, phi, c;
+          root(node_r2(f, n, r), rn, ri);
+          node_terms<POT, DM, R, KIND>(NodeR<POT, DM, R>(fun, rn, ri, eps), FP, FH, phi, c);
+          const R w = n[6];
           pe += w * phi;
-          const R u = w * c / rn;
+          const R u = w * c * ri;
           px += u * r[0];
           py += u * r[1];
           pz += u * r[2];
-          ps += u * (r[0] * nd[7 * k] + r[1] * nd[7 * k + 1] + r[2] * nd[7 * k + 2]);
+          ps += u * (r[0] * n[0] + r[1] * n[1] + r[2] * n[2]);
+          pt -= u * (r[0] * n[3] + r[1] * n[4] + r[2] * n[5]);
         }
-        const double wj = side == 0 ? 1.0 : xo[jl];  // H neighbors weigh by their occupancy
-        e += wj * (double)pe;
-        gq[0] += wj * (double)px;
-        gq[1] += wj * (double)py;
-        gq[2] += wj * (double)pz;
-        gs += wj * (double)(ps * f.fac);
-      }
+        if (g.rel) pt = ps;
+        o.e += wj * (double)pe;
+        o.g0 += wj * (double)px;
+        o.g1 += wj * (double)py;
+        o.g2 += wj * (double)pz;
+        o.gs += wj * (double)(ps * f.fi);
+        // the partner's share leaves weighted by the sender's occupancy
+        share[(size_t)rv * prows + jl] =
+            make_double4(-wme * (double)px, -wme * (double)py, -wme * (double)pz, wme * (double)(pt * f.fj));
+      });
+}
+
+template <int POT, int DM, class R>
+__global__ __launch_bounds__(TB) void k_gen_grad_own(const LatDev* __restrict__ lat, GenDev g, double eps, int KL) {
+  const R* nd = stage_nodes<R>(g);
+  const LatDev& S = *lat;
+  const OwnerLane ln(S, __builtin_amdgcn_readfirstlane(xcd_block()), KL);
+  if (ln.row >= ln.rows) return;  // whole lane groups
+  const RFun<POT, R> fun(g);
+  const Image img = image_of(S);
+  const int s = ln.pd ? ln.row : S.npd + ln.row;
+  const Site a = load_row(gmem((const double2*)S.qxy), gmem((const double2*)S.qzs), s);
+  const double Fi = gmem((const double*)S.Fp)[s];
+  Own o;
+  if (ln.pd) {
+    grad_list<POT, DM, R, 0>(S, g, fun, nd, ln, KL, a, Fi, img, 1.0, (R)eps, o);
+    grad_list<POT, DM, R, 1>(S, g, fun, nd, ln, KL, a, Fi, img, 1.0, (R)eps, o);
+  } else {
+    const double wme = gmem((const double*)S.xrow)[ln.row];
+    grad_list<POT, DM, R, 2>(S, g, fun, nd, ln, KL, a, Fi, img, wme, (R)eps, o);
+    grad_list<POT, DM, R, 3>(S, g, fun, nd, ln, KL, a, Fi, img, wme, (R)eps, o);
+  }
+  o.e = site_sum(o.e, KL);
+  o.g0 = site_sum(o.g0, KL);
+  o.g1 = site_sum(o.g1, KL);
+  o.g2 = site_sum(o.g2, KL);
+  o.gs = site_sum(o.gs, KL);
+  if (ln.ph != 0) return;
+  gmem(S.gown)[s] = make_double4(o.g0, o.g1, o.g2, o.gs);
+  gmem(S.epair)[s] = o.e;
+}
+
+__global__ __launch_bounds__(TB) void k_gen_grad_recv(const LatDev* __restrict__ lat) {
+  __shared__ double red[TB];
+  const LatDev& S = *lat;
+  const int lb = xcd_block();
+  const int s = lb * TB + threadIdx.x;
+  double fs = 0.0;
+  if (s < S.npd + S.nh) {
+    const bool pd = s < S.npd;
+    const int row = pd ? s : s - S.npd;
+    const size_t site = pd ? site_of_row(row, S.npd) : S.npd + site_of_row(row, S.nh);
+    double4 gr = S.gown[s];
+#pragma unroll
+    for (int side = 0; side < 2; ++side) {
+      const Ell& L = pd ? (side ? S.pdh : S.pdpd) : (side ? S.hh : S.hpd);
+      for_row_shares<RECV_RU_WIDE>(gmem(reinterpret_cast<const double4*>(L.rbuf)), L.rows, row, L.rcnt[row],
+                                   [&](const double4& v) {
+                                     gr.x += v.x; gr.y += v.y; gr.z += v.z;
+                                     gr.w += v.w;
+                                   });
     }
-    // V share of site s: embedding + half of every pair (minimizer.cpp:169-286)
-    const double V = S.emb[s] + 0.5 * xi * e;
-    const double T = S.T;
-    const double sc = xi / T;
-    double* __restrict__ G = S.G;
-    G[4 * (size_t)s + 0] = sc * gq[0];
-    G[4 * (size_t)s + 1] = sc * gq[1];
-    G[4 * (size_t)s + 2] = sc * gq[2];
-    G[4 * (size_t)s + 3] = sc * gs - 3.0 * KB * xi / a.s;
-    fs = V / T - 3.0 * KB * xi * log(a.s);
+    const double xi = pd ? 1.0 : S.xrow[row];
+    const double sg = S.qzs[s].y;
+    const double T = S.T, sc = xi / T;
+    const double V = S.emb[s] + xi * S.epair[s];  // owned pairs carry their full energy (minimizer.cpp:169-286)
+    double* __restrict__ G = S.G + 4 * site;  // the caller's: 8-byte aligned
+    G[0] = sc * gr.x;
+    G[1] = sc * gr.y;
+    G[2] = sc * gr.z;
+    G[3] = sc * gr.w - 3.0 * KB * xi / sg;
+    fs = V / T - 3.0 * KB * xi * log(sg);
   }
   red[threadIdx.x] = fs;
   __syncthreads();
@@ -328,12 +486,12 @@ __global__ __launch_bounds__(TB) void k_gen_chem(const LatDev* __restrict__ lat,
                                                  const double* __restrict__ corr, double ch0, double ch1, double ch2,
                                                  double ch3, double gamma_bd, double* __restrict__ gamma,
                                                  int32_t* __restrict__ full) {
-  __shared__ double nd[A2C_QUAD_MAX_NODES * 7];
-  stage_nodes(nd, g);
+  const double* nd = stage_nodes<double>(g);
   const LatDev& S = *lat;
   const int a = blockIdx.x * TB + threadIdx.x;
   if (a >= S.nh || full[a] == 1) return;  // fully occupied reservoir: gamma untouched
-  const RFun<POT, double> fun{g};
+  const RFun<POT, double> fun(g);
+  const Image img = image_of(S);
   const double* __restrict__ X = S.X;
   const double* __restrict__ xo = S.x;
   const double* __restrict__ Fp = S.Fp;
@@ -355,16 +513,16 @@ __global__ __launch_bounds__(TB) void k_gen_chem(const LatDev* __restrict__ lat,
       const int j = side == 0 ? jl : S.npd + jl;
       const Site b = load_site(X, j);
       double d[3];
-      pair_vec(S, si, b, d);
+      pair_vec(img, si, b, d);
       const PairFrame<double> f = frame<double>(g, d, si.s, b.s);
       double sf = 0.0, sp = 0.0;
       for (int k = 0; k < K; ++k) {
-        double r[3];
-        node_r(f, nd, k, r);
-        const double rn = sqrt(r[0] * r[0] + r[1] * r[1] + r[2] * r[2]);
-        const double w = nd[7 * k + 6];
-        sf += w * fun.val(GEN_RHO_H, rn);
-        sp += w * fun.val(side == 0 ? GEN_RPHI_PDH : GEN_RPHI_H, rn);
+        const double* n = nd + 8 * k;
+        double r[3], rn, ri;
+        root(node_r2(f, n, r), rn, ri);
+        const At<double> at = fun.at(rn, ri);
+        sf += n[6] * fun.template val<GEN_S_RHO_H>(at);
+        sp += n[6] * (side == 0 ? fun.template val<GEN_S_RPHI_PDH>(at) : fun.template val<GEN_S_RPHI_H>(at));
       }
       const double term = Fp[j] * sf + sp + corr[j];
       sum += side == 0 ? term : xo[jl] * term;
@@ -392,26 +550,42 @@ auto pick(const GenDev& g, int deriv_mode, bool fp32) {
   if (fp32) return tab ? Pick<1, A2C_DERIV_ANALYTIC, float>::fn : Pick<0, A2C_DERIV_ANALYTIC, float>::fn;
   return tab ? Pick<1, A2C_DERIV_ANALYTIC, double>::fn : Pick<0, A2C_DERIV_ANALYTIC, double>::fn;
 }
-template <int P, int D, class R> struct DensK { static constexpr auto fn = k_gen_density<P, D, R>; };
-template <int P, int D, class R> struct GradK { static constexpr auto fn = k_gen_grad<P, D, R>; };
+template <int P, int D, class R> struct DensK { static constexpr auto fn = k_gen_dens_own<P, R>; };
+template <int P, int D, class R> struct RecvK { static constexpr auto fn = k_gen_dens_recv<P, D>; };
+template <int P, int D, class R> struct GradK { static constexpr auto fn = k_gen_grad_own<P, D, R>; };
 
-}  // namespace
+bool general_fp32(int deriv_mode, bool fp32) { return fp32 && deriv_mode != A2C_DERIV_FD; }
+size_t lds_bytes(const GenDev& g, int deriv_mode, bool fp32) {
+  return general_fp32(deriv_mode, fp32) ? node_bytes<float>(g) : node_bytes<double>(g);
+}
 
-int run_density_gen(const LatDev* dlat, int N, const GenDev& g, int deriv_mode, double eps, hipStream_t st) {
-  if (N <= 0) return A2C_OK;
-  // the density feeding F' is FP64 in both precisions
-  hipLaunchKernelGGL(pick<DensK>(g, deriv_mode, false), dim3(site_blocks(N)), dim3(TB), 0, st, dlat, g, eps);
+// rho, F(rho), F'(rho) and the embedding energy at the state of *dlat.
+int run_density_gen(const LatDev* dlat, int npd, int nh, const GenDev& g, int deriv_mode, double eps, bool fp32,
+                    bool by_site, hipStream_t st, Timing* tm) {
+  if (npd + nh <= 0) return A2C_OK;
+  const int nblk = site_blocks(npd + nh), KL = lanes_per_site(npd + nh, true);
+  if (tm) tm->mark(st, "rows");
+  hipLaunchKernelGGL(k_gen_rows, dim3(nblk), dim3(TB), 0, st, dlat);
+  if (tm) tm->mark(st, "gen_dens_own");
+  hipLaunchKernelGGL(pick<DensK>(g, deriv_mode, fp32), dim3(owner_units(npd, nh, KL)), dim3(TB),
+                     lds_bytes(g, deriv_mode, fp32), st, dlat, g, KL);
+  if (tm) tm->mark(st, "gen_dens_recv");
+  hipLaunchKernelGGL(pick<RecvK>(g, deriv_mode, fp32), dim3(nblk), dim3(TB), 0, st, dlat, g, eps, (int)by_site);
   return hipGetLastError() == hipSuccess ? A2C_OK : A2C_EHIP;
 }
 
-int run_eval_gen(const LatDev* dlat, int N, const GenDev& g, int deriv_mode, double eps, bool fp32, hipStream_t st,
-                 Timing* tm) {
-  const int nblk = site_blocks(N);
-  if (nblk > 0) {
-    if (tm) tm->mark(st, "gen_density");
-    hipLaunchKernelGGL(pick<DensK>(g, deriv_mode, fp32), dim3(nblk), dim3(TB), 0, st, dlat, g, eps);
-    if (tm) tm->mark(st, "gen_grad");
-    hipLaunchKernelGGL(pick<GradK>(g, deriv_mode, fp32), dim3(nblk), dim3(TB), 0, st, dlat, g, eps);
+}  // namespace
+
+int run_eval_gen(const LatDev* dlat, int npd, int nh, const GenDev& g, int deriv_mode, double eps, bool fp32,
+                 hipStream_t st, Timing* tm) {
+  if (npd + nh > 0) {
+    const int nblk = site_blocks(npd + nh), KL = lanes_per_site(npd + nh, true);
+    if (int rc = run_density_gen(dlat, npd, nh, g, deriv_mode, eps, fp32, false, st, tm)) return rc;
+    if (tm) tm->mark(st, "gen_grad_own");
+    hipLaunchKernelGGL(pick<GradK>(g, deriv_mode, fp32), dim3(owner_units(npd, nh, KL)), dim3(TB),
+                       lds_bytes(g, deriv_mode, fp32), st, dlat, g, eps, KL);
+    if (tm) tm->mark(st, "gen_grad_recv");
+    hipLaunchKernelGGL(k_gen_grad_recv, dim3(nblk), dim3(TB), 0, st, dlat);
     if (hipGetLastError() != hipSuccess) return A2C_EHIP;
   }
   if (tm) tm->mark(st, "final_sum");
@@ -426,14 +600,16 @@ int run_eval_gen(const LatDev* dlat, int N, const GenDev& g, int deriv_mode, dou
 
 int launch_density_gen(a2c_fe_ctx* c, const double* dX) {
   if (int rc = sync_lattice(c, dX, c->dG, c->dF)) return rc;
-  if (run_density_gen(c->dlat, c->N, c->gen, c->desc.deriv_mode, c->desc.fd_eps, c->stream))
+  // the density feeding F' is FP64 in both precisions
+  if (run_density_gen(c->dlat, c->desc.n_pd, c->desc.n_h, c->gen, c->desc.deriv_mode, c->desc.fd_eps, false, true,
+                      c->stream, nullptr))
     return set_err(c, A2C_EHIP, "general density launch failed");
   return A2C_OK;
 }
 
 int launch_eval_gen(a2c_fe_ctx* c, const double* dX, double* dG, double* dF, bool timed, Timing* tm) {
   if (int rc = sync_lattice(c, dX, dG, dF)) return rc;
-  if (run_eval_gen(c->dlat, c->N, c->gen, c->desc.deriv_mode, c->desc.fd_eps,
+  if (run_eval_gen(c->dlat, c->desc.n_pd, c->desc.n_h, c->gen, c->desc.deriv_mode, c->desc.fd_eps,
                    c->desc.precision == A2C_PREC_MIXED, c->stream, timed ? tm : nullptr))
     return set_err(c, A2C_EHIP, "general eval launch failed");
   return A2C_OK;
@@ -444,8 +620,8 @@ int launch_chem_gen(a2c_fe_ctx* c, const double* dX, const double* coe_h, double
   (void)dX;  // the descriptor already points at dX (launch_density_gen)
   const int nh = c->desc.n_h;
   if (nh <= 0) return A2C_OK;
-  hipLaunchKernelGGL(c->gen.pot == 1 ? k_gen_chem<1> : k_gen_chem<0>, dim3((nh + TB - 1) / TB), dim3(TB), 0,
-                     c->stream, (const LatDev*)c->dlat, c->gen, dcorr, coe_h[0], coe_h[1], coe_h[2], coe_h[3],
+  hipLaunchKernelGGL(c->gen.pot == 1 ? k_gen_chem<1> : k_gen_chem<0>, dim3((nh + TB - 1) / TB), dim3(TB),
+                     node_bytes<double>(c->gen), c->stream, (const LatDev*)c->dlat, c->gen, dcorr, coe_h[0], coe_h[1], coe_h[2], coe_h[3],
                      gamma_bd, dgam, dfull);
   A2C_HIP(c, hipGetLastError());
   return A2C_OK;

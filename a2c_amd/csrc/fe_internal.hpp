@@ -210,12 +210,23 @@ __device__ inline void gh_node(int k, double z[3], double& w) {
 // and the rule as a node table.  Function order: F_Pd, F_H (embedding),
 // f_Pd, f_H (density), r phi_PdPd, r phi_PdH, r phi_HH (pair).
 enum { GEN_F_PD = 0, GEN_F_H, GEN_RHO_PD, GEN_RHO_H, GEN_RPHI_PD, GEN_RPHI_PDH, GEN_RPHI_H, GEN_NFN };
+// An embedding function: cubic pieces on its grid.
 struct GenFn {
   int32_t n = 0;        // nodes (n - 1 pieces), node k at k * h
-  int32_t off = 0;      // first piece in the coefficient arrays
+  int32_t off = 0;      // first piece in the coefficient array
   double ih = 0.0;      // 1 / h
-  double yend = 0.0;    // value and slope at the last node (embedding
-  double dend = 0.0;    // functions continue along it)
+  double yend = 0.0;    // value and slope at the last node (the function
+  double dend = 0.0;    // continues along it)
+};
+// The five r-functions share one grid and one table row per node (80 bytes),
+// so that a radius is located once and the two or three functions a pair needs
+// lie next to each other: r phi_PdPd f_Pd | r phi_PdH | f_H r phi_HH.
+enum { GEN_S_RPHI_PD = 0, GEN_S_RHO_PD, GEN_S_RPHI_PDH, GEN_S_RHO_H, GEN_S_RPHI_H, GEN_NS };
+template <class E>
+struct GenR {
+  const E* row = nullptr;  // GEN_NS entries per node (pieces: per interval, plus one unused row)
+  int32_t n = 0;           // nodes
+  double ih = 0.0;         // 1 / h
 };
 struct GenDev {
   int32_t pot = 0;      // 0: compiled-in Pd-H closed forms; 1: tabulated
@@ -224,10 +235,10 @@ struct GenDev {
                         //    s^2 = sigma_i^2 + sigma_j^2 (the Gauss-Hermite rule);
                         // 0: 6-D nodes, r = d + sqrt(2) (sigma_i xi1 - sigma_j xi2)
   const double* nodes = nullptr;  // K x 8: xi1[3] (or z), xi2[3], w, 0
-  const double4* tab = nullptr;   // FP64 piece coefficients (c0..c3 in u = x/h - k)
-  const float4* tab32 = nullptr;  // FP32 pieces of the five r-functions (mixed)
-  GenFn fn[GEN_NFN];
-  GenFn fn32[GEN_NFN];  // the FP32 pieces' grids (f_Pd .. r phi_HH)
+  const double4* tab = nullptr;   // embedding pieces (c0..c3 in u = x/h - k)
+  GenFn fn[2];                    // GEN_F_PD, GEN_F_H
+  GenR<double2> r64;  // FP64: node value and slope (times h); the pieces' coefficients follow from two nodes
+  GenR<float4> r32;   // FP32 (mixed): c0..c3 of each piece, rounded from FP64
 };
 
 // Minimum-image geometry of one lattice, copied out of its descriptor into
@@ -377,9 +388,10 @@ struct a2c_fe_ctx {
   bool gen_table_rule = false;  // a node table was set (else the descriptor's rule)
   a2c::GenDev gen{};
   double* gen_nodes = nullptr;  // device: K x 8
-  double4* gen_tab = nullptr;   // device: FP64 pieces
-  float4* gen_tab32 = nullptr;  // device: FP32 pieces
-  size_t gen_tab_n = 0, gen_tab32_n = 0;
+  double4* gen_tab = nullptr;   // device: embedding pieces
+  double2* gen_r64 = nullptr;   // device: r-functions, FP64
+  float4* gen_r32 = nullptr;    // device: r-functions, FP32
+  size_t gen_tab_n = 0, gen_r64_n = 0, gen_r32_n = 0;
 
   a2c::DevSys sys() const {
     a2c::DevSys s;
@@ -469,8 +481,7 @@ struct DeviceTables {
 hipError_t device_tables(int device, DeviceTables* out);
 int host_staging(a2c_fe_ctx* c);  // pinned hX, hG of the host-array entry points (capi.cpp)
 // General model (evalgen.hip, general.cpp)
-int run_density_gen(const LatDev* dlat, int N, const GenDev& g, int deriv_mode, double eps, hipStream_t st);
-int run_eval_gen(const LatDev* dlat, int N, const GenDev& g, int deriv_mode, double eps, bool fp32, hipStream_t st,
+int run_eval_gen(const LatDev* dlat, int npd, int nh, const GenDev& g, int deriv_mode, double eps, bool fp32, hipStream_t st,
                  Timing* tm);
 int launch_density_gen(a2c_fe_ctx* c, const double* dX);  // fills drho, dFp, demb
 int launch_eval_gen(a2c_fe_ctx* c, const double* dX, double* dG, double* dF, bool timed, Timing* tm);

@@ -10,6 +10,7 @@
 // second and second-to-last node, one-sided at the ends.  This is the
 // interpolation the setfl format is written for; it reproduces cubics
 // exactly on every interval not touching the two end intervals at either side.
+#include <algorithm>
 #include <cmath>
 #include <cstring>
 #include <fstream>
@@ -25,7 +26,8 @@ namespace a2c {
 namespace {
 
 struct Pieces {
-  std::vector<double> c;  // 4 per interval
+  std::vector<double> c;     // 4 per interval
+  std::vector<double> y, s;  // node values and slopes (times h)
   int n = 0;              // nodes
   double h = 0.0, yend = 0.0, dend = 0.0;
 };
@@ -51,8 +53,10 @@ bool make_pieces(const double* y, int n, double h, Pieces& P) {
     c[2] = 3.0 * dy - 2.0 * s[m] - s[m + 1];
     c[3] = s[m] + s[m + 1] - 2.0 * dy;
   }
+  P.y.assign(y, y + n);
   P.yend = y[n - 1];
   P.dend = s[n - 1] / h;
+  P.s = std::move(s);
   return true;
 }
 
@@ -92,41 +96,50 @@ int upload(a2c_fe_ctx* c, T** dst, size_t& cap, const std::vector<T>& v) {
   return A2C_OK;
 }
 
-// Pieces of the seven functions (FP64) and of the five r-functions (FP32);
-// fn[] null for the closed forms: FP64 kernels evaluate those directly.
+// Tables of the embedding functions (FP64 pieces) and of the five r-functions
+// (FP64 nodes, FP32 pieces); fn[] null for the closed forms: FP64 kernels
+// evaluate those directly.
 int install_potential(a2c_fe_ctx* c, const Pieces* fn) {
-  std::vector<double4> t64;
+  static const int slot_fn[GEN_NS] = {GEN_RPHI_PD, GEN_RHO_PD, GEN_RPHI_PDH, GEN_RHO_H, GEN_RPHI_H};
+  std::vector<double4> emb;
+  std::vector<double2> t64;
   std::vector<float4> t32;
   GenDev& g = c->gen;
   Pieces cf[GEN_NFN];
-  if (fn) {
-    for (int f = 0; f < GEN_NFN; ++f) {
-      set_fn(g.fn[f], fn[f], (int)t64.size());
-      for (int m = 0; m + 1 < fn[f].n; ++m) {
-        const double* q = &fn[f].c[4 * (size_t)m];
-        t64.push_back(make_double4(q[0], q[1], q[2], q[3]));
-      }
-    }
-  } else {
+  const bool tab = fn != nullptr;
+  if (!tab) {
     std::vector<double> y(CF_N);
     for (int f = GEN_RHO_PD; f < GEN_NFN; ++f) {
       for (int k = 0; k < CF_N; ++k) y[k] = closed_r_function(f, k * CF_H);
       make_pieces(y.data(), CF_N, CF_H, cf[f]);
     }
     fn = cf;
-    t64.push_back(make_double4(0, 0, 0, 0));  // unused by the closed-form FP64 kernels
+    emb.push_back(make_double4(0, 0, 0, 0));  // unused by the closed-form kernels
+    t64.push_back(make_double2(0, 0));
   }
-  for (int f = GEN_RHO_PD; f < GEN_NFN; ++f) {
-    set_fn(g.fn32[f], fn[f], (int)t32.size());
+  for (int f = 0; tab && f < GEN_RHO_PD; ++f) {
+    set_fn(g.fn[f], fn[f], (int)emb.size());
     for (int m = 0; m + 1 < fn[f].n; ++m) {
       const double* q = &fn[f].c[4 * (size_t)m];
-      t32.push_back(make_float4((float)q[0], (float)q[1], (float)q[2], (float)q[3]));
+      emb.push_back(make_double4(q[0], q[1], q[2], q[3]));
     }
   }
-  if (int rc = upload(c, &c->gen_tab, c->gen_tab_n, t64)) return rc;
-  if (int rc = upload(c, &c->gen_tab32, c->gen_tab32_n, t32)) return rc;
+  const int n = fn[GEN_RHO_PD].n;
+  for (int m = 0; m < n; ++m)
+    for (int s = 0; s < GEN_NS; ++s) {
+      const Pieces& P = fn[slot_fn[s]];
+      if (tab) t64.push_back(make_double2(P.y[m], P.s[m]));
+      const double* q = &P.c[4 * (size_t)std::min(m, n - 2)];
+      t32.push_back(make_float4((float)q[0], (float)q[1], (float)q[2], (float)q[3]));
+    }
+  if (int rc = upload(c, &c->gen_tab, c->gen_tab_n, emb)) return rc;
+  if (int rc = upload(c, &c->gen_r64, c->gen_r64_n, t64)) return rc;
+  if (int rc = upload(c, &c->gen_r32, c->gen_r32_n, t32)) return rc;
   g.tab = c->gen_tab;
-  g.tab32 = c->gen_tab32;
+  g.r64.row = c->gen_r64;
+  g.r32.row = c->gen_r32;
+  g.r64.n = g.r32.n = n;
+  g.r64.ih = g.r32.ih = 1.0 / fn[GEN_RHO_PD].h;
   return A2C_OK;
 }
 
@@ -181,7 +194,7 @@ int refresh(a2c_fe_ctx* c) {
     rule_nodes(c->desc.quad_rule, nd, rel);
     if (int rc = install_nodes(c, nd, rel)) return rc;
   }
-  if (c->gen_on && !c->gen_tab32)  // the closed forms' FP32 pieces
+  if (c->gen_on && !c->gen_r32)  // the closed forms' FP32 pieces
     if (int rc = install_potential(c, nullptr)) return rc;
   c->lat_dirty = true;
   return A2C_OK;
@@ -256,11 +269,13 @@ const std::vector<double>& pair_table(const Setfl& s, int a, int b) {
 void gen_free(a2c_fe_ctx* c) {
   dfree(c->gen_nodes);
   dfree(c->gen_tab);
-  dfree(c->gen_tab32);
+  dfree(c->gen_r64);
+  dfree(c->gen_r32);
   c->gen_nodes = nullptr;
   c->gen_tab = nullptr;
-  c->gen_tab32 = nullptr;
-  c->gen_tab_n = c->gen_tab32_n = 0;
+  c->gen_r64 = nullptr;
+  c->gen_r32 = nullptr;
+  c->gen_tab_n = c->gen_r64_n = c->gen_r32_n = 0;
 }
 
 }  // namespace a2c

@@ -23,6 +23,17 @@ __device__ __forceinline__ Site load_row(const A2C_GLOBAL double2* __restrict__ 
   return {{a.x, a.y, b.x}, b.y};
 }
 
+// the state and occupancy of site s to their place in row order
+__device__ __forceinline__ void copy_row(const LatDev& S, int s) {
+  const double4 v = reinterpret_cast<const double4*>(S.X)[s];
+  const bool pd = s < S.npd;
+  const int row = pd ? row_of_site(s, S.npd) : row_of_site(s - S.npd, S.nh);
+  const int p = pd ? row : S.npd + row;
+  S.qxy[p] = make_double2(v.x, v.y);
+  S.qzs[p] = make_double2(v.z, v.w);
+  if (!pd) S.xrow[row] = S.x[s - S.npd];
+}
+
 // Owned pairs of one list of one row, K lanes per row.  Software pipeline: at
 // a pair's turn the state of the next one and the index and slot of the one
 // after it are requested, then the pair is evaluated and its share stored.
