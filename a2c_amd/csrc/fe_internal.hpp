@@ -74,8 +74,8 @@ struct Ell {
   // by the partner's occupancy) and summed by this row's receive pass of the
   // same evaluation: rwidth * rows entries of a float (density) or float4
   // (gradient) in the mixed passes, a double or double4 in the FP64 passes --
-  // one buffer serves all four.  During the split it holds the map full-row
-  // slot -> received slot.
+  // one buffer serves all four.  During the build it holds the received
+  // half's site indices.
   void* rbuf = nullptr;
   int64_t ocap = 0;            // allocated entries of oj/orv
   int64_t bcap = 0;            // allocated bytes of rbuf

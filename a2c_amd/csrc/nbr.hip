@@ -12,16 +12,15 @@
 // after the count pass, the totals at the end):
 //   k_bin     cell of each site and the cell histogram
 //   k_scan    exclusive scan of the histogram (one workgroup)
-//   k_place   positions copied into cell order (with the site index), so a
-//             candidate is one load; three x-adjacent cells of a stencil row
-//             are one contiguous range
-//   k_site<false>  one lane per site: the candidates of its 27 cells (four
-//             loads in flight), row lengths, the owned/received split of each
-//             pair list, and their maxima
-//   k_site<true>   the same walk keeps each hit (neighbor index and shell
-//             bits) in the lane's LDS column; the wave sorts each row by
-//             ranking, then writes the rows slot by slot, 64 consecutive
-//             rows per store
+//   k_place   positions as floats in cell order, with the site index, so a
+//             candidate is one 16-byte load
+//   k_site<false>  one wave per site: its 27 cells' candidates filtered in FP32,
+//             the survivors tested in FP64; row lengths, the owned/received
+//             split of each pair list, and their maxima
+//   k_site<true>   the same walk keeps each hit (neighbor index and flags); the
+//             wave ranks the row's hits, then the workgroup writes its 32
+//             rows and their owned and received halves slot by slot
+//   k_orv     the owned pairs' slots in their partners' received halves
 // Rows come out sorted whatever order the cell placement used.
 #pragma clang fp contract(off)
 
@@ -87,30 +86,42 @@ __global__ __launch_bounds__(SCAN_T) void k_scan(const int* cnt, int n, int* __r
   if (threadIdx.x == SCAN_T - 1) start[n] = sm[SCAN_T - 1];
 }
 
-// positions in cell order, the site index in .w (exact in a double)
-__global__ void k_place(const double* __restrict__ X, int N, const int* __restrict__ cid, int* __restrict__ cursor,
-                        double4* __restrict__ qs) {
+// Position on one axis relative to the grid: wrapped into [0, L) or from the
+// lower bound, as a float (the filter's margin covers its rounding).
+__device__ __forceinline__ float grid_pos(const Grid& g, double x, int c) {
+  return (float)(g.periodic[c] ? x - g.box[c] * floor(x / g.box[c]) : x - g.lo[c]);
+}
+
+// positions in cell order, the site index in .w (its bits)
+__global__ void k_place(const double* __restrict__ X, int N, Grid g, const int* __restrict__ cid,
+                        int* __restrict__ cursor, float4* __restrict__ qs) {
   const int s = blockIdx.x * blockDim.x + threadIdx.x;
   if (s >= N) return;
   const int pos = atomicAdd(&cursor[cid[s]], 1);
-  qs[pos] = make_double4(X[4 * s], X[4 * s + 1], X[4 * s + 2], (double)s);
+  qs[pos] = make_float4(grid_pos(g, X[4 * s], 0), grid_pos(g, X[4 * s + 1], 1), grid_pos(g, X[4 * s + 2], 2),
+                        __int_as_float(s));
 }
 
 struct NbrArgs {
   const double* X;
-  const double4* qs;   // cell-ordered positions
+  const float4* qs;    // cell-ordered positions
   int npd, N;
   Grid g;
   double ibox[3];
+  double in0, in01;    // 1 / cells per row, 1 / cells per layer
+  float fbox[3], fibox[3];  // periodic axes: L and 1 / L, else 0
+  float rcf2;          // square of rc and the filter's margin
   const int* cid;
   const int* cstart;
   double rc2, sh1, sh2;
   int cap;
-  int width;           // fill pass: LDS slots per lane (the longest row)
+  int width;           // fill pass: LDS slots per row (the longest row)
   int32_t* cnt[5];     // row lengths: PdPd, PdH (Pd rows); HPd, HH, HH1 (H rows)
   int32_t* ocnt[4];    // owned entries of the four pair lists
   int32_t* rcnt[4];    // received entries
   int32_t* idx[5];     // ELL arrays (fill pass)
+  int32_t* oj[4];      // owned halves (fill pass; null: no split wanted)
+  int32_t* rj[4];      // received halves, species-local site indices (for k_orv)
   int32_t* pdpdnum;    // nPd*3 (fill pass)
   int32_t* maxw;       // 14 ints: width of the 5 lists, owned widths of the 4 pair lists, received
                        // widths, max total (count pass)
@@ -133,50 +144,22 @@ __device__ __forceinline__ double wrap(double d, double L, double iL) {
   return d - L * rint(fabs(f - 0.5) < 1e-9 ? d / L : q);
 }
 
-// Candidates of one stencil row (dy, dz) of cell (cx, cy, cz): the x cells
-// cx-1..cx+1 are consecutive cell indices, one range [b0, e0), unless the
-// row wraps a periodic x boundary (a second range [b1, e1)).  Axes with one
-// or two cells contribute each cell once.
-__device__ __forceinline__ void row_ranges(const NbrArgs& a, int cx, int yy, int zz, int& b0, int& e0, int& b1,
-                                           int& e1) {
-  const int n0 = a.g.nc[0];
-  const int base = (zz * a.g.nc[1] + yy) * n0;
-  int x0, x1, y0 = 0, y1 = -1;  // [x0, x1], then [y0, y1] (inclusive cell ranges)
-  if (n0 < 3) {
-    x0 = 0; x1 = n0 - 1;
-  } else if (a.g.periodic[0] && cx == 0) {
-    x0 = 0; x1 = 1; y0 = n0 - 1; y1 = n0 - 1;
-  } else if (a.g.periodic[0] && cx == n0 - 1) {
-    x0 = n0 - 2; x1 = n0 - 1; y0 = 0; y1 = 0;
-  } else {
-    x0 = max(cx - 1, 0); x1 = min(cx + 1, n0 - 1);
-  }
-  b0 = a.cstart[base + x0];
-  e0 = a.cstart[base + x1 + 1];
-  if (y1 >= y0) {
-    b1 = a.cstart[base + y0];
-    e1 = a.cstart[base + y1 + 1];
-  } else {
-    b1 = e1 = 0;
-  }
-}
-
 // stencil coordinate k in 0..2 of axis ax around c: the wrapped (periodic)
 // or clipped (-1: outside) cell, each distinct cell once
 __device__ __forceinline__ int stencil_axis(const NbrArgs& a, int ax, int c, int k) {
   const int n = a.g.nc[ax];
   if (a.g.periodic[ax]) {
     if (n == 1) return k == 1 ? 0 : -1;  // periodic axes have 1 or >= 3 cells
-    return (c + k - 1 + n) % n;
+    const int v = c + k - 1;
+    return v < 0 ? v + n : v >= n ? v - n : v;
   }
   const int v = c + k - 1;
   return (v >= 0 && v < n) ? v : -1;
 }
 
-constexpr int NT = 64;  // sites (rows) per workgroup of the site passes: one lane each
+constexpr int NT = 64;  // rows per workgroup of k_refresh: one lane each
 constexpr int CS = NT + 1;  // LDS: slot t of lane l at t * CS + l (a column and a slot row are both
                             // conflict-free)
-constexpr int MAXK = NBR_CAP / NT;  // keys of one row per lane in the ranking sort
 
 // Build counters (list widths and totals) in SPREAD copies, a workgroup
 // adding to copy blockIdx % SPREAD: tens of thousands of atomics on one
@@ -193,128 +176,223 @@ constexpr size_t MISC_BYTES = MISC_BBOX + 6 * sizeof(unsigned long long);
 __device__ __forceinline__ int32_t* maxw_copy(int32_t* m) { return m + (blockIdx.x % SPREAD) * 16; }
 __device__ __forceinline__ unsigned long long* tot_copy(unsigned long long* t) { return t + (blockIdx.x % SPREAD) * 5; }
 
-// Sort each row of the wave (lane l's row in LDS column l) by key, one row at
-// a time: every lane ranks its (at most K) keys of the row against all of the
-// row's keys, read by broadcast, then writes them to their ranks (keys are
-// distinct, so the ranks are a permutation).
-template <int K>
-__device__ __forceinline__ void rank_rows(uint32_t* buf, int n, int lane) {
-  for (int rl = 0; rl < NT; ++rl) {
-    const int nr = __shfl(n, rl);
-    if (nr < 2) continue;
-    uint32_t mine[K];
-    int rk[K];
-#pragma unroll
-    for (int q = 0; q < K; ++q) {
-      const int t = lane + NT * q;
-      mine[q] = t < nr ? buf[t * CS + rl] : 0u;
-      rk[q] = 0;
+// Orders a wave's own LDS writes before its reads of other lanes' words.
+__device__ __forceinline__ void wave_lds() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+__device__ __forceinline__ int below(uint64_t mask) {  // set bits of mask under this lane
+  return __builtin_amdgcn_mbcnt_hi((uint32_t)(mask >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)mask, 0));
+}
+
+// n distinct keys (16-byte aligned, padded to a multiple of four with words of
+// ones): the key of rank r to out[r * RS].
+constexpr int SR = 32, SW = 8, ST = 64 * SW;  // rows, waves and lanes per workgroup of k_site
+constexpr int RS = SR + 1;  // LDS: slot t of row l at t * RS + l (a column and a slot row are both conflict-free)
+__device__ __forceinline__ void rank_keys(const uint32_t* keys, int n, uint32_t* out, int lane) {
+  for (int q = 0; q < n; q += 64) {
+    const bool in = q + lane < n;
+    const uint32_t mine = in ? keys[q + lane] : 0u;
+    int rk = 0;
+    for (int t = 0; t < n; t += 4) {
+      const uint4 o = *reinterpret_cast<const uint4*>(keys + t);
+      rk += (o.x < mine) + (o.y < mine) + (o.z < mine) + (o.w < mine);
     }
-    for (int t = 0; t < nr; ++t) {
-      const uint32_t o = buf[t * CS + rl];
-#pragma unroll
-      for (int q = 0; q < K; ++q) rk[q] += o < mine[q];
-    }
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-#pragma unroll
-    for (int q = 0; q < K; ++q)
-      if (lane + NT * q < nr) buf[rk[q] * CS + rl] = mine[q];
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    if (in) out[rk * RS] = mine;
   }
 }
 
-// One lane per site (consecutive rows of one species per workgroup; Pd-row
-// workgroups first).  Each lane walks the candidates of its 27 cells from
-// the cell-ordered copy, four loads in flight.  Count pass (FILL = false):
-// row lengths, owned/received counts and their maxima.  Fill pass: each hit's
-// key (j << 2 | shell bits) goes into the lane's LDS column
-// (slot t of lane l at t * CS + l) in the order found, the wave ranks each
-// row's keys (the rows sorted by neighbor index), then the rows are written
-// slot by slot: 64 consecutive rows per store, one 256-byte line.
+// One wave per site, SR consecutive rows of one species per workgroup
+// (Pd-row workgroups first), SR / SW sites in turn to a wave.  The site's cells
+// share the wave's lanes evenly; each lane walks its cell's candidates, four
+// loads in flight, in FP32 against rc plus a margin that covers the floats'
+// rounding, and the survivors queue in LDS for the exact FP64 test, 64 at a time.
+// Count pass (FILL = false): row lengths, owned/received counts and their
+// maxima.  Fill pass: each hit's key (j << 2 | owned << 1 | first shell), Pd and
+// H apart, is ranked among the row's and goes to the row's LDS column, with the
+// order of the owned and received halves beside it; the workgroup then writes
+// lists and halves slot by slot, SR consecutive rows per store.
+// With one lane per site both passes were bound by latency at every size below
+// 50,000 sites, and by the divergent loads above (count / fill pass, then the
+// split, now part of the fill, and k_orv): 32,640 sites 322 / 467 / 70 / 231 us,
+// now 64 / 90 / - / 12; 262,144 sites at rc + 0.2 A 805 / 1648 us, now 405 / 591.
 template <bool FILL>
-__global__ __launch_bounds__(NT) void k_site(NbrArgs a, int nblk_pd) {
-  extern __shared__ uint32_t buf[];
-  const int lane = threadIdx.x;
-  const bool pdb = (int)blockIdx.x < nblk_pd;
-  const int nrows = pdb ? a.npd : a.N - a.npd;
-  const int row = (pdb ? (int)blockIdx.x : (int)blockIdx.x - nblk_pd) * NT + lane;
-  const bool live = row < nrows;
-  const int s = (pdb ? 0 : a.npd) + (live ? row : 0);
-  const A2C_GLOBAL double4* __restrict__ qs = gmem(a.qs);
-  int n = 0, npn = 0, nh1 = 0, op = 0, oh = 0, sh0 = 0, sh1n = 0;
-  if (live) {
-    const double qi0 = a.X[4 * (size_t)s], qi1 = a.X[4 * (size_t)s + 1], qi2 = a.X[4 * (size_t)s + 2];
-    const int c = a.cid[s];
-    const int cx = c % a.g.nc[0], cy = (c / a.g.nc[0]) % a.g.nc[1], cz = c / (a.g.nc[0] * a.g.nc[1]);
-    for (int kz = 0; kz < 3; ++kz) {
-      const int zz = stencil_axis(a, 2, cz, kz);
-      if (zz < 0) continue;
-      for (int ky = 0; ky < 3; ++ky) {
-        const int yy = stencil_axis(a, 1, cy, ky);
-        if (yy < 0) continue;
-        int b0, e0, b1, e1;
-        row_ranges(a, cx, yy, zz, b0, e0, b1, e1);
-        const int l0 = e0 - b0, tot = l0 + (e1 - b1);
-        for (int v0 = 0; v0 < tot; v0 += 4) {
-          double4 cq[4];
-#pragma unroll
-          for (int u = 0; u < 4; ++u) {
-            const int v = v0 + u;
-            cq[u] = make_double4(0.0, 0.0, 0.0, -1.0);
-            if (v < tot) cq[u] = qs[v < l0 ? b0 + v : b1 + (v - l0)];
+__global__ __launch_bounds__(ST) void k_site(NbrArgs a, int nblk_pd) {
+  extern __shared__ uint32_t buf[];  // fill pass: width columns' slots, then their halves' order (bytes)
+  __shared__ uint32_t queue[SW][128];
+  __shared__ __align__(16) uint32_t kp[SW][FILL ? NBR_CAP : 4], kh[SW][FILL ? NBR_CAP : 4];
+  __shared__ int2 cells[SW][32];
+  __shared__ int counts[7][SR];  // per row: Pd and H neighbors, owned ones, HH1, the Pd shells
+  const int tid = threadIdx.x, lane = tid & 63, wv = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int blk = xcd_block();
+  const bool pdb = blk < nblk_pd;
+  const int nrows = pdb ? a.npd : a.N - a.npd, soff = pdb ? 0 : a.npd;
+  const int row0 = (pdb ? blk : blk - nblk_pd) * SR;
+  uint8_t* const perm = reinterpret_cast<uint8_t*>(buf + (size_t)a.width * RS);
+  const A2C_GLOBAL float4* __restrict__ qs = gmem(a.qs);
+  const A2C_GLOBAL double4* __restrict__ X = gmem(reinterpret_cast<const double4*>(a.X));
+  const A2C_GLOBAL int* __restrict__ cstart = gmem(a.cstart);
+  const int kx = lane % 3, ky = (lane / 3) % 3, kz = lane / 9;  // lanes 0..26: the site's cells
+  uint32_t* const que = queue[wv];
+  for (int i = 0; i < SR / SW; ++i) {
+    const int rl = wv * (SR / SW) + i, row = row0 + rl;
+    int npn = 0, nhn = 0, op = 0, oh = 0, n1 = 0, sh0 = 0, sh1n = 0;
+    if (row < nrows) {
+      const int s = soff + row;
+      const double4 qi = X[s];
+      const float f0 = grid_pos(a.g, qi.x, 0), f1 = grid_pos(a.g, qi.y, 1), f2 = grid_pos(a.g, qi.z, 2);
+      // its cells that hold sites, a power of two of lanes to each
+      int start = 0, len = 0;
+      {
+        const int c = a.cid[s];
+        const int n0 = a.g.nc[0], n01 = n0 * a.g.nc[1];
+        const int cz = (int)(((double)c + 0.5) * a.in01), cyx = c - cz * n01;
+        const int cy = (int)(((double)cyx + 0.5) * a.in0), cx = cyx - cy * n0;
+        if (lane < 27) {
+          const int xx = stencil_axis(a, 0, cx, kx), yy = stencil_axis(a, 1, cy, ky), zz = stencil_axis(a, 2, cz, kz);
+          if (xx >= 0 && yy >= 0 && zz >= 0) {
+            const int e = zz * n01 + yy * n0 + xx;
+            start = cstart[e];
+            len = cstart[e + 1] - start;
           }
+        }
+      }
+      const uint64_t full = __ballot(len > 0);
+      const int m = __popcll(full);
+      const int lg = m > 1 ? 6 - (32 - __builtin_clz(m - 1)) : 6;  // log2 of the lanes per cell
+      if (len > 0) cells[wv][below(full)] = make_int2(start, len);
+      wave_lds();
+      const int g = lane >> lg;
+      const int2 mine = g < m ? cells[wv][g] : make_int2(0, 0);
+      int head = 0, qn = 0;
+      // exact test of the queue's first cnt (<= 64) candidates
+      auto drain = [&](int cnt) {
+        wave_lds();
+        const bool on = lane < cnt;
+        const int j = on ? (int)que[(head + lane) & 127] : s;
+        const double4 qj = X[j];
+        double d0 = qj.x - qi.x, d1 = qj.y - qi.y, dz = qj.z - qi.z;
+        if (a.g.periodic[0]) d0 = wrap(d0, a.g.box[0], a.ibox[0]);
+        if (a.g.periodic[1]) d1 = wrap(d1, a.g.box[1], a.ibox[1]);
+        if (a.g.periodic[2]) dz = wrap(dz, a.g.box[2], a.ibox[2]);
+        const double dd = d0 * d0 + d1 * d1 + dz * dz;
+        const bool hit = on && j != s && dd <= a.rc2, jpd = j < a.npd, own = pair_owner(s, j), first = dd < a.sh1;
+        const uint64_t mp = __ballot(hit && jpd), mh = __ballot(hit && !jpd), mo = __ballot(own), m1 = __ballot(first);
+        if (FILL && hit) {
+          const uint32_t key = ((uint32_t)j << 2) | (own ? 2u : 0u) | (first ? 1u : 0u);
+          const int at = jpd ? npn + below(mp) : nhn + below(mh);
+          if (at < NBR_CAP) (jpd ? kp : kh)[wv][at] = key;
+        }
+        npn += __popcll(mp);
+        nhn += __popcll(mh);
+        op += __popcll(mp & mo);
+        oh += __popcll(mh & mo);
+        n1 += __popcll(mh & m1);
+        if (FILL) {
+          sh0 += __popcll(mp & m1);
+          sh1n += __popcll(__ballot(hit && jpd && dd > a.sh1 && dd < a.sh2));
+        }
+        head = (head + cnt) & 127;
+        qn -= cnt;
+        wave_lds();
+      };
+      const int step = 1 << lg;
+      for (int e0 = lane & (step - 1); __ballot(e0 < mine.y); e0 += 4 * step) {
+        float4 cq[4];
 #pragma unroll
-          for (int u = 0; u < 4; ++u) {
-            const int j = (int)cq[u].w;
-            double d0 = cq[u].x - qi0, d1 = cq[u].y - qi1, dz = cq[u].z - qi2;
-            if (a.g.periodic[0]) d0 = wrap(d0, a.g.box[0], a.ibox[0]);
-            if (a.g.periodic[1]) d1 = wrap(d1, a.g.box[1], a.ibox[1]);
-            if (a.g.periodic[2]) dz = wrap(dz, a.g.box[2], a.ibox[2]);
-            const double d2 = d0 * d0 + d1 * d1 + dz * dz;
-            if (!(j >= 0 && j != s && d2 <= a.rc2)) continue;
-            const bool jpd = j < a.npd;
-            ++n;
-            if (jpd) ++npn;
-            if (!FILL) {
-              const bool own = pair_owner(s, j);
-              if (!jpd && d2 < a.sh1) ++nh1;
-              if (own) (jpd ? op : oh)++;
-            } else if (n <= a.width) {
-              if (jpd) {
-                if (d2 < a.sh1) ++sh0;
-                else if (d2 > a.sh1 && d2 < a.sh2) ++sh1n;
-              }
-              buf[(n - 1) * CS + lane] = ((uint32_t)j << 2) |
-                                         (jpd ? (d2 < a.sh1 ? 1u : ((d2 > a.sh1 && d2 < a.sh2) ? 2u : 0u))
-                                              : (d2 < a.sh1 ? 1u : 0u));
-            }
+        for (int u = 0; u < 4; ++u) {
+          const int e = e0 + u * step;
+          cq[u] = qs[mine.x + (e < mine.y ? e : 0)];
+        }
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+          float d0 = cq[u].x - f0, d1 = cq[u].y - f1, dz = cq[u].z - f2;
+          d0 = fmaf(-a.fbox[0], rintf(d0 * a.fibox[0]), d0);
+          d1 = fmaf(-a.fbox[1], rintf(d1 * a.fibox[1]), d1);
+          dz = fmaf(-a.fbox[2], rintf(dz * a.fibox[2]), dz);
+          const float dd = fmaf(d0, d0, fmaf(d1, d1, dz * dz));
+          const bool near = e0 + u * step < mine.y && !(dd > a.rcf2);  // NaN: left to the exact test
+          const uint64_t mask = __ballot(near);
+          if (near) que[(head + qn + below(mask)) & 127] = __float_as_uint(cq[u].w);
+          qn += __popcll(mask);
+          if (qn >= 64) drain(64);
+        }
+      }
+      if (qn > 0) drain(qn);
+      if (!FILL && lane == 0 && npn + nhn > a.cap) atomicOr(a.overflow, 1);
+      if (FILL && npn + nhn <= a.width) {
+        if (lane < 3 && npn + lane < NBR_CAP) kp[wv][npn + lane] = ~0u;
+        if (lane < 3 && nhn + lane < NBR_CAP) kh[wv][nhn + lane] = ~0u;
+        wave_lds();
+        rank_keys(kp[wv], npn, buf + rl, lane);
+        rank_keys(kh[wv], nhn, buf + (size_t)npn * RS + rl, lane);
+        wave_lds();
+        // order of the halves: owned Pd, received Pd, owned H, received H
+        const int n = npn + nhn;
+        int obp = 0, obh = 0, ob1 = 0;
+        for (int q = 0; q < n; q += 64) {
+          const int t = q + lane;
+          const uint32_t key = t < n ? buf[t * RS + rl] : 0u;
+          const bool own = (key & 2u) != 0, isp = t < npn;
+          const uint64_t mp = __ballot(own && isp), mh = __ballot(own && !isp);
+          const int bp = obp + below(mp), bh = obh + below(mh);
+          if (t < n) {
+            const int slot = isp ? (own ? bp : op + t - bp) : npn + (own ? bh : oh + t - npn - bh);
+            perm[slot * RS + rl] = (uint8_t)t;
+          }
+          obp += __popcll(mp);
+          obh += __popcll(mh);
+          if (!pdb) {  // HH1, in order
+            const uint64_t m1 = __ballot(t < n && !isp && (key & 1u));
+            if (t < n && !isp && (key & 1u))
+              a.idx[4][(size_t)(ob1 + below(m1)) * nrows + row] = (int)(key >> 2) - a.npd;
+            ob1 += __popcll(m1);
           }
         }
       }
     }
-    if (n > a.cap) atomicOr(a.overflow, 1);
+    if (lane == 0) {
+      counts[0][rl] = npn; counts[1][rl] = nhn; counts[2][rl] = op; counts[3][rl] = oh; counts[4][rl] = n1;
+      counts[5][rl] = sh0; counts[6][rl] = sh1n;
+    }
   }
-  const int nhn = n - npn;
+  __syncthreads();
+  const int rl = tid & (SR - 1), row = row0 + rl;
+  const int npn = counts[0][rl], nhn = counts[1][rl], op = counts[2][rl], oh = counts[3][rl], n1 = counts[4][rl];
   const int lp = pdb ? 0 : 2, lh = pdb ? 1 : 3;
+  const int p = row_of_site(row, nrows);
+  if (FILL && row < nrows && npn + nhn <= a.width) {
+    const int n = npn + nhn;
+    const bool split = a.oj[lp] != nullptr;
+    for (int t = tid / SR; t < n; t += ST / SR) {
+      const int j = (int)(buf[t * RS + rl] >> 2);
+      if (t < npn) a.idx[lp][(size_t)t * nrows + row] = j;
+      else a.idx[lh][(size_t)(t - npn) * nrows + row] = j - a.npd;
+      if (!split) continue;
+      const int k = (int)(buf[perm[t * RS + rl] * RS + rl] >> 2);
+      if (t < op) a.oj[lp][(size_t)t * nrows + p] = row_of_site(k, a.npd);
+      else if (t < npn) a.rj[lp][(size_t)(t - op) * nrows + p] = k;
+      else if (t < npn + oh) a.oj[lh][(size_t)(t - npn) * nrows + p] = row_of_site(k - a.npd, a.N - a.npd);
+      else a.rj[lh][(size_t)(t - npn - oh) * nrows + p] = k - a.npd;
+    }
+  }
+  if (tid >= 64) return;
+  const bool live = tid < SR && row < nrows;
   if (!FILL) {
     if (live) {
       a.cnt[lp][row] = npn;
       a.cnt[lh][row] = nhn;
-      const int p = row_of_site(row, nrows);
       a.ocnt[lp][p] = op;
       a.rcnt[lp][p] = npn - op;
       a.ocnt[lh][p] = oh;
       a.rcnt[lh][p] = nhn - oh;
-      if (!pdb) a.cnt[4][row] = nh1;
+      if (!pdb) a.cnt[4][row] = n1;
     }
-    // maxima over the wave, then one atomic per quantity
+    // maxima over the workgroup, then one atomic per quantity (rows past the end count 0)
     int v[14] = {0};
-    v[lp] = npn; v[lh] = nhn; v[4] = pdb ? 0 : nh1;
-    v[5 + lp] = op; v[5 + lh] = oh; v[9 + lp] = npn - op; v[9 + lh] = nhn - oh; v[13] = n;
+    v[lp] = npn; v[lh] = nhn; v[4] = pdb ? 0 : n1;
+    v[5 + lp] = op; v[5 + lh] = oh; v[9 + lp] = npn - op; v[9 + lh] = nhn - oh; v[13] = npn + nhn;
 #pragma unroll
     for (int k = 0; k < 14; ++k) {
       int m = v[k];
@@ -329,33 +407,13 @@ __global__ __launch_bounds__(NT) void k_site(NbrArgs a, int nblk_pd) {
     }
     return;
   }
-  // each row of the wave sorted by neighbor index
-  if (a.width <= 2 * NT) rank_rows<2>(buf, n, lane);
-  else rank_rows<MAXK>(buf, n, lane);
   if (live && pdb) {
-    a.pdpdnum[3 * (size_t)row] = sh0;
-    a.pdpdnum[3 * (size_t)row + 1] = sh1n;
-    a.pdpdnum[3 * (size_t)row + 2] = npn - sh0 - sh1n;
+    a.pdpdnum[3 * (size_t)row] = counts[5][rl];
+    a.pdpdnum[3 * (size_t)row + 1] = counts[6][rl];
+    a.pdpdnum[3 * (size_t)row + 2] = npn - counts[5][rl] - counts[6][rl];
   }
-  int mp = npn, mh = nhn;  // the wave's longest rows
-  for (int off = 32; off > 0; off >>= 1) {
-    mp = max(mp, __shfl_xor(mp, off));
-    mh = max(mh, __shfl_xor(mh, off));
-  }
-  int32_t* __restrict__ oP = a.idx[lp];
-  int32_t* __restrict__ oH = a.idx[lh];
-  for (int t = 0; t < mp; ++t)
-    if (t < npn) oP[(size_t)t * nrows + row] = (int)(buf[t * CS + lane] >> 2);
-  int k1 = 0;
-  for (int t = 0; t < mh; ++t)
-    if (t < nhn) {
-      const uint32_t key = buf[(npn + t) * CS + lane];
-      const int h = (int)(key >> 2) - a.npd;
-      oH[(size_t)t * nrows + row] = h;
-      if (!pdb && (key & 1u)) a.idx[4][(size_t)(k1++) * nrows + row] = h;  // HH1, in order
-    }
-  // totals of the five lists: wave sums, one atomic each
-  unsigned long long tp = npn, th = nhn, t1 = k1;
+  // totals of the five lists: sums over the workgroup, one atomic each
+  unsigned long long tp = live ? npn : 0, th = live ? nhn : 0, t1 = live && !pdb ? n1 : 0;
   for (int off = 32; off > 0; off >>= 1) {
     tp += __shfl_xor(tp, off);
     th += __shfl_xor(th, off);
@@ -369,60 +427,32 @@ __global__ __launch_bounds__(NT) void k_site(NbrArgs a, int nblk_pd) {
   }
 }
 
-// Split of each pair-list row into owned and received halves (pair-once
-// evaluation).  Ownership of {s, j} (global site indices):
-// (s < j) XOR ((s ^ j) & 1), which hands each site about half of every list.
-// Both halves keep the row's (sorted) order.
-
-// Both halves keep the row's index order: consecutive lanes (sites) then
-// gather consecutive neighbor sites at the same slot, so the state and F'
-// loads of a pair slot coalesce.  (Ordering the owned half by distance, to
-// align table rows across lanes, measured 40% slower: it scatters those
-// gathers.)
-__global__ void k_split(Ell L, int s_off, int j_off, int jrows) {
-  const int r = blockIdx.x * blockDim.x + threadIdx.x;
-  if (r >= L.rows) return;
-  int32_t* rpos = reinterpret_cast<int32_t*>(L.rbuf);  // full-row slot -> received slot (-1 if owned)
-  const int n = L.cnt[r];
-  const int s = s_off + r, p = row_of_site(r, L.rows);
-  int no = 0, nr = 0;
-  for (int t = 0; t < n; ++t) {
-    const size_t e = (size_t)t * L.rows + r;
-    const int j = L.idx[e];
-    if (pair_owner(s, j_off + j)) {
-      L.oj[(size_t)no * L.rows + p] = row_of_site(j, jrows);
-      rpos[e] = -1;
-      ++no;
-    } else {
-      rpos[e] = nr;
-      ++nr;
-    }
-  }
-}
-
-// For every owned entry (r, j): the received slot of r in the partner row j,
-// found by binary search of r in that sorted row (if absent, which the
-// symmetric lists never produce, a slot past the received half that nothing
-// reads: the owner passes store every share without a test).
-__global__ void k_orv(Ell L, Ell P) {
-  const int p = blockIdx.x * blockDim.x + threadIdx.x;
-  if (p >= L.rows) return;
+// For every owned entry, one thread each (slot blockIdx.y of list blockIdx.z):
+// the received slot of its row in the partner row, found by binary search of
+// the partner's received half (sorted site indices, in rbuf until the first
+// evaluation; if absent, which the symmetric lists never produce, a slot past
+// the received half that nothing reads: the owner passes store every share
+// without a test).
+struct OrvArgs {
+  Ell L[4];
+};
+__global__ void k_orv(OrvArgs a) {
+  const int w = blockIdx.z;
+  const Ell& L = a.L[w];
+  const int p = blockIdx.x * blockDim.x + threadIdx.x, t = blockIdx.y;
+  if (p >= L.rows || t >= L.owidth || t >= L.ocnt[p]) return;
+  const Ell& P = a.L[w == 1 ? 2 : w == 2 ? 1 : w];  // PdPd, PdH <-> HPd, HH
   const int r = site_of_row(p, L.rows);
-  const int32_t* prpos = reinterpret_cast<const int32_t*>(P.rbuf);
-  const int n = L.ocnt[p];
-  for (int t = 0; t < n; ++t) {
-    const size_t e = (size_t)t * L.rows + p;
-    const int j = site_of_row(L.oj[e], P.rows);
-    int lo = 0, hi = P.cnt[j] - 1, k = -1;
-    while (lo <= hi) {
-      const int mid = (lo + hi) >> 1;
-      const int v = P.idx[(size_t)mid * P.rows + j];
-      if (v == r) { k = mid; break; }
-      if (v < r) lo = mid + 1;
-      else hi = mid - 1;
-    }
-    L.orv[e] = k >= 0 ? prpos[(size_t)k * P.rows + j] : P.rwidth;
+  const size_t e = (size_t)t * L.rows + p;
+  const int j = L.oj[e];
+  const A2C_GLOBAL int32_t* rj = gmem(reinterpret_cast<const int32_t*>(P.rbuf)) + j;
+  int lo = 0, hi = P.rcnt[j];  // the slot is in [lo, hi) if the row holds r
+  while (hi - lo > 1) {
+    const int mid = (lo + hi) >> 1;
+    if (rj[(size_t)mid * P.rows] <= r) lo = mid;
+    else hi = mid;
   }
+  L.orv[e] = lo < hi && rj[(size_t)lo * P.rows] == r ? lo : P.rwidth;
 }
 
 // Bounding box of the positions (non-periodic axes): per block, then one
@@ -774,7 +804,7 @@ int size_lists(a2c_fe_ctx* c, Ell* L5, const int* w, const int* ow, const int* r
     if (k == 4 || !ow) continue;
     const int64_t on = (int64_t)std::max(ow[k], 1) * rows;
     const int64_t rn = (int64_t)(std::max(rw[k], 1) + 1) * rows;  // one slot to spare (k_orv)
-    const int64_t bn = std::max<int64_t>(32 * rn, 4 * (int64_t)std::max(w[k], 1) * rows);
+    const int64_t bn = 32 * rn;
     if (on > L.ocap) {
       (void)dfree(L.oj); (void)dfree(L.orv);
       L.oj = L.orv = nullptr;
@@ -792,15 +822,18 @@ int size_lists(a2c_fe_ctx* c, Ell* L5, const int* w, const int* ow, const int* r
   return A2C_OK;
 }
 
-// Reverse slots of the four pair lists (after their split).
+// Reverse slots of the four pair lists (after the fill pass).
 int reverse_slots(a2c_fe_ctx* c, Ell* L5) {
-  static const int partner[4] = {0, 2, 1, 3};  // PdPd, PdH<->HPd, HH
+  OrvArgs a;
+  int rows = 0, width = 0;
   for (int w = 0; w < 4; ++w) {
-    const Ell& L = L5[w];
-    if (L.rows == 0) continue;
-    hipLaunchKernelGGL(k_orv, dim3((L.rows + 255) / 256), dim3(256), 0, c->stream, L, L5[partner[w]]);
-    A2C_HIP(c, hipGetLastError());
+    a.L[w] = L5[w];
+    rows = std::max(rows, L5[w].rows);
+    width = std::max(width, L5[w].owidth);
   }
+  if (rows == 0 || width == 0) return A2C_OK;
+  hipLaunchKernelGGL(k_orv, dim3((rows + 255) / 256, width, 4), dim3(256), 0, c->stream, a);
+  A2C_HIP(c, hipGetLastError());
   return A2C_OK;
 }
 
@@ -823,7 +856,7 @@ int walk_cells(a2c_fe_ctx* c, double rc, Ell* L5, bool halves, int hm[16], unsig
   // scratch (grow-only): misc = 16 ints (widths, overflow) + 5 totals + 6 bbox keys
   if (!c->nb_cid) {
     A2C_HIP(c, dmalloc(&c->nb_cid, sizeof(int) * std::max(N, 1)));
-    A2C_HIP(c, dmalloc(&c->nb_order, sizeof(double4) * std::max(N, 1)));  // cell-ordered positions
+    A2C_HIP(c, dmalloc(&c->nb_order, sizeof(float4) * std::max(N, 1)));  // cell-ordered positions
   }
   if (!c->nb_misc) A2C_HIP(c, dmalloc(&c->nb_misc, MISC_BYTES));
   int* misc = c->nb_misc;
@@ -871,7 +904,7 @@ int walk_cells(a2c_fe_ctx* c, double rc, Ell* L5, bool halves, int hm[16], unsig
     c->nb_cap_cells = ncell + 1;
   }
   int *dcid = c->nb_cid, *dcc = c->nb_cc, *dcursor = c->nb_cursor;
-  double4* qs = reinterpret_cast<double4*>(c->nb_order);
+  float4* qs = reinterpret_cast<float4*>(c->nb_order);
   A2C_HIP(c, hipMemsetAsync(dcursor, 0, sizeof(int) * (ncell + 1), c->stream));  // the histogram
   A2C_HIP(c, hipMemsetAsync(misc, 0, MISC_DMAX, c->stream));
   if (N > 0) {
@@ -881,13 +914,24 @@ int walk_cells(a2c_fe_ctx* c, double rc, Ell* L5, bool halves, int hm[16], unsig
   hipLaunchKernelGGL(k_scan, dim3(1), dim3(SCAN_T), 0, c->stream, dcursor, (int)ncell, dcc, dcursor);
   A2C_HIP(c, hipGetLastError());
   if (N > 0) {
-    hipLaunchKernelGGL(k_place, dim3((N + TB - 1) / TB), dim3(TB), 0, c->stream, c->dX, N, dcid, dcursor, qs);
+    hipLaunchKernelGGL(k_place, dim3((N + TB - 1) / TB), dim3(TB), 0, c->stream, c->dX, N, g, dcid, dcursor, qs);
     A2C_HIP(c, hipGetLastError());
   }
   if (int rc2 = size_lists(c, L5, nullptr, nullptr, nullptr)) return rc2;  // row counts
   NbrArgs a{};
   a.X = c->dX; a.qs = qs; a.npd = npd; a.N = N; a.g = g; a.cid = dcid; a.cstart = dcc;
   for (int ax = 0; ax < 3; ++ax) a.ibox[ax] = g.box[ax] > 0.0 ? 1.0 / g.box[ax] : 0.0;
+  // the filter's margin: the floats' rounding over the grid's extent, with room to spare
+  double extent = 0.0;
+  for (int ax = 0; ax < 3; ++ax) {
+    extent = std::max(extent, g.w[ax] * g.nc[ax]);
+    a.fbox[ax] = g.periodic[ax] ? (float)g.box[ax] : 0.0f;
+    a.fibox[ax] = g.periodic[ax] ? (float)a.ibox[ax] : 0.0f;
+  }
+  const double rcf = rc + 1e-4 + extent * 0x1p-20;
+  a.rcf2 = (float)(rcf * rcf);
+  a.in0 = 1.0 / g.nc[0];
+  a.in01 = 1.0 / ((double)g.nc[0] * g.nc[1]);
   a.rc2 = rc * rc;
   a.sh1 = c->desc.a_pd * c->desc.a_pd * 0.75;
   a.sh2 = c->desc.a_pd * c->desc.a_pd * 1.25;
@@ -897,9 +941,9 @@ int walk_cells(a2c_fe_ctx* c, double rc, Ell* L5, bool halves, int hm[16], unsig
   a.maxw = misc;
   a.overflow = misc + 14;
   a.totals = totals;
-  const int nblk_pd = (npd + NT - 1) / NT, nblk_h = (nh + NT - 1) / NT;
+  const int nblk_pd = (npd + SR - 1) / SR, nblk_h = (nh + SR - 1) / SR;
   if (nblk_pd + nblk_h > 0) {
-    hipLaunchKernelGGL(k_site<false>, dim3(nblk_pd + nblk_h), dim3(NT), 0, c->stream, a, nblk_pd);
+    hipLaunchKernelGGL(k_site<false>, dim3(nblk_pd + nblk_h), dim3(ST), 0, c->stream, a, nblk_pd);
     A2C_HIP(c, hipGetLastError());
   }
   {
@@ -914,30 +958,22 @@ int walk_cells(a2c_fe_ctx* c, double rc, Ell* L5, bool halves, int hm[16], unsig
     a.idx[w] = L5[w].idx;
     L5[w].width = hm[w];
     if (w < 4) {
+      a.oj[w] = halves ? L5[w].oj : nullptr;
+      a.rj[w] = halves ? reinterpret_cast<int32_t*>(L5[w].rbuf) : nullptr;
       L5[w].owidth = hm[5 + w];
       L5[w].rwidth = hm[9 + w];
     }
   }
   if (!c->dpdpdnum) A2C_HIP(c, dmalloc(&c->dpdpdnum, sizeof(int32_t) * 3 * std::max(npd, 1)));
   a.pdpdnum = c->dpdpdnum;
-  a.width = std::max(hm[13], 1);  // LDS slots per lane: the longest row
+  a.width = std::max(hm[13], 1);
   if (nblk_pd + nblk_h > 0) {
-    hipLaunchKernelGGL(k_site<true>, dim3(nblk_pd + nblk_h), dim3(NT), sizeof(uint32_t) * CS * a.width, c->stream, a,
-                       nblk_pd);
+    hipLaunchKernelGGL(k_site<true>, dim3(nblk_pd + nblk_h), dim3(ST), (sizeof(uint32_t) + 1) * RS * (size_t)a.width,
+                       c->stream, a, nblk_pd);
     A2C_HIP(c, hipGetLastError());
   }
-  if (halves) {
-    // owned/received split of the four pair lists, then the partner slots
-    static const int s_sp[4] = {0, 0, 1, 1}, j_sp[4] = {0, 1, 0, 1};  // species of rows / of neighbors
-    for (int w = 0; w < 4; ++w) {
-      const Ell& L = L5[w];
-      if (L.rows == 0) continue;
-      hipLaunchKernelGGL(k_split, dim3((L.rows + TB - 1) / TB), dim3(TB), 0, c->stream, L, s_sp[w] * npd,
-                         j_sp[w] * npd, j_sp[w] ? nh : npd);
-      A2C_HIP(c, hipGetLastError());
-    }
+  if (halves)
     if (int rc2 = reverse_slots(c, L5)) return rc2;
-  }
   {
     std::vector<unsigned long long> tb(SPREAD * 5);
     A2C_HIP(c, hipMemcpyAsync(tb.data(), totals, sizeof(unsigned long long) * tb.size(), hipMemcpyDeviceToHost,
