@@ -239,7 +239,7 @@ int a2c_fe_density(a2c_fe_ctx* c, const double* X, double* rho) {
   if (int rc = check_ctx(c)) return rc;
   if (!c->have_nbr || !c->have_x) return set_err(c, A2C_ESTATE, "neighbors/occupancy not set");
   if (int rc = upload_state(c, X)) return rc;
-  if (int rc = launch_density64(c, c->dX)) return rc;
+  if (int rc = launch_density64(c, c->dX, true)) return rc;
   if (c->N) A2C_HIP(c, hipMemcpyAsync(rho, c->drho, 8 * (size_t)c->N, hipMemcpyDeviceToHost, c->stream));
   A2C_HIP(c, hipStreamSynchronize(c->stream));
   return A2C_OK;

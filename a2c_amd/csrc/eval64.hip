@@ -654,10 +654,14 @@ __global__ __launch_bounds__(TBO) __attribute__((amdgpu_waves_per_eu(4))) void k
     dens_list<RULE, true, true>(tab, tab + S_ROWS, S, ln, a, img, wme, rho);
   }
   rho = site_sum(rho, K);
-  if (ln.ph == 0) gmem(S.rho)[s] = rho;
+  if (ln.ph == 0) gmem(S.epair)[s] = rho;  // free until the gradient pass
 }
 
-__global__ __launch_bounds__(TB) void k_dens_recv64(const LatDev* __restrict__ lats, const int32_t* __restrict__ b2l) {
+// by_site: rho, F' and the embedding energy in site order (a caller's density),
+// else in row order (the passes that follow).
+template <int DM>
+__global__ __launch_bounds__(TB) void k_dens_recv64(const LatDev* __restrict__ lats, const int32_t* __restrict__ b2l,
+                                                    double eps, int by_site) {
   const int blk = xcd_block();
   const LatDev& S = lats[b2l[blk]];
   const int s = (blk - S.blk0) * TB + threadIdx.x;
@@ -666,7 +670,7 @@ __global__ __launch_bounds__(TB) void k_dens_recv64(const LatDev* __restrict__ l
   const double* __restrict__ xo = S.xrow;
   const bool pd = s < S.npd;
   const int row = pd ? s : s - S.npd;
-  double rho = S.rho[s];
+  double rho = S.epair[s];
 #pragma unroll
   for (int side = 0; side < 2; ++side) {
     const Ell& L = pd ? (side ? S.pdh : S.pdpd) : (side ? S.hh : S.hpd);
@@ -675,11 +679,12 @@ __global__ __launch_bounds__(TB) void k_dens_recv64(const LatDev* __restrict__ l
     for_row_shares<RECV_RU_SCALAR>(gmem(reinterpret_cast<const double*>(L.rbuf)), L.rows, row, n, [&](double v) { rho += v; });
   }
   rho *= S.rule == GH3 ? 1.0 : QW;
-  S.rho[s] = rho;
   const double xs = pd ? 1.0 : xo[row];
   const eam::VD F = pd ? eam::F_Pd_vd(rho) : eam::F_H_vd(rho);
-  S.Fp[s] = F.d;
-  S.emb[s] = xs * F.v;
+  const int o = !by_site ? s : pd ? site_of_row(row, S.npd) : S.npd + site_of_row(row, S.nh);
+  S.rho[o] = rho;
+  S.Fp[o] = DM == A2C_DERIV_FD ? dF<DM>(pd, rho, eps) : F.d;
+  S.emb[o] = xs * F.v;
 }
 
 // One node inside the tables: the pair energy phi and cu = SH dE/ds, E = F'_i f_j
@@ -996,6 +1001,162 @@ __global__ __launch_bounds__(TB) void k_grad_recv64(const LatDev* __restrict__ l
   if (threadIdx.x == 0) S.part[lb] = red[0];
 }
 
+// ================================================================ chemical potential
+// f_H and phi (phi_PdH, or phi_HH for an H neighbor) summed over a pair's nodes,
+// with the rule's weights; false, and zeros, if a node lies outside the tables.
+enum { C_PHPDH = 0, C_PHH = 1, NCTAB = 2 };  // this pass's order in LDS
+template <bool NB_H>
+__device__ __forceinline__ void node_fh_phi(const double* tab, const double* exptab, double x, double w, double& sf,
+                                            double& sp) {
+  double r, ri;
+  sf = fma(w, fH_s(exptab, s_of(x), r, ri), sf);
+  const double y = NB_H ? x : fma(r, RINV, -156.0);
+  sp = fma(w, poly<5>(s_row(tab, NB_H ? C_PHH : C_PHPDH, (int)y), __builtin_amdgcn_fract(y)), sp);
+}
+template <int RULE, bool NB_H>
+__device__ __forceinline__ bool pair_fh_phi(const double* tab, const double* exptab, const double d[3], double si,
+                                            double sj, double& sf, double& sp) {
+  sf = sp = 0.0;
+  if (RULE == GH3) {
+    const Nodes27 q(d, sqrt(fma(si, si, sj * sj)));
+    if (!inside(q.lo, q.hi)) return false;
+#pragma unroll 1
+    for (int k = 0; k < 9; ++k) {
+      const int a2 = k / 3 - 1, a1 = k % 3 - 1;
+      const double xb = q.x0 + q.n1 * (double)(a2 * a2 + a1 * a1) + ((double)a2 * q.t[2] + (double)a1 * q.t[1]);
+      const double w = (a2 ? 1.0 : 4.0) * (a1 ? 1.0 : 4.0);
+#pragma unroll
+      for (int a0 = -1; a0 <= 1; ++a0)
+        node_fh_phi<NB_H>(tab, exptab, a0 ? xb + q.n1 + a0 * q.t[0] : xb, a0 ? w : 4.0 * w, sf, sp);
+    }
+    sf *= 11.0025 / 216.0;
+    sp *= 1.0 / 216.0;
+  } else {
+    const Nodes12 q(d, SQ6 * si, SQ6 * sj);
+    if (!inside(q.lo, q.hi)) return false;
+    double d0 = d[0], d1 = d[1], d2 = d[2];
+#pragma unroll 1
+    for (int c = 0; c < 3; ++c) {
+      const double ti = q.gi * d0, tj = q.gj * d0;
+      const double x[4] = {q.xi + ti, q.xi - ti, q.xj - tj, q.xj + tj};
+#pragma unroll
+      for (int k = 0; k < 4; ++k) node_fh_phi<NB_H>(tab, exptab, x[k], 1.0, sf, sp);
+      d0 = d1;
+      d1 = d2;
+    }
+    sf *= 11.0025 * QW;
+    sp *= QW;
+  }
+  return true;
+}
+template <int RULE, bool NB_H>
+__device__ __forceinline__ void closed_fh_phi(const double d[3], double si, double sj, double& sf, double& sp) {
+  const Closed<RULE> q(d, si, sj);
+  sf = sp = 0.0;
+#pragma unroll 1
+  for (int k = 0; k < Closed<RULE>::N; ++k) {
+    double z[3], w;
+    const double r = q.node(k, z, w);
+    sf += w * eam::f_H(r);
+    sp += w * eam::phi_morse<NB_H>(r);
+  }
+  sf *= rule_qw<RULE>();
+  sp *= rule_qw<RULE>();
+}
+
+// The listed neighbors of H row `row` (full list L, site order), K lanes to a
+// row: sum += w_j (F'_j f_H + phi + corr_j), xs += w_j.  A pair's state is loaded a
+// pair ahead.
+template <int RULE, bool NB_H>
+__device__ __forceinline__ void chem_list(const double* tab, const double* exptab, const LatDev& S, const Ell& L,
+                                          const A2C_GLOBAL double* corr, int row, int ph, int K, const Site& a,
+                                          const Image& img, double& sum, double& xs) {
+  const A2C_GLOBAL double2* __restrict__ qxy = gmem((const double2*)S.qxy) + (NB_H ? S.npd : 0);
+  const A2C_GLOBAL double2* __restrict__ qzs = gmem((const double2*)S.qzs) + (NB_H ? S.npd : 0);
+  const A2C_GLOBAL double* __restrict__ Fp = gmem((const double*)S.Fp) + (NB_H ? S.npd : 0);
+  const A2C_GLOBAL double* __restrict__ w = gmem((const double*)S.xrow);
+  const int site = site_of_row(row, S.nh), jrows = NB_H ? S.nh : S.npd;
+  const A2C_GLOBAL int32_t* __restrict__ idx = gmem((const int32_t*)L.idx) + site;
+  const size_t rows = L.rows;
+  const int n = gmem((const int32_t*)L.cnt)[site];
+  corr += NB_H ? S.npd : 0;
+  if (ph >= n) return;
+  auto at = [&](int t) { return row_of_site(idx[(size_t)(t < n ? t : ph) * rows], jrows); };
+  int j = at(ph), jn = at(ph + K);
+  Site b = load_row(qxy, qzs, j);
+  double Fj = Fp[j], cj = corr[j], wj = NB_H ? w[j] : 1.0;
+  bool far = false;
+  for (int t = ph; t < n; t += K) {
+    Pair64 p;
+    pair_vec(img, a, b, p.d);
+    p.s = b.s;
+    const double Fc = Fj, cc = cj, wc = wj;
+    b = load_row(qxy, qzs, jn);
+    Fj = Fp[jn];
+    cj = corr[jn];
+    if (NB_H) wj = w[jn];
+    jn = at(t + 2 * K);
+    double sf, sp;
+    const bool in = pair_fh_phi<RULE, NB_H>(tab, exptab, p.d, a.s, p.s, sf, sp);
+    far |= !in;
+    const double v = fma(Fc, sf, sp) + cc;
+    xs += wc;
+    if (in) sum += NB_H ? wc * v : v;
+  }
+  if (!far) return;
+  for (int t = ph; t < n; t += K) {
+    j = at(t);
+    b = load_row(qxy, qzs, j);
+    double d[3], sf, sp;
+    pair_vec(img, a, b, d);
+    if (pair_inside<RULE>(d, a.s, b.s)) continue;
+    closed_fh_phi<RULE, NB_H>(d, a.s, b.s, sf, sp);
+    sum += (NB_H ? w[j] : 1.0) * (fma(Fp[j], sf, sp) + corr[j]);
+  }
+}
+
+// Chemical potential of the H sites (occupancy.hip has the formula), K lanes per
+// row over the full lists, from rho and F' in row order.  24^3 cells: one lane per
+// site and closed forms 353 us, this 117 us (4 waves per SIMD; LDS and FP64 units both busy);
+// error against 80-bit arithmetic 1e-12 before, 3e-15 now.
+template <int RULE, int TBO>
+__global__ __launch_bounds__(TBO) void k_chem64(const LatDev* __restrict__ lat, int units, int K,
+                                                const double* __restrict__ gtab, ChemArgs c) {
+  __shared__ __align__(16) double tab[NCTAB * S_ROWS + EXPN];
+  stage16(tab, gtab + S_PHPDH * S_ROWS, (NCTAB * S_ROWS + EXPN) / 2);  // phi_PdH, phi_HH, 2^(i/256)
+  __syncthreads();
+  const double* exptab = tab + NCTAB * S_ROWS;
+  const int u = xcd_block() * (TBO / TB) + __builtin_amdgcn_readfirstlane(threadIdx.x / TB);
+  if (u >= units) return;
+  const LatDev& S = *lat;
+  const int lane = (int)threadIdx.x % TB, sh = 31 - __builtin_clz(K);
+  const int row = u * (TB >> sh) + (lane >> sh), ph = lane & (K - 1);
+  if (row >= S.nh) return;  // whole lane groups
+  const int site = site_of_row(row, S.nh);
+  if (c.full[site] == 1) return;  // fully occupied reservoir: gamma untouched
+  const int s = S.npd + row;
+  const Image img = image_of(S);
+  const Site a = load_row(gmem((const double2*)S.qxy), gmem((const double2*)S.qzs), s);
+  const A2C_GLOBAL double* corr = gmem(c.corr);
+  double sum = 0.0, nP = 0.0, Xa = 0.0;
+  chem_list<RULE, false>(tab, exptab, S, S.hpd, corr, row, ph, K, a, img, sum, nP);
+  chem_list<RULE, true>(tab, exptab, S, S.hh, corr, row, ph, K, a, img, sum, Xa);
+  sum = site_sum(sum, K);
+  Xa = site_sum(Xa, K);
+  nP = site_sum(nP, K);
+  if (ph != 0) return;
+  const double T = S.T, x = S.xrow[row];
+  sum += eam::F_H(S.rho[s]);
+  sum += 0.5 * T * c.ch[0] * (c.ch[1] * nP * nP + 2.0 * c.ch[2] * nP * Xa + c.ch[3] * Xa * Xa);
+  const double raw = (x > 0.0 && x < 1.0) ? log(x / (1.0 - x)) + sum / (KB * T) : 0.0;
+  double g = raw + 1.5;
+  if (g > c.gamma_bd) {
+    g = c.gamma_bd;
+    if (x > 0.9999) c.full[site] = 1;
+  }
+  c.gamma[site] = g;
+}
+
 // Row-order copies of the state and the occupancy for the pair passes.
 __global__ __launch_bounds__(TB) void k_rows(const LatDev* __restrict__ lats, const int32_t* __restrict__ b2l) {
   const int blk = xcd_block();
@@ -1055,7 +1216,8 @@ template <int R, int T> struct DensOwn { static constexpr auto fn = k_dens_own64
 template <int R, int T> struct GradOwn { static constexpr auto fn = k_grad_own64<R, T>; };
 }  // namespace
 
-int run_density64(const Launch& L) {
+// rho, F', embedding energy from full lists, in site order
+static int run_density64(const Launch& L) {
   if (L.deriv_mode == A2C_DERIV_FD) return per_rule<DensFd>(L, L.nblk, L.lats, L.b2l, L.fd_eps);
   return per_rule<DensAn>(L, L.nblk, L.lats, L.b2l, L.fd_eps);
 }
@@ -1068,7 +1230,7 @@ int run_eval64(const Launch& L, Timing* tm) {
       if (tm) tm->mark(L.stream, "dens_own64");
       if (L.onblk > DENS_WIDE_UNITS ? owners<DensOwn, 512>(L) : owners<DensOwn, 256>(L)) return A2C_EHIP;
       if (tm) tm->mark(L.stream, "dens_recv64");
-      hipLaunchKernelGGL(k_dens_recv64, dim3(L.nblk), dim3(TB), 0, L.stream, L.lats, L.b2l);
+      hipLaunchKernelGGL(k_dens_recv64<A2C_DERIV_ANALYTIC>, dim3(L.nblk), dim3(TB), 0, L.stream, L.lats, L.b2l, 0.0, 0);
       if (hipGetLastError() != hipSuccess) return A2C_EHIP;
       if (tm) tm->mark(L.stream, "grad_own64");
       if (L.onblk > GRAD_WIDE_UNITS ? owners<GradOwn, 512>(L) : owners<GradOwn, 256>(L)) return A2C_EHIP;
@@ -1253,10 +1415,40 @@ static Launch single_launch(a2c_fe_ctx* c, bool fp64) {
   return L;
 }
 
-int launch_density64(a2c_fe_ctx* c, const double* dX) {
+// Density, F' and embedding energy of the context's lattice from the pair-once
+// passes, in site or in row order.
+int launch_density64(a2c_fe_ctx* c, const double* dX, bool by_site) {
   if (c->gen_on) return launch_density_gen(c, dX);
   if (int rc = sync_lattice(c, dX, c->dG, c->dF)) return rc;
-  if (run_density64(single_launch(c, true))) return set_err(c, A2C_EHIP, "density64 launch failed");
+  const Launch L = single_launch(c, true);
+  if (L.nblk == 0) return A2C_OK;
+  if (run_rows(L) || (L.onblk > DENS_WIDE_UNITS ? owners<DensOwn, 512>(L) : owners<DensOwn, 256>(L)))
+    return set_err(c, A2C_EHIP, "density64 launch failed");
+  hipLaunchKernelGGL(L.deriv_mode == A2C_DERIV_FD ? k_dens_recv64<A2C_DERIV_FD> : k_dens_recv64<A2C_DERIV_ANALYTIC>,
+                     dim3(L.nblk), dim3(TB), 0, L.stream, L.lats, L.b2l, L.fd_eps, (int)by_site);
+  A2C_HIP(c, hipGetLastError());
+  return A2C_OK;
+}
+
+// The chemical potential from what launch_density64 left in row order.  Up to a
+// unit of 256 lanes per CU the units go to workgroups of their own; beyond, two
+// or four share one, so that a CU's one copy of the tables serves all its waves.
+template <int RULE>
+static void launch_chem64_rule(a2c_fe_ctx* c, const ChemArgs& a) {
+  const int K = lanes_per_site(c->N, true), units = owner_units(c->desc.n_h, K);
+  auto go = [&](auto kernel, int tbo) {
+    hipLaunchKernelGGL(kernel, dim3((units + tbo / TB - 1) / (tbo / TB)), dim3(tbo), 0, c->stream,
+                       (const LatDev*)c->dlat, units, K, (const double*)c->dtab64, a);
+  };
+  if (units <= 256) go(k_chem64<RULE, 256>, 256);
+  else if (units <= 512) go(k_chem64<RULE, 512>, 512);
+  else go(k_chem64<RULE, 1024>, 1024);
+}
+int launch_chem64(a2c_fe_ctx* c, const ChemArgs& a) {
+  if (c->desc.n_h <= 0) return A2C_OK;
+  if (c->desc.quad_rule == A2C_QUAD_GH3) launch_chem64_rule<GH3>(c, a);
+  else launch_chem64_rule<A2C_QUAD_R12>(c, a);
+  A2C_HIP(c, hipGetLastError());
   return A2C_OK;
 }
 

@@ -445,14 +445,23 @@ struct Launch {
 };
 bool mixed_full_pairs();  // A2C_MIXED_PAIRS=full selects the both-ends kernels
 bool fp64_full_pairs();   // A2C_FP64_PAIRS=full likewise for the FP64 kernels
-int run_density64(const Launch& L);
 int run_eval64(const Launch& L, Timing* tm);
 int run_eval32(const Launch& L, Timing* tm);
 int run_final_sum(const Launch& L);
 int run_rows(const Launch& L);  // row-order copies of state and occupancy (pair-once evaluation)
 int sync_lattice(a2c_fe_ctx* c, const double* dX, double* dG, double* dF);  // refresh the one-lattice descriptor
 int launch_eval64(a2c_fe_ctx* c, const double* dX, double* dG, double* dF, bool timed, Timing* tm);
-int launch_density64(a2c_fe_ctx* c, const double* dX);  // fills drho, dFp, demb
+int launch_density64(a2c_fe_ctx* c, const double* dX, bool by_site);  // fills drho, dFp, demb
+// Chemical potential of the H sites: gamma and full in site order, corr
+// (k_chem_pre) in row order.
+struct ChemArgs {
+  const double* corr;
+  double ch[4];
+  double gamma_bd;
+  double* gamma;
+  int32_t* full;
+};
+int launch_chem64(a2c_fe_ctx* c, const ChemArgs& a);  // after launch_density64 in row order
 int launch_eval32(a2c_fe_ctx* c, const double* dX, double* dG, double* dF, bool timed, Timing* tm);
 int build_tables(a2c_fe_ctx* c);                        // eval32.hip
 int tables_download(a2c_fe_ctx* c, float* out);         // 5*500 float4

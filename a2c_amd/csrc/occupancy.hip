@@ -38,62 +38,10 @@ namespace a2c {
 namespace {
 
 constexpr int TB = 256;
-constexpr double QW = 1.0 / 12.0;
-constexpr double SQ6 = 2.449489742783178098;
-
-struct Site {
-  double q[3];
-  double s;
-};
-__device__ __forceinline__ Site load_site(const double* __restrict__ X, int s) {
-  const double4 v = *reinterpret_cast<const double4*>(X + 4 * (size_t)s);
-  return {{v.x, v.y, v.z}, v.w};
-}
-__device__ __forceinline__ void pair_vec(const DevSys& S, const Site& a, const Site& b, double d[3]) {
-#pragma unroll
-  for (int c = 0; c < 3; ++c) {
-    double qj = b.q[c];
-    if (S.periodic[c]) qj = qj - S.box[c] * rint((qj - a.q[c]) * S.ibox[c]);
-    d[c] = a.q[c] - qj;
-  }
-}
-
-// Sums of f_H and of phi (phi_PdH or phi_H) over the nodes of one pair:
-// unweighted over the 12 points (the caller applies 1/12), weighted over the
-// 27 Gauss-Hermite nodes.
-template <int HH, int RULE>
-__device__ __forceinline__ void pair_fh_phi(const double d[3], double si, double sj, double& sf, double& sp) {
-  sf = 0.0;
-  sp = 0.0;
-  if (RULE == A2C_QUAD_GH3) {
-    const double sd = sqrt(si * si + sj * sj);
-#pragma unroll 1
-    for (int k = 0; k < 27; ++k) {
-      double z[3], w;
-      gh_node(k, z, w);
-      const double r0 = d[0] + sd * z[0], r1 = d[1] + sd * z[1], r2 = d[2] + sd * z[2];
-      const double rn = sqrt(r0 * r0 + r1 * r1 + r2 * r2);
-      sf += w * eam::f_H(rn);
-      sp += w * eam::phi_morse<HH>(rn);
-    }
-    return;
-  }
-  const double ai = SQ6 * si, aj = SQ6 * sj;
-#pragma unroll
-  for (int p = 0; p < 12; ++p) {
-    const int c = (p >> 1) % 3;
-    const double sg = (p & 1) ? -1.0 : 1.0;
-    double r[3] = {d[0], d[1], d[2]};
-    r[c] += (p < 6) ? sg * ai : -sg * aj;
-    const double rn = sqrt(r[0] * r[0] + r[1] * r[1] + r[2] * r[2]);
-    sf += eam::f_H(rn);
-    sp += eam::phi_morse<HH>(rn);
-  }
-}
-
-// Per-site correction sums: P_j for Pd sites, Q_b for H sites.
+// Per-site correction sums: P_j for Pd sites, Q_b for H sites, in site order or
+// (by_row) row order.  Eight neighbors' occupancies are gathered together.
 __global__ void k_chem_pre(DevSys S, const double* __restrict__ xo, double T, double cp0, double cp2, double cp3,
-                           double ch0, double ch2, double ch3, double* __restrict__ corr) {
+                           double ch0, double ch2, double ch3, int by_row, double* __restrict__ corr) {
   const int s = blockIdx.x * blockDim.x + threadIdx.x;
   const int N = S.npd + S.nh;
   if (s >= N) return;
@@ -103,58 +51,18 @@ __global__ void k_chem_pre(DevSys S, const double* __restrict__ xo, double T, do
   const Ell LH = pd ? S.pdh : S.hh;
   double X = 0.0;
   const int nh = LH.cnt[row];
-  for (int t = 0; t < nh; ++t) X += xo[LH.idx[(size_t)t * LH.rows + row]];
+  constexpr int B = 8;
+  for (int t = 0; t < nh; t += B) {
+    double v[B];
+#pragma unroll
+    for (int u = 0; u < B; ++u) v[u] = xo[LH.idx[(size_t)min(t + u, nh - 1) * LH.rows + row]];
+#pragma unroll
+    for (int u = 0; u < B; ++u)
+      if (t + u < nh) X += v[u];
+  }
   const double n = (double)LP.cnt[row];
-  corr[s] = pd ? T * cp0 * (cp2 * n + cp3 * X) : T * ch0 * (ch2 * n + ch3 * X);
-}
-
-template <int RULE>
-__global__ __launch_bounds__(TB) void k_chem(DevSys S, const double* __restrict__ X, const double* __restrict__ xo,
-                                             const double* __restrict__ rho, const double* __restrict__ Fp,
-                                             const double* __restrict__ corr, double ch0, double ch1, double ch2,
-                                             double ch3, double gamma_bd, double* __restrict__ gamma,
-                                             int32_t* __restrict__ full) {
-  const int a = blockIdx.x * blockDim.x + threadIdx.x;
-  if (a >= S.nh) return;
-  if (full[a] == 1) return;  // fully occupied reservoir: gamma untouched
-  const int s = S.npd + a;
-  const Site si = load_site(X, s);
-  constexpr double qw = RULE == A2C_QUAD_GH3 ? 1.0 : QW;
-  const double T = S.T;
-  double sum = eam::F_H(rho[s]);
-  // correction of the site itself
-  const double n = (double)S.hpd.cnt[a];
-  double Xa = 0.0;
-  const int nhh = S.hh.cnt[a];
-  for (int t = 0; t < nhh; ++t) Xa += xo[S.hh.idx[(size_t)t * S.hh.rows + a]];
-  sum += 0.5 * T * ch0 * (ch1 * n * n + 2.0 * ch2 * n * Xa + ch3 * Xa * Xa);
-  const int npn = S.hpd.cnt[a];
-  for (int t = 0; t < npn; ++t) {  // H-Pd pairs (minimizer.cpp:679-698)
-    const int j = S.hpd.idx[(size_t)t * S.hpd.rows + a];
-    const Site b = load_site(X, j);
-    double d[3];
-    pair_vec(S, si, b, d);
-    double sf, sp;
-    pair_fh_phi<0, RULE>(d, si.s, b.s, sf, sp);
-    sum += qw * (Fp[j] * sf + sp) + corr[j];
-  }
-  for (int t = 0; t < nhh; ++t) {  // H-H pairs (:701-719)
-    const int h = S.hh.idx[(size_t)t * S.hh.rows + a];
-    const Site b = load_site(X, S.npd + h);
-    double d[3];
-    pair_vec(S, si, b, d);
-    double sf, sp;
-    pair_fh_phi<1, RULE>(d, si.s, b.s, sf, sp);
-    sum += xo[h] * (qw * (Fp[S.npd + h] * sf + sp) + corr[S.npd + h]);
-  }
-  const double x = xo[a];
-  const double raw = (x > 0.0 && x < 1.0) ? log(x / (1.0 - x)) + sum / (KB * T) : 0.0;
-  double g = raw + 1.5;
-  if (g > gamma_bd) {
-    g = gamma_bd;
-    if (x > 0.9999) full[a] = 1;
-  }
-  gamma[a] = g;
+  const int o = !by_row ? s : pd ? row_of_site(row, S.npd) : S.npd + row_of_site(row, S.nh);
+  corr[o] = pd ? T * cp0 * (cp2 * n + cp3 * X) : T * ch0 * (ch2 * n + ch3 * X);
 }
 
 constexpr double F_FACTOR_MAX = 700.0;  // |f| below which e^{+-f/2} and the edge products stay finite
@@ -294,19 +202,15 @@ int launch_chem(a2c_fe_ctx* c, const double* dX, const double* coe_pd, const dou
                 double* dgam, int32_t* dfull, double* dcorr) {
   const DevSys S = c->sys();
   const int N = c->N;
-  if (int rc = launch_density64(c, dX)) return rc;  // rho, F'(rho) at X
+  if (int rc = launch_density64(c, dX, false)) return rc;  // rho, F'(rho) at X
   if (N > 0) {
     hipLaunchKernelGGL(k_chem_pre, dim3((N + TB - 1) / TB), dim3(TB), 0, c->stream, S, c->dx, S.T, coe_pd[0],
-                       coe_pd[2], coe_pd[3], coe_h[0], coe_h[2], coe_h[3], dcorr);
+                       coe_pd[2], coe_pd[3], coe_h[0], coe_h[2], coe_h[3], (int)!c->gen_on, dcorr);
     A2C_HIP(c, hipGetLastError());
   }
   if (S.nh > 0 && c->gen_on) return launch_chem_gen(c, dX, coe_h, gamma_bd, dgam, dfull, dcorr);
-  if (S.nh > 0) {
-    hipLaunchKernelGGL(S.rule == A2C_QUAD_GH3 ? k_chem<A2C_QUAD_GH3> : k_chem<A2C_QUAD_R12>,
-                       dim3((S.nh + TB - 1) / TB), dim3(TB), 0, c->stream, S, dX, c->dx, c->drho, c->dFp, dcorr,
-                       coe_h[0], coe_h[1], coe_h[2], coe_h[3], gamma_bd, dgam, dfull);
-    A2C_HIP(c, hipGetLastError());
-  }
+  if (S.nh > 0)
+    return launch_chem64(c, ChemArgs{dcorr, {coe_h[0], coe_h[1], coe_h[2], coe_h[3]}, gamma_bd, dgam, dfull});
   return A2C_OK;
 }
 
