@@ -93,6 +93,7 @@ struct SegDot {  // out[0] = a1 . D^k1 b1, out[1] = a2 . D^k2 b2 (a2 may be null
   int32_t k1, k2;
   double* out;
   int32_t nsite, blk0;
+  int32_t done = 0;  // blocks arrived
 };
 
 // Coordinate groups of the scaled initial inverse Hessian: positions and
@@ -113,6 +114,8 @@ __host__ __device__ inline double group_gamma(const double* gs, double sy, doubl
 // recursion, m + 2 the second-loop dot, m + 3 and m + 4 g.D g and g.D^2 g of
 // scaled steepest descent, [m + 5, m + 5 + 2 NGROUP) s.y and y.D y of the
 // newest pair per coordinate group (m and m + 1 are unused).
+// Blocks of one op: a slot without sites keeps one, which writes its (zero) sums.
+__host__ __device__ inline int op_blocks(int nsite) { return nsite > 0 ? site_blocks(nsite) : 1; }
 constexpr int SCAL_PER_SLOT = 80;  // >= m + 5 + 2 NGROUP for m <= 64
 constexpr double SIGMA_STEP = 4.0;  // largest factor by which one line-search trial may change a width
 constexpr double Q_STEP = 0.25;     // largest displacement of a site in one line-search trial (A)
@@ -127,6 +130,16 @@ struct SegBound {  // sigma-bound operations: mode 0 project x, 1 gp = P g, 2 ze
   double lb, ub, stp;
   int32_t nsite, blk0;
 };
+
+// The four coordinates of a site at once (a slot's vectors are 256-byte aligned
+// allocations of its own).
+__device__ __forceinline__ void ld4(const double* p, size_t i, double (&v)[4]) {
+  const double4 t = *gmem(reinterpret_cast<const double4*>(p + i));
+  v[0] = t.x; v[1] = t.y; v[2] = t.z; v[3] = t.w;
+}
+__device__ __forceinline__ void st4(double* p, size_t i, const double (&v)[4]) {
+  *gmem(reinterpret_cast<double4*>(p + i)) = make_double4(v[0], v[1], v[2], v[3]);
+}
 
 __global__ __launch_bounds__(TB) void k_seg_axpby(const SegAx* __restrict__ ops, const int32_t* __restrict__ b2l) {
   const SegAx o = ops[b2l[blockIdx.x]];
@@ -144,8 +157,7 @@ __global__ __launch_bounds__(TB) void k_seg_axpby(const SegAx* __restrict__ ops,
   for (int c = 0; c < 4; ++c) o.z[i + c] = a * o.x[i + c] + bb * o.y[i + c];
 }
 
-__global__ __launch_bounds__(TB) void k_seg_dot(const SegDot* __restrict__ ops, const int32_t* __restrict__ b2l,
-                                                double* __restrict__ part, int nblk) {
+__global__ __launch_bounds__(TB) void k_seg_dot(SegDot* ops, const int32_t* __restrict__ b2l, double* part, int nblk) {
   __shared__ double r1[TB], r2[TB];
   const SegDot o = ops[b2l[blockIdx.x]];
   const int s = (blockIdx.x - o.blk0) * TB + threadIdx.x;
@@ -153,12 +165,17 @@ __global__ __launch_bounds__(TB) void k_seg_dot(const SegDot* __restrict__ ops, 
   if (s < o.nsite) {
     const size_t i = 4 * (size_t)s;
     const double di = metric_inv(o.met, s);
+    double a[4], b[4];
+    ld4(o.a1, i, a);
+    ld4(o.b1, i, b);
 #pragma unroll
-    for (int c = 0; c < 4; ++c) v1 += o.a1[i + c] * o.b1[i + c];
+    for (int c = 0; c < 4; ++c) v1 += a[c] * b[c];
     if (o.k1) v1 *= o.k1 == 1 ? di : di * di;
     if (o.a2) {
+      ld4(o.a2, i, a);
+      ld4(o.b2, i, b);
 #pragma unroll
-      for (int c = 0; c < 4; ++c) v2 += o.a2[i + c] * o.b2[i + c];
+      for (int c = 0; c < 4; ++c) v2 += a[c] * b[c];
       if (o.k2) v2 *= o.k2 == 1 ? di : di * di;
     }
   }
@@ -173,36 +190,13 @@ __global__ __launch_bounds__(TB) void k_seg_dot(const SegDot* __restrict__ ops, 
     __syncthreads();
   }
   if (threadIdx.x == 0) {
-    part[blockIdx.x] = r1[0];
-    part[nblk + blockIdx.x] = r2[0];
+    put_part(part + blockIdx.x, r1[0]);
+    put_part(part + nblk + blockIdx.x, r2[0]);
   }
-}
-
-// one block per op: fixed-order sum of the op's block partials
-__global__ __launch_bounds__(1024) void k_seg_dot_final(const SegDot* __restrict__ ops, const double* __restrict__ part,
-                                                        int nblk) {
-  __shared__ double r1[1024], r2[1024];
-  const SegDot o = ops[blockIdx.x];
-  const int n = site_blocks(o.nsite);
-  double v1 = 0.0, v2 = 0.0;
-  for (int i = threadIdx.x; i < n; i += 1024) {
-    v1 += part[o.blk0 + i];
-    v2 += part[nblk + o.blk0 + i];
-  }
-  r1[threadIdx.x] = v1;
-  r2[threadIdx.x] = v2;
-  __syncthreads();
-  for (int w = 512; w > 0; w >>= 1) {
-    if (threadIdx.x < w) {
-      r1[threadIdx.x] += r1[threadIdx.x + w];
-      r2[threadIdx.x] += r2[threadIdx.x + w];
-    }
-    __syncthreads();
-  }
-  if (threadIdx.x == 0) {
-    o.out[0] = r1[0];
-    if (o.a2) o.out[1] = r2[0];  // single dots write one scalar (device scalars are packed)
-  }
+  if (!last_block(&ops[b2l[blockIdx.x]].done, op_blocks(o.nsite))) return;
+  sum_parts<2>(part + o.blk0, nblk, op_blocks(o.nsite), [&](int k, double v) {
+    if (k == 0 || o.a2) o.out[k] = v;  // single dots write one scalar (device scalars are packed)
+  });
 }
 
 // block sum in a fixed order: wave trees, then the NT / 64 wave partials in order
@@ -224,8 +218,9 @@ template <int NT, int K>
 __device__ __forceinline__ void bsum_n(double (&v)[K], double* red) {
   constexpr int W = NT / 64;
 #pragma unroll
-  for (int k = 0; k < K; ++k)
-    for (int off = 32; off > 0; off >>= 1) v[k] += __shfl_down(v[k], off);
+  for (int off = 32; off > 0; off >>= 1)
+#pragma unroll
+    for (int k = 0; k < K; ++k) v[k] += __shfl_down(v[k], off);
   __syncthreads();  // the previous sum's readers are done with red
   if ((threadIdx.x & 63) == 0)
 #pragma unroll
@@ -357,38 +352,43 @@ struct SegPair {
   double* out;   // s.y
   double* out2;  // gp.gp
   int32_t nsite, blk0;
+  int32_t done = 0;  // blocks arrived
 };
 
-__global__ __launch_bounds__(TB) void k_seg_pair(const SegPair* __restrict__ ops, const int32_t* __restrict__ b2l,
-                                                 double* __restrict__ part, int nblk) {
+__global__ __launch_bounds__(TB) void k_seg_pair(SegPair* ops, const int32_t* __restrict__ b2l, double* part,
+                                                 int nblk) {
   __shared__ double red[TB / 64];
   const SegPair o = ops[b2l[blockIdx.x]];
   const int s = (blockIdx.x - o.blk0) * TB + threadIdx.x;
   double sy = 0.0, gg = 0.0;
   if (s < o.nsite) {
     const size_t i = 4 * (size_t)s;
+    double x[4], xo[4], g[4], go[4];
+    ld4(o.x, i, x);
+    ld4(o.xo, i, xo);
+    ld4(o.g, i, g);
+    ld4(o.go, i, go);
 #pragma unroll
     for (int c = 0; c < 4; ++c) {
-      const double gi = o.g[i + c];
-      const double si = o.x[i + c] - o.xo[i + c], yi = gi - o.go[i + c];
-      o.S[i + c] = si;
-      o.Y[i + c] = yi;
+      const double si = x[c] - xo[c], yi = g[c] - go[c];
       sy += si * yi;
-      double pi = gi;
-      if (c == 3) {
-        const double xs = o.x[i + 3];
-        if ((xs <= o.lb && gi > 0.0) || (xs >= o.ub && gi < 0.0)) pi = 0.0;
-      }
-      o.gp[i + c] = pi;
-      gg += pi * pi;
+      xo[c] = si;
+      go[c] = yi;
+      if (c == 3 && ((x[3] <= o.lb && g[3] > 0.0) || (x[3] >= o.ub && g[3] < 0.0))) g[3] = 0.0;
+      gg += g[c] * g[c];
     }
+    st4(o.S, i, xo);
+    st4(o.Y, i, go);
+    st4(o.gp, i, g);
   }
   sy = bsum<TB>(sy, red);
   gg = bsum<TB>(gg, red);
   if (threadIdx.x == 0) {
-    part[blockIdx.x] = sy;
-    part[nblk + blockIdx.x] = gg;
+    put_part(part + blockIdx.x, sy);
+    put_part(part + nblk + blockIdx.x, gg);
   }
+  if (!last_block(&ops[b2l[blockIdx.x]].done, op_blocks(o.nsite))) return;
+  sum_parts<2>(part + o.blk0, nblk, op_blocks(o.nsite), [&](int k, double v) { *(k ? o.out2 : o.out) = v; });
 }
 
 // one block per op: fixed-order sums of the op's NOUT block partials
@@ -417,11 +417,11 @@ __global__ __launch_bounds__(TB) void k_seg_bound(const SegBound* __restrict__ o
   if (MODE == 0) {
     o.z[i + 3] = fmin(fmax(o.z[i + 3], o.lb), o.ub);
   } else if (MODE == 1) {
-    o.z[i] = o.y[i];
-    o.z[i + 1] = o.y[i + 1];
-    o.z[i + 2] = o.y[i + 2];
-    const double gs = o.y[i + 3], xs = o.x[i + 3];
-    o.z[i + 3] = ((xs <= o.lb && gs > 0.0) || (xs >= o.ub && gs < 0.0)) ? 0.0 : gs;
+    double g[4];
+    ld4(o.y, i, g);
+    const double xs = o.x[i + 3];
+    if ((xs <= o.lb && g[3] > 0.0) || (xs >= o.ub && g[3] < 0.0)) g[3] = 0.0;
+    st4(o.z, i, g);
   } else if (MODE == 2) {
     const double xs = o.x[i + 3], ds = o.z[i + 3];
     if ((xs <= o.lb && ds < 0.0) || (xs >= o.ub && ds > 0.0)) o.z[i + 3] = 0.0;
@@ -434,21 +434,23 @@ __global__ __launch_bounds__(TB) void k_seg_bound(const SegBound* __restrict__ o
     // the -3 kB x ln(sigma) wall near zero).  The realised direction is built
     // from d and the scale factors, never as x - x_old, which would lose
     // digits to the ~100 A coordinates once steps are small.
-    const double d0 = o.y[i], d1 = o.y[i + 1], d2 = o.y[i + 2];
-    const double len = o.stp * sqrt(d0 * d0 + d1 * d1 + d2 * d2);
+    double x[4], d[4], w[4];
+    ld4(o.x, i, x);
+    ld4(o.y, i, d);
+    const double len = o.stp * sqrt(d[0] * d[0] + d[1] * d[1] + d[2] * d[2]);
     const double sc = len > Q_STEP ? Q_STEP / len : 1.0;  // a site moves at most Q_STEP per trial
-    const double w0 = sc * d0, w1 = sc * d1, w2 = sc * d2;
-    o.w[i] = w0;
-    o.w[i + 1] = w1;
-    o.w[i + 2] = w2;
-    o.z[i] = o.x[i] + o.stp * w0;
-    o.z[i + 1] = o.x[i + 1] + o.stp * w1;
-    o.z[i + 2] = o.x[i + 2] + o.stp * w2;
-    const double so = o.x[i + 3], ds = o.y[i + 3];
+#pragma unroll
+    for (int c = 0; c < 3; ++c) {
+      w[c] = sc * d[c];
+      x[c] += o.stp * w[c];
+    }
+    const double so = x[3], ds = d[3];
     const double lo = fmax(o.lb, so * (1.0 / SIGMA_STEP)), hi = fmin(o.ub, so * SIGMA_STEP);
     const double xs = so + o.stp * ds, cs = fmin(fmax(xs, lo), hi);
-    o.z[i + 3] = cs;
-    o.w[i + 3] = cs == xs ? ds : (cs - so) / o.stp;
+    x[3] = cs;
+    w[3] = cs == xs ? ds : (cs - so) / o.stp;
+    st4(o.w, i, w);
+    st4(o.z, i, x);
   }
 }
 
@@ -680,105 +682,15 @@ __device__ __forceinline__ void vf_coef(const double* acc, const double* yr, con
   }
 }
 
-__global__ __launch_bounds__(TL_THREADS) void k_two_loop_vf(const TwoLoop* __restrict__ ops) {
-  __shared__ double red[VF_SUMS * (TL_THREADS / 64)];
-  const TwoLoop& o = ops[blockIdx.x];
-  const int n = 4 * o.nsite, np = o.np, npd = o.npd;
-  const Metric met = o.met;
-  const double* __restrict__ g = o.g;
-  double* __restrict__ q = o.q;
-  const double* S[VF_PAIRS];
-  const double* Y[VF_PAIRS];
-  double rho[VF_PAIRS];
-#pragma unroll
-  for (int t = 0; t < VF_PAIRS; ++t) {
-    S[t] = t < np ? o.S[t] : nullptr;
-    Y[t] = t < np ? o.Y[t] : nullptr;
-    rho[t] = t < np ? o.rho[t] : 0.0;
-  }
-  // pass 1: [0, np) s_t . g; vf_tri(a, b) s_a . y_b; then s_0 . y_0 and
-  // y_0 . D y_0 per coordinate group
-  double acc[VF_SUMS] = {};
-  for (int i = threadIdx.x; i < n; i += TL_THREADS) {
-    double sv[VF_PAIRS], yv[VF_PAIRS];
-    const double gi = g[i];
-#pragma unroll
-    for (int t = 0; t < VF_PAIRS; ++t)
-      if (t < np) {
-        sv[t] = S[t][i];
-        yv[t] = Y[t][i];
-      }
-#pragma unroll
-    for (int a = 0; a < VF_PAIRS; ++a)
-      if (a < np) {
-        acc[a] += sv[a] * gi;
-#pragma unroll
-        for (int b = 0; b < a; ++b) acc[vf_tri(a, b)] += sv[a] * yv[b];
-      }
-    const int gr = group_of(i >> 2, i & 3, npd);
-    const double di = metric_inv(met, i >> 2);
-#pragma unroll
-    for (int k = 0; k < NGROUP; ++k) {
-      acc[VF_PAIRS + VF_TRI + 2 * k] += k == gr ? sv[0] * yv[0] : 0.0;
-      acc[VF_PAIRS + VF_TRI + 2 * k + 1] += k == gr ? yv[0] * yv[0] * di : 0.0;
-    }
-  }
-  tl_sum_n(acc, red);
-  double al[VF_PAIRS], gam[NGROUP];
-  vf_alpha(acc, rho, np, al);
-  vf_gamma(acc, gam);
-  // pass 2: r = diag(gamma_g) D (g - sum_t alpha_t y_t) into q; y_t . r
-  double yr[VF_PAIRS] = {};
-  for (int i = threadIdx.x; i < n; i += TL_THREADS) {
-    double yv[VF_PAIRS];
-#pragma unroll
-    for (int t = 0; t < VF_PAIRS; ++t)
-      if (t < np) yv[t] = Y[t][i];
-    double qi = g[i];
-#pragma unroll
-    for (int t = 0; t < VF_PAIRS; ++t)
-      if (t < np) qi -= al[t] * yv[t];
-    const double ri = vf_pick(gam, group_of(i >> 2, i & 3, npd)) * metric_inv(met, i >> 2) * qi;
-    q[i] = ri;
-#pragma unroll
-    for (int t = 0; t < VF_PAIRS; ++t)
-      if (t < np) yr[t] += yv[t] * ri;
-  }
-  tl_sum_n(yr, red);
-  double c[VF_PAIRS];
-  vf_coef(acc, yr, rho, np, al, c);
-  // pass 3: d = -(r + sum_t c_t s_t) (oldest first), widths at an active bound not moved; g . d
-  const double* __restrict__ x = o.x;
-  double* __restrict__ d = o.d;
-  const double lb = o.lb, ub = o.ub;
-  double gd = 0.0;
-  for (int i = threadIdx.x; i < n; i += TL_THREADS) {
-    double sv[VF_PAIRS];
-#pragma unroll
-    for (int t = 0; t < VF_PAIRS; ++t)
-      if (t < np) sv[t] = S[t][i];
-    const double gi = g[i], xs = (i & 3) == 3 ? x[i] : 0.0;
-    double ri = q[i];
-#pragma unroll
-    for (int t = VF_PAIRS - 1; t >= 0; --t)
-      if (t < np) ri += c[t] * sv[t];
-    double di = -ri;
-    if ((i & 3) == 3 && ((xs <= lb && di < 0.0) || (xs >= ub && di > 0.0))) di = 0.0;
-    d[i] = di;
-    gd += gi * di;
-  }
-  gd = tl_sum(gd, red);
-  if (threadIdx.x == 0) o.out[0] = gd;
-}
-
-// The vector-free recursion for slots too large for one workgroup: the three
-// passes as grid launches over all such slots, each followed by a
-// fixed-order reduction of its block partials into the slot's device
-// scalars (the VF_SUMS first-pass sums, then the y_t . r), which the next
-// pass reads to run the loops on the scalars itself.
+// The three passes as grid launches over all such slots.  A pass's last block
+// per slot sums the block partials into the slot's device scalars (the VF_SUMS
+// first-pass sums, then the y_t . r), which the next pass reads to run the loops
+// on the scalars itself.  1,728 sites, 5 pairs: one workgroup running the three
+// passes took 43 us, most of it one memory latency after another; a launch per
+// pass 22 us together (8,192 sites and more: 28 us, six launches before 55).
 struct SegVF {
   const double* g;
-  const double* S[VF_PAIRS];  // step t = 0 is the newest pair
+  const double* S[VF_PAIRS];  // step t = 0 is the newest pair (again past np)
   const double* Y[VF_PAIRS];
   double rho[VF_PAIRS];
   double* q;                  // r
@@ -790,10 +702,10 @@ struct SegVF {
   double lb, ub;
   int32_t np, npd;
   int32_t nsite, blk0;
+  int32_t done[3];            // blocks arrived, per pass
 };
 
-__global__ __launch_bounds__(TB) void k_seg_vf1(const SegVF* __restrict__ ops, const int32_t* __restrict__ b2l,
-                                                double* __restrict__ part, int nblk) {
+__global__ __launch_bounds__(TB) void k_seg_vf1(SegVF* ops, const int32_t* __restrict__ b2l, double* part, int nblk) {
   __shared__ double red[VF_SUMS * (TB / 64)];
   const SegVF o = ops[b2l[blockIdx.x]];
   const int s = (blockIdx.x - o.blk0) * TB + threadIdx.x;
@@ -802,40 +714,42 @@ __global__ __launch_bounds__(TB) void k_seg_vf1(const SegVF* __restrict__ ops, c
   if (s < o.nsite) {
     const size_t i0 = 4 * (size_t)s;
     const double di = metric_inv(o.met, s);
+    double g[4], sv[VF_PAIRS][4], yv[VF_PAIRS][4];
+    ld4(o.g, i0, g);
+#pragma unroll
+    for (int t = 0; t < VF_PAIRS; ++t) {  // past np the newest pair again: no branch around a load
+      ld4(o.S[t], i0, sv[t]);
+      ld4(o.Y[t], i0, yv[t]);
+    }
+#pragma unroll
+    for (int a = 0; a < VF_PAIRS; ++a)
+      if (a < np) {
+#pragma unroll
+        for (int c = 0; c < 4; ++c) {
+          acc[a] += sv[a][c] * g[c];
+#pragma unroll
+          for (int b = 0; b < a; ++b) acc[vf_tri(a, b)] += sv[a][c] * yv[b][c];
+        }
+      }
 #pragma unroll
     for (int c = 0; c < 4; ++c) {
-      const size_t i = i0 + c;
-      double sv[VF_PAIRS], yv[VF_PAIRS];
-      const double gi = o.g[i];
-#pragma unroll
-      for (int t = 0; t < VF_PAIRS; ++t)
-        if (t < np) {
-          sv[t] = o.S[t][i];
-          yv[t] = o.Y[t][i];
-        }
-#pragma unroll
-      for (int a = 0; a < VF_PAIRS; ++a)
-        if (a < np) {
-          acc[a] += sv[a] * gi;
-#pragma unroll
-          for (int b = 0; b < a; ++b) acc[vf_tri(a, b)] += sv[a] * yv[b];
-        }
       const int gr = group_of(s, c, o.npd);
 #pragma unroll
       for (int k = 0; k < NGROUP; ++k) {
-        acc[VF_PAIRS + VF_TRI + 2 * k] += k == gr ? sv[0] * yv[0] : 0.0;
-        acc[VF_PAIRS + VF_TRI + 2 * k + 1] += k == gr ? yv[0] * yv[0] * di : 0.0;
+        acc[VF_PAIRS + VF_TRI + 2 * k] += k == gr ? sv[0][c] * yv[0][c] : 0.0;
+        acc[VF_PAIRS + VF_TRI + 2 * k + 1] += k == gr ? yv[0][c] * yv[0][c] * di : 0.0;
       }
     }
   }
   bsum_n<TB>(acc, red);
   if (threadIdx.x == 0)
 #pragma unroll
-    for (int k = 0; k < VF_SUMS; ++k) part[(size_t)k * nblk + blockIdx.x] = acc[k];
+    for (int k = 0; k < VF_SUMS; ++k) put_part(part + (size_t)k * nblk + blockIdx.x, acc[k]);
+  if (!last_block(&ops[b2l[blockIdx.x]].done[0], op_blocks(o.nsite))) return;
+  sum_parts<VF_SUMS>(part + o.blk0, nblk, op_blocks(o.nsite), [&](int k, double v) { o.sums[k] = v; });
 }
 
-__global__ __launch_bounds__(TB) void k_seg_vf2(const SegVF* __restrict__ ops, const int32_t* __restrict__ b2l,
-                                                double* __restrict__ part, int nblk) {
+__global__ __launch_bounds__(TB) void k_seg_vf2(SegVF* ops, const int32_t* __restrict__ b2l, double* part, int nblk) {
   __shared__ double red[VF_PAIRS * (TB / 64)];
   const SegVF o = ops[b2l[blockIdx.x]];
   const int s = (blockIdx.x - o.blk0) * TB + threadIdx.x;
@@ -847,32 +761,31 @@ __global__ __launch_bounds__(TB) void k_seg_vf2(const SegVF* __restrict__ ops, c
   if (s < o.nsite) {
     const size_t i0 = 4 * (size_t)s;
     const double di = metric_inv(o.met, s);
+    double q[4], yv[VF_PAIRS][4];
+    ld4(o.g, i0, q);
+#pragma unroll
+    for (int t = 0; t < VF_PAIRS; ++t) ld4(o.Y[t], i0, yv[t]);
 #pragma unroll
     for (int c = 0; c < 4; ++c) {
-      const size_t i = i0 + c;
-      double yv[VF_PAIRS];
 #pragma unroll
       for (int t = 0; t < VF_PAIRS; ++t)
-        if (t < np) yv[t] = o.Y[t][i];
-      double qi = o.g[i];
+        if (t < np) q[c] -= al[t] * yv[t][c];
+      q[c] *= vf_pick(gam, group_of(s, c, o.npd)) * di;
 #pragma unroll
       for (int t = 0; t < VF_PAIRS; ++t)
-        if (t < np) qi -= al[t] * yv[t];
-      const double ri = vf_pick(gam, group_of(s, c, o.npd)) * di * qi;
-      o.q[i] = ri;
-#pragma unroll
-      for (int t = 0; t < VF_PAIRS; ++t)
-        if (t < np) yr[t] += yv[t] * ri;
+        if (t < np) yr[t] += yv[t][c] * q[c];
     }
+    st4(o.q, i0, q);
   }
   bsum_n<TB>(yr, red);
   if (threadIdx.x == 0)
 #pragma unroll
-    for (int k = 0; k < VF_PAIRS; ++k) part[(size_t)k * nblk + blockIdx.x] = yr[k];
+    for (int k = 0; k < VF_PAIRS; ++k) put_part(part + (size_t)k * nblk + blockIdx.x, yr[k]);
+  if (!last_block(&ops[b2l[blockIdx.x]].done[1], op_blocks(o.nsite))) return;
+  sum_parts<VF_PAIRS>(part + o.blk0, nblk, op_blocks(o.nsite), [&](int k, double v) { o.sums[VF_SUMS + k] = v; });
 }
 
-__global__ __launch_bounds__(TB) void k_seg_vf3(const SegVF* __restrict__ ops, const int32_t* __restrict__ b2l,
-                                                double* __restrict__ part) {
+__global__ __launch_bounds__(TB) void k_seg_vf3(SegVF* ops, const int32_t* __restrict__ b2l, double* part) {
   __shared__ double red[TB / 64];
   const SegVF o = ops[b2l[blockIdx.x]];
   const int s = (blockIdx.x - o.blk0) * TB + threadIdx.x;
@@ -883,41 +796,27 @@ __global__ __launch_bounds__(TB) void k_seg_vf3(const SegVF* __restrict__ ops, c
   double gd = 0.0;
   if (s < o.nsite) {
     const size_t i0 = 4 * (size_t)s;
+    double r[4], g[4], sv[VF_PAIRS][4];
+    ld4(o.q, i0, r);
+    ld4(o.g, i0, g);
+    const double xs = o.x[i0 + 3];
+#pragma unroll
+    for (int t = 0; t < VF_PAIRS; ++t) ld4(o.S[t], i0, sv[t]);
 #pragma unroll
     for (int k = 0; k < 4; ++k) {
-      const size_t i = i0 + k;
-      double ri = o.q[i];
 #pragma unroll
       for (int t = VF_PAIRS - 1; t >= 0; --t)
-        if (t < np) ri += c[t] * o.S[t][i];
-      double di = -ri;
-      if (k == 3) {
-        const double xs = o.x[i];
-        if ((xs <= o.lb && di < 0.0) || (xs >= o.ub && di > 0.0)) di = 0.0;
-      }
-      o.d[i] = di;
-      gd += o.g[i] * di;
+        if (t < np) r[k] += c[t] * sv[t][k];
+      r[k] = -r[k];
+      if (k == 3 && ((xs <= o.lb && r[3] < 0.0) || (xs >= o.ub && r[3] > 0.0))) r[3] = 0.0;
+      gd += g[k] * r[k];
     }
+    st4(o.d, i0, r);
   }
   gd = bsum<TB>(gd, red);
-  if (threadIdx.x == 0) part[blockIdx.x] = gd;
-}
-
-// one block per op: fixed-order sums of the K block partials of pass PASS
-template <int K, int PASS>
-__global__ __launch_bounds__(256) void k_seg_vf_final(const SegVF* __restrict__ ops, const double* __restrict__ part,
-                                                      int nblk) {
-  __shared__ double red[4];
-  const SegVF o = ops[blockIdx.x];
-  const int n = site_blocks(o.nsite);
-  double* out = PASS == 1 ? o.sums : (PASS == 2 ? o.sums + VF_SUMS : o.out);
-#pragma unroll
-  for (int k = 0; k < K; ++k) {
-    double v = 0.0;
-    for (int j = threadIdx.x; j < n; j += 256) v += part[(size_t)k * nblk + o.blk0 + j];
-    v = bsum<256>(v, red);
-    if (threadIdx.x == 0) out[k] = v;
-  }
+  if (threadIdx.x == 0) put_part(part + blockIdx.x, gd);
+  if (!last_block(&ops[b2l[blockIdx.x]].done[2], op_blocks(o.nsite))) return;
+  sum_parts<1>(part + o.blk0, 0, op_blocks(o.nsite), [&](int, double v) { o.out[0] = v; });
 }
 
 }  // namespace
@@ -997,8 +896,8 @@ struct a2c_batch {
   a2c::Arena arena;
   a2c::GraphCache graphs;
   int qrc = 0;  // first error of a queued operation
-  bool fused_two_loop = true;  // small slots run the two-loop recursion in one workgroup
-  bool vector_free = true;     // slots of at most VF_PAIRS pairs take the vector-free form
+  bool vector_free = true;     // slots of at most VF_PAIRS pairs take the vector-free form of the recursion
+  bool fused_two_loop = true;  // of the others, small ones run it in one workgroup
   double* dF = nullptr;    // objective per slot (device)
   double* hF = nullptr;    // pinned mirror
   double* dres = nullptr;  // 2 doubles per slot (device dot results read by the host)
@@ -1143,7 +1042,7 @@ int seg_launch_prep(a2c_batch* b, const std::vector<int>& ids, Fill fill, Op** d
     fill(ops[k], s);
     ops[k].nsite = s.N();
     ops[k].blk0 = cum;
-    const int nb = site_blocks(s.N());
+    const int nb = op_blocks(s.N());
     map.insert(map.end(), nb, (int32_t)k);
     cum += nb;
   }
@@ -1178,16 +1077,12 @@ int seg_axpby(a2c_batch* b, const std::vector<int>& ids, Fill fill) {
   return A2C_OK;
 }
 
-// block partials, then one fixed-order sum per op
-void enqueue_dot(a2c_batch* b, const SegDot* ops, const int32_t* map, int nblk, unsigned nops) {
+void enqueue_dot(a2c_batch* b, SegDot* ops, const int32_t* map, int nblk) {
   double* part = b->dpart;
   if (nblk)
     enqueue(b, {2, u64(ops), u64(map), u64(part), (uint64_t)nblk}, [=](hipStream_t st) {
       hipLaunchKernelGGL(k_seg_dot, dim3(nblk), dim3(TB), 0, st, ops, map, part, nblk);
     });
-  enqueue(b, {3, u64(ops), u64(part), (uint64_t)nblk, nops}, [=](hipStream_t st) {
-    hipLaunchKernelGGL(k_seg_dot_final, dim3(nops), dim3(1024), 0, st, ops, part, nblk);
-  });
 }
 
 // dot products per slot; results (2 per slot) returned in out[k*2 + 0/1]
@@ -1206,7 +1101,7 @@ int seg_dot(a2c_batch* b, const std::vector<int>& ids, Fill fill, std::vector<do
   int32_t* map;
   int nblk;
   if (int rc = seg_launch_prep<SegDot>(b, ids, fill2, &ops, &map, &nblk)) return rc;
-  enqueue_dot(b, ops, map, nblk, (unsigned)ids.size());
+  enqueue_dot(b, ops, map, nblk);
   enqueue_d2h(b, b->hres, b->dres, sizeof(double) * 2 * b->slots.size());
   if (int rc = bsync(b)) return rc;
   for (size_t k = 0; k < ids.size(); ++k) {
@@ -1230,7 +1125,7 @@ int seg_dot_dev(a2c_batch* b, const std::vector<int>& ids, Fill fill) {
   int32_t* map;
   int nblk;
   if (int rc = seg_launch_prep<SegDot>(b, ids, fill2, &ops, &map, &nblk)) return rc;
-  enqueue_dot(b, ops, map, nblk, (unsigned)ids.size());
+  enqueue_dot(b, ops, map, nblk);
   return A2C_OK;
 }
 
@@ -1269,7 +1164,7 @@ int seg_tl(a2c_batch* b, const std::vector<int>& ids, bool first, Fill fill) {
   return A2C_OK;
 }
 
-// the three passes of the segmented vector-free recursion and their reductions
+// the three passes of the vector-free recursion
 template <class Fill>
 int seg_vf(a2c_batch* b, const std::vector<int>& ids, Fill fill) {
   if (ids.empty()) return A2C_OK;
@@ -1282,28 +1177,12 @@ int seg_vf(a2c_batch* b, const std::vector<int>& ids, Fill fill) {
   int nblk;
   if (int rc = seg_launch_prep<SegVF>(b, ids, fill0, &ops, &map, &nblk)) return rc;
   double* part = b->dpart;
-  const unsigned nops = (unsigned)ids.size();
   if (nblk)
     enqueue(b, {14, u64(ops), u64(map), u64(part), (uint64_t)nblk}, [=](hipStream_t st) {
       hipLaunchKernelGGL(k_seg_vf1, dim3(nblk), dim3(TB), 0, st, ops, map, part, nblk);
-    });
-  enqueue(b, {15, u64(ops), u64(part), (uint64_t)nblk, nops}, [=](hipStream_t st) {
-    hipLaunchKernelGGL((k_seg_vf_final<VF_SUMS, 1>), dim3(nops), dim3(256), 0, st, ops, part, nblk);
-  });
-  if (nblk)
-    enqueue(b, {16, u64(ops), u64(map), u64(part), (uint64_t)nblk}, [=](hipStream_t st) {
       hipLaunchKernelGGL(k_seg_vf2, dim3(nblk), dim3(TB), 0, st, ops, map, part, nblk);
-    });
-  enqueue(b, {17, u64(ops), u64(part), (uint64_t)nblk, nops}, [=](hipStream_t st) {
-    hipLaunchKernelGGL((k_seg_vf_final<VF_PAIRS, 2>), dim3(nops), dim3(256), 0, st, ops, part, nblk);
-  });
-  if (nblk)
-    enqueue(b, {18, u64(ops), u64(map), u64(part), (uint64_t)nblk}, [=](hipStream_t st) {
       hipLaunchKernelGGL(k_seg_vf3, dim3(nblk), dim3(TB), 0, st, ops, map, part);
     });
-  enqueue(b, {19, u64(ops), u64(part), (uint64_t)nblk, nops}, [=](hipStream_t st) {
-    hipLaunchKernelGGL((k_seg_vf_final<1, 3>), dim3(nops), dim3(256), 0, st, ops, part, nblk);
-  });
   return A2C_OK;
 }
 
@@ -1324,14 +1203,10 @@ int seg_pair(a2c_batch* b, const std::vector<int>& ids, std::vector<double>& out
   int nblk;
   if (int rc = seg_launch_prep<SegPair>(b, ids, fill, &ops, &map, &nblk)) return rc;
   double* part = b->dpart;
-  const unsigned nops = (unsigned)ids.size();
   if (nblk)
     enqueue(b, {12, u64(ops), u64(map), u64(part), (uint64_t)nblk}, [=](hipStream_t st) {
       hipLaunchKernelGGL(k_seg_pair, dim3(nblk), dim3(TB), 0, st, ops, map, part, nblk);
     });
-  enqueue(b, {13, u64(ops), u64(part), (uint64_t)nblk, nops}, [=](hipStream_t st) {
-    hipLaunchKernelGGL((k_seg_final<SegPair, 2>), dim3(nops), dim3(256), 0, st, ops, part, nblk);
-  });
   enqueue_d2h(b, b->hres, b->dres, sizeof(double) * 2 * b->slots.size());
   if (int rc = bsync(b)) return rc;
   for (size_t k = 0; k < ids.size(); ++k) {
@@ -1597,27 +1472,22 @@ int directions(a2c_batch* b, const std::vector<int>& ids) {
     if (s.steepest || s.npairs == 0) {
       s.npairs = 0;
       sd.push_back(i);
-    } else if (b->fused_two_loop && s.N() <= TL_MAX_SITES) {
-      small.push_back(i);
     } else if (b->vector_free && s.npairs <= VF_PAIRS) {
       tlvf.push_back(i);
+    } else if (b->fused_two_loop && s.N() <= TL_MAX_SITES) {
+      small.push_back(i);
     } else {
       tl.push_back(i);
       maxp = std::max(maxp, s.npairs);
     }
   }
-  // fused recursion: vector-free for up to VF_PAIRS pairs, one pass per step above
-  for (int vf = 1; vf >= 0; --vf) {
-    std::vector<int> part;
-    for (int i : small)
-      if ((b->vector_free && b->slots[i].npairs <= VF_PAIRS) == (vf == 1)) part.push_back(i);
-    if (part.empty()) continue;
-    std::vector<TwoLoop> ops(part.size());
-    for (size_t k = 0; k < part.size(); ++k) {
-      Slot& s = b->slots[part[k]];
+  if (!small.empty()) {  // fused recursion, one pass per step
+    std::vector<TwoLoop> ops(small.size());
+    for (size_t k = 0; k < small.size(); ++k) {
+      Slot& s = b->slots[small[k]];
       TwoLoop& o = ops[k];
       o.g = s.g; o.q = s.q; o.d = s.d; o.x = s.x;
-      o.out = b->dres + 2 * part[k];
+      o.out = b->dres + 2 * small[k];
       for (int t = 0; t < s.npairs; ++t) {
         const int p = (s.head - 1 - t + s.m) % s.m;
         o.S[t] = s.S[p]; o.Y[t] = s.Y[p]; o.rho[t] = s.rho[p];
@@ -1632,9 +1502,8 @@ int directions(a2c_batch* b, const std::vector<int>& ids) {
     const TwoLoop* dops = b->arena.push(ops.data(), ops.size());
     if (!dops) return berr(b, A2C_ENOMEM, "staging arena too small");
     const unsigned nops = (unsigned)ops.size();
-    enqueue(b, {6, (uint64_t)vf, u64(dops), nops}, [=](hipStream_t st) {
-      if (vf) hipLaunchKernelGGL(k_two_loop_vf, dim3(nops), dim3(TL_THREADS), 0, st, dops);
-      else hipLaunchKernelGGL(k_two_loop, dim3(nops), dim3(TL_THREADS), 0, st, dops);
+    enqueue(b, {6, u64(dops), nops}, [=](hipStream_t st) {
+      hipLaunchKernelGGL(k_two_loop, dim3(nops), dim3(TL_THREADS), 0, st, dops);
     });
   }
   std::vector<double> v;
@@ -1642,9 +1511,9 @@ int directions(a2c_batch* b, const std::vector<int>& ids) {
   static_assert(VF_SUMS + VF_PAIRS <= SCAL_PER_SLOT, "device scalars of the vector-free recursion");
   if (int rc = seg_vf(b, tlvf, [&](SegVF& o, Slot& s) {
         o.g = s.g; o.q = s.q; o.d = s.d; o.x = s.x;
-        for (int t = 0; t < s.npairs; ++t) {
-          const int p = (s.head - 1 - t + s.m) % s.m;
-          o.S[t] = s.S[p]; o.Y[t] = s.Y[p]; o.rho[t] = s.rho[p];
+        for (int t = 0; t < VF_PAIRS; ++t) {
+          const int p = (s.head - 1 - (t < s.npairs ? t : 0) + s.m) % s.m;
+          o.S[t] = s.S[p]; o.Y[t] = s.Y[p]; o.rho[t] = t < s.npairs ? s.rho[p] : 0.0;
         }
         o.np = s.npairs; o.npd = s.fe->desc.n_pd; o.met = s.metric();
         o.lb = s.opts.sigma_lb; o.ub = s.opts.sigma_ub;

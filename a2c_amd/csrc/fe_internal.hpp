@@ -303,6 +303,59 @@ __device__ inline int xcd_block() {
   return x * q + (x < r ? x : r) + b / NUM_XCD;
 }
 
+// Block partials summed by the block of their group that arrives last, instead of
+// by a launch of its own (~4 us and a gap for a few kilobytes).  Thread 0 puts its
+// block's partials with put_part, then the whole block calls last_block; where
+// it returns true, every partial of the group's n blocks is visible to get_part
+// (device-scope accesses, which pass the XCDs' separate L2s by; the wait orders the
+// partials before the count without writing those caches back).  sum_parts adds
+// in an order that depends on n alone.  done starts at 0.
+__device__ __forceinline__ void put_part(double* p, double v) {
+  __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ double get_part(const double* p) {
+  return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ bool last_block(int32_t* done, int n) {
+  __shared__ int last;
+  if (threadIdx.x == 0) {
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    last = __hip_atomic_fetch_add(done, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == n - 1;
+  }
+  __syncthreads();
+  return last != 0;
+}
+// out(k, sum of part[k stride + j], j < n) for k < K, by a block of SITE_BLOCK:
+// wave w takes k = w, w + 4, ..., all of its sums' loads and trees in flight
+// together.
+template <int K, class Out>
+__device__ __forceinline__ void sum_parts(const double* part, size_t stride, int n, Out out) {
+  constexpr int W = SITE_BLOCK / 64, KW = (K + W - 1) / W, U = KW > 4 ? 1 : 8 / KW;  // sums per wave, loads per sum
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+  double v[KW] = {};
+  for (int j0 = lane; j0 < n; j0 += 64 * U) {
+    double p[KW][U];
+#pragma unroll
+    for (int i = 0; i < KW; ++i)
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        const int k = w + W * i, j = j0 + 64 * u;
+        p[i][u] = k < K && j < n ? get_part(part + k * stride + j) : 0.0;
+      }
+#pragma unroll
+    for (int i = 0; i < KW; ++i)
+#pragma unroll
+      for (int u = 0; u < U; ++u) v[i] += p[i][u];
+  }
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1)
+#pragma unroll
+    for (int i = 0; i < KW; ++i) v[i] += __shfl_down(v[i], off);
+#pragma unroll
+  for (int i = 0; i < KW; ++i)
+    if (lane == 0 && w + W * i < K) out(w + W * i, v[i]);
+}
+
 struct Timing;
 
 // a2c_fe_create on a stream of the caller's (a batch's own lattices share
