@@ -114,8 +114,6 @@ __host__ __device__ inline double group_gamma(const double* gs, double sy, doubl
 // recursion, m + 2 the second-loop dot, m + 3 and m + 4 g.D g and g.D^2 g of
 // scaled steepest descent, [m + 5, m + 5 + 2 NGROUP) s.y and y.D y of the
 // newest pair per coordinate group (m and m + 1 are unused).
-// Blocks of one op: a slot without sites keeps one, which writes its (zero) sums.
-__host__ __device__ inline int op_blocks(int nsite) { return nsite > 0 ? site_blocks(nsite) : 1; }
 constexpr int SCAL_PER_SLOT = 80;  // >= m + 5 + 2 NGROUP for m <= 64
 constexpr double SIGMA_STEP = 4.0;  // largest factor by which one line-search trial may change a width
 constexpr double Q_STEP = 0.25;     // largest displacement of a site in one line-search trial (A)
@@ -193,8 +191,8 @@ __global__ __launch_bounds__(TB) void k_seg_dot(SegDot* ops, const int32_t* __re
     put_part(part + blockIdx.x, r1[0]);
     put_part(part + nblk + blockIdx.x, r2[0]);
   }
-  if (!last_block(&ops[b2l[blockIdx.x]].done, op_blocks(o.nsite))) return;
-  sum_parts<2>(part + o.blk0, nblk, op_blocks(o.nsite), [&](int k, double v) {
+  if (!last_block(&ops[b2l[blockIdx.x]].done, lattice_blocks(o.nsite))) return;
+  sum_parts<2>(part + o.blk0, nblk, lattice_blocks(o.nsite), [&](int k, double v) {
     if (k == 0 || o.a2) o.out[k] = v;  // single dots write one scalar (device scalars are packed)
   });
 }
@@ -387,8 +385,8 @@ __global__ __launch_bounds__(TB) void k_seg_pair(SegPair* ops, const int32_t* __
     put_part(part + blockIdx.x, sy);
     put_part(part + nblk + blockIdx.x, gg);
   }
-  if (!last_block(&ops[b2l[blockIdx.x]].done, op_blocks(o.nsite))) return;
-  sum_parts<2>(part + o.blk0, nblk, op_blocks(o.nsite), [&](int k, double v) { *(k ? o.out2 : o.out) = v; });
+  if (!last_block(&ops[b2l[blockIdx.x]].done, lattice_blocks(o.nsite))) return;
+  sum_parts<2>(part + o.blk0, nblk, lattice_blocks(o.nsite), [&](int k, double v) { *(k ? o.out2 : o.out) = v; });
 }
 
 // one block per op: fixed-order sums of the op's NOUT block partials
@@ -745,8 +743,8 @@ __global__ __launch_bounds__(TB) void k_seg_vf1(SegVF* ops, const int32_t* __res
   if (threadIdx.x == 0)
 #pragma unroll
     for (int k = 0; k < VF_SUMS; ++k) put_part(part + (size_t)k * nblk + blockIdx.x, acc[k]);
-  if (!last_block(&ops[b2l[blockIdx.x]].done[0], op_blocks(o.nsite))) return;
-  sum_parts<VF_SUMS>(part + o.blk0, nblk, op_blocks(o.nsite), [&](int k, double v) { o.sums[k] = v; });
+  if (!last_block(&ops[b2l[blockIdx.x]].done[0], lattice_blocks(o.nsite))) return;
+  sum_parts<VF_SUMS>(part + o.blk0, nblk, lattice_blocks(o.nsite), [&](int k, double v) { o.sums[k] = v; });
 }
 
 __global__ __launch_bounds__(TB) void k_seg_vf2(SegVF* ops, const int32_t* __restrict__ b2l, double* part, int nblk) {
@@ -781,8 +779,8 @@ __global__ __launch_bounds__(TB) void k_seg_vf2(SegVF* ops, const int32_t* __res
   if (threadIdx.x == 0)
 #pragma unroll
     for (int k = 0; k < VF_PAIRS; ++k) put_part(part + (size_t)k * nblk + blockIdx.x, yr[k]);
-  if (!last_block(&ops[b2l[blockIdx.x]].done[1], op_blocks(o.nsite))) return;
-  sum_parts<VF_PAIRS>(part + o.blk0, nblk, op_blocks(o.nsite), [&](int k, double v) { o.sums[VF_SUMS + k] = v; });
+  if (!last_block(&ops[b2l[blockIdx.x]].done[1], lattice_blocks(o.nsite))) return;
+  sum_parts<VF_PAIRS>(part + o.blk0, nblk, lattice_blocks(o.nsite), [&](int k, double v) { o.sums[VF_SUMS + k] = v; });
 }
 
 __global__ __launch_bounds__(TB) void k_seg_vf3(SegVF* ops, const int32_t* __restrict__ b2l, double* part) {
@@ -815,8 +813,8 @@ __global__ __launch_bounds__(TB) void k_seg_vf3(SegVF* ops, const int32_t* __res
   }
   gd = bsum<TB>(gd, red);
   if (threadIdx.x == 0) put_part(part + blockIdx.x, gd);
-  if (!last_block(&ops[b2l[blockIdx.x]].done[2], op_blocks(o.nsite))) return;
-  sum_parts<1>(part + o.blk0, 0, op_blocks(o.nsite), [&](int, double v) { o.out[0] = v; });
+  if (!last_block(&ops[b2l[blockIdx.x]].done[2], lattice_blocks(o.nsite))) return;
+  sum_parts<1>(part + o.blk0, 0, lattice_blocks(o.nsite), [&](int, double v) { o.out[0] = v; });
 }
 
 }  // namespace
@@ -1042,7 +1040,7 @@ int seg_launch_prep(a2c_batch* b, const std::vector<int>& ids, Fill fill, Op** d
     fill(ops[k], s);
     ops[k].nsite = s.N();
     ops[k].blk0 = cum;
-    const int nb = op_blocks(s.N());
+    const int nb = lattice_blocks(s.N());
     map.insert(map.end(), nb, (int32_t)k);
     cum += nb;
   }
@@ -1279,7 +1277,7 @@ int fused_eval(a2c_batch* b, const std::vector<int>& ids_in, bool fp64, StateOf 
   }
   std::vector<LatDev> lats(ids.size());
   std::vector<int32_t> map, omap;  // site block -> lattice; pair-owner workgroup -> lattice
-  int cum = 0, ocum = 0, rules = 0;
+  int cum = 0, ocum = 0, rules = 0, rq = 1;
   for (size_t k = 0; k < ids.size(); ++k) {
     Slot& s = b->slots[ids[k]];
     LatDev L = s.fe->sys();
@@ -1296,7 +1294,8 @@ int fused_eval(a2c_batch* b, const std::vector<int>& ids_in, bool fp64, StateOf 
     const int kl = fp64 ? L.kl64 : L.kl32;
     L.owg0_32 = L.owg0_64 = ocum;
     lats[k] = L;
-    const int nb = site_blocks(s.N());
+    const int nb = lattice_blocks(s.N());
+    rq = std::max(rq, (int)L.rl);
     map.insert(map.end(), nb, (int32_t)k);
     const int no = owner_units(L.npd, L.nh, kl);
     omap.insert(omap.end(), (size_t)no, (int32_t)k);
@@ -1315,6 +1314,7 @@ int fused_eval(a2c_batch* b, const std::vector<int>& ids_in, bool fp64, StateOf 
   L.lats = dl;
   L.b2l = dm;
   L.nblk = cum;
+  L.rq = rq;
   L.ob2l = dom;
   L.onblk = ocum;
   L.nlat = (int)ids.size();
@@ -1326,7 +1326,7 @@ int fused_eval(a2c_batch* b, const std::vector<int>& ids_in, bool fp64, StateOf 
   L.tab64 = b->dtab64;
   L.mixed_full = mixed_full_pairs();
   L.full_pairs64 = fp64_full_pairs();
-  enqueue(b, {5, (uint64_t)fp64, u64(L.lats), u64(L.b2l), u64(L.ob2l), (uint64_t)L.nblk, (uint64_t)L.onblk,
+  enqueue(b, {5, (uint64_t)fp64, u64(L.lats), u64(L.b2l), u64(L.ob2l), (uint64_t)L.nblk, (uint64_t)L.rq, (uint64_t)L.onblk,
               (uint64_t)L.nlat, (uint64_t)L.rules, (uint64_t)L.deriv_mode, u64(L.fd_eps), u64(L.tab), u64(L.tab64),
               (uint64_t)L.mixed_full, (uint64_t)L.full_pairs64},
           [=](hipStream_t st) {

@@ -663,24 +663,24 @@ __global__ __launch_bounds__(TB) __attribute__((amdgpu_waves_per_eu(6))) void k_
   if (ln.ph == 0) gmem(S.rho)[s] = rho;
 }
 
-__global__ __launch_bounds__(TB) void k_dens_recv(const LatDev* __restrict__ lats, const int32_t* __restrict__ b2l) {
-  const int blk = xcd_block();
+__global__ __launch_bounds__(TB) void k_dens_recv(const LatDev* __restrict__ lats, const int32_t* __restrict__ b2l,
+                                                  int rq) {
+  const int v = xcd_block(), blk = v / rq;
   const LatDev& S = lats[b2l[blk]];
-  const int s = (blk - S.blk0) * TB + threadIdx.x;
-  const int N = S.npd + S.nh;
-  if (s >= N) return;
+  const RecvLane ln(S, blk - S.blk0, v % rq);
+  const int s = ln.s;
+  if (ln.idle || s >= S.npd + S.nh) return;
   const double* __restrict__ xo = S.xrow;
   const bool pd = s < S.npd;
   const int row = pd ? s : s - S.npd;
-  double rho = S.rho[s];
+  double rho = 0.0;
 #pragma unroll
-  for (int side = 0; side < 2; ++side) {
-    const int list = pd ? side : 2 + side;
-    const Ell& L = list == 0 ? S.pdpd : (list == 1 ? S.pdh : (list == 2 ? S.hpd : S.hh));
-    const int n = L.rcnt[row];
-    // shares arrive weighted by their senders
-    for_row_shares<RECV_RU_SCALAR>(gmem(reinterpret_cast<const float*>(L.rbuf)), L.rows, row, n, [&](float v) { rho += (double)v; });
+  for (int side = 0; side < 2; ++side) {  // shares arrive weighted by their senders
+    const Ell& L = pd ? (side ? S.pdh : S.pdpd) : (side ? S.hh : S.hpd);
+    row_shares<RECV_RU_SCALAR, float>(L, row, ln.ph, ln.G, [&](float v) { rho += (double)v; });
   }
+  rho = ln.sum(rho) + S.rho[s];
+  if (ln.ph) return;
   rho *= S.rule == GH3 ? GHQW : QW;
   S.rho[s] = rho;
   const double xs = pd ? 1.0 : xo[row];
@@ -953,33 +953,34 @@ __global__ __launch_bounds__(TBO) __attribute__((amdgpu_waves_per_eu(TBO / 128))
   gmem(S.epair)[s] = o.e;
 }
 
-__global__ __launch_bounds__(TB) void k_grad_recv(const LatDev* __restrict__ lats, const int32_t* __restrict__ b2l) {
-  __shared__ double red[TB];
-  const int blk = xcd_block();
+__global__ __launch_bounds__(TB) void k_grad_recv(const LatDev* __restrict__ lats, const int32_t* __restrict__ b2l,
+                                                 int rq) {
+  const int v = xcd_block(), blk = v / rq;
   const LatDev& S = lats[b2l[blk]];
-  const int lb = blk - S.blk0;
-  const int s = lb * TB + threadIdx.x;
-  const int N = S.npd + S.nh;
+  const RecvLane ln(S, blk - S.blk0, v % rq);
+  if (ln.idle) return;
+  const int s = ln.s;
   double fs = 0.0;
-  if (s < N) {
+  if (s < S.npd + S.nh) {
     const double* __restrict__ xo = S.xrow;
     const bool pd = s < S.npd;
     const int row = pd ? s : s - S.npd;
     double* __restrict__ G = S.G;
     const size_t site = pd ? site_of_row(row, S.npd) : S.npd + site_of_row(row, S.nh);
-    const double4 own = S.gown[s];
-    double g0 = own.x, g1 = own.y, g2 = own.z, gs = own.w;
+    double g0 = 0.0, g1 = 0.0, g2 = 0.0, gs = 0.0;
+    if (ln.ph == 0) {
+      const double4 own = S.gown[s];
+      g0 = own.x; g1 = own.y; g2 = own.z; gs = own.w;
+    }
 #pragma unroll
-    for (int side = 0; side < 2; ++side) {
-      const int list = pd ? side : 2 + side;
-      const Ell& L = list == 0 ? S.pdpd : (list == 1 ? S.pdh : (list == 2 ? S.hpd : S.hh));
-      const int n = L.rcnt[row];
-      // shares arrive weighted by their senders
-      for_row_shares<RECV_RU_WIDE>(gmem(reinterpret_cast<const float4*>(L.rbuf)), L.rows, row, n, [&](const float4& v) {
+    for (int side = 0; side < 2; ++side) {  // shares arrive weighted by their senders
+      const Ell& L = pd ? (side ? S.pdh : S.pdpd) : (side ? S.hh : S.hpd);
+      row_shares<RECV_RU_WIDE, float4>(L, row, ln.ph, ln.G, [&](const float4& v) {
         g0 += v.x; g1 += v.y; g2 += v.z;
         gs += v.w;
       });
     }
+    g0 = ln.sum(g0); g1 = ln.sum(g1); g2 = ln.sum(g2); gs = ln.sum(gs);
     const double xi = pd ? 1.0 : xo[row];
     const double sg = S.qzs[s].y;
     const double T = S.T;
@@ -987,20 +988,15 @@ __global__ __launch_bounds__(TB) void k_grad_recv(const LatDev* __restrict__ lat
     const double qw = gh ? GHQW : QW, sq = gh ? 1.0 : SQ6;
     const double V = S.emb[s] + qw * xi * S.epair[s];  // owned pairs carry their full energy
     const double sc = qw * xi / T;
-    G[4 * site + 0] = sc * g0;
-    G[4 * site + 1] = sc * g1;
-    G[4 * site + 2] = sc * g2;
-    G[4 * site + 3] = sq * sc * gs - 3.0 * KB * xi / sg;
-    fs = V / T - 3.0 * KB * xi * log(sg);
+    if (ln.ph == 0) {
+      G[4 * site + 0] = sc * g0;
+      G[4 * site + 1] = sc * g1;
+      G[4 * site + 2] = sc * g2;
+      G[4 * site + 3] = sq * sc * gs - 3.0 * KB * xi / sg;
+      fs = V / T - 3.0 * KB * xi * log(sg);
+    }
   }
-  red[threadIdx.x] = fs;
-  __syncthreads();
-#pragma unroll
-  for (int w = TB / 2; w > 0; w >>= 1) {
-    if (threadIdx.x < w) red[threadIdx.x] += red[threadIdx.x + w];
-    __syncthreads();
-  }
-  if (threadIdx.x == 0) S.part[lb] = red[0];
+  finish_objective(S, ln, fs);
 }
 
 }  // namespace
@@ -1140,22 +1136,23 @@ int run_eval32(const Launch& L, Timing* tm) {
     if (tm) tm->mark(L.stream, "rows");
     if (run_rows(L)) return A2C_EHIP;
     if (tm) tm->mark(L.stream, "dens_own");
-    if (L.rules & (1 << A2C_QUAD_R12))
+    if (L.onblk > 0 && (L.rules & (1 << A2C_QUAD_R12)))
       hipLaunchKernelGGL(k_dens_own<A2C_QUAD_R12>, dim3(L.onblk), dim3(TB), 0, L.stream, L.lats, L.ob2l, L.tab);
-    if (L.rules & (1 << GH3))
+    if (L.onblk > 0 && (L.rules & (1 << GH3)))
       hipLaunchKernelGGL(k_dens_own<GH3>, dim3(L.onblk), dim3(TB), 0, L.stream, L.lats, L.ob2l, L.tab);
     if (hipGetLastError() != hipSuccess) return A2C_EHIP;
     if (tm) tm->mark(L.stream, "dens_recv");
-    hipLaunchKernelGGL(k_dens_recv, dim3(L.nblk), dim3(TB), 0, L.stream, L.lats, L.b2l);
+    hipLaunchKernelGGL(k_dens_recv, dim3(L.nblk * L.rq), dim3(TB), 0, L.stream, L.lats, L.b2l, L.rq);
     if (hipGetLastError() != hipSuccess) return A2C_EHIP;
     if (tm) tm->mark(L.stream, "grad_own");
-    if (L.rules & (1 << A2C_QUAD_R12))
-      launch_grad_own<A2C_QUAD_R12>(L);
-    if (L.rules & (1 << GH3)) launch_grad_own<GH3>(L);
+    if (L.onblk > 0 && (L.rules & (1 << A2C_QUAD_R12))) launch_grad_own<A2C_QUAD_R12>(L);
+    if (L.onblk > 0 && (L.rules & (1 << GH3))) launch_grad_own<GH3>(L);
     if (hipGetLastError() != hipSuccess) return A2C_EHIP;
     if (tm) tm->mark(L.stream, "grad_recv");
-    hipLaunchKernelGGL(k_grad_recv, dim3(L.nblk), dim3(TB), 0, L.stream, L.lats, L.b2l);
+    hipLaunchKernelGGL(k_grad_recv, dim3(L.nblk * L.rq), dim3(TB), 0, L.stream, L.lats, L.b2l, L.rq);
     if (hipGetLastError() != hipSuccess) return A2C_EHIP;
+    if (tm) tm->mark(L.stream, nullptr);
+    return A2C_OK;
   }
   if (tm) tm->mark(L.stream, "final_sum");
   if (int rc = run_final_sum(L)) return rc;

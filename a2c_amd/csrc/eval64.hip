@@ -661,23 +661,23 @@ __global__ __launch_bounds__(TBO) __attribute__((amdgpu_waves_per_eu(4))) void k
 // else in row order (the passes that follow).
 template <int DM>
 __global__ __launch_bounds__(TB) void k_dens_recv64(const LatDev* __restrict__ lats, const int32_t* __restrict__ b2l,
-                                                    double eps, int by_site) {
-  const int blk = xcd_block();
+                                                    int rq, double eps, int by_site) {
+  const int v = xcd_block(), blk = v / rq;
   const LatDev& S = lats[b2l[blk]];
-  const int s = (blk - S.blk0) * TB + threadIdx.x;
-  const int N = S.npd + S.nh;
-  if (s >= N) return;
+  const RecvLane ln(S, blk - S.blk0, v % rq);
+  const int s = ln.s;
+  if (ln.idle || s >= S.npd + S.nh) return;
   const double* __restrict__ xo = S.xrow;
   const bool pd = s < S.npd;
   const int row = pd ? s : s - S.npd;
-  double rho = S.epair[s];
+  double rho = 0.0;
 #pragma unroll
-  for (int side = 0; side < 2; ++side) {
+  for (int side = 0; side < 2; ++side) {  // shares arrive weighted by their senders
     const Ell& L = pd ? (side ? S.pdh : S.pdpd) : (side ? S.hh : S.hpd);
-    const int n = L.rcnt[row];
-    // shares arrive weighted by their senders
-    for_row_shares<RECV_RU_SCALAR>(gmem(reinterpret_cast<const double*>(L.rbuf)), L.rows, row, n, [&](double v) { rho += v; });
+    row_shares<RECV_RU_SCALAR, double>(L, row, ln.ph, ln.G, [&](double v) { rho += v; });
   }
+  rho = ln.sum(rho) + S.epair[s];
+  if (ln.ph) return;
   rho *= S.rule == GH3 ? 1.0 : QW;
   const double xs = pd ? 1.0 : xo[row];
   const eam::VD F = pd ? eam::F_Pd_vd(rho) : eam::F_H_vd(rho);
@@ -952,32 +952,34 @@ __global__ __launch_bounds__(TBO) __attribute__((amdgpu_waves_per_eu(TBO / 256))
   gmem(S.epair)[s] = o.e;
 }
 
-__global__ __launch_bounds__(TB) void k_grad_recv64(const LatDev* __restrict__ lats, const int32_t* __restrict__ b2l) {
-  __shared__ double red[TB];
-  const int blk = xcd_block();
+__global__ __launch_bounds__(TB) void k_grad_recv64(const LatDev* __restrict__ lats, const int32_t* __restrict__ b2l,
+                                                 int rq) {
+  const int v = xcd_block(), blk = v / rq;
   const LatDev& S = lats[b2l[blk]];
-  const int lb = blk - S.blk0;
-  const int s = lb * TB + threadIdx.x;
-  const int N = S.npd + S.nh;
+  const RecvLane ln(S, blk - S.blk0, v % rq);
+  if (ln.idle) return;
+  const int s = ln.s;
   double fs = 0.0;
-  if (s < N) {
+  if (s < S.npd + S.nh) {
     const double* __restrict__ xo = S.xrow;
     const bool pd = s < S.npd;
     const int row = pd ? s : s - S.npd;
     double* __restrict__ G = S.G;
     const size_t site = pd ? site_of_row(row, S.npd) : S.npd + site_of_row(row, S.nh);
-    const double4 own = S.gown[s];
-    double g0 = own.x, g1 = own.y, g2 = own.z, gs = own.w;
+    double g0 = 0.0, g1 = 0.0, g2 = 0.0, gs = 0.0;
+    if (ln.ph == 0) {
+      const double4 own = S.gown[s];
+      g0 = own.x; g1 = own.y; g2 = own.z; gs = own.w;
+    }
 #pragma unroll
-    for (int side = 0; side < 2; ++side) {
+    for (int side = 0; side < 2; ++side) {  // shares arrive weighted by their senders
       const Ell& L = pd ? (side ? S.pdh : S.pdpd) : (side ? S.hh : S.hpd);
-      const int n = L.rcnt[row];
-      // shares arrive weighted by their senders
-      for_row_shares<RECV_RU_WIDE>(gmem(reinterpret_cast<const double4*>(L.rbuf)), L.rows, row, n, [&](const double4& v) {
+      row_shares<RECV_RU_WIDE, double4>(L, row, ln.ph, ln.G, [&](const double4& v) {
         g0 += v.x; g1 += v.y; g2 += v.z;
         gs += v.w;
       });
     }
+    g0 = ln.sum(g0); g1 = ln.sum(g1); g2 = ln.sum(g2); gs = ln.sum(gs);
     const double xi = pd ? 1.0 : xo[row];
     const double sg = S.qzs[s].y;
     const double T = S.T;
@@ -985,20 +987,15 @@ __global__ __launch_bounds__(TB) void k_grad_recv64(const LatDev* __restrict__ l
     const double qw = gh ? 1.0 : QW, sq = gh ? 1.0 : SQ6;
     const double V = S.emb[s] + qw * xi * S.epair[s];  // owned pairs carry their full energy
     const double sc = qw * xi / T;
-    G[4 * site + 0] = sc * g0;
-    G[4 * site + 1] = sc * g1;
-    G[4 * site + 2] = sc * g2;
-    G[4 * site + 3] = sq * sc * gs - 3.0 * KB * xi / sg;
-    fs = V / T - 3.0 * KB * xi * log(sg);
+    if (ln.ph == 0) {
+      G[4 * site + 0] = sc * g0;
+      G[4 * site + 1] = sc * g1;
+      G[4 * site + 2] = sc * g2;
+      G[4 * site + 3] = sq * sc * gs - 3.0 * KB * xi / sg;
+      fs = V / T - 3.0 * KB * xi * log(sg);
+    }
   }
-  red[threadIdx.x] = fs;
-  __syncthreads();
-#pragma unroll
-  for (int w = TB / 2; w > 0; w >>= 1) {
-    if (threadIdx.x < w) red[threadIdx.x] += red[threadIdx.x + w];
-    __syncthreads();
-  }
-  if (threadIdx.x == 0) S.part[lb] = red[0];
+  finish_objective(S, ln, fs);
 }
 
 // ================================================================ chemical potential
@@ -1162,7 +1159,6 @@ __global__ __launch_bounds__(TB) void k_rows(const LatDev* __restrict__ lats, co
   const int blk = xcd_block();
   const LatDev& S = lats[b2l[blk]];
   const int s = (blk - S.blk0) * TB + threadIdx.x;
-  if (s >= S.npd + S.nh) return;
   copy_row(S, s);
 }
 
@@ -1201,6 +1197,7 @@ template <int R> struct GradAn { static constexpr auto fn = k_grad64<A2C_DERIV_A
 // Owner launches: workgroups of TBO lanes, TBO / 256 units each.
 template <template <int, int> class K, int TBO>
 int owners(const Launch& L) {
+  if (L.onblk == 0) return A2C_OK;
   const dim3 grid((L.onblk + TBO / TB - 1) / (TBO / TB));
   if (L.rules & (1 << A2C_QUAD_R12))
     hipLaunchKernelGGL((K<A2C_QUAD_R12, TBO>::fn), grid, dim3(TBO), 0, L.stream, L.lats, L.ob2l, L.onblk, L.tab64);
@@ -1230,16 +1227,15 @@ int run_eval64(const Launch& L, Timing* tm) {
       if (tm) tm->mark(L.stream, "dens_own64");
       if (L.onblk > DENS_WIDE_UNITS ? owners<DensOwn, 512>(L) : owners<DensOwn, 256>(L)) return A2C_EHIP;
       if (tm) tm->mark(L.stream, "dens_recv64");
-      hipLaunchKernelGGL(k_dens_recv64<A2C_DERIV_ANALYTIC>, dim3(L.nblk), dim3(TB), 0, L.stream, L.lats, L.b2l, 0.0, 0);
+      hipLaunchKernelGGL(k_dens_recv64<A2C_DERIV_ANALYTIC>, dim3(L.nblk * L.rq), dim3(TB), 0, L.stream, L.lats, L.b2l,
+                         L.rq, 0.0, 0);
       if (hipGetLastError() != hipSuccess) return A2C_EHIP;
       if (tm) tm->mark(L.stream, "grad_own64");
       if (L.onblk > GRAD_WIDE_UNITS ? owners<GradOwn, 512>(L) : owners<GradOwn, 256>(L)) return A2C_EHIP;
       if (tm) tm->mark(L.stream, "grad_recv64");
-      hipLaunchKernelGGL(k_grad_recv64, dim3(L.nblk), dim3(TB), 0, L.stream, L.lats, L.b2l);
+      hipLaunchKernelGGL(k_grad_recv64, dim3(L.nblk * L.rq), dim3(TB), 0, L.stream, L.lats, L.b2l, L.rq);
       if (hipGetLastError() != hipSuccess) return A2C_EHIP;
     }
-    if (tm) tm->mark(L.stream, "final_sum");
-    if (int rc = run_final_sum(L)) return rc;
     if (tm) tm->mark(L.stream, nullptr);
     return A2C_OK;
   }
@@ -1404,7 +1400,8 @@ static Launch single_launch(a2c_fe_ctx* c, bool fp64) {
   L.b2l = c->db2l;
   L.ob2l = c->db2l;
   L.onblk = owner_units(c->desc.n_pd, c->desc.n_h, lanes_per_site(c->N, fp64));
-  L.nblk = site_blocks(c->N);
+  L.nblk = lattice_blocks(c->N);
+  L.rq = recv_lanes(c->N);
   L.nlat = 1;
   L.rules = 1 << c->desc.quad_rule;
   L.stream = c->stream;
@@ -1421,11 +1418,10 @@ int launch_density64(a2c_fe_ctx* c, const double* dX, bool by_site) {
   if (c->gen_on) return launch_density_gen(c, dX);
   if (int rc = sync_lattice(c, dX, c->dG, c->dF)) return rc;
   const Launch L = single_launch(c, true);
-  if (L.nblk == 0) return A2C_OK;
   if (run_rows(L) || (L.onblk > DENS_WIDE_UNITS ? owners<DensOwn, 512>(L) : owners<DensOwn, 256>(L)))
     return set_err(c, A2C_EHIP, "density64 launch failed");
   hipLaunchKernelGGL(L.deriv_mode == A2C_DERIV_FD ? k_dens_recv64<A2C_DERIV_FD> : k_dens_recv64<A2C_DERIV_ANALYTIC>,
-                     dim3(L.nblk), dim3(TB), 0, L.stream, L.lats, L.b2l, L.fd_eps, (int)by_site);
+                     dim3(L.nblk * L.rq), dim3(TB), 0, L.stream, L.lats, L.b2l, L.rq, L.fd_eps, (int)by_site);
   A2C_HIP(c, hipGetLastError());
   return A2C_OK;
 }

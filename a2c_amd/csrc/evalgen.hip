@@ -13,8 +13,7 @@
 //   k_gen_grad_own   owned pairs' energy and coefficient c = F'_i f_j' +
 //                    F'_j f_i' + phi' at each node, both ends' q- and
 //                    sigma-gradient
-//   k_gen_grad_recv  gradient, the site's share of f, and a fixed-shape block
-//                    sum (k_final_sum completes f)
+//   k_gen_grad_recv  gradient, the site's share of f, block sums and f
 //   k_gen_chem       per H site over its full lists: dV/dx_a + the correction
 //                    terms, gamma, cap
 //
@@ -259,7 +258,6 @@ __device__ __forceinline__ GenPair gen_pair(const Image& img, const Site& a, con
 __global__ __launch_bounds__(TB) void k_gen_rows(const LatDev* __restrict__ lat) {
   const LatDev& S = *lat;
   const int s = xcd_block() * TB + threadIdx.x;
-  if (s >= S.npd + S.nh) return;
   copy_row(S, s);
 }
 
@@ -327,17 +325,20 @@ template <int POT, int DM>
 __global__ __launch_bounds__(TB) void k_gen_dens_recv(const LatDev* __restrict__ lat, GenDev g, double eps,
                                                       int by_site) {
   const LatDev& S = *lat;
-  const int s = xcd_block() * TB + threadIdx.x;
+  const int v = xcd_block(), rq = S.rl;
+  const RecvLane ln(S, v / rq, v % rq);
+  const int s = ln.s;
   if (s >= S.npd + S.nh) return;
   const bool pd = s < S.npd;
   const int row = pd ? s : s - S.npd;
-  double rho = S.epair[s];
+  double rho = 0.0;
 #pragma unroll
   for (int side = 0; side < 2; ++side) {
     const Ell& L = pd ? (side ? S.pdh : S.pdpd) : (side ? S.hh : S.hpd);
-    for_row_shares<RECV_RU_SCALAR>(gmem(reinterpret_cast<const double*>(L.rbuf)), L.rows, row, L.rcnt[row],
-                                   [&](double v) { rho += v; });
+    row_shares<RECV_RU_SCALAR, double>(L, row, ln.ph, ln.G, [&](double v) { rho += v; });
   }
+  rho = ln.sum(rho) + S.epair[s];
+  if (ln.ph) return;
   const double F = F_val<POT>(g, pd, rho);
   const int o = !by_site ? s : pd ? site_of_row(row, S.npd) : S.npd + site_of_row(row, S.nh);
   S.rho[o] = rho;
@@ -437,44 +438,39 @@ __global__ __launch_bounds__(TB) void k_gen_grad_own(const LatDev* __restrict__ 
 }
 
 __global__ __launch_bounds__(TB) void k_gen_grad_recv(const LatDev* __restrict__ lat) {
-  __shared__ double red[TB];
   const LatDev& S = *lat;
-  const int lb = xcd_block();
-  const int s = lb * TB + threadIdx.x;
+  const int v = xcd_block(), rq = S.rl;
+  const RecvLane ln(S, v / rq, v % rq);
+  const int s = ln.s;
   double fs = 0.0;
   if (s < S.npd + S.nh) {
     const bool pd = s < S.npd;
     const int row = pd ? s : s - S.npd;
     const size_t site = pd ? site_of_row(row, S.npd) : S.npd + site_of_row(row, S.nh);
-    double4 gr = S.gown[s];
+    double4 gr = ln.ph ? make_double4(0.0, 0.0, 0.0, 0.0) : S.gown[s];
 #pragma unroll
     for (int side = 0; side < 2; ++side) {
       const Ell& L = pd ? (side ? S.pdh : S.pdpd) : (side ? S.hh : S.hpd);
-      for_row_shares<RECV_RU_WIDE>(gmem(reinterpret_cast<const double4*>(L.rbuf)), L.rows, row, L.rcnt[row],
-                                   [&](const double4& v) {
-                                     gr.x += v.x; gr.y += v.y; gr.z += v.z;
-                                     gr.w += v.w;
-                                   });
+      row_shares<RECV_RU_WIDE, double4>(L, row, ln.ph, ln.G, [&](const double4& v) {
+        gr.x += v.x; gr.y += v.y; gr.z += v.z;
+        gr.w += v.w;
+      });
     }
-    const double xi = pd ? 1.0 : S.xrow[row];
-    const double sg = S.qzs[s].y;
-    const double T = S.T, sc = xi / T;
-    const double V = S.emb[s] + xi * S.epair[s];  // owned pairs carry their full energy (minimizer.cpp:169-286)
-    double* __restrict__ G = S.G + 4 * site;  // the caller's: 8-byte aligned
-    G[0] = sc * gr.x;
-    G[1] = sc * gr.y;
-    G[2] = sc * gr.z;
-    G[3] = sc * gr.w - 3.0 * KB * xi / sg;
-    fs = V / T - 3.0 * KB * xi * log(sg);
+    gr = make_double4(ln.sum(gr.x), ln.sum(gr.y), ln.sum(gr.z), ln.sum(gr.w));
+    if (ln.ph == 0) {
+      const double xi = pd ? 1.0 : S.xrow[row];
+      const double sg = S.qzs[s].y;
+      const double T = S.T, sc = xi / T;
+      const double V = S.emb[s] + xi * S.epair[s];  // owned pairs carry their full energy (minimizer.cpp:169-286)
+      double* __restrict__ G = S.G + 4 * site;  // the caller's: 8-byte aligned
+      G[0] = sc * gr.x;
+      G[1] = sc * gr.y;
+      G[2] = sc * gr.z;
+      G[3] = sc * gr.w - 3.0 * KB * xi / sg;
+      fs = V / T - 3.0 * KB * xi * log(sg);
+    }
   }
-  red[threadIdx.x] = fs;
-  __syncthreads();
-#pragma unroll
-  for (int w = TB / 2; w > 0; w >>= 1) {
-    if (threadIdx.x < w) red[threadIdx.x] += red[threadIdx.x + w];
-    __syncthreads();
-  }
-  if (threadIdx.x == 0) S.part[lb] = red[0];
+  finish_objective(S, ln, fs);
 }
 
 // ------------------------------------------------------------ chemical potential
@@ -570,7 +566,7 @@ int run_density_gen(const LatDev* dlat, int npd, int nh, const GenDev& g, int de
   hipLaunchKernelGGL(pick<DensK>(g, deriv_mode, fp32), dim3(owner_units(npd, nh, KL)), dim3(TB),
                      lds_bytes(g, deriv_mode, fp32), st, dlat, g, KL);
   if (tm) tm->mark(st, "gen_dens_recv");
-  hipLaunchKernelGGL(pick<RecvK>(g, deriv_mode, fp32), dim3(nblk), dim3(TB), 0, st, dlat, g, eps, (int)by_site);
+  hipLaunchKernelGGL(pick<RecvK>(g, deriv_mode, fp32), dim3(nblk * recv_lanes(npd + nh)), dim3(TB), 0, st, dlat, g, eps, (int)by_site);
   return hipGetLastError() == hipSuccess ? A2C_OK : A2C_EHIP;
 }
 
@@ -585,8 +581,10 @@ int run_eval_gen(const LatDev* dlat, int npd, int nh, const GenDev& g, int deriv
     hipLaunchKernelGGL(pick<GradK>(g, deriv_mode, fp32), dim3(owner_units(npd, nh, KL)), dim3(TB),
                        lds_bytes(g, deriv_mode, fp32), st, dlat, g, eps, KL);
     if (tm) tm->mark(st, "gen_grad_recv");
-    hipLaunchKernelGGL(k_gen_grad_recv, dim3(nblk), dim3(TB), 0, st, dlat);
+    hipLaunchKernelGGL(k_gen_grad_recv, dim3(nblk * recv_lanes(npd + nh)), dim3(TB), 0, st, dlat);
     if (hipGetLastError() != hipSuccess) return A2C_EHIP;
+    if (tm) tm->mark(st, nullptr);
+    return A2C_OK;
   }
   if (tm) tm->mark(st, "final_sum");
   Launch L{};

@@ -106,7 +106,9 @@ struct LatDev {
   float2* aux = nullptr;      // N {F'(rho), x} (mixed path)
   double* emb = nullptr;      // N embedding energy (x-weighted for H)
   double* epair = nullptr;    // N pair-energy partial (mixed path)
-  double* part = nullptr;     // ceil(N/256) block partial sums of f
+  double* part = nullptr;     // block partial sums of f: one per 256 sites, or per 64 (recv_lanes)
+  int32_t* done = nullptr;    // blocks of the gradient receive pass that have put theirs (k_rows clears it)
+  int32_t rl = 1;             // lanes per row in the receive passes (recv_lanes)
   double* f = nullptr;        // objective
   // pair-once evaluation, per species in row order (Pd rows, then H rows; rho,
   // Fp, aux, emb and epair are in this order too while it runs):
@@ -118,6 +120,18 @@ struct LatDev {
 using DevSys = LatDev;
 constexpr int SITE_BLOCK = 256;  // sites per block of every site-parallel kernel
 __host__ __device__ inline int site_blocks(int n) { return (n + SITE_BLOCK - 1) / SITE_BLOCK; }
+// Blocks of a lattice in a launch that must write its results even if it has no
+// sites (zeros then).
+__host__ __device__ inline int lattice_blocks(int n) { return n > 0 ? site_blocks(n) : 1; }
+
+// Lanes per row of the receive passes.  Up to RECV_SPLIT_SITES a pass is bound by
+// the memory latency of one row's ~20 shares per list, and RECV_LANES lanes
+// take them in turn; beyond, it streams, and one lane per row reads whole
+// lines.  Mixed gradient pass, 1 / 4 lanes: 1,728 sites 16.5 / 9.9 us, 21,952
+// sites 17.0 / 13.7, 46,656 sites 17.8 / 20.3, 512,000 sites 90 / 131; FP64 16.0 /
+// 11.3, 17.3 / 15.3, 18.4 / 23.1, 174 / 186.
+constexpr int RECV_LANES = 4, RECV_SPLIT_SITES = 32768;
+__host__ __device__ inline int recv_lanes(int n) { return n <= RECV_SPLIT_SITES ? RECV_LANES : 1; }
 
 // Global-memory views.  Pointers read from a descriptor in memory are
 // generic to the compiler, which then issues flat_* instructions: those count
@@ -134,32 +148,62 @@ __device__ __forceinline__ A2C_GLOBAL T* gmem(T* p) {
   return (A2C_GLOBAL T*)p;
 }
 
-// The n received shares of one row of a slot-major buffer (share t at
-// base[t * rows + row]) passed to add in slot order.  The loads of RU
-// consecutive shares are issued before any of them is added, so a row costs
-// one memory latency per RU shares rather than one per share; the order of
-// the additions, and so the result, is that of a plain loop.
+// The shares ph, ph + G, ... of the n received by one row of a slot-major
+// buffer (share t at base[t * rows + row]) passed to add in slot order.  The
+// loads of RU of them are issued before any is added, so a row costs one
+// memory latency per RU shares rather than one per share; the order of the
+// additions, and so the result, is that of a plain loop.
 template <int RU, class T, class Add>
 __device__ __forceinline__ void for_row_shares(const A2C_GLOBAL T* __restrict__ base, size_t rows, int row, int n,
-                                               Add add) {
-  for (int t = 0; t < n; t += RU) {
+                                               int ph, int G, Add add) {
+  for (int t = ph; t < n; t += RU * G) {
     T v[RU];
 #pragma unroll
     for (int u = 0; u < RU; ++u)
-      if (t + u < n) v[u] = base[(size_t)(t + u) * rows + row];
+      if (t + u * G < n) v[u] = base[(size_t)(t + u * G) * rows + row];
 #pragma unroll
     for (int u = 0; u < RU; ++u)
-      if (t + u < n) add(v[u]);
+      if (t + u * G < n) add(v[u]);
   }
 }
-// Loads in flight per lane: 8 for the density pass's scalar shares (faster
-// at every size measured), 2 for the gradient pass's shares of 16 or 32
-// bytes.  Measured on
-// the mixed gradient receive pass, RU = 1/2/4/8: a 6^3-cell lattice (latency-
-// bound) 19.6/15.0/12.2/10.9 us, a 40^3-cell one (streaming at HBM speed,
-// where more rows in flight and the registers they hold cost waves)
-// 74.6/76.3/83.0/87.9 us.
-constexpr int RECV_RU_SCALAR = 8, RECV_RU_WIDE = 2;
+// Loads in flight per lane with one lane per row: 8 for the density pass's
+// scalar shares (faster at every size measured), 2 for the gradient pass's
+// shares of 16 or 32 bytes (a 40^3-cell lattice, streaming at HBM speed: RU =
+// 1/2/4/8 took 74.6/76.3/83.0/87.9 us, where the registers they hold cost
+// waves).  With RECV_LANES lanes per row 6, a lane's part of ~20, or 3 of 32 bytes.
+constexpr int RECV_RU_SCALAR = 8, RECV_RU_WIDE = 2, RECV_RU_SPLIT = 6;
+template <int RU, class T, class Add>
+__device__ __forceinline__ void row_shares(const Ell& L, int row, int ph, int G, Add add) {
+  const A2C_GLOBAL T* base = gmem(reinterpret_cast<const T*>(L.rbuf));
+  const int n = L.rcnt[row];
+  if (G == 1) for_row_shares<RU>(base, L.rows, row, n, 0, 1, add);
+  else for_row_shares<(sizeof(T) > 16 ? RECV_RU_SPLIT / 2 : RECV_RU_SPLIT)>(base, L.rows, row, n, ph, G, add);
+}
+
+// Place of a lane in a receive pass: rq blocks of 256 lanes per 256 rows, of
+// which a lattice with one lane per row uses the first.
+struct RecvLane {
+  int lb, q, G;  // block of 256 rows within the lattice, quarter of it, lanes per row
+  int s, ph;     // row (row order) and phase
+  bool idle;     // a block without work
+  __device__ __forceinline__ RecvLane(const LatDev& S, int lblk, int quarter)
+      : lb(lblk), q(quarter), G(S.rl), ph(0), idle(false) {
+    const int t = threadIdx.x;
+    if (G == 1) {
+      idle = q != 0;
+      s = lb * SITE_BLOCK + t;
+    } else {
+      s = lb * SITE_BLOCK + q * (SITE_BLOCK / RECV_LANES) + t / RECV_LANES;
+      ph = t % RECV_LANES;
+    }
+  }
+  __device__ __forceinline__ double sum(double v) const { return G == 1 ? v : site_sum_row(v); }
+  static __device__ __forceinline__ double site_sum_row(double v) {
+#pragma unroll
+    for (int off = RECV_LANES / 2; off > 0; off >>= 1) v += __shfl_down(v, off, RECV_LANES);
+    return v;
+  }
+};
 
 // Lanes per site of the pair-owner passes.  A small lattice gives too few
 // waves to fill the GPU with one lane per site, and each lane would walk its
@@ -356,6 +400,20 @@ __device__ __forceinline__ void sum_parts(const double* part, size_t stride, int
     if (lane == 0 && w + W * i < K) out(w + W * i, v[i]);
 }
 
+// End of a gradient receive pass: the block's sum of fs, and of all blocks' sums
+// by the last one, into the objective.  Every lane of a working block calls it.
+__device__ __forceinline__ void finish_objective(const LatDev& S, const RecvLane& ln, double fs) {
+  __shared__ double red[SITE_BLOCK / 64];
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1) fs += __shfl_down(fs, off);
+  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = fs;
+  __syncthreads();
+  const int n = (ln.G == 1 ? 1 : RECV_LANES) * lattice_blocks(S.npd + S.nh);
+  if (threadIdx.x == 0) put_part(S.part + (ln.G == 1 ? ln.lb : RECV_LANES * ln.lb + ln.q), (red[0] + red[1]) + (red[2] + red[3]));
+  if (!last_block(S.done, n)) return;
+  sum_parts<1>(S.part, 0, n, [&](int, double v) { *S.f = v; });
+}
+
 struct Timing;
 
 // a2c_fe_create on a stream of the caller's (a batch's own lattices share
@@ -459,6 +517,8 @@ struct a2c_fe_ctx {
     s.rule = desc.quad_rule;
     s.pdpd = ell[0]; s.pdh = ell[1]; s.hpd = ell[2]; s.hh = ell[3]; s.hh1 = ell[4];
     s.x = dx; s.rho = drho; s.Fp = dFp; s.aux = daux; s.emb = demb; s.part = dpart; s.epair = depair;
+    s.done = reinterpret_cast<int32_t*>(dpart + (size_t)a2c::RECV_LANES * nblk_red);
+    s.rl = a2c::recv_lanes(N);
     s.qxy = dqxy; s.qzs = dqzs; s.xrow = dxrow; s.gown = dgown;
     return s;
   }
@@ -485,6 +545,7 @@ struct Launch {
   const LatDev* lats;
   const int32_t* b2l;
   int nblk, nlat;
+  int rq = 1;  // blocks per site block in the receive passes: RECV_LANES if some lattice takes that many
   hipStream_t stream;
   int deriv_mode;
   double fd_eps;

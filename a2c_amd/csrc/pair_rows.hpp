@@ -23,8 +23,11 @@ __device__ __forceinline__ Site load_row(const A2C_GLOBAL double2* __restrict__ 
   return {{a.x, a.y, b.x}, b.y};
 }
 
-// the state and occupancy of site s to their place in row order
+// the state and occupancy of site s to their place in row order; site 0's lane
+// also clears the count of finished blocks
 __device__ __forceinline__ void copy_row(const LatDev& S, int s) {
+  if (s == 0) *S.done = 0;
+  if (s >= S.npd + S.nh) return;
   const double4 v = reinterpret_cast<const double4*>(S.X)[s];
   const bool pd = s < S.npd;
   const int row = pd ? row_of_site(s, S.npd) : row_of_site(s - S.npd, S.nh);
