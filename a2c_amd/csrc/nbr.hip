@@ -427,32 +427,43 @@ __global__ __launch_bounds__(ST) void k_site(NbrArgs a, int nblk_pd) {
   }
 }
 
-// For every owned entry, one thread each (slot blockIdx.y of list blockIdx.z):
+// For every owned entry (list blockIdx.z; a row's entries dealt to ORV_Y threads):
 // the received slot of its row in the partner row, found by binary search of
 // the partner's received half (sorted site indices, in rbuf until the first
 // evaluation; if absent, which the symmetric lists never produce, a slot past
 // the received half that nothing reads: the owner passes store every share
-// without a test).
+// without a test).  Neighboring rows' entries of one slot probe neighboring rows.
+constexpr int ORV_Y = 16;
 struct OrvArgs {
   Ell L[4];
+  int spare[4];   // that slot, per partner list
+  int32_t* maxw;  // after a refresh: the longest total row (Pd rows: PdPd + PdH, H rows: HPd + HH) goes to maxw[13]
 };
 __global__ void k_orv(OrvArgs a) {
   const int w = blockIdx.z;
   const Ell& L = a.L[w];
-  const int p = blockIdx.x * blockDim.x + threadIdx.x, t = blockIdx.y;
-  if (p >= L.rows || t >= L.owidth || t >= L.ocnt[p]) return;
-  const Ell& P = a.L[w == 1 ? 2 : w == 2 ? 1 : w];  // PdPd, PdH <-> HPd, HH
-  const int r = site_of_row(p, L.rows);
-  const size_t e = (size_t)t * L.rows + p;
-  const int j = L.oj[e];
-  const A2C_GLOBAL int32_t* rj = gmem(reinterpret_cast<const int32_t*>(P.rbuf)) + j;
-  int lo = 0, hi = P.rcnt[j];  // the slot is in [lo, hi) if the row holds r
-  while (hi - lo > 1) {
-    const int mid = (lo + hi) >> 1;
-    if (rj[(size_t)mid * P.rows] <= r) lo = mid;
-    else hi = mid;
+  const int p = blockIdx.x * blockDim.x + threadIdx.x;
+  if (a.maxw && blockIdx.y == 0 && w % 2 == 0) {
+    int m = p < L.rows ? L.cnt[p] + a.L[w + 1].cnt[p] : 0;
+    for (int off = 32; off > 0; off >>= 1) m = max(m, __shfl_xor(m, off));
+    if ((threadIdx.x & 63) == 0 && m) atomicMax(&maxw_copy(a.maxw)[13], m);
   }
-  L.orv[e] = lo < hi && rj[(size_t)lo * P.rows] == r ? lo : P.rwidth;
+  if (p >= L.rows) return;
+  const int pw = w == 1 ? 2 : w == 2 ? 1 : w;  // PdPd, PdH <-> HPd, HH
+  const Ell& P = a.L[pw];
+  const int r = site_of_row(p, L.rows), n = L.ocnt[p];
+  for (int t = blockIdx.y; t < n; t += ORV_Y) {
+    const size_t e = (size_t)t * L.rows + p;
+    const int j = L.oj[e];
+    const A2C_GLOBAL int32_t* rj = gmem(reinterpret_cast<const int32_t*>(P.rbuf)) + j;
+    int lo = 0, hi = P.rcnt[j];  // the slot is in [lo, hi) if the row holds r
+    while (hi - lo > 1) {
+      const int mid = (lo + hi) >> 1;
+      if (rj[(size_t)mid * P.rows] <= r) lo = mid;
+      else hi = mid;
+    }
+    L.orv[e] = lo < hi && rj[(size_t)lo * P.rows] == r ? lo : a.spare[pw];
+  }
 }
 
 // Bounding box of the positions (non-periodic axes): per block, then one
@@ -529,13 +540,18 @@ struct RefreshArgs {
   Grid g;
   double ibox[3];
   double rc2, sh1, sh2;
-  Ell sup[4];          // skin lists: PdPd, PdH (Pd rows), HPd, HH (H rows); rbuf: per entry its fate (below)
-  Ell out[5];          // lists at rc (idx, cnt; pair lists also ocnt, rcnt, oj)
+  Ell sup[4];          // skin lists: PdPd, PdH (Pd rows), HPd, HH (H rows)
+  Ell out[5];          // lists at rc (idx, cnt; pair lists also ocnt, rcnt, oj, and the received half in rbuf)
   int32_t* pdpdnum;
   int32_t* maxw;       // 14 ints as in the count pass
   unsigned long long* totals;
   const unsigned long long* dmax;  // squared largest displacement (a double's bits), 0 after a skin build
 };
+
+__device__ __forceinline__ int wave_max(int v) {
+  for (int off = 32; off > 0; off >>= 1) v = max(v, __shfl_xor(v, off));
+  return v;
+}
 
 // One lane per row of one list (one wave per workgroup; the workgroups of
 // PdPd, PdH, HPd and HH rows in that order): the row's skin-list entries
@@ -547,12 +563,13 @@ struct RefreshArgs {
 // shell radii, delta the largest displacement since then, is decided by that
 // distance alone: no site pair moved closer or apart by more than 2 delta,
 // and the float carries 3e-7 A of rounding.  The others are tested with the
-// current FP64 positions exactly as the cell walk tests them.  The fate of
-// every skin entry goes to the skin list's rbuf: -2 dropped, -3 - k kept as
-// the row's k-th owned entry, else its slot in the received half.  Kept
+// current FP64 positions exactly as the cell walk tests them.  Kept
 // entries are staged in the lane's LDS column (neighbor << 2 | owned << 1 |
 // first shell), then each output array is written slot by slot, 64
 // consecutive rows per store.
+// 262,144 sites, rebuilt in place: 176 us with one entry's positions at a time, 124
+// with a batch's (the lists' own bytes take 70); the reverse slots 73 us from the
+// received halves, where per-entry fates and twins took 157 us in four launches.
 __global__ __launch_bounds__(NT) void k_refresh(RefreshArgs a, int4 blk0) {
   extern __shared__ uint32_t col[];
   const int b = blockIdx.x;
@@ -576,64 +593,82 @@ __global__ __launch_bounds__(NT) void k_refresh(RefreshArgs a, int4 blk0) {
   const Ell L = a.out[w];
   const A2C_GLOBAL int32_t* __restrict__ sidx = gmem(S.idx);
   const A2C_GLOBAL float* __restrict__ sdist = gmem(reinterpret_cast<const float*>(S.oj));
-  A2C_GLOBAL int32_t* __restrict__ fate = gmem(reinterpret_cast<int32_t*>(S.rbuf));
   const size_t srows = S.rows, orows = L.rows;
   const int n = live ? gmem(S.cnt)[row] : 0;
   int nk = 0, no = 0, nr = 0, nf = 0, sh0 = 0, sh1n = 0;
-  constexpr int B = 8;  // entries whose index and distance are loaded before any is tested
-  int jb[B];
-  float db[B];
-  for (int t = 0; t < n; ++t) {
-    const size_t se = (size_t)t * srows + row;
-    if (t % B == 0) {
+  // Entries in batches of B: the next batch's indices and distances are
+  // requested before this one is decided, and where some lane needs positions, all
+  // of the batch's are requested together.
+  constexpr int B = 8;
+  const int nw = wave_max(n);
+  int jb[B], jn[B];
+  float db[B], dn[B];
+  auto load = [&](int t0, int (&jv)[B], float (&dv)[B]) {
+#pragma unroll
+    for (int u = 0; u < B; ++u) {  // past the row's end its last entry again
+      const size_t se = (size_t)max(min(t0 + u, n - 1), 0) * srows + (live ? row : 0);
+      jv[u] = sidx[se];
+      dv[u] = sdist[se];
+    }
+  };
+  if (nw > 0) load(0, jn, dn);
+  for (int t0 = 0; t0 < nw; t0 += B) {
+#pragma unroll
+    for (int u = 0; u < B; ++u) {
+      jb[u] = jn[u];
+      db[u] = dn[u];
+    }
+    load(t0 + B, jn, dn);
+    bool near[B], keep[B], some = false;
+    int cls[B];  // shell class: 0 below r1, 1 between, 2 beyond
+#pragma unroll
+    for (int u = 0; u < B; ++u) {
+      const double df = (double)db[u];
+      const bool near_rc = fabs(df - rc) <= band;
+      const bool near_sh = (shells || first) && (fabs(df - r1) <= band || (shells && fabs(df - r2) <= band));
+      near[u] = t0 + u < n && (near_rc || near_sh);
+      some |= near[u];
+      keep[u] = t0 + u < n && df < rc;
+      cls[u] = df < r1 ? 0 : (df < r2 ? 1 : 2);
+    }
+    if (__ballot(some)) {
+      double4 q[B];
+#pragma unroll
+      for (int u = 0; u < B; ++u) q[u] = X[near[u] ? joff + jb[u] : s];
 #pragma unroll
       for (int u = 0; u < B; ++u) {
-        const bool in = t + u < n;
-        jb[u] = in ? sidx[se + (size_t)u * srows] : 0;
-        db[u] = in ? sdist[se + (size_t)u * srows] : 0.0f;
+        double d0 = q[u].x - qi.x, d1 = q[u].y - qi.y, dz = q[u].z - qi.z;
+        if (a.g.periodic[0]) d0 = wrap(d0, a.g.box[0], a.ibox[0]);
+        if (a.g.periodic[1]) d1 = wrap(d1, a.g.box[1], a.ibox[1]);
+        if (a.g.periodic[2]) dz = wrap(dz, a.g.box[2], a.ibox[2]);
+        const double d2 = d0 * d0 + d1 * d1 + dz * dz;
+        if (near[u]) {
+          keep[u] = d2 <= a.rc2;
+          cls[u] = d2 < a.sh1 ? 0 : ((d2 > a.sh1 && d2 < a.sh2) ? 1 : 2);
+        }
       }
     }
-    const int jl = jb[t % B];
-    const int j = joff + jl;
-    const double df = (double)db[t % B];
-    const bool near_rc = fabs(df - rc) <= band;
-    const bool near_sh = (shells || first) && (fabs(df - r1) <= band || (shells && fabs(df - r2) <= band));
-    bool keep;
-    int cls;  // shell class: 0 below r1, 1 between, 2 beyond
-    if (near_rc || near_sh) {
-      const double4 qj = X[j];
-      double d0 = qj.x - qi.x, d1 = qj.y - qi.y, dz = qj.z - qi.z;
-      if (a.g.periodic[0]) d0 = wrap(d0, a.g.box[0], a.ibox[0]);
-      if (a.g.periodic[1]) d1 = wrap(d1, a.g.box[1], a.ibox[1]);
-      if (a.g.periodic[2]) dz = wrap(dz, a.g.box[2], a.ibox[2]);
-      const double d2 = d0 * d0 + d1 * d1 + dz * dz;
-      keep = d2 <= a.rc2;
-      cls = d2 < a.sh1 ? 0 : ((d2 > a.sh1 && d2 < a.sh2) ? 1 : 2);
-    } else {
-      keep = df < rc;
-      cls = df < r1 ? 0 : (df < r2 ? 1 : 2);
+#pragma unroll
+    for (int u = 0; u < B; ++u) {
+      if (!keep[u]) continue;
+      const bool owned = pair_owner(s, joff + jb[u]);
+      owned ? ++no : ++nr;
+      if (shells) {
+        if (cls[u] == 0) ++sh0;
+        else if (cls[u] == 1) ++sh1n;
+      }
+      const bool f1 = first && cls[u] == 0;
+      nf += f1;
+      col[nk * CS + lane] = ((uint32_t)jb[u] << 2) | (owned ? 2u : 0u) | (f1 ? 1u : 0u);
+      ++nk;
     }
-    if (!keep) {
-      fate[se] = -2;
-      continue;
-    }
-    const bool owned = pair_owner(s, j);
-    fate[se] = owned ? -3 - no : nr;
-    owned ? ++no : ++nr;
-    if (shells) {
-      if (cls == 0) ++sh0;
-      else if (cls == 1) ++sh1n;
-    }
-    const bool f1 = first && cls == 0;
-    nf += f1;
-    col[nk * CS + lane] = ((uint32_t)jl << 2) | (owned ? 2u : 0u) | (f1 ? 1u : 0u);
-    ++nk;
   }
-  // the wave's longest row, owned half and HH1 row: slot loops every lane joins
-  int mk = nk, mo = no, mf = nf;
+  // the wave's longest row, halves and HH1 row: slot loops every lane joins
+  int mk = nk, mo = no, mr = nr, mf = nf;
   for (int off = 32; off > 0; off >>= 1) {
     mk = max(mk, __shfl_xor(mk, off));
     mo = max(mo, __shfl_xor(mo, off));
+    mr = max(mr, __shfl_xor(mr, off));
     mf = max(mf, __shfl_xor(mf, off));
   }
   A2C_GLOBAL int32_t* __restrict__ oidx = gmem(L.idx);
@@ -644,6 +679,13 @@ __global__ __launch_bounds__(NT) void k_refresh(RefreshArgs a, int4 blk0) {
     if (u >= no) continue;
     while (!(col[q * CS + lane] & 2u)) ++q;
     ooj[(size_t)u * orows + prow] = row_of_site((int)(col[q * CS + lane] >> 2), jrows);
+    ++q;
+  }
+  A2C_GLOBAL int32_t* __restrict__ orj = gmem(reinterpret_cast<int32_t*>(L.rbuf));
+  for (int u = 0, q = 0; u < mr; ++u) {
+    if (u >= nr) continue;
+    while (col[q * CS + lane] & 2u) ++q;
+    orj[(size_t)u * orows + prow] = (int)(col[q * CS + lane] >> 2);
     ++q;
   }
   if (first) {
@@ -693,15 +735,6 @@ __global__ __launch_bounds__(NT) void k_refresh(RefreshArgs a, int4 blk0) {
   }
 }
 
-// The longest total row (Pd rows: PdPd + PdH, H rows: HPd + HH) after a
-// refresh, into maxw[13].
-__global__ void k_rowmax(const int32_t* __restrict__ c0, const int32_t* __restrict__ c1, int n, int32_t* maxw) {
-  const int r = blockIdx.x * blockDim.x + threadIdx.x;
-  int m = r < n ? c0[r] + c1[r] : 0;
-  for (int off = 32; off > 0; off >>= 1) m = max(m, __shfl_xor(m, off));
-  if ((threadIdx.x & 63) == 0 && m) atomicMax(&maxw_copy(maxw)[13], m);
-}
-
 // Skin build: the FP64 distance of every skin entry (as the cell walk
 // computes it), rounded to a float, into the skin list's oj.
 __global__ void k_sdist(Ell L, const double* __restrict__ X, int s_off, int j_off, Grid g, double ix, double iy,
@@ -717,45 +750,6 @@ __global__ void k_sdist(Ell L, const double* __restrict__ X, int s_off, int j_of
   if (g.periodic[1]) d1 = wrap(d1, g.box[1], iy);
   if (g.periodic[2]) dz = wrap(dz, g.box[2], iz);
   reinterpret_cast<float*>(L.oj)[e] = (float)sqrt(d0 * d0 + d1 * d1 + dz * dz);
-}
-
-// Skin build: for every skin entry (row r, slot t = blockIdx.y, neighbor j)
-// the slot of r in j's row of the partner skin list (binary search of the
-// sorted row; -1 if absent, which the symmetric lists never produce), into
-// the skin list's orv.
-__global__ void k_srev(Ell L, Ell P) {
-  const int r = blockIdx.x * blockDim.x + threadIdx.x;
-  const int t = blockIdx.y;
-  if (r >= L.rows || t >= L.cnt[r]) return;
-  const size_t e = (size_t)t * L.rows + r;
-  const int j = L.idx[e];
-  int lo = 0, hi = P.cnt[j] - 1, k = -1;
-  while (lo <= hi) {
-    const int mid = (lo + hi) >> 1;
-    const int v = P.idx[(size_t)mid * P.rows + j];
-    if (v == r) { k = mid; break; }
-    if (v < r) lo = mid + 1;
-    else hi = mid - 1;
-  }
-  L.orv[e] = k;
-}
-
-// Reverse slots after a refresh, one thread per skin entry (slot t =
-// blockIdx.y): a kept, owned entry (fate -3 - k) takes the fate of its twin
-// in the partner's skin row -- the slot of this pair in the partner's
-// received half -- as the reverse slot of the row's k-th owned entry (spare:
-// the slot past every received half, as in k_orv).
-__global__ void k_orv_skin(Ell S, Ell SP, Ell L, int spare) {
-  const int r = blockIdx.x * blockDim.x + threadIdx.x;
-  const int t = blockIdx.y;
-  if (r >= S.rows || t >= gmem(S.cnt)[r]) return;
-  const size_t e = (size_t)t * S.rows + r;
-  const int f = gmem(reinterpret_cast<const int32_t*>(S.rbuf))[e];
-  if (f > -3) return;
-  const int j = gmem(S.idx)[e];
-  const int u = gmem(S.orv)[e];
-  gmem(L.orv)[(size_t)(-3 - f) * L.rows + row_of_site(r, L.rows)] =
-      u >= 0 ? gmem(reinterpret_cast<const int32_t*>(SP.rbuf))[(size_t)u * SP.rows + j] : spare;
 }
 
 }  // namespace
@@ -822,17 +816,19 @@ int size_lists(a2c_fe_ctx* c, Ell* L5, const int* w, const int* ow, const int* r
   return A2C_OK;
 }
 
-// Reverse slots of the four pair lists (after the fill pass).
-int reverse_slots(a2c_fe_ctx* c, Ell* L5) {
+// Reverse slots of the four pair lists (after the fill pass or a refresh);
+// spare[w]: an allocated slot past list w's received halves.
+int reverse_slots(a2c_fe_ctx* c, const Ell* L5, const int* spare, int32_t* maxw) {
   OrvArgs a;
-  int rows = 0, width = 0;
+  a.maxw = maxw;
+  int rows = 0;
   for (int w = 0; w < 4; ++w) {
     a.L[w] = L5[w];
+    a.spare[w] = spare[w];
     rows = std::max(rows, L5[w].rows);
-    width = std::max(width, L5[w].owidth);
   }
-  if (rows == 0 || width == 0) return A2C_OK;
-  hipLaunchKernelGGL(k_orv, dim3((rows + 255) / 256, width, 4), dim3(256), 0, c->stream, a);
+  if (rows == 0) return A2C_OK;
+  hipLaunchKernelGGL(k_orv, dim3((rows + 255) / 256, ORV_Y, 4), dim3(256), 0, c->stream, a);
   A2C_HIP(c, hipGetLastError());
   return A2C_OK;
 }
@@ -973,7 +969,7 @@ int walk_cells(a2c_fe_ctx* c, double rc, Ell* L5, bool halves, int hm[16], unsig
     A2C_HIP(c, hipGetLastError());
   }
   if (halves)
-    if (int rc2 = reverse_slots(c, L5)) return rc2;
+    if (int rc2 = reverse_slots(c, L5, hm + 9, nullptr)) return rc2;
   {
     std::vector<unsigned long long> tb(SPREAD * 5);
     A2C_HIP(c, hipMemcpyAsync(tb.data(), totals, sizeof(unsigned long long) * tb.size(), hipMemcpyDeviceToHost,
@@ -987,26 +983,16 @@ int walk_cells(a2c_fe_ctx* c, double rc, Ell* L5, bool halves, int hm[16], unsig
   return A2C_OK;
 }
 
-// Per-entry arrays of the skin lists, filled at the skin build: the
-// distance at the build as a float (oj), the partner slot (orv); and room
-// for the fate of every entry in a refresh (rbuf, one int32 each).
+// Distance of every skin entry at the skin build, as a float, in oj.
 int size_skin_extras(a2c_fe_ctx* c) {
   for (int k = 0; k < 4; ++k) {
     Ell& S = c->nb_sup[k];
     const int64_t n = (int64_t)std::max(S.width, 1) * std::max(S.rows, 1);
     if (n > S.ocap) {
-      (void)dfree(S.orv);
       (void)dfree(S.oj);
-      S.orv = S.oj = nullptr;
+      S.oj = nullptr;
       S.ocap = n + 4 * (int64_t)std::max(S.rows, 1);
-      A2C_HIP(c, dmalloc(&S.orv, sizeof(int32_t) * S.ocap));
       A2C_HIP(c, dmalloc(&S.oj, sizeof(float) * S.ocap));
-    }
-    if ((int64_t)sizeof(int32_t) * n > S.bcap) {
-      (void)dfree(S.rbuf);
-      S.rbuf = nullptr;
-      S.bcap = (int64_t)sizeof(int32_t) * (n + 4 * (int64_t)std::max(S.rows, 1));
-      A2C_HIP(c, dmalloc(&S.rbuf, S.bcap));
     }
   }
   const Grid g = box_grid(c);
@@ -1018,14 +1004,6 @@ int size_skin_extras(a2c_fe_ctx* c) {
     if (S.rows == 0 || S.width == 0) continue;
     hipLaunchKernelGGL(k_sdist, dim3((S.rows + 255) / 256, S.width), dim3(256), 0, c->stream, S, c->dX,
                        s_sp[k] * c->desc.n_pd, j_sp[k] * c->desc.n_pd, g, ib[0], ib[1], ib[2]);
-    A2C_HIP(c, hipGetLastError());
-  }
-  static const int partner[4] = {0, 2, 1, 3};
-  for (int k = 0; k < 4; ++k) {
-    const Ell& S = c->nb_sup[k];
-    if (S.rows == 0) continue;
-    if (S.width == 0) continue;
-    hipLaunchKernelGGL(k_srev, dim3((S.rows + 255) / 256, S.width), dim3(256), 0, c->stream, S, c->nb_sup[partner[k]]);
     A2C_HIP(c, hipGetLastError());
   }
   return A2C_OK;
@@ -1075,25 +1053,7 @@ int refresh(a2c_fe_ctx* c, bool check, int hm[16], unsigned long long ht[5], dou
     hipLaunchKernelGGL(k_refresh, dim3(2 * (bp + bh)), dim3(NT), sizeof(uint32_t) * CS * wmax, c->stream, a, blk0);
     A2C_HIP(c, hipGetLastError());
   }
-  if (npd > 0) {
-    hipLaunchKernelGGL(k_rowmax, dim3((npd + 255) / 256), dim3(256), 0, c->stream, c->ell[0].cnt, c->ell[1].cnt, npd,
-                       misc);
-    A2C_HIP(c, hipGetLastError());
-  }
-  if (nh > 0) {
-    hipLaunchKernelGGL(k_rowmax, dim3((nh + 255) / 256), dim3(256), 0, c->stream, c->ell[2].cnt, c->ell[3].cnt, nh,
-                       misc);
-    A2C_HIP(c, hipGetLastError());
-  }
-  static const int partner[4] = {0, 2, 1, 3};
-  for (int k = 0; k < 4; ++k) {
-    const Ell& S = c->nb_sup[k];
-    if (S.rows == 0) continue;
-    if (S.width == 0) continue;
-    hipLaunchKernelGGL(k_orv_skin, dim3((S.rows + 255) / 256, S.width), dim3(256), 0, c->stream, S,
-                       c->nb_sup[partner[k]], c->ell[k], c->nb_sup[partner[k]].width);
-    A2C_HIP(c, hipGetLastError());
-  }
+  if (int rc = reverse_slots(c, c->ell, rw, misc)) return rc;  // rw + 1 slots are allocated
   std::vector<unsigned char> hb(MISC_BBOX);
   A2C_HIP(c, hipMemcpyAsync(hb.data(), misc, MISC_BBOX, hipMemcpyDeviceToHost, c->stream));
   A2C_HIP(c, hipStreamSynchronize(c->stream));
