@@ -50,6 +50,7 @@
 #include "linesearch.hpp"
 
 namespace a2c {
+int batch_create(const a2c_batch_desc* desc, hipStream_t shared, a2c_batch** out);
 namespace {
 
 constexpr int TB = SITE_BLOCK;
@@ -889,6 +890,8 @@ struct GraphCache {
 struct a2c_batch {
   a2c_batch_desc desc{};
   hipStream_t stream = nullptr;
+  bool own_stream = true;
+  a2c::HostTransfer xfer;
   std::string err;
   std::vector<a2c::Slot> slots;
   a2c::Arena arena;
@@ -896,10 +899,9 @@ struct a2c_batch {
   int qrc = 0;  // first error of a queued operation
   bool vector_free = true;     // slots of at most VF_PAIRS pairs take the vector-free form of the recursion
   bool fused_two_loop = true;  // of the others, small ones run it in one workgroup
-  double* dF = nullptr;    // objective per slot (device)
-  double* hF = nullptr;    // pinned mirror
-  double* dres = nullptr;  // 2 doubles per slot (device dot results read by the host)
-  double* hres = nullptr;  // pinned mirror
+  // results the host reads after a synchronisation, in pinned memory that the kernels write
+  double* hF = nullptr;    // objective per slot
+  double* hres = nullptr;  // 2 doubles per slot: dot results
   double* dscal = nullptr;  // SCAL_PER_SLOT doubles per slot: optimizer scalars that stay on the device
   double* dpart = nullptr;  // PART_PER_BLOCK * max blocks
   size_t part_cap = 0;      // blocks
@@ -934,12 +936,6 @@ void enqueue(a2c_batch* b, std::initializer_list<uint64_t> key, std::function<vo
   b->arena.key.insert(b->arena.key.end(), key);
   b->arena.q.push_back(std::move(fn));
 }
-void enqueue_d2h(a2c_batch* b, void* dst, const void* src, size_t bytes) {
-  enqueue(b, {7, u64(dst), u64(src), (uint64_t)bytes}, [=](hipStream_t st) {
-    (void)hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, st);
-  });
-}
-
 uint64_t key_hash(const std::vector<uint64_t>& k) {  // FNV-1a over the words
   uint64_t h = 1469598103934665603ull;
   for (uint64_t w : k) h = (h ^ w) * 1099511628211ull;
@@ -1093,14 +1089,13 @@ int seg_dot(a2c_batch* b, const std::vector<int>& ids, Fill fill, std::vector<do
     o.met = Metric{};
     o.k1 = o.k2 = 0;
     fill(o, s);
-    o.out = b->dres + 2 * (&s - b->slots.data());
+    o.out = b->hres + 2 * (&s - b->slots.data());
   };
   SegDot* ops;
   int32_t* map;
   int nblk;
   if (int rc = seg_launch_prep<SegDot>(b, ids, fill2, &ops, &map, &nblk)) return rc;
   enqueue_dot(b, ops, map, nblk);
-  enqueue_d2h(b, b->hres, b->dres, sizeof(double) * 2 * b->slots.size());
   if (int rc = bsync(b)) return rc;
   for (size_t k = 0; k < ids.size(); ++k) {
     out[2 * k] = b->hres[2 * ids[k]];
@@ -1193,7 +1188,7 @@ int seg_pair(a2c_batch* b, const std::vector<int>& ids, std::vector<double>& out
     o.x = s.x; o.xo = s.xo; o.g = s.g; o.go = s.go;
     o.S = s.S[s.head]; o.Y = s.Y[s.head]; o.gp = s.gp;
     o.lb = s.opts.sigma_lb; o.ub = s.opts.sigma_ub;
-    o.out = b->dres + 2 * (&s - b->slots.data());
+    o.out = b->hres + 2 * (&s - b->slots.data());
     o.out2 = o.out + 1;
   };
   SegPair* ops;
@@ -1205,7 +1200,6 @@ int seg_pair(a2c_batch* b, const std::vector<int>& ids, std::vector<double>& out
     enqueue(b, {12, u64(ops), u64(map), u64(part), (uint64_t)nblk}, [=](hipStream_t st) {
       hipLaunchKernelGGL(k_seg_pair, dim3(nblk), dim3(TB), 0, st, ops, map, part, nblk);
     });
-  enqueue_d2h(b, b->hres, b->dres, sizeof(double) * 2 * b->slots.size());
   if (int rc = bsync(b)) return rc;
   for (size_t k = 0; k < ids.size(); ++k) {
     out[2 * k] = b->hres[2 * ids[k]];
@@ -1242,7 +1236,7 @@ int gen_eval(a2c_batch* b, int id, bool fp64, StateOf state_of) {
   state_of(s, &X, &G);
   L.X = X;
   L.G = G;
-  L.f = b->dF + id;
+  L.f = b->hF + id;
   if (b->arena.used + 256 + sizeof(LatDev) > b->arena.cap)
     if (int rc = bsync(b)) return rc;
   LatDev* dl = b->arena.push(&L, 1);
@@ -1272,7 +1266,6 @@ int fused_eval(a2c_batch* b, const std::vector<int>& ids_in, bool fp64, StateOf 
   }
   if (ids.empty()) {
     if (!sync || ids_in.empty()) return A2C_OK;
-    enqueue_d2h(b, b->hF, b->dF, sizeof(double) * b->slots.size());
     return bsync(b);
   }
   std::vector<LatDev> lats(ids.size());
@@ -1287,7 +1280,7 @@ int fused_eval(a2c_batch* b, const std::vector<int>& ids_in, bool fp64, StateOf 
     state_of(s, &X, &G);
     L.X = X;
     L.G = G;
-    L.f = b->dF + ids[k];
+    L.f = b->hF + ids[k];
     L.blk0 = cum;
     L.kl32 = lanes_per_site(s.N(), false);
     L.kl64 = lanes_per_site(s.N(), true);
@@ -1336,7 +1329,6 @@ int fused_eval(a2c_batch* b, const std::vector<int>& ids_in, bool fp64, StateOf 
             if (rc && !b->qrc) b->qrc = rc;
           });
   if (!sync) return A2C_OK;
-  enqueue_d2h(b, b->hF, b->dF, sizeof(double) * b->slots.size());
   return bsync(b);
 }
 
@@ -1390,8 +1382,8 @@ int converged_reason(const Slot& s) {
 }
 
 // evaluate f, g at x for the listed slots, each in its own precision; with
-// sync = false the objective copy is only enqueued (the caller's next
-// synchronising step completes it, then take_f reads it)
+// sync = false the launches are only enqueued (after the caller's next
+// synchronising step take_f reads the objectives)
 int eval_slots(a2c_batch* b, const std::vector<int>& ids, bool sync = true) {
   std::vector<int> m32, m64;
   for (int i : ids) {
@@ -1402,7 +1394,6 @@ int eval_slots(a2c_batch* b, const std::vector<int>& ids, bool sync = true) {
   }
   if (int rc = fused_eval(b, m32, false, lmvm_state, false)) return rc;
   if (int rc = fused_eval(b, m64, true, lmvm_state, false)) return rc;
-  enqueue_d2h(b, b->hF, b->dF, sizeof(double) * b->slots.size());
   if (!sync) return A2C_OK;
   if (int rc = bsync(b)) return rc;
   for (int i : ids) b->slots[i].f = b->hF[i];
@@ -1487,7 +1478,7 @@ int directions(a2c_batch* b, const std::vector<int>& ids) {
       Slot& s = b->slots[small[k]];
       TwoLoop& o = ops[k];
       o.g = s.g; o.q = s.q; o.d = s.d; o.x = s.x;
-      o.out = b->dres + 2 * small[k];
+      o.out = b->hres + 2 * small[k];
       for (int t = 0; t < s.npairs; ++t) {
         const int p = (s.head - 1 - t + s.m) % s.m;
         o.S[t] = s.S[p]; o.Y[t] = s.Y[p]; o.rho[t] = s.rho[p];
@@ -1517,7 +1508,7 @@ int directions(a2c_batch* b, const std::vector<int>& ids) {
         }
         o.np = s.npairs; o.npd = s.fe->desc.n_pd; o.met = s.metric();
         o.lb = s.opts.sigma_lb; o.ub = s.opts.sigma_ub;
-        o.sums = scal(s); o.out = b->dres + 2 * (&s - b->slots.data());
+        o.sums = scal(s); o.out = b->hres + 2 * (&s - b->slots.data());
       }))
     return rc;
   if (!tl.empty()) {
@@ -1553,7 +1544,7 @@ int directions(a2c_batch* b, const std::vector<int>& ids) {
               if (t > 0) { o.w = s.Y[pidx(s, t - 1)]; o.out = scal(s) + s.m + 2; }
               else {  // d = -q, widths at an active bound not moved; g . d
                 o.mode = 2; o.d = s.d; o.g = s.g; o.x = s.x; o.lb = s.opts.sigma_lb; o.ub = s.opts.sigma_ub;
-                o.out = b->dres + 2 * (&s - b->slots.data());
+                o.out = b->hres + 2 * (&s - b->slots.data());
               }
             }
           }))
@@ -1583,7 +1574,6 @@ int directions(a2c_batch* b, const std::vector<int>& ids) {
     if (int rc = seg_dot(b, sd, [](SegDot& o, Slot& s) { o.a1 = s.g; o.b1 = s.d; }, v)) return rc;
     for (size_t k = 0; k < sd.size(); ++k) b->slots[sd[k]].gd = v[2 * k];
   } else {
-    enqueue_d2h(b, b->hres, b->dres, sizeof(double) * 2 * b->slots.size());
     if (int rc = bsync(b)) return rc;
   }
   for (int i : small) b->slots[i].gd = b->hres[2 * i];
@@ -1786,7 +1776,12 @@ void a2c_batch_desc_default(a2c_batch_desc* d) {
   d->graphs = (g && std::string(g) == "1") ? 1 : 0;
 }
 
-int a2c_batch_create(const a2c_batch_desc* desc, a2c_batch** out) {
+int a2c_batch_create(const a2c_batch_desc* desc, a2c_batch** out) { return batch_create(desc, nullptr, out); }
+
+}  // extern "C"
+
+// On a stream of the caller's, or on one of its own when shared is null
+int a2c::batch_create(const a2c_batch_desc* desc, hipStream_t shared, a2c_batch** out) {
   if (!desc || !out || desc->max_lattices <= 0 || desc->max_lattices > (1 << 20)) return A2C_EINVAL;
   if (desc->precision != A2C_PREC_FP64 && desc->precision != A2C_PREC_MIXED) return A2C_EINVAL;
   if (desc->graphs != 0 && desc->graphs != 1) return A2C_EINVAL;
@@ -1803,13 +1798,18 @@ int a2c_batch_create(const a2c_batch_desc* desc, a2c_batch** out) {
   b->vector_free = tls.find("perstep") == std::string::npos;
   auto fail = [&](int rc) { a2c_batch_destroy(b); return rc; };
   if (hipSetDevice(desc->device) != hipSuccess) return fail(A2C_EHIP);
-  if (hipStreamCreateWithFlags(&b->stream, hipStreamNonBlocking) != hipSuccess) return fail(A2C_EHIP);
+  if (shared) {
+    b->stream = shared;
+    b->own_stream = false;
+  } else if (hipStreamCreateWithFlags(&b->stream, hipStreamNonBlocking) != hipSuccess) {
+    return fail(A2C_EHIP);
+  }
   const size_t cap = desc->max_lattices;
   b->slots.resize(cap);
   b->arena.cap = (size_t)32 << 20;
   bool ok = hmalloc(&b->arena.h, b->arena.cap) == hipSuccess && dmalloc(&b->arena.d, b->arena.cap) == hipSuccess &&
-            dmalloc(&b->dF, 8 * cap) == hipSuccess && hmalloc(&b->hF, 8 * cap) == hipSuccess &&
-            dmalloc(&b->dres, 16 * cap) == hipSuccess && hmalloc(&b->hres, 16 * cap) == hipSuccess &&
+            hmalloc(&b->hF, 8 * cap) == hipSuccess &&
+            hmalloc(&b->hres, 16 * cap) == hipSuccess &&
             dmalloc(&b->dscal, sizeof(double) * SCAL_PER_SLOT * cap) == hipSuccess;
   if (!ok) return fail(A2C_ENOMEM);
   DeviceTables tabs;
@@ -1820,9 +1820,12 @@ int a2c_batch_create(const a2c_batch_desc* desc, a2c_batch** out) {
   return A2C_OK;
 }
 
+extern "C" {
+
 void a2c_batch_destroy(a2c_batch* b) {
   if (!b) return;
   if (b->stream) (void)hipStreamSynchronize(b->stream);
+  const ReleaseScope released(b->desc.device);
   for (auto& e : b->graphs.map) (void)hipGraphExecDestroy(e.second.exec);
   for (auto& s : b->slots) {
     lmvm_free(s);
@@ -1830,13 +1833,11 @@ void a2c_batch_destroy(a2c_batch* b) {
   }
   (void)dfree(b->arena.d);
   if (b->arena.h) (void)hfree(b->arena.h);
-  (void)dfree(b->dF);
   if (b->hF) (void)hfree(b->hF);
-  (void)dfree(b->dres);
   (void)dfree(b->dscal);
   if (b->hres) (void)hfree(b->hres);
   (void)dfree(b->dpart);
-  if (b->stream) (void)hipStreamDestroy(b->stream);
+  if (b->stream && b->own_stream) (void)hipStreamDestroy(b->stream);
   delete b;
 }
 
@@ -1884,7 +1885,16 @@ int a2c_batch_add(a2c_batch* b, const a2c_fe_desc* lat, const double* X, const d
   a2c_fe_ctx* fe = nullptr;
   int rc = fe_create(&d, b->stream, &fe);
   if (rc) return berr(b, rc, "lattice context creation failed");
-  if ((rc = a2c_fe_set_occupancy(fe, x)) || (rc = a2c_fe_build_neighbors(fe, X, nullptr))) {
+  if ((rc = bsync(b))) {  // the state goes up through the arena
+    a2c_fe_destroy(fe);
+    return rc;
+  }
+  if (b->xfer.upload(b->stream, b->arena.h, b->arena.cap, fe->dX, X, 32 * (size_t)fe->N) != hipSuccess) {
+    (void)hipStreamSynchronize(b->stream);
+    a2c_fe_destroy(fe);
+    return berr(b, A2C_EHIP, "state upload failed");
+  }
+  if ((rc = a2c_fe_set_occupancy(fe, x)) || (rc = a2c_fe_build_neighbors_device(fe, fe->dX, nullptr))) {
     b->err = a2c_fe_last_error(fe);
     a2c_fe_destroy(fe);
     return rc;
@@ -1906,6 +1916,7 @@ int a2c_batch_remove(a2c_batch* b, int32_t slot) {
   if (int rc = bsync(b)) return rc;
   Slot& s = b->slots[slot];
   b->mem_used -= std::min(b->mem_used, s.charged);
+  const ReleaseScope released(b->desc.device);
   lmvm_free(s);
   if (s.owned) a2c_fe_destroy(s.fe);
   s = Slot();
@@ -1916,7 +1927,9 @@ int a2c_batch_set_state(a2c_batch* b, int32_t slot, const double* X) {
   if (!b || slot < 0 || slot >= (int)b->slots.size() || !b->slots[slot].used || !X) return A2C_EINVAL;
   if (int rc = bsync(b)) return rc;  // no launch may still read the state
   Slot& s = b->slots[slot];
-  B_HIP(b, hipMemcpy(s.fe->dX, X, 32 * (size_t)s.N(), hipMemcpyHostToDevice));
+  // through the arena, which is idle after bsync until the next queued launch
+  B_HIP(b, b->xfer.upload(b->stream, b->arena.h, b->arena.cap, s.fe->dX, X, 32 * (size_t)s.N()));
+  B_HIP(b, hipStreamSynchronize(b->stream));
   return A2C_OK;
 }
 
@@ -1926,8 +1939,9 @@ int a2c_batch_get_state(a2c_batch* b, int32_t slot, double* X, double* G) {
   Slot& s = b->slots[slot];
   const double* src = s.x ? s.x : s.fe->dX;
   const double* gsrc = s.x ? s.g : s.fe->dG;
-  if (X) B_HIP(b, hipMemcpy(X, src, 32 * (size_t)s.N(), hipMemcpyDeviceToHost));
-  if (G) B_HIP(b, hipMemcpy(G, gsrc, 32 * (size_t)s.N(), hipMemcpyDeviceToHost));
+  const size_t n = 32 * (size_t)s.N();
+  if (X) B_HIP(b, b->xfer.download(b->stream, b->arena.h, b->arena.cap, X, src, n));
+  if (G) B_HIP(b, b->xfer.download(b->stream, b->arena.h, b->arena.cap, G, gsrc, n));
   return A2C_OK;
 }
 
@@ -2008,11 +2022,10 @@ int lmvm_minimize(a2c_fe_ctx* c, const double* X0, const a2c_lmvm_opts* o, doubl
   bd.deriv_mode = c->desc.deriv_mode;
   bd.fd_eps = c->desc.fd_eps;
   bd.max_lattices = 1;
-  // the context's stream may still run work that uses the buffers the
+  // on the context's stream, behind any work that uses the buffers the
   // optimizer shares with it (state, scratch of the evaluation)
-  A2C_HIP(c, hipStreamSynchronize(c->stream));
   a2c_batch* b = nullptr;
-  if (int rc = a2c_batch_create(&bd, &b)) return set_err(c, rc, "batch creation failed");
+  if (int rc = batch_create(&bd, c->stream, &b)) return set_err(c, rc, "batch creation failed");
   struct Guard {
     a2c_batch* b;
     ~Guard() { a2c_batch_destroy(b); }
@@ -2023,7 +2036,7 @@ int lmvm_minimize(a2c_fe_ctx* c, const double* X0, const a2c_lmvm_opts* o, doubl
   s.fe = c;
   s.owned = false;
   s.used = true;
-  A2C_HIP(c, hipMemcpy(c->dX, X0, 32 * (size_t)c->N, hipMemcpyHostToDevice));
+  if (int rc = upload_state(c, X0)) return rc;
   c->lat_dirty = true;
   int rc = a2c_batch_lmvm_start(b, 0, o);
   if (!rc) {
@@ -2032,8 +2045,7 @@ int lmvm_minimize(a2c_fe_ctx* c, const double* X0, const a2c_lmvm_opts* o, doubl
   }
   if (rc) return set_err(c, rc, b->err);
   *rep = s.rep;
-  A2C_HIP(c, hipMemcpy(Xout, s.x, 32 * (size_t)c->N, hipMemcpyDeviceToHost));
-  return A2C_OK;
+  return download_state(c, Xout, s.x);
 }
 }  // namespace a2c
 

@@ -24,8 +24,24 @@ int set_err(a2c_fe_ctx* c, int code, const std::string& msg) {
 int host_staging(a2c_fe_ctx* c) {
   if (c->hX && c->hG) return A2C_OK;
   const size_t N = std::max(c->N, 1);
-  if ((!c->hX && hmalloc(&c->hX, 32 * N) != hipSuccess) || (!c->hG && hmalloc(&c->hG, 32 * N) != hipSuccess))
+  if ((!c->hX && hmalloc(&c->hX, 32 * N) != hipSuccess) || (!c->hG && hmalloc(&c->hG, 32 * N + 32) != hipSuccess))
     return set_err(c, A2C_ENOMEM, "pinned host staging");
+  return A2C_OK;
+}
+
+int upload_state(a2c_fe_ctx* c, const double* X) {
+  const size_t n = 32 * (size_t)c->N;
+  if (n == 0) return A2C_OK;
+  if (int rc = host_staging(c)) return rc;
+  A2C_HIP(c, c->xfer.upload(c->stream, reinterpret_cast<char*>(c->hX), n, c->dX, X, n));
+  return A2C_OK;
+}
+
+int download_state(a2c_fe_ctx* c, double* out, const double* dsrc) {
+  const size_t n = 32 * (size_t)c->N;
+  if (n == 0) return A2C_OK;
+  if (int rc = host_staging(c)) return rc;
+  A2C_HIP(c, c->xfer.download(c->stream, reinterpret_cast<char*>(c->hG), n, out, dsrc, n));
   return A2C_OK;
 }
 
@@ -34,15 +50,6 @@ namespace {
 int check_ctx(a2c_fe_ctx* c) {
   if (!c) return A2C_EINVAL;
   c->err.clear();
-  return A2C_OK;
-}
-
-int upload_state(a2c_fe_ctx* c, const double* X) {
-  const size_t n = 4 * (size_t)c->N;
-  if (n == 0) return A2C_OK;
-  if (int rc = host_staging(c)) return rc;
-  std::memcpy(c->hX, X, n * sizeof(double));
-  A2C_HIP(c, hipMemcpyAsync(c->dX, c->hX, n * sizeof(double), hipMemcpyHostToDevice, c->stream));
   return A2C_OK;
 }
 
@@ -116,7 +123,7 @@ int a2c::fe_create(const a2c_fe_desc* desc, hipStream_t shared, a2c_fe_ctx** out
   bool ok = dmalloc(&c->dX, 32 * N) == hipSuccess && dmalloc(&c->dG, 32 * N) == hipSuccess &&
             dmalloc(&c->dx, 8 * nh) == hipSuccess && dmalloc(&c->drho, 8 * N) == hipSuccess &&
             dmalloc(&c->dFp, 8 * N) == hipSuccess && dmalloc(&c->demb, 8 * N) == hipSuccess &&
-            dmalloc(&c->dpart, 8 * (RECV_LANES * (size_t)c->nblk_red + 1)) == hipSuccess && dmalloc(&c->dF, 64) == hipSuccess &&
+            dmalloc(&c->dpart, 8 * (RECV_LANES * (size_t)c->nblk_red + 1)) == hipSuccess && hmalloc(&c->dF, 64) == hipSuccess &&
             dmalloc(&c->dlat, sizeof(LatDev)) == hipSuccess &&
             dmalloc(&c->dqxy, 16 * N) == hipSuccess && dmalloc(&c->dqzs, 16 * N) == hipSuccess &&
             dmalloc(&c->dxrow, 8 * nh) == hipSuccess && dmalloc(&c->dgown, 32 * N) == hipSuccess &&
@@ -140,8 +147,9 @@ extern "C" {
 void a2c_fe_destroy(a2c_fe_ctx* c) {
   if (!c) return;
   if (c->stream) hipStreamSynchronize(c->stream);
+  const ReleaseScope released(c->desc.device);
   dfree(c->dX); dfree(c->dG); dfree(c->dx); dfree(c->drho); dfree(c->dFp);
-  dfree(c->demb); dfree(c->dpart); dfree(c->dF); dfree(c->dpdpdnum); dfree(c->daux);
+  dfree(c->demb); dfree(c->dpart); hfree(c->dF); dfree(c->dpdpdnum); dfree(c->daux);
   dfree(c->dqxy); dfree(c->dqzs); dfree(c->dxrow); dfree(c->dgown);  // dtab, dtab64: shared
   gen_free(c);
   for (int w = 0; w < 5; ++w) {
@@ -251,12 +259,9 @@ int a2c_fe_eval(a2c_fe_ctx* c, const double* X, double* f, double* G) {
   if (!f) return set_err(c, A2C_EINVAL, "null f");
   if (int rc = upload_state(c, X)) return rc;
   if (int rc = eval_dispatch(c, c->dX, c->dG, c->dF, false, nullptr)) return rc;
-  const size_t n = 4 * (size_t)c->N;  // upload_state allocated hG with hX
-  if (n) A2C_HIP(c, hipMemcpyAsync(c->hG, c->dG, 8 * n, hipMemcpyDeviceToHost, c->stream));
-  double fh = 0.0;
-  A2C_HIP(c, hipMemcpyAsync(&fh, c->dF, 8, hipMemcpyDeviceToHost, c->stream));
-  A2C_HIP(c, hipStreamSynchronize(c->stream));
-  if (n) std::memcpy(G, c->hG, 8 * n);
+  if (int rc = download_state(c, G, c->dG)) return rc;
+  if (c->N == 0) A2C_HIP(c, hipStreamSynchronize(c->stream));
+  const double fh = *c->dF;
   *f = fh;
   if (!std::isfinite(fh)) return set_err(c, A2C_ENONFINITE, "non-finite objective");
   return A2C_OK;

@@ -115,6 +115,19 @@ hipError_t dmalloc(void** ptr, size_t bytes) {
   return hipSuccess;
 }
 
+namespace {
+thread_local int t_released = -1;  // device of this thread's innermost ReleaseScope
+}
+
+ReleaseScope::ReleaseScope(int device) : prev_(t_released) {
+  int cur = 0;
+  if (hipGetDevice(&cur) != hipSuccess) return;
+  if (cur != device) (void)hipSetDevice(device);
+  if (hipDeviceSynchronize() == hipSuccess) t_released = device;
+  if (cur != device) (void)hipSetDevice(cur);
+}
+ReleaseScope::~ReleaseScope() { t_released = prev_; }
+
 hipError_t dfree(const void* ptr) {
   if (!ptr) return hipSuccess;
   Pool& P = pool();
@@ -125,11 +138,14 @@ hipError_t dfree(const void* ptr) {
     if (it == P.owner.end()) return hipErrorInvalidValue;
     o = it->second;
   }
-  int cur = 0;
-  if (hipError_t e = hipGetDevice(&cur)) return e;
-  if (cur != o.first) (void)hipSetDevice(o.first);
-  const hipError_t e = hipDeviceSynchronize();  // work in flight may still use the block
-  if (cur != o.first) (void)hipSetDevice(cur);
+  hipError_t e = hipSuccess;
+  if (t_released != o.first) {
+    int cur = 0;
+    if (hipError_t g = hipGetDevice(&cur)) return g;
+    if (cur != o.first) (void)hipSetDevice(o.first);
+    e = hipDeviceSynchronize();  // work in flight may still use the block
+    if (cur != o.first) (void)hipSetDevice(cur);
+  }
   std::lock_guard<std::mutex> lk(P.mu);
   P.owner.erase(ptr);
   P.free_blocks[o].push_back(const_cast<void*>(ptr));
@@ -163,7 +179,8 @@ hipError_t hfree(const void* ptr) {
     if (it == P.host_owner.end()) return hipErrorInvalidValue;
     sz = it->second;
   }
-  const hipError_t e = hipDeviceSynchronize();  // copies in flight may still read it
+  // copies in flight may still read it
+  const hipError_t e = t_released >= 0 ? hipSuccess : hipDeviceSynchronize();
   std::lock_guard<std::mutex> lk(P.mu);
   P.host_owner.erase(ptr);
   P.free_host[sz].push_back(const_cast<void*>(ptr));

@@ -24,6 +24,41 @@ inline hipError_t hmalloc(T** ptr, size_t bytes) {
   return hmalloc(reinterpret_cast<void**>(ptr), bytes);
 }
 hipError_t hfree(const void* ptr);
+// While one lives, this thread's releases on its device (dfree, hfree) do not
+// wait for the device again: it waited when it was made, and nothing that uses
+// the released blocks is issued during its life (a context's teardown, ~50
+// blocks at ~1 us each).
+class ReleaseScope {
+ public:
+  explicit ReleaseScope(int device);
+  ~ReleaseScope();
+  ReleaseScope(const ReleaseScope&) = delete;
+  ReleaseScope& operator=(const ReleaseScope&) = delete;
+
+ private:
+  int prev_;
+};
+
+// Transfers between pageable memory of a caller and the device through pinned
+// staging, in parts, so that the copy on the host and the transfer overlap.  stage
+// (cap bytes, a multiple of 16) must be idle.  Device buffers are the library's own
+// (whole 16-byte words).  upload returns with transfers in flight from stage
+// unless it had to reuse it; download returns when dst is complete.  A kernel writes
+// the pinned words: for the small transfers that is ~20 us sooner than the
+// copy engine, for large ones as fast.
+class HostTransfer {
+ public:
+  hipError_t upload(hipStream_t st, char* stage, size_t cap, void* ddst, const void* src, size_t bytes);
+  hipError_t download(hipStream_t st, char* stage, size_t cap, void* dst, const void* dsrc, size_t bytes);
+  ~HostTransfer();
+
+ private:
+  static constexpr int PARTS = 8;
+  static constexpr size_t PART_MIN = (size_t)512 << 10;
+  hipEvent_t ev_[PARTS] = {};
+};
+// device words to pinned memory by a kernel on st, rounded up to 16 bytes
+hipError_t copy_to_pinned(hipStream_t st, void* pinned, const void* dsrc, size_t bytes);
 
 constexpr double KB = 8.6173324e-5;  // Boltzmann constant, eV/K (minimizer.cpp:92)
 constexpr int NBR_CAP = 256;          // per-site neighbor cap of the build kernel
@@ -439,7 +474,7 @@ struct a2c_fe_ctx {
   double* demb = nullptr;    // N  embedding energy per site (x-weighted for H)
   double* depair = nullptr;  // N  pair-energy partial of the mixed path
   double* dpart = nullptr;   // block partial sums
-  double* dF = nullptr;      // 1 objective (device)
+  double* dF = nullptr;      // 1 objective, in pinned memory that the kernels write
   int32_t nblk_red = 0;
   bool have_x = false;
   bool have_nbr = false;
@@ -482,6 +517,7 @@ struct a2c_fe_ctx {
   // host staging (pinned)
   double* hX = nullptr;
   double* hG = nullptr;
+  a2c::HostTransfer xfer;
 
   // occupancy scratch of the chemical potential and the diffusion step
   // (allocated at their first call, kept for the context's lifetime)
@@ -603,6 +639,8 @@ struct DeviceTables {
 };
 hipError_t device_tables(int device, DeviceTables* out);
 int host_staging(a2c_fe_ctx* c);  // pinned hX, hG of the host-array entry points (capi.cpp)
+int upload_state(a2c_fe_ctx* c, const double* X);  // X to the context state dX through hX, on the context stream
+int download_state(a2c_fe_ctx* c, double* out, const double* dsrc);  // 4N doubles through hG; complete on return
 // General model (evalgen.hip, general.cpp)
 int run_eval_gen(const LatDev* dlat, int npd, int nh, const GenDev& g, int deriv_mode, double eps, bool fp32, hipStream_t st,
                  Timing* tm);

@@ -28,6 +28,26 @@ int occ_scratch(a2c_fe_ctx* c) {
   return A2C_OK;
 }
 
+// Pinned staging of the occupancy arrays in hG (32 N bytes, at least 64):
+// gamma or the new occupancy, and full_H or the balance, each in whole 16-byte words.
+struct OccStage {
+  double* g;
+  int32_t* full;
+  explicit OccStage(const a2c_fe_ctx* c)
+      : g(c->hG), full(reinterpret_cast<int32_t*>(c->hG + (c->desc.n_h + 1) / 2 * 2)) {}
+};
+int upload_occ(a2c_fe_ctx* c, const double* gamma, const int32_t* full_h) {
+  const size_t nh = c->desc.n_h;
+  if (!nh) return A2C_OK;
+  if (int rc = host_staging(c)) return rc;
+  const OccStage h(c);
+  std::memcpy(h.g, gamma, 8 * nh);
+  std::memcpy(h.full, full_h, 4 * nh);
+  A2C_HIP(c, hipMemcpyAsync(c->occ_g, h.g, 8 * nh, hipMemcpyHostToDevice, c->stream));
+  A2C_HIP(c, hipMemcpyAsync(c->occ_full, h.full, 4 * nh, hipMemcpyHostToDevice, c->stream));
+  return A2C_OK;
+}
+
 }  // namespace
 
 extern "C" int a2c_fe_chem_potential(a2c_fe_ctx* c, const double* X, const double* coe_pd, const double* coe_h,
@@ -37,25 +57,23 @@ extern "C" int a2c_fe_chem_potential(a2c_fe_ctx* c, const double* X, const doubl
   if (!c->have_nbr || !c->have_x) return set_err(c, A2C_ESTATE, "neighbors/occupancy not set");
   if ((!X && c->N) || !coe_pd || !coe_h || (c->desc.n_h && (!gamma || !full_h)))
     return set_err(c, A2C_EINVAL, "null argument");
-  const size_t nh = c->desc.n_h, N = c->N;
+  const size_t nh = c->desc.n_h;
   if (int rc = occ_scratch(c)) return rc;
   double *dg = c->occ_g, *dcorr = c->occ_corr;
   int32_t* dfull = c->occ_full;
-  if (N) {
-    if (int rc = host_staging(c)) return rc;
-    std::copy(X, X + 4 * N, c->hX);
-    A2C_HIP(c, hipMemcpyAsync(c->dX, c->hX, 32 * N, hipMemcpyHostToDevice, c->stream));
-  }
-  if (nh) {
-    A2C_HIP(c, hipMemcpyAsync(dg, gamma, 8 * nh, hipMemcpyHostToDevice, c->stream));
-    A2C_HIP(c, hipMemcpyAsync(dfull, full_h, 4 * nh, hipMemcpyHostToDevice, c->stream));
-  }
+  if (int rc = upload_state(c, X)) return rc;
+  if (int rc = upload_occ(c, gamma, full_h)) return rc;
   if (int rc = launch_chem(c, c->dX, coe_pd, coe_h, gamma_bd, dg, dfull, dcorr)) return rc;
   if (nh) {
-    A2C_HIP(c, hipMemcpyAsync(gamma, dg, 8 * nh, hipMemcpyDeviceToHost, c->stream));
-    A2C_HIP(c, hipMemcpyAsync(full_h, dfull, 4 * nh, hipMemcpyDeviceToHost, c->stream));
+    const OccStage h(c);
+    A2C_HIP(c, copy_to_pinned(c->stream, h.g, dg, 8 * nh));
+    A2C_HIP(c, copy_to_pinned(c->stream, h.full, dfull, 4 * nh));
+    A2C_HIP(c, hipStreamSynchronize(c->stream));
+    std::memcpy(gamma, h.g, 8 * nh);
+    std::memcpy(full_h, h.full, 4 * nh);
+  } else {
+    A2C_HIP(c, hipStreamSynchronize(c->stream));
   }
-  A2C_HIP(c, hipStreamSynchronize(c->stream));
   return A2C_OK;
 }
 
@@ -72,15 +90,16 @@ extern "C" int a2c_fe_diffuse(a2c_fe_ctx* c, double dt, double nu, double Qm, do
   if (int rc = occ_scratch(c)) return rc;
   double *dg = c->occ_g, *dxn = c->occ_xn;
   int32_t* dfull = c->occ_full;
-  A2C_HIP(c, hipMemcpyAsync(dg, gamma, 8 * nh, hipMemcpyHostToDevice, c->stream));
-  A2C_HIP(c, hipMemcpyAsync(dfull, full_h, 4 * nh, hipMemcpyHostToDevice, c->stream));
+  if (int rc = upload_occ(c, gamma, full_h)) return rc;
   const DiffuseScratch w{c->occ_uv, c->occ_part, c->occ_bal};
   if (int rc = launch_diffuse(c, dt, pref, xLb, xUb, dg, dfull, w, dxn)) return rc;
   A2C_HIP(c, hipMemcpyAsync(c->dx, dxn, 8 * nh, hipMemcpyDeviceToDevice, c->stream));
-  A2C_HIP(c, hipMemcpyAsync(x, dxn, 8 * nh, hipMemcpyDeviceToHost, c->stream));
-  double bal[4];
-  A2C_HIP(c, hipMemcpyAsync(bal, c->occ_bal, sizeof(bal), hipMemcpyDeviceToHost, c->stream));
+  const OccStage h(c);
+  A2C_HIP(c, copy_to_pinned(c->stream, h.g, dxn, 8 * nh));
+  double* bal = reinterpret_cast<double*>(h.full);
+  A2C_HIP(c, copy_to_pinned(c->stream, bal, c->occ_bal, 32));
   A2C_HIP(c, hipStreamSynchronize(c->stream));
+  std::memcpy(x, h.g, 8 * nh);
   c->last_balance = a2c_diffusion_balance{bal[0], bal[1], bal[2], bal[3]};
   return A2C_OK;
 }
