@@ -350,6 +350,7 @@ struct SegPair {
   double lb, ub;
   double* out;   // s.y
   double* out2;  // gp.gp
+  double* sy;    // s.y again, on the device
   int32_t nsite, blk0;
   int32_t done = 0;  // blocks arrived
 };
@@ -387,7 +388,10 @@ __global__ __launch_bounds__(TB) void k_seg_pair(SegPair* ops, const int32_t* __
     put_part(part + nblk + blockIdx.x, gg);
   }
   if (!last_block(&ops[b2l[blockIdx.x]].done, lattice_blocks(o.nsite))) return;
-  sum_parts<2>(part + o.blk0, nblk, lattice_blocks(o.nsite), [&](int k, double v) { *(k ? o.out2 : o.out) = v; });
+  sum_parts<2>(part + o.blk0, nblk, lattice_blocks(o.nsite), [&](int k, double v) {
+    *(k ? o.out2 : o.out) = v;
+    if (k == 0) *o.sy = v;
+  });
 }
 
 // one block per op: fixed-order sums of the op's NOUT block partials
@@ -638,6 +642,13 @@ constexpr int VF_TRI = VF_PAIRS * (VF_PAIRS - 1) / 2;
 constexpr int VF_SUMS = VF_PAIRS + VF_TRI + 2 * NGROUP;
 __device__ __forceinline__ constexpr int vf_tri(int a, int b) { return VF_PAIRS + a * (a - 1) / 2 + b; }  // a > b
 
+// rho with the newest pair's from the device
+__device__ __forceinline__ void vf_rho(const double (&host)[VF_PAIRS], const double* sy, double (&rho)[VF_PAIRS]) {
+#pragma unroll
+  for (int t = 0; t < VF_PAIRS; ++t) rho[t] = host[t];
+  if (sy) rho[0] = 1.0 / *sy;
+}
+
 // The loops on the scalars.  acc: the VF_SUMS sums of the first pass.
 // First loop, newest to oldest: alpha_t = rho_t s_t . (g - sum_{u<t} alpha_u y_u).
 __device__ __forceinline__ void vf_alpha(const double* acc, const double* rho, int np, double (&al)[VF_PAIRS]) {
@@ -692,6 +703,7 @@ struct SegVF {
   const double* S[VF_PAIRS];  // step t = 0 is the newest pair (again past np)
   const double* Y[VF_PAIRS];
   double rho[VF_PAIRS];
+  const double* sy;           // s_0 . y_0 on the device where the host does not know rho[0] yet, else null
   double* q;                  // r
   double* d;
   const double* x;
@@ -753,8 +765,9 @@ __global__ __launch_bounds__(TB) void k_seg_vf2(SegVF* ops, const int32_t* __res
   const SegVF o = ops[b2l[blockIdx.x]];
   const int s = (blockIdx.x - o.blk0) * TB + threadIdx.x;
   const int np = o.np;
-  double al[VF_PAIRS], gam[NGROUP];
-  vf_alpha(o.sums, o.rho, np, al);
+  double al[VF_PAIRS], gam[NGROUP], rho[VF_PAIRS];
+  vf_rho(o.rho, o.sy, rho);
+  vf_alpha(o.sums, rho, np, al);
   vf_gamma(o.sums, gam);
   double yr[VF_PAIRS] = {};
   if (s < o.nsite) {
@@ -789,9 +802,10 @@ __global__ __launch_bounds__(TB) void k_seg_vf3(SegVF* ops, const int32_t* __res
   const SegVF o = ops[b2l[blockIdx.x]];
   const int s = (blockIdx.x - o.blk0) * TB + threadIdx.x;
   const int np = o.np;
-  double al[VF_PAIRS], c[VF_PAIRS];
-  vf_alpha(o.sums, o.rho, np, al);
-  vf_coef(o.sums, o.sums + VF_SUMS, o.rho, np, al, c);
+  double al[VF_PAIRS], c[VF_PAIRS], rho[VF_PAIRS];
+  vf_rho(o.rho, o.sy, rho);
+  vf_alpha(o.sums, rho, np, al);
+  vf_coef(o.sums, o.sums + VF_SUMS, rho, np, al, c);
   double gd = 0.0;
   if (s < o.nsite) {
     const size_t i0 = 4 * (size_t)s;
@@ -859,6 +873,8 @@ struct Slot {
   std::vector<double> rho, alpha;
   double f = 0, fold = 0, gnorm = 0, gnorm0 = 0, gd = 0, stp = 0;
   bool steepest = false;
+  bool dir_ready = false;  // d and gd_next hold the next iteration's direction and slope
+  double gd_next = 0;
   int lsstat = 0, nfev = 0;
   MoreThuente ls;
   int N() const { return fe->N; }
@@ -902,6 +918,7 @@ struct a2c_batch {
   // results the host reads after a synchronisation, in pinned memory that the kernels write
   double* hF = nullptr;    // objective per slot
   double* hres = nullptr;  // 2 doubles per slot: dot results
+  double* hgd = nullptr;   // slope of a direction queued behind its pair
   double* dscal = nullptr;  // SCAL_PER_SLOT doubles per slot: optimizer scalars that stay on the device
   double* dpart = nullptr;  // PART_PER_BLOCK * max blocks
   size_t part_cap = 0;      // blocks
@@ -1179,9 +1196,28 @@ int seg_vf(a2c_batch* b, const std::vector<int>& ids, Fill fill) {
   return A2C_OK;
 }
 
+double* slot_scal(a2c_batch* b, const Slot& s) { return b->dscal + SCAL_PER_SLOT * (&s - b->slots.data()); }
+constexpr int SCAL_SY = SCAL_PER_SLOT - 1;  // s.y of the newest pair
+static_assert(VF_SUMS + VF_PAIRS <= SCAL_SY, "device scalars of the vector-free recursion");
+
+// The recursion over the np newest of the pairs that end before head.
+void fill_vf(a2c_batch* b, SegVF& o, Slot& s, int np, int head, const double* sy, double* out) {
+  o.g = s.g; o.q = s.q; o.d = s.d; o.x = s.x;
+  for (int t = 0; t < VF_PAIRS; ++t) {
+    const int p = (head - 1 - (t < np ? t : 0) + 2 * s.m) % s.m;
+    o.S[t] = s.S[p]; o.Y[t] = s.Y[p]; o.rho[t] = t < np ? s.rho[p] : 0.0;
+  }
+  o.sy = sy;
+  o.np = np; o.npd = s.fe->desc.n_pd; o.met = s.metric();
+  o.lb = s.opts.sigma_lb; o.ub = s.opts.sigma_ub;
+  o.sums = slot_scal(b, s); o.out = out;
+}
+
 // s, y, gp of the accepted step and the dots s.y, gp.gp per slot, returned in
-// out[2k], out[2k + 1] (one round trip)
-int seg_pair(a2c_batch* b, const std::vector<int>& ids, std::vector<double>& out) {
+// out[2k], out[2k + 1]; behind them, in the same round trip, the next
+// directions of the slots in next, as if their pairs are kept (a pair that is
+// not makes its slot's d and hgd meaningless)
+int seg_pair(a2c_batch* b, const std::vector<int>& ids, const std::vector<int>& next, std::vector<double>& out) {
   out.assign(2 * ids.size(), 0.0);
   if (ids.empty()) return A2C_OK;
   auto fill = [&](SegPair& o, Slot& s) {
@@ -1190,6 +1226,7 @@ int seg_pair(a2c_batch* b, const std::vector<int>& ids, std::vector<double>& out
     o.lb = s.opts.sigma_lb; o.ub = s.opts.sigma_ub;
     o.out = b->hres + 2 * (&s - b->slots.data());
     o.out2 = o.out + 1;
+    o.sy = slot_scal(b, s) + SCAL_SY;
   };
   SegPair* ops;
   int32_t* map;
@@ -1200,6 +1237,11 @@ int seg_pair(a2c_batch* b, const std::vector<int>& ids, std::vector<double>& out
     enqueue(b, {12, u64(ops), u64(map), u64(part), (uint64_t)nblk}, [=](hipStream_t st) {
       hipLaunchKernelGGL(k_seg_pair, dim3(nblk), dim3(TB), 0, st, ops, map, part, nblk);
     });
+  if (int rc = seg_vf(b, next, [&](SegVF& o, Slot& s) {
+        fill_vf(b, o, s, std::min(s.npairs + 1, s.m), (s.head + 1) % s.m, slot_scal(b, s) + SCAL_SY,
+                b->hgd + (&s - b->slots.data()));
+      }))
+    return rc;
   if (int rc = bsync(b)) return rc;
   for (size_t k = 0; k < ids.size(); ++k) {
     out[2 * k] = b->hres[2 * ids[k]];
@@ -1417,7 +1459,10 @@ int proj_gnorm(a2c_batch* b, const std::vector<int>& ids) {
 // slots whose mixed phase ended: re-evaluate in FP64 at the same point
 int switch_to_fp64(a2c_batch* b, const std::vector<int>& ids) {
   if (ids.empty()) return A2C_OK;
-  for (int i : ids) b->slots[i].mixed = false;
+  for (int i : ids) {
+    b->slots[i].mixed = false;
+    b->slots[i].dir_ready = false;  // its gradient is replaced
+  }
   if (int rc = eval_slots(b, ids)) return rc;
   return proj_gnorm(b, ids);
 }
@@ -1455,7 +1500,18 @@ int lmvm_init(a2c_batch* b, const std::vector<int>& ids) {
 
 // d = -H g for the listed slots (two-loop recursion, or scaled steepest
 // descent for slots with no pairs or marked steepest)
-int directions(a2c_batch* b, const std::vector<int>& ids) {
+int directions(a2c_batch* b, const std::vector<int>& all) {
+  std::vector<int> ids;
+  for (int i : all) {
+    Slot& s = b->slots[i];
+    if (!s.dir_ready || s.steepest) {
+      ids.push_back(i);
+    } else {
+      s.gd = s.gd_next;
+    }
+    s.dir_ready = false;
+  }
+  if (ids.empty()) return A2C_OK;
   std::vector<int> tl, tlvf, sd, small;  // segmented two-loop (per step / vector-free), steepest descent, fused
   int maxp = 0;
   for (int i : ids) {
@@ -1498,17 +1554,9 @@ int directions(a2c_batch* b, const std::vector<int>& ids) {
     });
   }
   std::vector<double> v;
-  auto scal = [b](const Slot& s) { return b->dscal + SCAL_PER_SLOT * (&s - b->slots.data()); };
-  static_assert(VF_SUMS + VF_PAIRS <= SCAL_PER_SLOT, "device scalars of the vector-free recursion");
+  auto scal = [b](const Slot& s) { return slot_scal(b, s); };
   if (int rc = seg_vf(b, tlvf, [&](SegVF& o, Slot& s) {
-        o.g = s.g; o.q = s.q; o.d = s.d; o.x = s.x;
-        for (int t = 0; t < VF_PAIRS; ++t) {
-          const int p = (s.head - 1 - (t < s.npairs ? t : 0) + s.m) % s.m;
-          o.S[t] = s.S[p]; o.Y[t] = s.Y[p]; o.rho[t] = t < s.npairs ? s.rho[p] : 0.0;
-        }
-        o.np = s.npairs; o.npd = s.fe->desc.n_pd; o.met = s.metric();
-        o.lb = s.opts.sigma_lb; o.ub = s.opts.sigma_ub;
-        o.sums = scal(s); o.out = b->hres + 2 * (&s - b->slots.data());
+        fill_vf(b, o, s, s.npairs, s.head, nullptr, b->hres + 2 * (&s - b->slots.data()));
       }))
     return rc;
   if (!tl.empty()) {
@@ -1570,7 +1618,7 @@ int directions(a2c_batch* b, const std::vector<int>& ids) {
         o.z = s.d; o.x = s.x; o.lb = s.opts.sigma_lb; o.ub = s.opts.sigma_ub;
       }))
     return rc;
-  if (!sd.empty()) {  // its copy of the results also brings the two-loop slots' g . d
+  if (!sd.empty()) {  // its round trip also brings the two-loop slots' g . d
     if (int rc = seg_dot(b, sd, [](SegDot& o, Slot& s) { o.a1 = s.g; o.b1 = s.d; }, v)) return rc;
     for (size_t k = 0; k < sd.size(); ++k) b->slots[sd[k]].gd = v[2 * k];
   } else {
@@ -1680,8 +1728,14 @@ int lmvm_iteration(a2c_batch* b, std::vector<int>& act) {
     if (s.rep.reason) s.running = false;
   }
   if (!ok.empty()) {
-    // the new pair, s.y and the projected-gradient norm in one round trip
-    if (int rc = seg_pair(b, ok, v)) return rc;
+    // the new pair, s.y and the projected-gradient norm, and the direction that
+    // follows, in one round trip
+    std::vector<int> next;
+    for (int i : ok) {
+      const Slot& s = b->slots[i];
+      if (b->vector_free && std::min(s.npairs + 1, s.m) <= VF_PAIRS) next.push_back(i);
+    }
+    if (int rc = seg_pair(b, ok, next, v)) return rc;
     for (size_t k = 0; k < ok.size(); ++k) {
       Slot& s = b->slots[ok[k]];
       s.gnorm = std::sqrt(v[2 * k + 1]);
@@ -1689,6 +1743,8 @@ int lmvm_iteration(a2c_batch* b, std::vector<int>& act) {
         s.rho[s.head] = 1.0 / v[2 * k];
         s.head = (s.head + 1) % s.m;
         s.npairs = std::min(s.npairs + 1, s.m);
+        s.dir_ready = b->vector_free && s.npairs <= VF_PAIRS;
+        s.gd_next = b->hgd[ok[k]];
       } else if (s.npairs == s.m) {
         // k_seg_pair wrote the rejected s, y over S[head], Y[head], which with
         // a full history held the oldest pair still in use: that pair is gone,
@@ -1810,6 +1866,7 @@ int a2c::batch_create(const a2c_batch_desc* desc, hipStream_t shared, a2c_batch*
   bool ok = hmalloc(&b->arena.h, b->arena.cap) == hipSuccess && dmalloc(&b->arena.d, b->arena.cap) == hipSuccess &&
             hmalloc(&b->hF, 8 * cap) == hipSuccess &&
             hmalloc(&b->hres, 16 * cap) == hipSuccess &&
+            hmalloc(&b->hgd, 8 * cap) == hipSuccess &&
             dmalloc(&b->dscal, sizeof(double) * SCAL_PER_SLOT * cap) == hipSuccess;
   if (!ok) return fail(A2C_ENOMEM);
   DeviceTables tabs;
@@ -1836,6 +1893,7 @@ void a2c_batch_destroy(a2c_batch* b) {
   if (b->hF) (void)hfree(b->hF);
   (void)dfree(b->dscal);
   if (b->hres) (void)hfree(b->hres);
+  if (b->hgd) (void)hfree(b->hgd);
   (void)dfree(b->dpart);
   if (b->stream && b->own_stream) (void)hipStreamDestroy(b->stream);
   delete b;
@@ -1982,6 +2040,7 @@ int a2c_batch_lmvm_start(a2c_batch* b, int32_t slot, const a2c_lmvm_opts* o) {
   s.mixed = s.fe->desc.precision == A2C_PREC_MIXED;
   s.running = true;
   s.started = false;
+  s.dir_ready = false;  // a direction left by the last relaxation
   return A2C_OK;
 }
 

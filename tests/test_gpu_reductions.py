@@ -54,3 +54,24 @@ def test_blocks():
         assert np.max(np.abs(X - Y)) <= 1e-7
         ra, Xa = relax((n,), "")[n]
         assert ra["f"] == r["f"] and np.array_equal(Xa, X)
+
+
+@pytest.mark.parametrize("precision", ["fp64", "mixed"])
+@pytest.mark.parametrize("first", [1, 6, 400])
+def test_a_slot_relaxes_again_as_the_first_time(precision, first):
+    """A relaxation leaves nothing to the next one of its slot: stopped after
+    `first` iterations or converged, a new start from the same state gives the
+    same report and state, bit for bit."""
+    X, x, box, per, npd, nh = cut(513)
+    with A.Batch(precision=precision, max_lattices=1) as b:
+        s = b.add(X, x, npd, nh, box, per, T=400.0)
+        runs = []
+        for it in (first, 400, 400):
+            b.set_state(s, X)
+            b.start(s, max_it=it)
+            while b.step(7):
+                pass
+            runs.append((b.report(s), b.get_state(s)[0]))
+    assert runs[1][0] == runs[2][0] and np.array_equal(runs[1][1], runs[2][1])
+    if first == 400:
+        assert runs[0][0] == runs[1][0] and np.array_equal(runs[0][1], runs[1][1])
