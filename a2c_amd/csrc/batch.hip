@@ -1947,12 +1947,18 @@ int a2c_batch_add(a2c_batch* b, const a2c_fe_desc* lat, const double* X, const d
     a2c_fe_destroy(fe);
     return rc;
   }
-  if (b->xfer.upload(b->stream, b->arena.h, b->arena.cap, fe->dX, X, 32 * (size_t)fe->N) != hipSuccess) {
+  // the occupancy behind the state if both fit
+  const size_t nX = 32 * (size_t)fe->N, nx = 8 * (size_t)lat->n_h;
+  const bool both = nX + nx <= b->arena.cap;
+  if (b->xfer.upload(b->stream, b->arena.h, both ? std::max<size_t>(nX, 16) : b->arena.cap, fe->dX, X, nX) != hipSuccess ||
+      (both && b->xfer.upload(b->stream, b->arena.h + nX, std::max<size_t>(nx, 16), fe->dx, x, nx) != hipSuccess)) {
     (void)hipStreamSynchronize(b->stream);
     a2c_fe_destroy(fe);
     return berr(b, A2C_EHIP, "state upload failed");
   }
-  if ((rc = a2c_fe_set_occupancy(fe, x)) || (rc = a2c_fe_build_neighbors_device(fe, fe->dX, nullptr))) {
+  fe->have_x = true;
+  // the build's synchronisation frees the arena again
+  if ((!both && (rc = a2c_fe_set_occupancy(fe, x))) || (rc = a2c_fe_build_neighbors_device(fe, fe->dX, nullptr))) {
     b->err = a2c_fe_last_error(fe);
     a2c_fe_destroy(fe);
     return rc;

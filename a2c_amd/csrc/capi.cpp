@@ -53,10 +53,6 @@ int check_ctx(a2c_fe_ctx* c) {
   return A2C_OK;
 }
 
-// entries of the block -> lattice map: site blocks or the units of a
-// pair-owner pass at any lanes per site
-int map_units(int N) { return owner_units(N, MAX_LANES_PER_SITE) + 1; }
-
 bool aligned32(const void* p) { return ((uintptr_t)p & 31u) == 0; }
 
 }  // namespace
@@ -126,16 +122,13 @@ int a2c::fe_create(const a2c_fe_desc* desc, hipStream_t shared, a2c_fe_ctx** out
             dmalloc(&c->dpart, 8 * (RECV_LANES * (size_t)c->nblk_red + 1)) == hipSuccess && hmalloc(&c->dF, 64) == hipSuccess &&
             dmalloc(&c->dlat, sizeof(LatDev)) == hipSuccess &&
             dmalloc(&c->dqxy, 16 * N) == hipSuccess && dmalloc(&c->dqzs, 16 * N) == hipSuccess &&
-            dmalloc(&c->dxrow, 8 * nh) == hipSuccess && dmalloc(&c->dgown, 32 * N) == hipSuccess &&
-            dmalloc(&c->db2l, 4 * (size_t)map_units(c->N)) == hipSuccess;
+            dmalloc(&c->dxrow, 8 * nh) == hipSuccess && dmalloc(&c->dgown, 32 * N) == hipSuccess;
   if (!ok) return fail(A2C_ENOMEM);
   {
     DeviceTables t;
     if (device_tables(desc->device, &t) != hipSuccess) return fail(A2C_EHIP);
     c->dtab64 = t.t64;  // shared, not freed with the context
   }
-  // all-zero block -> lattice map, long enough for the pair-owner launches too
-  if (hipMemset(c->db2l, 0, 4 * (size_t)map_units(c->N)) != hipSuccess) return fail(A2C_EHIP);
   c->lat_dirty = true;
   if (desc->precision == A2C_PREC_MIXED && build_tables(c) != A2C_OK) return fail(A2C_EHIP);
   *out = c;
@@ -167,6 +160,7 @@ void a2c_fe_destroy(a2c_fe_ctx* c) {
   if (c->hX) hfree(c->hX);
   if (c->hG) hfree(c->hG);
   if (c->hlat) hfree(c->hlat);
+  hfree(c->nb_host);
   dfree(c->dlat);
   dfree(c->db2l);
   if (c->stream && c->own_stream) hipStreamDestroy(c->stream);
@@ -189,8 +183,13 @@ int a2c_fe_set_precision(a2c_fe_ctx* c, int32_t precision) {
 int a2c_fe_set_occupancy(a2c_fe_ctx* c, const double* x) {
   if (int rc = check_ctx(c)) return rc;
   if (!x && c->desc.n_h > 0) return set_err(c, A2C_EINVAL, "x is null");
-  if (c->desc.n_h > 0)
-    A2C_HIP(c, hipMemcpy(c->dx, x, 8 * (size_t)c->desc.n_h, hipMemcpyHostToDevice));
+  const size_t n = 8 * (size_t)c->desc.n_h;
+  if (n > 0 && c->hX) {  // through the pinned staging if the context has it
+    A2C_HIP(c, c->xfer.upload(c->stream, reinterpret_cast<char*>(c->hX), 32 * (size_t)c->N, c->dx, x, n));
+    A2C_HIP(c, hipStreamSynchronize(c->stream));
+  } else if (n > 0) {
+    A2C_HIP(c, hipMemcpy(c->dx, x, n, hipMemcpyHostToDevice));
+  }
   c->have_x = true;
   return A2C_OK;
 }
@@ -223,6 +222,7 @@ int a2c_fe_get_neighbors(a2c_fe_ctx* c, int32_t which, int32_t* offsets, int32_t
   if (!c->have_nbr) return set_err(c, A2C_ESTATE, "no neighbor lists");
   if (which < 0 || which > 4 || !offsets) return set_err(c, A2C_EINVAL, "bad list id");
   const Ell& L = c->ell[which];
+  A2C_HIP(c, hipStreamSynchronize(c->stream));  // the build's last kernels may still run
   std::vector<int32_t> cnt(L.rows), idx((size_t)L.width * L.rows);
   if (L.rows) A2C_HIP(c, hipMemcpy(cnt.data(), L.cnt, 4 * cnt.size(), hipMemcpyDeviceToHost));
   if (!idx.empty()) A2C_HIP(c, hipMemcpy(idx.data(), L.idx, 4 * idx.size(), hipMemcpyDeviceToHost));
@@ -238,6 +238,7 @@ int a2c_fe_get_neighbors(a2c_fe_ctx* c, int32_t which, int32_t* offsets, int32_t
 int a2c_fe_get_pdpdnum(a2c_fe_ctx* c, int32_t* pdpdnum) {
   if (int rc = check_ctx(c)) return rc;
   if (!c->have_nbr) return set_err(c, A2C_ESTATE, "no neighbor lists");
+  A2C_HIP(c, hipStreamSynchronize(c->stream));
   if (c->desc.n_pd)
     A2C_HIP(c, hipMemcpy(pdpdnum, c->dpdpdnum, 12 * (size_t)c->desc.n_pd, hipMemcpyDeviceToHost));
   return A2C_OK;

@@ -1469,6 +1469,11 @@ int sync_lattice(a2c_fe_ctx* c, const double* dX, double* dG, double* dF) {
     new (c->hlat) LatDev();
     c->lat_dirty = true;
   }
+  if (!c->db2l) {  // all-zero block -> lattice map: site blocks, or owner units at any lanes per site
+    const size_t n = 4 * (size_t)(owner_units(c->N, MAX_LANES_PER_SITE) + 1);
+    A2C_HIP(c, dmalloc(&c->db2l, n));
+    A2C_HIP(c, hipMemsetAsync(c->db2l, 0, n, c->stream));
+  }
   LatDev& h = *c->hlat;
   const int kl32 = lanes_per_site(c->N, false), kl64 = lanes_per_site(c->N, true);
   if (!c->lat_dirty && h.X == dX && h.G == dG && h.f == dF && h.kl32 == kl32 && h.kl64 == kl64) return A2C_OK;

@@ -449,6 +449,14 @@ __device__ __forceinline__ void finish_objective(const LatDev& S, const RecvLane
   sum_parts<1>(S.part, 0, n, [&](int, double v) { *S.f = v; });
 }
 
+// What a neighbor build tells the host: the 14 maxima and the overflow flag of
+// the count pass (nbr.hip), list totals, squared largest displacement.
+struct NbrCounters {
+  int32_t max[16];
+  unsigned long long total[5];
+  double d2;
+};
+
 struct Timing;
 
 // a2c_fe_create on a stream of the caller's (a batch's own lattices share
@@ -486,6 +494,7 @@ struct a2c_fe_ctx {
   void* nb_order = nullptr;  // N double4: positions in cell order, site index in .w
   int* nb_cc = nullptr;      // cells + 1: cell starts
   int* nb_cursor = nullptr;  // cells + 1: histogram, then placement cursors
+  a2c::NbrCounters* nb_host = nullptr;  // pinned: the reduced counters
   int* nb_misc = nullptr;    // build counters (list widths, totals; copies per workgroup group), displacement, bounding box
   int64_t nb_cap_cells = 0;
   // skin lists: the pair lists at rc + skin and the positions they were built

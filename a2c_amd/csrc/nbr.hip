@@ -8,8 +8,8 @@
 // 0.75a^2 < d2 < 1.25a^2, else (minimizer.cpp:935-947); HH1 = H neighbors with
 // d2 < 0.75a^2 (:999-1004).
 //
-// Passes, all on the device (two host synchronisations: the list widths
-// after the count pass, the totals at the end):
+// Passes, all on the device (one host synchronisation, for the list widths after
+// the count pass; the caller's positions have been read by then):
 //   k_bin     cell of each site and the cell histogram
 //   k_scan    exclusive scan of the histogram (one workgroup)
 //   k_place   positions as floats in cell order, with the site index, so a
@@ -102,6 +102,12 @@ __global__ void k_place(const double* __restrict__ X, int N, Grid g, const int* 
                         __int_as_float(s));
 }
 
+// clears the cell histogram and the build's counters
+__global__ void k_clear(int* __restrict__ a, int na, int* __restrict__ b, int nb) {
+  for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < na + nb; i += gridDim.x * blockDim.x)
+    (i < na ? a[i] : b[i - na]) = 0;
+}
+
 struct NbrArgs {
   const double* X;
   const float4* qs;    // cell-ordered positions
@@ -126,7 +132,7 @@ struct NbrArgs {
   int32_t* maxw;       // 14 ints: width of the 5 lists, owned widths of the 4 pair lists, received
                        // widths, max total (count pass)
   int32_t* overflow;   // 1 if a site exceeds cap
-  unsigned long long* totals;  // entries of the 5 lists (fill pass)
+  unsigned long long* totals;  // entries of the 5 lists (count pass)
 };
 
 // Ownership of the unordered pair {s, j} (global site indices) in the
@@ -173,6 +179,29 @@ constexpr size_t MISC_TOT = SPREAD * 16 * sizeof(int32_t);
 constexpr size_t MISC_DMAX = MISC_TOT + SPREAD * 5 * sizeof(unsigned long long);
 constexpr size_t MISC_BBOX = MISC_DMAX + sizeof(unsigned long long);
 constexpr size_t MISC_BYTES = MISC_BBOX + 6 * sizeof(unsigned long long);
+// The copies reduced, one lane each, to pinned memory.
+__global__ __launch_bounds__(SPREAD) void k_counters(const int32_t* __restrict__ m,
+                                                     const unsigned long long* __restrict__ tot,
+                                                     const double* __restrict__ dmax, NbrCounters* out) {
+  const int c = threadIdx.x;
+#pragma unroll
+  for (int k = 0; k < 14; ++k) {
+    int v = m[c * 16 + k];
+    for (int off = SPREAD / 2; off > 0; off >>= 1) v = max(v, __shfl_xor(v, off));
+    if (c == 0) out->max[k] = v;
+  }
+#pragma unroll
+  for (int k = 0; k < 5; ++k) {
+    unsigned long long v = tot[c * 5 + k];
+    for (int off = SPREAD / 2; off > 0; off >>= 1) v += __shfl_xor(v, off);
+    if (c == 0) out->total[k] = v;
+  }
+  if (c == 0) {
+    out->max[14] = m[14];
+    out->max[15] = 0;
+    out->d2 = *dmax;
+  }
+}
 __device__ __forceinline__ int32_t* maxw_copy(int32_t* m) { return m + (blockIdx.x % SPREAD) * 16; }
 __device__ __forceinline__ unsigned long long* tot_copy(unsigned long long* t) { return t + (blockIdx.x % SPREAD) * 5; }
 
@@ -405,25 +434,25 @@ __global__ __launch_bounds__(ST) void k_site(NbrArgs a, int nblk_pd) {
       for (int k = 0; k < 14; ++k)
         if (v[k]) atomicMax(&mw[k], v[k]);
     }
+    // totals of the five lists: sums over the workgroup, one atomic each
+    unsigned long long tp = live ? npn : 0, th = live ? nhn : 0, t1 = live && !pdb ? n1 : 0;
+    for (int off = 32; off > 0; off >>= 1) {
+      tp += __shfl_xor(tp, off);
+      th += __shfl_xor(th, off);
+      t1 += __shfl_xor(t1, off);
+    }
+    if (lane == 0) {
+      unsigned long long* tt = tot_copy(a.totals);
+      atomicAdd(&tt[lp], tp);
+      atomicAdd(&tt[lh], th);
+      if (!pdb) atomicAdd(&tt[4], t1);
+    }
     return;
   }
   if (live && pdb) {
     a.pdpdnum[3 * (size_t)row] = counts[5][rl];
     a.pdpdnum[3 * (size_t)row + 1] = counts[6][rl];
     a.pdpdnum[3 * (size_t)row + 2] = npn - counts[5][rl] - counts[6][rl];
-  }
-  // totals of the five lists: sums over the workgroup, one atomic each
-  unsigned long long tp = live ? npn : 0, th = live ? nhn : 0, t1 = live && !pdb ? n1 : 0;
-  for (int off = 32; off > 0; off >>= 1) {
-    tp += __shfl_xor(tp, off);
-    th += __shfl_xor(th, off);
-    t1 += __shfl_xor(t1, off);
-  }
-  if (lane == 0) {
-    unsigned long long* tt = tot_copy(a.totals);
-    atomicAdd(&tt[lp], tp);
-    atomicAdd(&tt[lh], th);
-    if (!pdb) atomicAdd(&tt[4], t1);
   }
 }
 
@@ -756,20 +785,24 @@ __global__ void k_sdist(Ell L, const double* __restrict__ X, int s_off, int j_of
 
 namespace {
 
-// The counters of a build read back from the misc buffer (the first bytes
-// of it): maxima over the copies, the overflow flag, totals summed.
-void reduce_counters(const unsigned char* hb, size_t bytes, int hm[16], unsigned long long ht[5]) {
-  const int32_t* m = reinterpret_cast<const int32_t*>(hb);
-  for (int k = 0; k < 16; ++k) hm[k] = 0;
-  for (int c = 0; c < SPREAD; ++c)
-    for (int k = 0; k < 14; ++k) hm[k] = std::max(hm[k], m[c * 16 + k]);
-  hm[14] = m[14];
-  if (!ht || bytes < MISC_DMAX) return;
-  const unsigned long long* t = reinterpret_cast<const unsigned long long*>(hb + MISC_TOT);
-  for (int k = 0; k < 5; ++k) {
-    ht[k] = 0;
-    for (int c = 0; c < SPREAD; ++c) ht[k] += t[c * 5 + k];
-  }
+// The counters of a build on the host: c->nb_host, pinned, written by k_counters
+// and valid after a synchronisation.
+void read_counters(const a2c_fe_ctx* c, int hm[16], unsigned long long ht[5]) {
+  std::memcpy(hm, c->nb_host->max, sizeof(c->nb_host->max));
+  for (int k = 0; k < 5; ++k) ht[k] = c->nb_host->total[k];
+}
+int launch_counters(a2c_fe_ctx* c) {
+  const char* m = reinterpret_cast<const char*>(c->nb_misc);
+  hipLaunchKernelGGL(k_counters, dim3(1), dim3(SPREAD), 0, c->stream, c->nb_misc,
+                     reinterpret_cast<const unsigned long long*>(m + MISC_TOT),
+                     reinterpret_cast<const double*>(m + MISC_DMAX), c->nb_host);
+  A2C_HIP(c, hipGetLastError());
+  return A2C_OK;
+}
+int nbr_counters(a2c_fe_ctx* c) {  // the buffers of a build's counters
+  if (!c->nb_misc) A2C_HIP(c, dmalloc(&c->nb_misc, MISC_BYTES));
+  if (!c->nb_host) A2C_HIP(c, hmalloc(&c->nb_host, sizeof(NbrCounters)));
+  return A2C_OK;
 }
 
 // Device buffers of one set of five lists for rows of npd / nh sites: row
@@ -849,12 +882,12 @@ Grid box_grid(a2c_fe_ctx* c) {
 int walk_cells(a2c_fe_ctx* c, double rc, Ell* L5, bool halves, int hm[16], unsigned long long ht[5]) {
   const int N = c->N, npd = c->desc.n_pd, nh = c->desc.n_h;
   const int TB = 256;
-  // scratch (grow-only): misc = 16 ints (widths, overflow) + 5 totals + 6 bbox keys
+  // scratch (grow-only)
   if (!c->nb_cid) {
     A2C_HIP(c, dmalloc(&c->nb_cid, sizeof(int) * std::max(N, 1)));
     A2C_HIP(c, dmalloc(&c->nb_order, sizeof(float4) * std::max(N, 1)));  // cell-ordered positions
   }
-  if (!c->nb_misc) A2C_HIP(c, dmalloc(&c->nb_misc, MISC_BYTES));
+  if (int rc2 = nbr_counters(c)) return rc2;
   int* misc = c->nb_misc;
   unsigned long long* totals = reinterpret_cast<unsigned long long*>(reinterpret_cast<char*>(misc) + MISC_TOT);
   unsigned long long* bbox = reinterpret_cast<unsigned long long*>(reinterpret_cast<char*>(misc) + MISC_BBOX);
@@ -901,8 +934,12 @@ int walk_cells(a2c_fe_ctx* c, double rc, Ell* L5, bool halves, int hm[16], unsig
   }
   int *dcid = c->nb_cid, *dcc = c->nb_cc, *dcursor = c->nb_cursor;
   float4* qs = reinterpret_cast<float4*>(c->nb_order);
-  A2C_HIP(c, hipMemsetAsync(dcursor, 0, sizeof(int) * (ncell + 1), c->stream));  // the histogram
-  A2C_HIP(c, hipMemsetAsync(misc, 0, MISC_DMAX, c->stream));
+  {
+    const int nm = (int)(MISC_BBOX / sizeof(int)), n = (int)ncell + 1 + nm;
+    hipLaunchKernelGGL(k_clear, dim3(std::min((n + TB - 1) / TB, 1024)), dim3(TB), 0, c->stream, dcursor,
+                       (int)ncell + 1, misc, nm);
+    A2C_HIP(c, hipGetLastError());
+  }
   if (N > 0) {
     hipLaunchKernelGGL(k_bin, dim3((N + TB - 1) / TB), dim3(TB), 0, c->stream, c->dX, N, g, dcid, dcursor);
     A2C_HIP(c, hipGetLastError());
@@ -942,12 +979,9 @@ int walk_cells(a2c_fe_ctx* c, double rc, Ell* L5, bool halves, int hm[16], unsig
     hipLaunchKernelGGL(k_site<false>, dim3(nblk_pd + nblk_h), dim3(ST), 0, c->stream, a, nblk_pd);
     A2C_HIP(c, hipGetLastError());
   }
-  {
-    std::vector<unsigned char> hb(MISC_TOT);
-    A2C_HIP(c, hipMemcpyAsync(hb.data(), misc, MISC_TOT, hipMemcpyDeviceToHost, c->stream));
-    A2C_HIP(c, hipStreamSynchronize(c->stream));
-    reduce_counters(hb.data(), MISC_TOT, hm, nullptr);
-  }
+  if (int rc2 = launch_counters(c)) return rc2;
+  A2C_HIP(c, hipStreamSynchronize(c->stream));
+  read_counters(c, hm, ht);
   if (hm[14]) return A2C_ENBR_OVERFLOW;
   if (int rc2 = size_lists(c, L5, hm, halves ? hm + 5 : nullptr, hm + 9)) return rc2;
   for (int w = 0; w < 5; ++w) {
@@ -970,16 +1004,6 @@ int walk_cells(a2c_fe_ctx* c, double rc, Ell* L5, bool halves, int hm[16], unsig
   }
   if (halves)
     if (int rc2 = reverse_slots(c, L5, hm + 9, nullptr)) return rc2;
-  {
-    std::vector<unsigned long long> tb(SPREAD * 5);
-    A2C_HIP(c, hipMemcpyAsync(tb.data(), totals, sizeof(unsigned long long) * tb.size(), hipMemcpyDeviceToHost,
-                              c->stream));
-    A2C_HIP(c, hipStreamSynchronize(c->stream));
-    for (int k = 0; k < 5; ++k) {
-      ht[k] = 0;
-      for (int cp = 0; cp < SPREAD; ++cp) ht[k] += tb[cp * 5 + k];
-    }
-  }
   return A2C_OK;
 }
 
@@ -1022,7 +1046,8 @@ int refresh(a2c_fe_ctx* c, bool check, int hm[16], unsigned long long ht[5], dou
   int* misc = c->nb_misc;
   unsigned long long* totals = reinterpret_cast<unsigned long long*>(reinterpret_cast<char*>(misc) + MISC_TOT);
   unsigned long long* dmax = reinterpret_cast<unsigned long long*>(reinterpret_cast<char*>(misc) + MISC_DMAX);
-  A2C_HIP(c, hipMemsetAsync(misc, 0, MISC_BBOX, c->stream));
+  hipLaunchKernelGGL(k_clear, dim3(8), dim3(256), 0, c->stream, misc, (int)(MISC_BBOX / sizeof(int)), misc, 0);
+  A2C_HIP(c, hipGetLastError());
   if (!c->dpdpdnum) A2C_HIP(c, dmalloc(&c->dpdpdnum, sizeof(int32_t) * 3 * std::max(npd, 1)));
   const Grid g = box_grid(c);
   if (check && N > 0) {
@@ -1054,13 +1079,10 @@ int refresh(a2c_fe_ctx* c, bool check, int hm[16], unsigned long long ht[5], dou
     A2C_HIP(c, hipGetLastError());
   }
   if (int rc = reverse_slots(c, c->ell, rw, misc)) return rc;  // rw + 1 slots are allocated
-  std::vector<unsigned char> hb(MISC_BBOX);
-  A2C_HIP(c, hipMemcpyAsync(hb.data(), misc, MISC_BBOX, hipMemcpyDeviceToHost, c->stream));
+  if (int rc = launch_counters(c)) return rc;
   A2C_HIP(c, hipStreamSynchronize(c->stream));
-  reduce_counters(hb.data(), MISC_BBOX, hm, ht);
-  double d2;
-  std::memcpy(&d2, hb.data() + MISC_DMAX, sizeof(d2));
-  *maxd = std::sqrt(d2);
+  read_counters(c, hm, ht);
+  *maxd = std::sqrt(c->nb_host->d2);
   for (int k = 0; k < 5; ++k) {
     c->ell[k].width = hm[k];
     if (k < 4) {
@@ -1094,7 +1116,7 @@ int nbr_build(a2c_fe_ctx* c) {
   unsigned long long ht[5] = {0, 0, 0, 0, 0};
   bool refreshed = false;
   double maxd = 0.0;
-  if (!c->nb_misc) A2C_HIP(c, dmalloc(&c->nb_misc, MISC_BYTES));
+  if (int rc2 = nbr_counters(c)) return rc2;
   if (c->nb_sup_ok) {
     if (int rc2 = refresh(c, true, hm, ht, &maxd)) return rc2;
     refreshed = 2.0 * maxd < skin * (1.0 - 1e-9);  // else the filtered lists may miss a pair
