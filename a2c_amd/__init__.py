@@ -457,13 +457,13 @@ class FreeEntropy:
 
     def density(self, X):
         X = _f64(X, 4 * self.N)
-        rho = np.zeros(max(self.N, 1))
+        rho = np.empty(max(self.N, 1))
         self._check(lib.a2c_fe_density(self._ctx, _dptr(X), _dptr(rho)))
         return rho[: self.N]
 
     def formFunctionAndGradient(self, X):
         X = _f64(X, 4 * self.N)
-        G = np.zeros(max(4 * self.N, 1))
+        G = np.empty(max(4 * self.N, 1))  # filled by the call
         f = C.c_double()
         self._check(lib.a2c_fe_eval(self._ctx, _dptr(X), C.byref(f), _dptr(G)))
         return f.value, G[: 4 * self.N]
@@ -503,7 +503,7 @@ class FreeEntropy:
         for k, v in opts.items():
             setattr(o, k, v)
         X0 = _f64(X0, 4 * self.N)
-        Xo = np.zeros_like(X0)
+        Xo = np.empty_like(X0)
         rep = LmvmReport()
         self._check(lib.a2c_fe_minimize(self._ctx, _dptr(X0), C.byref(o), _dptr(Xo), C.byref(rep)))
         return Xo, {k: getattr(rep, k) for k, _ in LmvmReport._fields_}
@@ -726,7 +726,7 @@ class Batch:
 
     def get_state(self, slot):
         n = 4 * self.sizes[slot]
-        X, G = np.zeros(n), np.zeros(n)
+        X, G = np.empty(n), np.empty(n)
         self._check(lib.a2c_batch_get_state(self._b, slot, _dptr(X), _dptr(G)))
         return X, G
 
