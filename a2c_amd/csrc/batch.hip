@@ -1313,6 +1313,7 @@ int fused_eval(a2c_batch* b, const std::vector<int>& ids_in, bool fp64, StateOf 
   std::vector<LatDev> lats(ids.size());
   std::vector<int32_t> map, omap;  // site block -> lattice; pair-owner workgroup -> lattice
   int cum = 0, ocum = 0, rules = 0, rq = 1;
+  bool empty = false;
   for (size_t k = 0; k < ids.size(); ++k) {
     Slot& s = b->slots[ids[k]];
     LatDev L = s.fe->sys();
@@ -1331,6 +1332,7 @@ int fused_eval(a2c_batch* b, const std::vector<int>& ids_in, bool fp64, StateOf 
     lats[k] = L;
     const int nb = lattice_blocks(s.N());
     rq = std::max(rq, (int)L.rl);
+    empty |= s.N() == 0;
     map.insert(map.end(), nb, (int32_t)k);
     const int no = owner_units(L.npd, L.nh, kl);
     omap.insert(omap.end(), (size_t)no, (int32_t)k);
@@ -1350,6 +1352,7 @@ int fused_eval(a2c_batch* b, const std::vector<int>& ids_in, bool fp64, StateOf 
   L.b2l = dm;
   L.nblk = cum;
   L.rq = rq;
+  L.empty = empty;
   L.ob2l = dom;
   L.onblk = ocum;
   L.nlat = (int)ids.size();

@@ -605,7 +605,7 @@ struct Pair32 {
   float d[3], bs;
 };
 
-template <int RULE, bool NB_H, bool ME_H>
+template <int RULE, bool BY_SITE, bool NB_H, bool ME_H>
 __device__ __forceinline__ void dens_list(const float4* tab, const LatDev& S, const OwnerLane& ln, const Site& a,
                                           const Image& img, double wme, double& rho) {
   const Ell& L = ME_H ? (NB_H ? S.hh : S.hpd) : (NB_H ? S.pdh : S.pdpd);
@@ -613,7 +613,7 @@ __device__ __forceinline__ void dens_list(const float4* tab, const LatDev& S, co
   A2C_GLOBAL float* __restrict__ prb = gmem(reinterpret_cast<float*>(P.rbuf));
   const size_t prows = P.rows;
   const float as = (float)a.s;
-  owned_pairs<NB_H>(
+  owned_pairs<NB_H, BY_SITE>(
       L, ln, S.kl32, S, [](int) { return 0.0f; },
       [&](const Site& b) {
         Pair32 p;
@@ -635,7 +635,7 @@ __device__ __forceinline__ void dens_list(const float4* tab, const LatDev& S, co
 // rules' node blocks without spills.  40^3 cells, 12-point / Gauss-Hermite rule:
 // 214 / 340 us with tables in |r|, sites in lattice order and the loads of a
 // pair in its own turn, 147 / 255 us as it is.
-template <int RULE>
+template <int RULE, bool BY_SITE>
 __global__ __launch_bounds__(TB) __attribute__((amdgpu_waves_per_eu(6))) void k_dens_own(
     const LatDev* __restrict__ lats, const int32_t* __restrict__ ob2l, const float4* __restrict__ gtab) {
   __shared__ float4 tab[SNT];  // f_Pd (f_H is evaluated directly)
@@ -649,15 +649,15 @@ __global__ __launch_bounds__(TB) __attribute__((amdgpu_waves_per_eu(6))) void k_
   if (ln.row >= ln.rows) return;  // whole lane groups
   const Image img = image_of(S);
   const int s = ln.pd ? ln.row : S.npd + ln.row;
-  const Site a = load_row(gmem((const double2*)S.qxy), gmem((const double2*)S.qzs), s);
+  double wme;
+  const Site a = own_site<BY_SITE>(S, ln, wme);
   double rho = 0.0;
   if (ln.pd) {
-    dens_list<RULE, false, false>(tab, S, ln, a, img, 1.0, rho);
-    dens_list<RULE, true, false>(tab, S, ln, a, img, 1.0, rho);
+    dens_list<RULE, BY_SITE, false, false>(tab, S, ln, a, img, 1.0, rho);
+    dens_list<RULE, BY_SITE, true, false>(tab, S, ln, a, img, 1.0, rho);
   } else {
-    const double wme = gmem((const double*)S.xrow)[ln.row];
-    dens_list<RULE, false, true>(tab, S, ln, a, img, wme, rho);
-    dens_list<RULE, true, true>(tab, S, ln, a, img, wme, rho);
+    dens_list<RULE, BY_SITE, false, true>(tab, S, ln, a, img, wme, rho);
+    dens_list<RULE, BY_SITE, true, true>(tab, S, ln, a, img, wme, rho);
   }
   rho = site_sum(rho, K);
   if (ln.ph == 0) gmem(S.rho)[s] = rho;
@@ -1133,13 +1133,18 @@ int run_eval32(const Launch& L, Timing* tm) {
       if (hipGetLastError() != hipSuccess) return A2C_EHIP;
     }
   } else if (L.nblk > 0) {
-    if (tm) tm->mark(L.stream, "rows");
-    if (run_rows(L)) return A2C_EHIP;
+    const bool fold = fold_rows(L);
+    if (!fold) {
+      if (tm) tm->mark(L.stream, "rows");
+      if (run_rows(L)) return A2C_EHIP;
+    }
     if (tm) tm->mark(L.stream, "dens_own");
+    auto own = [&](auto kernel) {
+      hipLaunchKernelGGL(kernel, dim3(L.onblk), dim3(TB), 0, L.stream, L.lats, L.ob2l, L.tab);
+    };
     if (L.onblk > 0 && (L.rules & (1 << A2C_QUAD_R12)))
-      hipLaunchKernelGGL(k_dens_own<A2C_QUAD_R12>, dim3(L.onblk), dim3(TB), 0, L.stream, L.lats, L.ob2l, L.tab);
-    if (L.onblk > 0 && (L.rules & (1 << GH3)))
-      hipLaunchKernelGGL(k_dens_own<GH3>, dim3(L.onblk), dim3(TB), 0, L.stream, L.lats, L.ob2l, L.tab);
+      fold ? own(k_dens_own<A2C_QUAD_R12, true>) : own(k_dens_own<A2C_QUAD_R12, false>);
+    if (L.onblk > 0 && (L.rules & (1 << GH3))) fold ? own(k_dens_own<GH3, true>) : own(k_dens_own<GH3, false>);
     if (hipGetLastError() != hipSuccess) return A2C_EHIP;
     if (tm) tm->mark(L.stream, "dens_recv");
     hipLaunchKernelGGL(k_dens_recv, dim3(L.nblk * L.rq), dim3(TB), 0, L.stream, L.lats, L.b2l, L.rq);

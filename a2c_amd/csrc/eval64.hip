@@ -589,7 +589,7 @@ __device__ __forceinline__ bool pair_inside(const double d[3], double si, double
 struct Pair64 {
   double d[3], s;
 };
-template <int RULE, bool NB_H, bool ME_H>
+template <int RULE, bool BY_SITE, bool NB_H, bool ME_H>
 __device__ __forceinline__ void dens_list(const double* tab, const double* exptab, const LatDev& S,
                                           const OwnerLane& ln, const Site& a, const Image& img, double wme,
                                           double& rho) {
@@ -598,7 +598,7 @@ __device__ __forceinline__ void dens_list(const double* tab, const double* expta
   A2C_GLOBAL double* __restrict__ share = gmem(reinterpret_cast<double*>(P.rbuf));
   const size_t prows = P.rows;
   bool far = false;
-  owned_pairs<NB_H>(
+  owned_pairs<NB_H, BY_SITE>(
       L, ln, S.kl64, S, [](int) { return 0.0f; },
       [&](const Site& b) {
         Pair64 p;
@@ -614,20 +614,21 @@ __device__ __forceinline__ void dens_list(const double* tab, const double* expta
         share[(size_t)rv * prows + jl] = ME_H ? wme * theirs : theirs;
       });
   if (far)
-    far_pairs<NB_H>(L, ln, S.kl64, S, [&](int jl, int rv, int j) {
-      const Site b = load_row(gmem((const double2*)S.qxy), gmem((const double2*)S.qzs), j);
+    far_pairs<NB_H>(L, ln, S.kl64, S, [&](int jl, int rv, int) {
+      const RowState<BY_SITE, NB_H> st(S);
+      const Site b = st.site(jl);
       double d[3];
       pair_vec(img, a, b, d);
       if (pair_inside<RULE>(d, a.s, b.s)) return;
       const double2 v = closed_dens<RULE>(d, a.s, b.s);
-      rho += (NB_H ? S.xrow[jl] : 1.0) * (NB_H ? v.y : v.x);
+      rho += (NB_H ? st.occ(jl) : 1.0) * (NB_H ? v.y : v.x);
       share[(size_t)rv * prows + jl] = wme * (ME_H ? v.y : v.x);
     });
 }
 
 // Bound by the LDS and the vector ALUs (40^3 cells: 60% and 75% busy): 654 us
 // with the tables in |r|, 276 us; Gauss-Hermite rule 1386 and 604 us.
-template <int RULE, int TBO>
+template <int RULE, int TBO, bool BY_SITE>
 __global__ __launch_bounds__(TBO) __attribute__((amdgpu_waves_per_eu(4))) void k_dens_own64(
     const LatDev* __restrict__ lats, const int32_t* __restrict__ ob2l, int nblk, const double* __restrict__ gtab) {
   __shared__ __align__(16) double tab[S_ROWS + EXPN];  // f_Pd, 2^(i/256)
@@ -643,15 +644,15 @@ __global__ __launch_bounds__(TBO) __attribute__((amdgpu_waves_per_eu(4))) void k
   if (ln.row >= ln.rows) return;  // whole lane groups
   const Image img = image_of(S);
   const int s = ln.pd ? ln.row : S.npd + ln.row;
-  const Site a = load_row(gmem((const double2*)S.qxy), gmem((const double2*)S.qzs), s);
+  double wme;
+  const Site a = own_site<BY_SITE>(S, ln, wme);
   double rho = 0.0;
   if (ln.pd) {
-    dens_list<RULE, false, false>(tab, tab + S_ROWS, S, ln, a, img, 1.0, rho);
-    dens_list<RULE, true, false>(tab, tab + S_ROWS, S, ln, a, img, 1.0, rho);
+    dens_list<RULE, BY_SITE, false, false>(tab, tab + S_ROWS, S, ln, a, img, 1.0, rho);
+    dens_list<RULE, BY_SITE, true, false>(tab, tab + S_ROWS, S, ln, a, img, 1.0, rho);
   } else {
-    const double wme = gmem((const double*)S.xrow)[ln.row];
-    dens_list<RULE, false, true>(tab, tab + S_ROWS, S, ln, a, img, wme, rho);
-    dens_list<RULE, true, true>(tab, tab + S_ROWS, S, ln, a, img, wme, rho);
+    dens_list<RULE, BY_SITE, false, true>(tab, tab + S_ROWS, S, ln, a, img, wme, rho);
+    dens_list<RULE, BY_SITE, true, true>(tab, tab + S_ROWS, S, ln, a, img, wme, rho);
   }
   rho = site_sum(rho, K);
   if (ln.ph == 0) gmem(S.epair)[s] = rho;  // free until the gradient pass
@@ -1209,7 +1210,19 @@ int owners(const Launch& L) {
 // pass) the units go to workgroups of their own; beyond, two to a workgroup, so
 // that a CU holds 8 waves on one copy of the tables.
 constexpr int GRAD_WIDE_UNITS = 256, DENS_WIDE_UNITS = 512;
-template <int R, int T> struct DensOwn { static constexpr auto fn = k_dens_own64<R, T>; };
+template <int R, int T> struct DensOwn { static constexpr auto fn = k_dens_own64<R, T, false>; };
+template <int R, int T> struct DensOwnFold { static constexpr auto fn = k_dens_own64<R, T, true>; };
+// the row-order copies and the density pass
+int run_dens_own(const Launch& L, Timing* tm) {
+  const bool fold = fold_rows(L), wide = L.onblk > DENS_WIDE_UNITS;
+  if (!fold) {
+    if (tm) tm->mark(L.stream, "rows");
+    if (run_rows(L)) return A2C_EHIP;
+  }
+  if (tm) tm->mark(L.stream, "dens_own64");
+  if (fold) return wide ? owners<DensOwnFold, 512>(L) : owners<DensOwnFold, 256>(L);
+  return wide ? owners<DensOwn, 512>(L) : owners<DensOwn, 256>(L);
+}
 template <int R, int T> struct GradOwn { static constexpr auto fn = k_grad_own64<R, T>; };
 }  // namespace
 
@@ -1222,10 +1235,7 @@ static int run_density64(const Launch& L) {
 int run_eval64(const Launch& L, Timing* tm) {
   if (L.deriv_mode == A2C_DERIV_ANALYTIC && !L.full_pairs64) {
     if (L.nblk > 0) {
-      if (tm) tm->mark(L.stream, "rows");
-      if (run_rows(L)) return A2C_EHIP;
-      if (tm) tm->mark(L.stream, "dens_own64");
-      if (L.onblk > DENS_WIDE_UNITS ? owners<DensOwn, 512>(L) : owners<DensOwn, 256>(L)) return A2C_EHIP;
+      if (run_dens_own(L, tm)) return A2C_EHIP;
       if (tm) tm->mark(L.stream, "dens_recv64");
       hipLaunchKernelGGL(k_dens_recv64<A2C_DERIV_ANALYTIC>, dim3(L.nblk * L.rq), dim3(TB), 0, L.stream, L.lats, L.b2l,
                          L.rq, 0.0, 0);
@@ -1253,6 +1263,7 @@ int run_eval64(const Launch& L, Timing* tm) {
   return A2C_OK;
 }
 
+bool fold_rows(const Launch& L) { return L.nblk <= FOLD_BLOCKS && !L.empty; }
 int run_rows(const Launch& L) {
   hipLaunchKernelGGL(k_rows, dim3(L.nblk), dim3(TB), 0, L.stream, L.lats, L.b2l);
   return hipGetLastError() == hipSuccess ? A2C_OK : A2C_EHIP;
@@ -1402,6 +1413,7 @@ static Launch single_launch(a2c_fe_ctx* c, bool fp64) {
   L.onblk = owner_units(c->desc.n_pd, c->desc.n_h, lanes_per_site(c->N, fp64));
   L.nblk = lattice_blocks(c->N);
   L.rq = recv_lanes(c->N);
+  L.empty = c->N == 0;
   L.nlat = 1;
   L.rules = 1 << c->desc.quad_rule;
   L.stream = c->stream;
@@ -1418,7 +1430,7 @@ int launch_density64(a2c_fe_ctx* c, const double* dX, bool by_site) {
   if (c->gen_on) return launch_density_gen(c, dX);
   if (int rc = sync_lattice(c, dX, c->dG, c->dF)) return rc;
   const Launch L = single_launch(c, true);
-  if (run_rows(L) || (L.onblk > DENS_WIDE_UNITS ? owners<DensOwn, 512>(L) : owners<DensOwn, 256>(L)))
+  if (run_dens_own(L, nullptr))
     return set_err(c, A2C_EHIP, "density64 launch failed");
   hipLaunchKernelGGL(L.deriv_mode == A2C_DERIV_FD ? k_dens_recv64<A2C_DERIV_FD> : k_dens_recv64<A2C_DERIV_ANALYTIC>,
                      dim3(L.nblk * L.rq), dim3(TB), 0, L.stream, L.lats, L.b2l, L.rq, L.fd_eps, (int)by_site);

@@ -262,7 +262,7 @@ __global__ __launch_bounds__(TB) void k_gen_rows(const LatDev* __restrict__ lat)
 }
 
 // ------------------------------------------------------------ density
-template <int POT, class R, bool NB_H, bool ME_H>
+template <int POT, class R, bool BY_SITE, bool NB_H, bool ME_H>
 __device__ __forceinline__ void dens_list(const LatDev& S, const GenDev& g, const RFun<POT, R>& fun, const R* nd,
                                           const OwnerLane& ln, int KL, const Site& a, const Image& img, double wme,
                                           double& rho) {
@@ -271,7 +271,7 @@ __device__ __forceinline__ void dens_list(const LatDev& S, const GenDev& g, cons
   const Ell& P = ME_H ? (NB_H ? S.hh : S.pdh) : (NB_H ? S.hpd : S.pdpd);  // partner rows
   A2C_GLOBAL double* __restrict__ share = gmem(reinterpret_cast<double*>(P.rbuf));
   const size_t prows = P.rows;
-  owned_pairs<NB_H>(
+  owned_pairs<NB_H, BY_SITE>(
       L, ln, KL, S, [](int) { return 0.0f; }, [&](const Site& b) { return gen_pair(img, a, b); },
       [&](const GenPair& p, float, double wj, int jl, int rv) {
         const PairFrame<R> f = frame<R>(g, p.d, a.s, p.s);
@@ -296,7 +296,7 @@ __device__ __forceinline__ void dens_list(const LatDev& S, const GenDev& g, cons
 // gathers (two 16-byte words per function) touch a line per lane.  5^3 cells (memory
 // latency): 62 us with a branch around the table's end, 52 without, 41 with two
 // nodes in flight; more nodes only take registers.
-template <int POT, class R>
+template <int POT, class R, bool BY_SITE>
 __global__ __launch_bounds__(TB) void k_gen_dens_own(const LatDev* __restrict__ lat, GenDev g, int KL) {
   const R* nd = stage_nodes<R>(g);
   const LatDev& S = *lat;
@@ -305,15 +305,15 @@ __global__ __launch_bounds__(TB) void k_gen_dens_own(const LatDev* __restrict__ 
   const RFun<POT, R> fun(g);
   const Image img = image_of(S);
   const int s = ln.pd ? ln.row : S.npd + ln.row;
-  const Site a = load_row(gmem((const double2*)S.qxy), gmem((const double2*)S.qzs), s);
+  double wme;
+  const Site a = own_site<BY_SITE>(S, ln, wme);
   double rho = 0.0;
   if (ln.pd) {
-    dens_list<POT, R, false, false>(S, g, fun, nd, ln, KL, a, img, 1.0, rho);
-    dens_list<POT, R, true, false>(S, g, fun, nd, ln, KL, a, img, 1.0, rho);
+    dens_list<POT, R, BY_SITE, false, false>(S, g, fun, nd, ln, KL, a, img, 1.0, rho);
+    dens_list<POT, R, BY_SITE, true, false>(S, g, fun, nd, ln, KL, a, img, 1.0, rho);
   } else {
-    const double wme = gmem((const double*)S.xrow)[ln.row];
-    dens_list<POT, R, false, true>(S, g, fun, nd, ln, KL, a, img, wme, rho);
-    dens_list<POT, R, true, true>(S, g, fun, nd, ln, KL, a, img, wme, rho);
+    dens_list<POT, R, BY_SITE, false, true>(S, g, fun, nd, ln, KL, a, img, wme, rho);
+    dens_list<POT, R, BY_SITE, true, true>(S, g, fun, nd, ln, KL, a, img, wme, rho);
   }
   rho = site_sum(rho, KL);
   if (ln.ph == 0) gmem(S.epair)[s] = rho;
@@ -546,7 +546,8 @@ auto pick(const GenDev& g, int deriv_mode, bool fp32) {
   if (fp32) return tab ? Pick<1, A2C_DERIV_ANALYTIC, float>::fn : Pick<0, A2C_DERIV_ANALYTIC, float>::fn;
   return tab ? Pick<1, A2C_DERIV_ANALYTIC, double>::fn : Pick<0, A2C_DERIV_ANALYTIC, double>::fn;
 }
-template <int P, int D, class R> struct DensK { static constexpr auto fn = k_gen_dens_own<P, R>; };
+template <int P, int D, class R> struct DensK { static constexpr auto fn = k_gen_dens_own<P, R, false>; };
+template <int P, int D, class R> struct DensFoldK { static constexpr auto fn = k_gen_dens_own<P, R, true>; };
 template <int P, int D, class R> struct RecvK { static constexpr auto fn = k_gen_dens_recv<P, D>; };
 template <int P, int D, class R> struct GradK { static constexpr auto fn = k_gen_grad_own<P, D, R>; };
 
@@ -560,11 +561,14 @@ int run_density_gen(const LatDev* dlat, int npd, int nh, const GenDev& g, int de
                     bool by_site, hipStream_t st, Timing* tm) {
   if (npd + nh <= 0) return A2C_OK;
   const int nblk = site_blocks(npd + nh), KL = lanes_per_site(npd + nh, true);
-  if (tm) tm->mark(st, "rows");
-  hipLaunchKernelGGL(k_gen_rows, dim3(nblk), dim3(TB), 0, st, dlat);
+  const bool fold = nblk <= FOLD_BLOCKS;
+  if (!fold) {
+    if (tm) tm->mark(st, "rows");
+    hipLaunchKernelGGL(k_gen_rows, dim3(nblk), dim3(TB), 0, st, dlat);
+  }
   if (tm) tm->mark(st, "gen_dens_own");
-  hipLaunchKernelGGL(pick<DensK>(g, deriv_mode, fp32), dim3(owner_units(npd, nh, KL)), dim3(TB),
-                     lds_bytes(g, deriv_mode, fp32), st, dlat, g, KL);
+  hipLaunchKernelGGL(fold ? pick<DensFoldK>(g, deriv_mode, fp32) : pick<DensK>(g, deriv_mode, fp32),
+                     dim3(owner_units(npd, nh, KL)), dim3(TB), lds_bytes(g, deriv_mode, fp32), st, dlat, g, KL);
   if (tm) tm->mark(st, "gen_dens_recv");
   hipLaunchKernelGGL(pick<RecvK>(g, deriv_mode, fp32), dim3(nblk * recv_lanes(npd + nh)), dim3(TB), 0, st, dlat, g, eps, (int)by_site);
   return hipGetLastError() == hipSuccess ? A2C_OK : A2C_EHIP;

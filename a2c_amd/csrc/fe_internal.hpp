@@ -600,6 +600,7 @@ struct Launch {
   int onblk = 0;                  // pair-owner workgroups
   bool mixed_full = false;    // mixed path: every pair from both ends (A/B reference)
   bool full_pairs64 = false;  // FP64 analytic path: every pair from both ends (A/B reference)
+  bool empty = false;         // some lattice of the launch has no sites
   int rules = 1;              // bit r set: some lattice of the launch uses quadrature rule r
 };
 bool mixed_full_pairs();  // A2C_MIXED_PAIRS=full selects the both-ends kernels
@@ -607,6 +608,7 @@ bool fp64_full_pairs();   // A2C_FP64_PAIRS=full likewise for the FP64 kernels
 int run_eval64(const Launch& L, Timing* tm);
 int run_eval32(const Launch& L, Timing* tm);
 int run_final_sum(const Launch& L);
+bool fold_rows(const Launch& L);  // the density pass makes the row-order copies itself (pair_rows.hpp)
 int run_rows(const Launch& L);  // row-order copies of state and occupancy (pair-once evaluation)
 int sync_lattice(a2c_fe_ctx* c, const double* dX, double* dG, double* dF);  // refresh the one-lattice descriptor
 int launch_eval64(a2c_fe_ctx* c, const double* dX, double* dG, double* dF, bool timed, Timing* tm);
