@@ -1269,8 +1269,9 @@ int seg_bound(a2c_batch* b, const std::vector<int>& ids, Fill fill) {
 // A slot whose context has a general model (a tabulated potential or a node
 // table: a2c_fe_set_potential_*, a2c_fe_set_quadrature) is evaluated by the
 // general kernels, on its own; the fused launch takes the others.
+// slopes: also G . q of every slot, into its first double of hres (slopes_in_eval).
 template <class StateOf>
-int gen_eval(a2c_batch* b, int id, bool fp64, StateOf state_of) {
+int gen_eval(a2c_batch* b, int id, bool fp64, bool slopes, StateOf state_of) {
   Slot& s = b->slots[id];
   LatDev L = s.fe->sys();
   const double* X;
@@ -1279,6 +1280,7 @@ int gen_eval(a2c_batch* b, int id, bool fp64, StateOf state_of) {
   L.X = X;
   L.G = G;
   L.f = b->hF + id;
+  if (slopes) L.w = s.q, L.slope = b->hres + 2 * id;
   if (b->arena.used + 256 + sizeof(LatDev) > b->arena.cap)
     if (int rc = bsync(b)) return rc;
   LatDev* dl = b->arena.push(&L, 1);
@@ -1296,13 +1298,19 @@ int gen_eval(a2c_batch* b, int id, bool fp64, StateOf state_of) {
   return A2C_OK;
 }
 
+// The pair-once evaluations can sum G . q as they write G; central differences and
+// the both-ends kernels leave it to a pass of its own.
+bool slopes_in_eval(const a2c_batch* b) {
+  return b->desc.deriv_mode == A2C_DERIV_ANALYTIC && !mixed_full_pairs() && !fp64_full_pairs();
+}
 template <class StateOf>
-int fused_eval(a2c_batch* b, const std::vector<int>& ids_in, bool fp64, StateOf state_of, bool sync = true) {
+int fused_eval(a2c_batch* b, const std::vector<int>& ids_in, bool fp64, StateOf state_of, bool sync = true,
+               bool slopes = false) {
   std::vector<int> ids;
   for (int i : ids_in) {
     if (!b->slots[i].fe->gen_on) {
       ids.push_back(i);
-    } else if (int rc = gen_eval(b, i, fp64, state_of)) {
+    } else if (int rc = gen_eval(b, i, fp64, slopes, state_of)) {
       return rc;
     }
   }
@@ -1324,6 +1332,7 @@ int fused_eval(a2c_batch* b, const std::vector<int>& ids_in, bool fp64, StateOf 
     L.X = X;
     L.G = G;
     L.f = b->hF + ids[k];
+    if (slopes) L.w = s.q, L.slope = b->hres + 2 * ids[k];
     L.blk0 = cum;
     L.kl32 = lanes_per_site(s.N(), false);
     L.kl64 = lanes_per_site(s.N(), true);
@@ -1429,7 +1438,7 @@ int converged_reason(const Slot& s) {
 // evaluate f, g at x for the listed slots, each in its own precision; with
 // sync = false the launches are only enqueued (after the caller's next
 // synchronising step take_f reads the objectives)
-int eval_slots(a2c_batch* b, const std::vector<int>& ids, bool sync = true) {
+int eval_slots(a2c_batch* b, const std::vector<int>& ids, bool sync = true, bool slopes = false) {
   std::vector<int> m32, m64;
   for (int i : ids) {
     Slot& s = b->slots[i];
@@ -1437,8 +1446,8 @@ int eval_slots(a2c_batch* b, const std::vector<int>& ids, bool sync = true) {
     s.rep.evals++;
     if (!s.mixed) s.rep.evals_fp64++;
   }
-  if (int rc = fused_eval(b, m32, false, lmvm_state, false)) return rc;
-  if (int rc = fused_eval(b, m64, true, lmvm_state, false)) return rc;
+  if (int rc = fused_eval(b, m32, false, lmvm_state, false, slopes)) return rc;
+  if (int rc = fused_eval(b, m64, true, lmvm_state, false, slopes)) return rc;
   if (!sync) return A2C_OK;
   if (int rc = bsync(b)) return rc;
   for (int i : ids) b->slots[i].f = b->hF[i];
@@ -1683,8 +1692,16 @@ int lmvm_iteration(a2c_batch* b, std::vector<int>& act) {
           o.lb = s.opts.sigma_lb; o.ub = s.opts.sigma_ub; o.stp = s.stp;
         }))
       return rc;
-    if (int rc = eval_slots(b, run, false)) return rc;  // f and the slope come back in one round trip
-    if (int rc = seg_dot(b, run, [](SegDot& o, Slot& s) { o.a1 = s.g; o.b1 = s.q; }, v)) return rc;
+    // f and the slope along the realised direction come back in one round trip
+    const bool slopes = slopes_in_eval(b);
+    if (int rc = eval_slots(b, run, false, slopes)) return rc;
+    if (slopes) {
+      if (int rc = bsync(b)) return rc;
+      v.resize(2 * run.size());
+      for (size_t k = 0; k < run.size(); ++k) v[2 * k] = b->hres[2 * run[k]];
+    } else if (int rc = seg_dot(b, run, [](SegDot& o, Slot& s) { o.a1 = s.g; o.b1 = s.q; }, v)) {
+      return rc;
+    }
     take_f(b, run);
     std::vector<int> next;
     for (size_t k = 0; k < run.size(); ++k) {

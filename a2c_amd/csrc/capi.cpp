@@ -119,7 +119,7 @@ int a2c::fe_create(const a2c_fe_desc* desc, hipStream_t shared, a2c_fe_ctx** out
   bool ok = dmalloc(&c->dX, 32 * N) == hipSuccess && dmalloc(&c->dG, 32 * N) == hipSuccess &&
             dmalloc(&c->dx, 8 * nh) == hipSuccess && dmalloc(&c->drho, 8 * N) == hipSuccess &&
             dmalloc(&c->dFp, 8 * N) == hipSuccess && dmalloc(&c->demb, 8 * N) == hipSuccess &&
-            dmalloc(&c->dpart, 8 * (RECV_LANES * (size_t)c->nblk_red + 1)) == hipSuccess && hmalloc(&c->dF, 64) == hipSuccess &&
+            dmalloc(&c->dpart, 8 * (2 * RECV_LANES * (size_t)c->nblk_red + 1)) == hipSuccess && hmalloc(&c->dF, 64) == hipSuccess &&
             dmalloc(&c->dlat, sizeof(LatDev)) == hipSuccess &&
             dmalloc(&c->dqxy, 16 * N) == hipSuccess && dmalloc(&c->dqzs, 16 * N) == hipSuccess &&
             dmalloc(&c->dxrow, 8 * nh) == hipSuccess && dmalloc(&c->dgown, 32 * N) == hipSuccess;

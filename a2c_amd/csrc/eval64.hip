@@ -960,7 +960,7 @@ __global__ __launch_bounds__(TB) void k_grad_recv64(const LatDev* __restrict__ l
   const RecvLane ln(S, blk - S.blk0, v % rq);
   if (ln.idle) return;
   const int s = ln.s;
-  double fs = 0.0;
+  double fs = 0.0, sl = 0.0;
   if (s < S.npd + S.nh) {
     const double* __restrict__ xo = S.xrow;
     const bool pd = s < S.npd;
@@ -989,14 +989,19 @@ __global__ __launch_bounds__(TB) void k_grad_recv64(const LatDev* __restrict__ l
     const double V = S.emb[s] + qw * xi * S.epair[s];  // owned pairs carry their full energy
     const double sc = qw * xi / T;
     if (ln.ph == 0) {
-      G[4 * site + 0] = sc * g0;
-      G[4 * site + 1] = sc * g1;
-      G[4 * site + 2] = sc * g2;
-      G[4 * site + 3] = sq * sc * gs - 3.0 * KB * xi / sg;
+      g0 *= sc;
+      g1 *= sc;
+      g2 *= sc;
+      gs = sq * sc * gs - 3.0 * KB * xi / sg;
+      G[4 * site + 0] = g0;
+      G[4 * site + 1] = g1;
+      G[4 * site + 2] = g2;
+      G[4 * site + 3] = gs;
       fs = V / T - 3.0 * KB * xi * log(sg);
+      sl = site_slope(S, site, g0, g1, g2, gs);
     }
   }
-  finish_objective(S, ln, fs);
+  finish_objective(S, ln, fs, sl);
 }
 
 // ================================================================ chemical potential

@@ -442,7 +442,7 @@ __global__ __launch_bounds__(TB) void k_gen_grad_recv(const LatDev* __restrict__
   const int v = xcd_block(), rq = S.rl;
   const RecvLane ln(S, v / rq, v % rq);
   const int s = ln.s;
-  double fs = 0.0;
+  double fs = 0.0, sl = 0.0;
   if (s < S.npd + S.nh) {
     const bool pd = s < S.npd;
     const int row = pd ? s : s - S.npd;
@@ -463,14 +463,16 @@ __global__ __launch_bounds__(TB) void k_gen_grad_recv(const LatDev* __restrict__
       const double T = S.T, sc = xi / T;
       const double V = S.emb[s] + xi * S.epair[s];  // owned pairs carry their full energy (minimizer.cpp:169-286)
       double* __restrict__ G = S.G + 4 * site;  // the caller's: 8-byte aligned
-      G[0] = sc * gr.x;
-      G[1] = sc * gr.y;
-      G[2] = sc * gr.z;
-      G[3] = sc * gr.w - 3.0 * KB * xi / sg;
+      gr = make_double4(sc * gr.x, sc * gr.y, sc * gr.z, sc * gr.w - 3.0 * KB * xi / sg);
+      G[0] = gr.x;
+      G[1] = gr.y;
+      G[2] = gr.z;
+      G[3] = gr.w;
       fs = V / T - 3.0 * KB * xi * log(sg);
+      sl = site_slope(S, site, gr.x, gr.y, gr.z, gr.w);
     }
   }
-  finish_objective(S, ln, fs);
+  finish_objective(S, ln, fs, sl);
 }
 
 // ------------------------------------------------------------ chemical potential

@@ -141,7 +141,9 @@ struct LatDev {
   float2* aux = nullptr;      // N {F'(rho), x} (mixed path)
   double* emb = nullptr;      // N embedding energy (x-weighted for H)
   double* epair = nullptr;    // N pair-energy partial (mixed path)
-  double* part = nullptr;     // block partial sums of f: one per 256 sites, or per 64 (recv_lanes)
+  const double* w = nullptr;  // 4N direction (site order), or null: the gradient receive pass then also sums
+  double* slope = nullptr;    // G . w into slope
+  double* part = nullptr;     // block partial sums of f and G . w: one of each per 256 sites, or per 64 (recv_lanes)
   int32_t* done = nullptr;    // blocks of the gradient receive pass that have put theirs (k_rows clears it)
   int32_t rl = 1;             // lanes per row in the receive passes (recv_lanes)
   double* f = nullptr;        // objective
@@ -435,18 +437,36 @@ __device__ __forceinline__ void sum_parts(const double* part, size_t stride, int
     if (lane == 0 && w + W * i < K) out(w + W * i, v[i]);
 }
 
-// End of a gradient receive pass: the block's sum of fs, and of all blocks' sums
-// by the last one, into the objective.  Every lane of a working block calls it.
-__device__ __forceinline__ void finish_objective(const LatDev& S, const RecvLane& ln, double fs) {
-  __shared__ double red[SITE_BLOCK / 64];
+// End of a gradient receive pass: the block's sums of fs and sl, and of all blocks'
+// sums by the last one, into the objective and (S.w) the slope.  Every lane of a
+// working block calls it.
+__device__ __forceinline__ void finish_objective(const LatDev& S, const RecvLane& ln, double fs, double sl) {
+  __shared__ double red[2][SITE_BLOCK / 64];
 #pragma unroll
-  for (int off = 32; off > 0; off >>= 1) fs += __shfl_down(fs, off);
-  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = fs;
+  for (int off = 32; off > 0; off >>= 1) {
+    fs += __shfl_down(fs, off);
+    sl += __shfl_down(sl, off);
+  }
+  if ((threadIdx.x & 63) == 0) {
+    red[0][threadIdx.x >> 6] = fs;
+    red[1][threadIdx.x >> 6] = sl;
+  }
   __syncthreads();
   const int n = (ln.G == 1 ? 1 : RECV_LANES) * lattice_blocks(S.npd + S.nh);
-  if (threadIdx.x == 0) put_part(S.part + (ln.G == 1 ? ln.lb : RECV_LANES * ln.lb + ln.q), (red[0] + red[1]) + (red[2] + red[3]));
+  if (threadIdx.x == 0) {
+    double* p = S.part + (ln.G == 1 ? ln.lb : RECV_LANES * ln.lb + ln.q);
+    put_part(p, (red[0][0] + red[0][1]) + (red[0][2] + red[0][3]));
+    if (S.w) put_part(p + n, (red[1][0] + red[1][1]) + (red[1][2] + red[1][3]));
+  }
   if (!last_block(S.done, n)) return;
-  sum_parts<1>(S.part, 0, n, [&](int, double v) { *S.f = v; });
+  if (S.w) sum_parts<2>(S.part, n, n, [&](int k, double v) { *(k ? S.slope : S.f) = v; });
+  else sum_parts<1>(S.part, 0, n, [&](int, double v) { *S.f = v; });
+}
+// G . w of one site
+__device__ __forceinline__ double site_slope(const LatDev& S, size_t site, double g0, double g1, double g2, double g3) {
+  if (!S.w) return 0.0;
+  const A2C_GLOBAL double* w = gmem(S.w) + 4 * site;
+  return (g0 * w[0] + g1 * w[1]) + (g2 * w[2] + g3 * w[3]);
 }
 
 // What a neighbor build tells the host: the 14 maxima and the overflow flag of
@@ -562,7 +582,7 @@ struct a2c_fe_ctx {
     s.rule = desc.quad_rule;
     s.pdpd = ell[0]; s.pdh = ell[1]; s.hpd = ell[2]; s.hh = ell[3]; s.hh1 = ell[4];
     s.x = dx; s.rho = drho; s.Fp = dFp; s.aux = daux; s.emb = demb; s.part = dpart; s.epair = depair;
-    s.done = reinterpret_cast<int32_t*>(dpart + (size_t)a2c::RECV_LANES * nblk_red);
+    s.done = reinterpret_cast<int32_t*>(dpart + 2 * (size_t)a2c::RECV_LANES * nblk_red);
     s.rl = a2c::recv_lanes(N);
     s.qxy = dqxy; s.qzs = dqzs; s.xrow = dxrow; s.gown = dgown;
     return s;
