@@ -1290,7 +1290,7 @@ int gen_eval(a2c_batch* b, int id, bool fp64, bool slopes, StateOf state_of) {
   const double eps = b->desc.fd_eps;
   enqueue(b, {8, (uint64_t)fp64, u64(dl), (uint64_t)npd, (uint64_t)nh, u64(g.nodes), u64(g.tab), u64(g.r64.row),
               u64(g.r32.row), (uint64_t)g.r64.n, u64(g.r64.ih), (uint64_t)g.K, (uint64_t)g.rel, (uint64_t)g.pot,
-              (uint64_t)dm, u64(eps), (uint64_t)lanes_per_site(npd + nh, true)},
+              (uint64_t)dm, u64(eps), (uint64_t)lanes_per_site(npd + nh, false)},
           [=](hipStream_t st) {
             const int rc = run_eval_gen(dl, npd, nh, g, dm, eps, !fp64, st, nullptr);
             if (rc && !b->qrc) b->qrc = rc;

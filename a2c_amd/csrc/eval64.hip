@@ -1448,7 +1448,8 @@ int launch_density64(a2c_fe_ctx* c, const double* dX, bool by_site) {
 // or four share one, so that a CU's one copy of the tables serves all its waves.
 template <int RULE>
 static void launch_chem64_rule(a2c_fe_ctx* c, const ChemArgs& a) {
-  const int K = lanes_per_site(c->N, true), units = owner_units(c->desc.n_h, K);
+  // lanes per row as in the mixed passes: one species' full lists are a smaller, longer launch than the FP64 passes'
+  const int K = lanes_per_site(c->N, false), units = owner_units(c->desc.n_h, K);
   auto go = [&](auto kernel, int tbo) {
     hipLaunchKernelGGL(kernel, dim3((units + tbo / TB - 1) / (tbo / TB)), dim3(tbo), 0, c->stream,
                        (const LatDev*)c->dlat, units, K, (const double*)c->dtab64, a);

@@ -558,11 +558,16 @@ size_t lds_bytes(const GenDev& g, int deriv_mode, bool fp32) {
   return general_fp32(deriv_mode, fp32) ? node_bytes<float>(g) : node_bytes<double>(g);
 }
 
+// Lanes per site: the mixed passes' table in either precision.  These kernels
+// wait for gathers where the FP64 passes compute (16^3 cells, FP64, K = 1/2/4/8:
+// 580/333/238/251 us).
+int gen_lanes(int n) { return lanes_per_site(n, false); }
+
 // rho, F(rho), F'(rho) and the embedding energy at the state of *dlat.
 int run_density_gen(const LatDev* dlat, int npd, int nh, const GenDev& g, int deriv_mode, double eps, bool fp32,
                     bool by_site, hipStream_t st, Timing* tm) {
   if (npd + nh <= 0) return A2C_OK;
-  const int nblk = site_blocks(npd + nh), KL = lanes_per_site(npd + nh, true);
+  const int nblk = site_blocks(npd + nh), KL = gen_lanes(npd + nh);
   const bool fold = nblk <= FOLD_BLOCKS;
   if (!fold) {
     if (tm) tm->mark(st, "rows");
@@ -581,7 +586,7 @@ int run_density_gen(const LatDev* dlat, int npd, int nh, const GenDev& g, int de
 int run_eval_gen(const LatDev* dlat, int npd, int nh, const GenDev& g, int deriv_mode, double eps, bool fp32,
                  hipStream_t st, Timing* tm) {
   if (npd + nh > 0) {
-    const int nblk = site_blocks(npd + nh), KL = lanes_per_site(npd + nh, true);
+    const int nblk = site_blocks(npd + nh), KL = gen_lanes(npd + nh);
     if (int rc = run_density_gen(dlat, npd, nh, g, deriv_mode, eps, fp32, false, st, tm)) return rc;
     if (tm) tm->mark(st, "gen_grad_own");
     hipLaunchKernelGGL(pick<GradK>(g, deriv_mode, fp32), dim3(owner_units(npd, nh, KL)), dim3(TB),

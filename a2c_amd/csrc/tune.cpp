@@ -1,9 +1,9 @@
 // Launch-shape table of the pair-owner passes (lanes per site by lattice
 // size and precision) and the autotuner that measures it.
 //
-// The built-in table is the outcome of a2c_autotune on one MI355X with the
-// default options (evaluations of 6^3..40^3-cell lattices, in fused launches
-// filling about one million sites and alone).
+// The built-in table was measured on one MI355X (below); a2c_autotune measures
+// one with a class per given size (evaluations of 6^3..40^3-cell lattices by
+// default, in fused launches filling about one million sites and alone).
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -22,19 +22,21 @@ namespace a2c {
 namespace {
 
 a2c_tune_table default_table() {
-  // a2c_autotune with the default options on one MI355X.  Up to 11^3 cells a
-  // lattice alone fills fewer SIMDs than the device has and takes the K that
-  // finishes it soonest within 25% of the best throughput: 6^3 cells, K =
-  // 1/2/4/8/16, alone mixed 294/143/98/80/67 us and FP64 687/270/165/124/96
-  // us per evaluation, in launches of 256 copies mixed 1.99/1.75/1.67/1.85/
-  // 2.30 and FP64 5.39/4.72/4.70/5.11/6.04 ns per site (K = 16 costs 37%
-  // there).  Larger lattices take the fastest K alone within 5% of the best
-  // throughput (24^3 cells FP64: 4.13/4.18 ns per site at K = 2/4 in a full
-  // launch, 602/528 us alone; 40^3 cells mixed 1.74/1.58/1.60/1.79/2.33 ns
-  // per site, 871/807/818/915/1193 us alone).
-  static const int32_t max_sites[] = {2660, 6604, 15288, 32003, 71831, 170267, 366357, INT_MAX};
-  static const int32_t lanes_mixed[] = {8, 8, 8, 4, 4, 4, 2, 2};
-  static const int32_t lanes_fp64[] = {8, 8, 8, 4, 4, 4, 4, 2};
+  // The FP64 gradient pass runs 512 lanes per CU at a time (its tables fill the
+  // LDS), 131,072 on 256 CUs, and a lattice takes ceil(sites K / 131072) rounds of
+  // length ~ 1/K: alone it finishes soonest at the K whose last round is
+  // fullest, so the classes end at multiples of 1/8 of that capacity.  FP64, 12-point
+  // rule, K = 1/2/4/8, us per evaluation: 13,824 sites 195/129/100/90, 32,768
+  // sites 205/143/123/136, 64,000 sites 211/174/181/215, 85,184 sites 277/283/252/
+  // 301, 110,592 sites 292/290/316/346, 140,608 sites 486/410/391/441, 175,616
+  // sites 499/424/465/531, 373,248 sites 820/860/942/1113.  The mixed passes hold
+  // twice the lanes in smaller workgroups and want K = 8 up to 16,384 sites (13,824
+  // sites 128/87/68/63), 2 on the largest (373,248 sites 410/407/433/509), and
+  // 4 between, where 8 gains little alone (27,000 sites 135/95/83/80) and costs
+  // 15% in a batch's full launches.
+  static const int32_t max_sites[] = {16384, 32768, 65536, 98304, 131072, 163840, 196608, INT_MAX};
+  static const int32_t lanes_mixed[] = {8, 4, 4, 4, 4, 4, 4, 2};
+  static const int32_t lanes_fp64[] = {8, 4, 2, 4, 1, 4, 2, 1};
   a2c_tune_table t;
   std::memset(&t, 0, sizeof t);
   t.n_classes = 8;
@@ -52,8 +54,8 @@ constexpr int NLANES = 5;
 // Largest per-site cost in a full launch that a choice for the lone-lattice
 // time may add: for a lattice that alone fills fewer SIMDs than the device
 // has, and for one that fills them (where near-equal throughputs differ
-// alone: at 24^3 cells FP64, K = 2 beat K = 4 by 1% per site in a full
-// launch and lost by 14% alone, in the tail of a lockstep run).
+// alone: at 24^3 cells mixed, K = 2 and 4 are within 5% per site in a full
+// launch, and 158 and 154 us alone).
 constexpr double LATENCY_COST = 1.25, THROUGHPUT_SLACK = 1.05;
 const int LANES[NLANES] = {1, 2, 4, 8, 16};
 bool valid_lanes(int k) { return k == 1 || k == 2 || k == 4 || k == 8 || k == 16; }

@@ -32,8 +32,8 @@ typedef struct a2c_tune_table {
   int32_t lanes_fp64[A2C_TUNE_MAX_CLASSES];  /* K of the FP64 passes */
 } a2c_tune_table;
 
-/* The table in effect; the built-in default is the result of a2c_autotune
- * on MI355X. */
+/* The table in effect; the built-in default was measured on one MI355X, with
+ * classes that end where the FP64 gradient pass's last round of workgroups fills. */
 void a2c_tune_get(a2c_tune_table* out);
 /* Replace the table (A2C_EINVAL if malformed); null restores the default. */
 int a2c_tune_set(const a2c_tune_table* t);
