@@ -115,6 +115,17 @@ hipError_t dmalloc(void** ptr, size_t bytes) {
   return hipSuccess;
 }
 
+DeviceScope::DeviceScope(int device) {
+  int cur = 0;
+  err_ = hipGetDevice(&cur);
+  if (err_ != hipSuccess || cur == device) return;
+  err_ = hipSetDevice(device);
+  if (err_ == hipSuccess) prev_ = cur;
+}
+DeviceScope::~DeviceScope() {
+  if (prev_ >= 0) (void)hipSetDevice(prev_);
+}
+
 namespace {
 thread_local int t_released = -1;  // device of this thread's innermost ReleaseScope
 }

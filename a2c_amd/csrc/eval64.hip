@@ -1489,6 +1489,8 @@ int sync_lattice(a2c_fe_ctx* c, const double* dX, double* dG, double* dF) {
   }
   if (!c->db2l) {  // all-zero block -> lattice map: site blocks, or owner units at any lanes per site
     const size_t n = 4 * (size_t)(owner_units(c->N, MAX_LANES_PER_SITE) + 1);
+    const DeviceScope on(c->desc.device);
+    A2C_HIP(c, on.status());
     A2C_HIP(c, dmalloc(&c->db2l, n));
     A2C_HIP(c, hipMemsetAsync(c->db2l, 0, n, c->stream));
   }

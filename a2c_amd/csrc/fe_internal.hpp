@@ -24,6 +24,21 @@ inline hipError_t hmalloc(T** ptr, size_t bytes) {
   return hmalloc(reinterpret_cast<void**>(ptr), bytes);
 }
 hipError_t hfree(const void* ptr);
+// While one lives, this thread's current device is the given one: what a context
+// makes at its first use (memory, events) belongs to the context's device,
+// whichever is current in the calling thread.
+class DeviceScope {
+ public:
+  explicit DeviceScope(int device);
+  ~DeviceScope();
+  DeviceScope(const DeviceScope&) = delete;
+  DeviceScope& operator=(const DeviceScope&) = delete;
+  hipError_t status() const { return err_; }
+
+ private:
+  int prev_ = -1;  // the device to go back to, -1 if it is the given one
+  hipError_t err_;
+};
 // While one lives, this thread's releases on its device (dfree, hfree) do not
 // wait for the device again: it waited when it was made, and nothing that uses
 // the released blocks is issued during its life (a context's teardown, ~50

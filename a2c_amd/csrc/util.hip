@@ -52,8 +52,13 @@ hipError_t HostTransfer::download(hipStream_t st, char* stage, size_t cap, void*
       if (hipError_t e = copy_to_pinned(st, stage + o, static_cast<const char*>(dsrc) + r + o, std::min(part, n - o)))
         return e;
       if (o + part >= n) break;  // the last part is waited for with the stream
-      if (!ev_[k])
+      if (!ev_[k]) {  // an event belongs to its stream's device
+        hipDevice_t dev;
+        if (hipError_t e = hipStreamGetDevice(st, &dev)) return e;
+        const DeviceScope on(dev);
+        if (hipError_t e = on.status()) return e;
         if (hipError_t e = hipEventCreateWithFlags(&ev_[k], hipEventDisableTiming)) return e;
+      }
       if (hipError_t e = hipEventRecord(ev_[k], st)) return e;
     }
     k = 0;
