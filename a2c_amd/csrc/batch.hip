@@ -1373,8 +1373,8 @@ int fused_eval(a2c_batch* b, const std::vector<int>& ids_in, bool fp64, StateOf 
   L.tab64 = b->dtab64;
   L.mixed_full = mixed_full_pairs();
   L.full_pairs64 = fp64_full_pairs();
-  enqueue(b, {5, (uint64_t)fp64, u64(L.lats), u64(L.b2l), u64(L.ob2l), (uint64_t)L.nblk, (uint64_t)L.rq, (uint64_t)L.onblk,
-              (uint64_t)L.nlat, (uint64_t)L.rules, (uint64_t)L.deriv_mode, u64(L.fd_eps), u64(L.tab), u64(L.tab64),
+  enqueue(b, {5, (uint64_t)fp64, u64(L.lats), u64(L.b2l), u64(L.ob2l), (uint64_t)L.nblk, (uint64_t)L.rq, (uint64_t)L.empty,
+              (uint64_t)L.onblk, (uint64_t)L.nlat, (uint64_t)L.rules, (uint64_t)L.deriv_mode, u64(L.fd_eps), u64(L.tab), u64(L.tab64),
               (uint64_t)L.mixed_full, (uint64_t)L.full_pairs64},
           [=](hipStream_t st) {
             Launch l = L;
