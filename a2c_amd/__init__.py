@@ -203,6 +203,7 @@ def _load():
         "a2c_philox4x32_10": (None, [P(C.c_uint32), P(C.c_uint32), P(C.c_uint32)]),
         "a2c_eam_tables": (I, [P(C.c_float), C.c_int32]),
         "a2c_eam_tables64": (I, [dp, C.c_int32]),
+        "a2c_eam_pass": (I, [C.c_int32, C.c_int32, C.c_int32, dp, dp, dp, dp]),
         "a2c_enforce_boundary_conditions": (I, [C.c_int32, ip, D, D, dp, dp, ip]),
         "a2c_macro_results": (I, [C.c_int32, dp, C.c_int32, ip, dp, dp]),
         "a2c_read_results": (I, [C.c_char_p, C.c_int32, C.c_int32, D, D, dp, dp, dp, ip]),
@@ -310,6 +311,17 @@ def eam_tables64():
     out = np.zeros(n)
     lib.a2c_eam_tables64(_dptr(out), n)
     return out[:3000].reshape(3, 100, 10), out[3000:].reshape(2, 100, 12)
+
+
+def eam_pass(fn, r, precision="fp64"):
+    """An EAM function (0..4: f_Pd, f_H, phi_Pd, phi_PdH, phi_H) at the radii r as
+    the pair-once passes of a precision take it from their tables: (radii the
+    arguments stand for, values, slopes)."""
+    r = _f64(r, len(r))
+    at, v, d = np.empty_like(r), np.empty_like(r), np.empty_like(r)
+    if lib.a2c_eam_pass(PREC[precision], fn, len(r), _dptr(r), _dptr(at), _dptr(v), _dptr(d)):
+        raise ValueError("function 0..4, radii in [1, 5.999)")
+    return at, v, d
 
 
 def eam_tables():

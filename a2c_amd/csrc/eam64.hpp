@@ -11,6 +11,7 @@
 #include <hip/hip_runtime.h>
 
 #include <cmath>
+#include <cstdint>
 
 namespace a2c {
 namespace eam {
@@ -19,6 +20,24 @@ template <typename T>
 struct VDT { T v, d; };
 using VD = VDT<double>;
 #define A2C_HD __host__ __device__ __forceinline__
+
+// Operations with an instruction of their own on the device; the host forms let
+// the passes' table code be evaluated on the host (a2c_eam_pass).
+#ifdef __HIP_DEVICE_COMPILE__
+A2C_HD double fract(double x) { return __builtin_amdgcn_fract(x); }
+A2C_HD float fract(float x) { return __builtin_amdgcn_fractf(x); }
+A2C_HD double rsq_est(double x) { return __builtin_amdgcn_rsq(x); }
+A2C_HD float rsq_est(float x) { return __builtin_amdgcn_rsqf(x); }
+A2C_HD float exp2_est(float x) { return __builtin_amdgcn_exp2f(x); }
+A2C_HD uint32_t mul24(uint32_t a, uint32_t b) { return __umul24(a, b); }
+#else
+A2C_HD double fract(double x) { return x - std::floor(x); }
+A2C_HD float fract(float x) { return x - std::floor(x); }
+A2C_HD double rsq_est(double x) { return 1.0 / std::sqrt(x); }
+A2C_HD float rsq_est(float x) { return 1.0f / std::sqrt(x); }
+A2C_HD float exp2_est(float x) { return std::exp2(x); }
+A2C_HD uint32_t mul24(uint32_t a, uint32_t b) { return a * b; }
+#endif
 
 template <typename T>
 struct same { using type = T; };  // keeps an argument out of template deduction

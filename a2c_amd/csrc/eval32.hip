@@ -57,7 +57,7 @@ __constant__ float TAIL[NTAB][3] = {
     {-3.353001113951400e-04f, (float)(7.147062196813336e-04 / -3.353001113951400e-04), 5.35f},
     {-0.003702722457147f, (float)(0.005465945471933 / -0.003702722457147), 5.35f}};
 
-__device__ __forceinline__ float rsq(float x) { return __builtin_amdgcn_rsqf(x); }
+A2C_HD float rsq(float x) { return eam::rsq_est(x); }
 
 // Position of r in the tables: interval k and local coordinate u in [0, 1),
 // computed once per quadrature point and shared by every function evaluated
@@ -80,9 +80,9 @@ __device__ __forceinline__ Pos tab_pos(float r) {
   return p;
 }
 // value of a cubic row {c0, c1, c2, c3}
-__device__ __forceinline__ float cubic(const float4 c, float u) { return fmaf(u, fmaf(u, fmaf(u, c.w, c.z), c.y), c.x); }
+A2C_HD float cubic(const float4 c, float u) { return fmaf(u, fmaf(u, fmaf(u, c.w, c.z), c.y), c.x); }
 // value and d/du of a cubic row (Horner with derivative: 5 FMAs)
-__device__ __forceinline__ void cubic_vd(const float4 c, float u, float& v, float& du) {
+A2C_HD void cubic_vd(const float4 c, float u, float& v, float& du) {
   const float v1 = fmaf(u, c.w, c.z);
   const float v2 = fmaf(u, v1, c.y);
   const float d2 = fmaf(u, c.w, v1);
@@ -90,7 +90,7 @@ __device__ __forceinline__ void cubic_vd(const float4 c, float u, float& v, floa
   du = fmaf(u, d2, v2);
 }
 // value of a derivative row {c1, 2 c2, 3 c3, 0} (d/du of a cubic row)
-__device__ __forceinline__ float quad(const float4 c, float u) { return fmaf(u, fmaf(u, c.z, c.y), c.x); }
+A2C_HD float quad(const float4 c, float u) { return fmaf(u, fmaf(u, c.z, c.y), c.x); }
 // exponential tail of function w (its slope is TAIL[w][1] times the value);
 // NaN below the table (see tab_pos)
 __device__ __forceinline__ float tail(int w, float r) {
@@ -481,19 +481,19 @@ struct Edge {
 // f_H / 11.0025 at s, and 1/|r|: 2^(K r), K = -1.30927 log2(e) split into
 // FP32 hi and lo parts, with the rounding of K r carried into a first-order
 // correction (within about an ulp of FP32).  Callers scale their sums.
-__device__ __forceinline__ float fH_s(float s, float& rinv) {
+A2C_HD float fH_s(float s, float& rinv) {
   rinv = rsq(s);
   const float r = s * rinv;
   const float e = FH_KHI * r;
   const float el = fmaf(FH_KLO, r, fmaf(FH_KHI, r, -e));
-  return __builtin_amdgcn_exp2f(e) * fmaf(el, LN2F, 1.0f);
+  return eam::exp2_est(e) * fmaf(el, LN2F, 1.0f);
 }
 // Row position of table coordinate x: interval k and u in [0, 1).
 struct SPos {
   int k;
   float u;
 };
-__device__ __forceinline__ SPos s_pos(float x) { return {(int)x, __builtin_amdgcn_fractf(x)}; }
+A2C_HD SPos s_pos(float x) { return {(int)x, eam::fract(x)}; }
 // s of a table coordinate, and whether the tables serve it (a pair with a
 // node outside is evaluated node by node: the exponential tails from 6 A on,
 // NaN below 1 A -- no physical configuration comes that close, and the
@@ -1097,6 +1097,28 @@ void host_tables(std::vector<float4>& t) {
     return u;
   }();
   t = built;
+}
+
+// One EAM function (order of a2c_eam_tables) at r in [1, 6) as the pair-once passes
+// take it from the tables t: value, and slope in r.
+void pass_eval32(const std::vector<float4>& t, int fn, float s, double& v, double& d) {
+  const SPos p = s_pos(fmaf(s, SINV, SB));
+  const double r = std::sqrt((double)s);
+  float vf = 0.0f, df = 0.0f, ri;
+  if (fn == T_FH) {
+    vf = fH_s(s, ri);
+    v = (double)FH_C * vf;
+    d = FH_K * FH_C * vf;
+    return;
+  }
+  if (fn == T_FPD) {
+    vf = cubic(t[S_FPD * SNT + p.k], p.u);
+    df = quad(t[S_DFPD * SNT + p.k], p.u);
+  } else {
+    cubic_vd(t[(fn == T_PHPD ? S_PHPD : fn == T_PHPDH ? S_PHPDH : S_PHH) * SNT + p.k], p.u, vf, df);
+  }
+  v = vf;
+  d = 2.0 * SINV * r * df;
 }
 
 int build_tables(a2c_fe_ctx* c) {

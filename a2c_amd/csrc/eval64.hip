@@ -380,20 +380,18 @@ struct SPos {
   int k;
   double u;
 };
-__device__ __forceinline__ SPos s_pos(double x) { return {(int)x, __builtin_amdgcn_fract(x)}; }
-__device__ __forceinline__ double s_of(double x) { return fma(x, SH, S0); }
-__device__ __forceinline__ const double* s_row(const double* tab, int f, int k) {
-  return tab + f * S_ROWS + __umul24(k, SP);
-}
+A2C_HD SPos s_pos(double x) { return {(int)x, eam::fract(x)}; }
+A2C_HD double s_of(double x) { return fma(x, SH, S0); }
+A2C_HD const double* s_row(const double* tab, int f, int k) { return tab + f * S_ROWS + eam::mul24(k, SP); }
 template <int D>
-__device__ __forceinline__ double poly(const double* c, double u) {
+A2C_HD double poly(const double* c, double u) {
   double v = c[D];
 #pragma unroll
   for (int j = D - 1; j >= 0; --j) v = fma(v, u, c[j]);
   return v;
 }
 // value and d/du
-__device__ __forceinline__ void poly_vd(const double* c, double u, double& v, double& d) {
+A2C_HD void poly_vd(const double* c, double u, double& v, double& d) {
   v = fma(c[5], u, c[4]);
   d = fma(c[5], u, v);
 #pragma unroll
@@ -404,10 +402,12 @@ __device__ __forceinline__ void poly_vd(const double* c, double u, double& v, do
   v = fma(v, u, c[0]);
 }
 // the same for a degree-6 row whose last two coefficients share a double (phi_Pd)
-__device__ __forceinline__ void poly6_vd(const double* c, double u, double& v, double& d) {
+A2C_HD void poly6_vd(const double* c, double u, double& v, double& d) {
   const double2 c45 = *reinterpret_cast<const double2*>(c + 4);  // one 16-byte read
-  const double hy = __int_as_float(__double2hiint(c45.y));
-  v = fma(hy, u, (double)__int_as_float(__double2loint(c45.y)));
+  float f2[2];
+  __builtin_memcpy(f2, &c45.y, 8);
+  const double hy = f2[1];
+  v = fma(hy, u, (double)f2[0]);
   d = fma(hy, u, v);
   v = fma(v, u, c45.x);
   d = fma(d, u, v);
@@ -418,27 +418,43 @@ __device__ __forceinline__ void poly6_vd(const double* c, double u, double& v, d
   }
   v = fma(v, u, c[0]);
 }
+A2C_HD long long double_bits(double x) {
+  long long b;
+  __builtin_memcpy(&b, &x, sizeof b);
+  return b;
+}
 // 1/sqrt(x): the hardware estimate y (relative error below 2^-20), then one
 // step of y <- y (1 + e/2 + 3 e^2 / 8), e = 1 - x y^2 (third order).
-__device__ __forceinline__ double rsqrt3(double x) {
-  const double y = __builtin_amdgcn_rsq(x);
+A2C_HD double rsqrt3(double x) {
+  const double y = eam::rsq_est(x);
   const double e = fma(-(x * y), y, 1.0);
   return fma(y * e, fma(e, 0.375, 0.5), y);
 }
-// f_H / 11.0025 = 2^(K r) at s = r^2, r and 1/r: n = rint(256 K r) picks 2^(n/256)
-// from the table, the remainder f in [-1/2, 1/2] goes through the series of
-// 2^(f/256) (next term 4e-17).
-__device__ __forceinline__ double fH_s(const double* exptab, double s, double& r, double& ri) {
-  constexpr double K = -1.30927 * 1.4426950408889634074 * EXPN, MAGIC = 6755399441055744.0;
+// f_H / 11.0025 = 2^(E / 256), E = 256 log2(e) ln(f_H / 11.0025), at s = r^2, with r
+// and 1/r; sl = f_H' / (-1.30927 11.0025).  n = rint(E) picks 2^(n/256) from the
+// table, the remainder f in [-1/2, 1/2] goes through the series of 2^(f/256) (next
+// term 4e-17).  E = K r up to 5.35 A and K2 r + B2 on the tail beyond, which
+// potential.cpp gives another amplitude (5e-14 off at 5.35 A) and decay (2.5e-11): 256
+// log2(e) ln(0.009986990526578 / 11.0025 exp(5.35 FH_K2)) is B2.  The choice costs
+// 7% of an evaluation, so a wave's pairs make it (TAIL) only if one of them has
+// a node there (40^3 cells: 1069 us without it, 1142 with it in every pair).
+constexpr double FH_K = -1.30927, FH_K2 = -0.013075667086408 / 0.009986990526578;
+template <bool TAIL>
+A2C_HD double fH_s(const double* exptab, double s, double& r, double& ri, double& sl) {
+  constexpr double C = 1.4426950408889634074 * EXPN, MAGIC = 6755399441055744.0;
+  constexpr double K = FH_K * C, K2 = FH_K2 * C, B2 = -6.42743196697137263e-8;
   constexpr double L1 = 0.69314718055994530942 / EXPN;
   ri = rsqrt3(s);
   r = s * ri;
-  const double t = fma(r, K, MAGIC);
-  const int n = (int)(unsigned)__double_as_longlong(t);
-  const double f = fma(r, K, -(t - MAGIC));
+  const bool tail = TAIL && r > 5.35;
+  const double k = tail ? K2 : K;
+  const double t = fma(r, k, MAGIC);
+  const int n = (int)(unsigned)double_bits(t);
+  const double f = fma(r, k, (tail ? B2 : 0.0) - (t - MAGIC));
   const double p = f * fma(f, fma(f, fma(f, L1 * L1 * L1 * L1 / 24.0, L1 * L1 * L1 / 6.0), L1 * L1 / 2.0), L1);
-  const double T = ldexp(exptab[n & (EXPN - 1)], n >> 8);
-  return fma(T, p, T);
+  const double T = ldexp(exptab[n & (EXPN - 1)], n >> 8), v = fma(T, p, T);
+  sl = v * (tail ? FH_K2 / FH_K : 1.0);
+  return v;
 }
 
 // Table coordinates of one pair: 12-point rule (site e's nodes have
@@ -477,17 +493,19 @@ struct Nodes27 {
   }
 };
 __device__ __forceinline__ bool inside(double lo, double hi) { return lo >= SLO && hi < SHI; }
+// some pair of the wave has a node on f_H's tail (a margin over the roundings of hi and r)
+__device__ __forceinline__ bool on_tail(double hi) { return __ballot(hi > 5.35 * 5.35 - 1e-9) != 0; }
 
 // densities at one node inside the tables
-template <bool WANT_PD, bool WANT_H>
+template <bool WANT_PD, bool WANT_H, bool TAIL>
 __device__ __forceinline__ void node_dens(const double* tab, const double* exptab, double x, double& fpd, double& fh) {
   if (WANT_PD) {
     const SPos p = s_pos(x);
     fpd = poly<5>(s_row(tab, 0, p.k), p.u);
   }
   if (WANT_H) {
-    double r, ri;
-    fh = fH_s(exptab, s_of(x), r, ri);
+    double r, ri, sl;
+    fh = fH_s<TAIL>(exptab, s_of(x), r, ri, sl);
   }
 }
 
@@ -506,6 +524,53 @@ __device__ __forceinline__ double2 closed_dens(const double d[3], double si, dou
   return make_double2(sp, sh);
 }
 
+// Sums over a pair's nodes of f_Pd and of f_H / 11.0025, as wanted.
+template <bool WP, bool WH, bool TAIL>
+__device__ __forceinline__ void dens_sums27(const double* tab, const double* exptab, const Nodes27& q, double& sp,
+                                            double& sh) {
+#pragma unroll 1
+  for (int a2 = -1; a2 <= 1; ++a2) {
+#pragma unroll 1
+    for (int a1 = -1; a1 <= 1; ++a1) {
+      const double xb = q.x0 + q.n1 * (double)(a2 * a2 + a1 * a1) + ((double)a2 * q.t[2] + (double)a1 * q.t[1]);
+      const double w = (a2 ? 1.0 : 4.0) * (a1 ? 1.0 : 4.0);
+      double pp = 0.0, ph = 0.0;
+#pragma unroll
+      for (int a0 = -1; a0 <= 1; ++a0) {
+        double fp = 0.0, fh = 0.0;
+        node_dens<WP, WH, TAIL>(tab, exptab, a0 ? xb + q.n1 + a0 * q.t[0] : xb, fp, fh);
+        pp += a0 ? fp : 4.0 * fp;
+        ph += a0 ? fh : 4.0 * fh;
+      }
+      sp = fma(w, pp, sp);
+      sh = fma(w, ph, sh);
+    }
+  }
+  sp *= 1.0 / 216.0;
+  sh *= 1.0 / 216.0;
+}
+template <bool WP, bool WH, bool TAIL>
+__device__ __forceinline__ void dens_sums12(const double* tab, const double* exptab, const Nodes12& q,
+                                            const double d[3], double& sp, double& sh) {
+  double d0 = d[0], d1 = d[1], d2 = d[2];
+  constexpr int UN = TAIL ? 1 : 3;  // the rare instance would spill unrolled
+#pragma unroll UN
+  for (int c = 0; c < 3; ++c) {
+    const double ti = q.gi * d0, tj = q.gj * d0;
+    const double x[4] = {q.xi + ti, q.xi - ti, q.xj - tj, q.xj + tj};
+    constexpr int UK = TAIL ? 1 : 4;
+#pragma unroll UK
+    for (int k = 0; k < 4; ++k) {
+      double fp = 0.0, fh = 0.0;
+      node_dens<WP, WH, TAIL>(tab, exptab, k == 0 ? x[0] : k == 1 ? x[1] : k == 2 ? x[2] : x[3], fp, fh);
+      if (WP) sp += fp;
+      if (WH) sh += fh;
+    }
+    d0 = d1;
+    d1 = d2;
+  }
+}
+
 // Sums over a pair's nodes of the density of the neighbor's species (mine) and
 // of this site's species (theirs); NB_H / ME_H: neighbor / this site is an H
 // site.  False, and zeros, if a node lies outside the tables.
@@ -516,47 +581,18 @@ __device__ __forceinline__ bool pair_dens(const double* tab, const double* expta
   double sp = 0.0, sh = 0.0;
   bool in;
   if (RULE == GH3) {
-    const double sd = sqrt(fma(si, si, sj * sj));
-    const Nodes27 q(d, sd);
+    const Nodes27 q(d, sqrt(fma(si, si, sj * sj)));
     in = inside(q.lo, q.hi);
     if (in) {
-#pragma unroll 1
-      for (int a2 = -1; a2 <= 1; ++a2) {
-#pragma unroll 1
-        for (int a1 = -1; a1 <= 1; ++a1) {
-          const double xb = q.x0 + q.n1 * (double)(a2 * a2 + a1 * a1) + ((double)a2 * q.t[2] + (double)a1 * q.t[1]);
-          const double w = (a2 ? 1.0 : 4.0) * (a1 ? 1.0 : 4.0);
-          double pp = 0.0, ph = 0.0;
-#pragma unroll
-          for (int a0 = -1; a0 <= 1; ++a0) {
-            double fp = 0.0, fh = 0.0;
-            node_dens<WP, WH>(tab, exptab, a0 ? xb + q.n1 + a0 * q.t[0] : xb, fp, fh);
-            pp += a0 ? fp : 4.0 * fp;
-            ph += a0 ? fh : 4.0 * fh;
-          }
-          sp = fma(w, pp, sp);
-          sh = fma(w, ph, sh);
-        }
-      }
-      sp *= 1.0 / 216.0;
-      sh *= 1.0 / 216.0;
+      if (WH && on_tail(q.hi)) dens_sums27<WP, WH, true>(tab, exptab, q, sp, sh);
+      else dens_sums27<WP, WH, false>(tab, exptab, q, sp, sh);
     }
   } else {
     const Nodes12 q(d, SQ6 * si, SQ6 * sj);
     in = inside(q.lo, q.hi);
     if (in) {
-#pragma unroll
-      for (int c = 0; c < 3; ++c) {
-        const double ti = q.gi * d[c], tj = q.gj * d[c];
-        const double x[4] = {q.xi + ti, q.xi - ti, q.xj - tj, q.xj + tj};
-#pragma unroll
-        for (int k = 0; k < 4; ++k) {
-          double fp = 0.0, fh = 0.0;
-          node_dens<WP, WH>(tab, exptab, x[k], fp, fh);
-          if (WP) sp += fp;
-          if (WH) sh += fh;
-        }
-      }
+      if (WH && on_tail(q.hi)) dens_sums12<WP, WH, true>(tab, exptab, q, d, sp, sh);
+      else dens_sums12<WP, WH, false>(tab, exptab, q, d, sp, sh);
     }
   }
   sh *= 11.0025;
@@ -690,8 +726,8 @@ __global__ __launch_bounds__(TB) void k_dens_recv64(const LatDev* __restrict__ l
 
 // One node inside the tables: the pair energy phi and cu = SH dE/ds, E = F'_i f_j
 // + F'_j f_i + phi.  FP multiplies f_Pd', FH f_H' / |r| (it carries FH_D).
-constexpr double FH_D = 0.5 * SH * -1.30927 * 11.0025;
-template <int KIND>
+constexpr double FH_D = 0.5 * SH * FH_K * 11.0025;
+template <int KIND, bool TAIL>
 __device__ __forceinline__ void node_coef(const double* tab, const double* exptab, double x, double FP, double FH,
                                           double& phi, double& cu) {
   const SPos p = s_pos(x);
@@ -699,14 +735,14 @@ __device__ __forceinline__ void node_coef(const double* tab, const double* expta
   if (KIND == 3) poly_vd(s_row(tab, G_PHH, p.k), p.u, phi, cu);
   if (KIND == 0) cu = fma(FP, poly<5>(s_row(tab, G_DFPD, p.k), p.u), cu);
   if (KIND != 0) {
-    double r, ri;
-    const double fh = fH_s(exptab, s_of(x), r, ri);
+    double r, ri, fh;
+    (void)fH_s<TAIL>(exptab, s_of(x), r, ri, fh);
     if (KIND == 3) {
       cu = fma(FH, fh * ri, cu);
     } else {  // phi_PdH from its rows in r
       const double y = fma(r, RINV, -156.0);
       double d;
-      poly_vd(s_row(tab, G_PHPDH, (int)y), __builtin_amdgcn_fract(y), phi, d);
+      poly_vd(s_row(tab, G_PHPDH, (int)y), eam::fract(y), phi, d);
       cu = fma(fma(FH, fh, (0.5 * SH * RINV) * d), ri, FP * poly<5>(s_row(tab, G_DFPD, p.k), p.u));
     }
   }
@@ -724,7 +760,7 @@ struct PairSums {
 //   sigma terms d . T + a U (site i), its negative (partner).
 // One axis of one site (2 nodes) per trip, the components rotating through d0
 // and h2: more rows in flight would not fit the registers of 4 waves per SIMD.
-template <int KIND>
+template <int KIND, bool TAIL>
 __device__ __forceinline__ PairSums pair_sums12(const double* tab, const double* exptab, const Nodes12& n,
                                                 const double d[3], double ai, double aj, double FP, double FH) {
   double pe = 0.0, su = 0.0, d0 = d[0], d1 = d[1], d2 = d[2], h0 = 0.0, h1 = 0.0, h2 = 0.0;
@@ -737,8 +773,8 @@ __device__ __forceinline__ PairSums pair_sums12(const double* tab, const double*
     for (int c = 0; c < 3; ++c) {
       const double t = g * d0;
       double phi0, phi1, u0, u1;
-      node_coef<KIND>(tab, exptab, xb + t, FP, FH, phi0, u0);
-      node_coef<KIND>(tab, exptab, xb - t, FP, FH, phi1, u1);
+      node_coef<KIND, TAIL>(tab, exptab, xb + t, FP, FH, phi0, u0);
+      node_coef<KIND, TAIL>(tab, exptab, xb - t, FP, FH, phi1, u1);
       pe += phi0 + phi1;
       const double T = u0 - u1;
       ue += u0 + u1;
@@ -769,7 +805,7 @@ __device__ __forceinline__ PairSums pair_sums12(const double* tab, const double*
 //   q-gradient  sum u r = d U + sqrt(3) s V,
 //   Sz = sum u (r . z) = sqrt(3) d . V + 3 s Wn,  d/dsigma_k = Sz sigma_k / s.
 // Weights 4 and 1 per axis, divided by 216 at the end; three nodes per trip.
-template <int KIND>
+template <int KIND, bool TAIL>
 __device__ __forceinline__ PairSums pair_sums27(const double* tab, const double* exptab, const Nodes27& q,
                                                 const double d[3], double sd, double si, double sj, double FP,
                                                 double FH) {
@@ -782,9 +818,9 @@ __device__ __forceinline__ PairSums pair_sums27(const double* tab, const double*
       const double xb = q.x0 + q.n1 * n2 + ((double)a2 * q.t[2] + (double)a1 * q.t[1]);
       const double w = (a2 ? 1.0 : 4.0) * (a1 ? 1.0 : 4.0);
       double f0, fm, fp, c0, cm, cp;
-      node_coef<KIND>(tab, exptab, xb, FP, FH, f0, c0);
-      node_coef<KIND>(tab, exptab, xb + q.n1 - q.t[0], FP, FH, fm, cm);
-      node_coef<KIND>(tab, exptab, xb + q.n1 + q.t[0], FP, FH, fp, cp);
+      node_coef<KIND, TAIL>(tab, exptab, xb, FP, FH, f0, c0);
+      node_coef<KIND, TAIL>(tab, exptab, xb + q.n1 - q.t[0], FP, FH, fm, cm);
+      node_coef<KIND, TAIL>(tab, exptab, xb + q.n1 + q.t[0], FP, FH, fp, cp);
       pe = fma(w, fma(4.0, f0, fm + fp), pe);
       const double e = cm + cp, u = w * fma(4.0, c0, e);
       U += u;
@@ -848,12 +884,18 @@ __device__ __forceinline__ bool pair_both(const double* tab, const double* expta
     const double sd = sqrt(fma(si, si, sj * sj));
     const Nodes27 n(d, sd);
     in = inside(n.lo, n.hi);
-    if (in) p = pair_sums27<KIND>(tab, exptab, n, d, sd, si, sj, FP, FH);
+    if (in) {
+      if (KIND != 0 && on_tail(n.hi)) p = pair_sums27<KIND, true>(tab, exptab, n, d, sd, si, sj, FP, FH);
+      else p = pair_sums27<KIND, false>(tab, exptab, n, d, sd, si, sj, FP, FH);
+    }
   } else {
     const double ai = SQ6 * si, aj = SQ6 * sj;
     const Nodes12 n(d, ai, aj);
     in = inside(n.lo, n.hi);
-    if (in) p = pair_sums12<KIND>(tab, exptab, n, d, ai, aj, FP, FH);
+    if (in) {
+      if (KIND != 0 && on_tail(n.hi)) p = pair_sums12<KIND, true>(tab, exptab, n, d, ai, aj, FP, FH);
+      else p = pair_sums12<KIND, false>(tab, exptab, n, d, ai, aj, FP, FH);
+    }
   }
   return in;
 }
@@ -1011,10 +1053,10 @@ enum { C_PHPDH = 0, C_PHH = 1, NCTAB = 2 };  // this pass's order in LDS
 template <bool NB_H>
 __device__ __forceinline__ void node_fh_phi(const double* tab, const double* exptab, double x, double w, double& sf,
                                             double& sp) {
-  double r, ri;
-  sf = fma(w, fH_s(exptab, s_of(x), r, ri), sf);
+  double r, ri, sl;
+  sf = fma(w, fH_s<true>(exptab, s_of(x), r, ri, sl), sf);
   const double y = NB_H ? x : fma(r, RINV, -156.0);
-  sp = fma(w, poly<5>(s_row(tab, NB_H ? C_PHH : C_PHPDH, (int)y), __builtin_amdgcn_fract(y)), sp);
+  sp = fma(w, poly<5>(s_row(tab, NB_H ? C_PHH : C_PHPDH, (int)y), eam::fract(y)), sp);
 }
 template <int RULE, bool NB_H>
 __device__ __forceinline__ bool pair_fh_phi(const double* tab, const double* exptab, const double d[3], double si,
@@ -1348,6 +1390,38 @@ void host_tables64_s(std::vector<double>& t) {
   t = built;
 }
 
+// One EAM function (order of a2c_eam_tables) at r in [1, 6) as the passes take it
+// from the tables t: value, and slope in r.
+void pass_eval64(const std::vector<double>& t, int fn, double r, double& v, double& d) {
+  const double s = r * r, x = fma(s, SINV, SB), *exptab = &t[S_EXP];
+  const SPos p = s_pos(x);
+  double r1, ri, sl;
+  const double fh = fH_s<true>(exptab, s, r1, ri, sl);
+  switch (fn) {
+    case 0:
+      v = poly<5>(s_row(t.data(), S_FPD, p.k), p.u);
+      d = 2.0 * SINV * r * poly<5>(s_row(t.data(), S_DFPD, p.k), p.u);
+      return;
+    case 1:
+      v = 11.0025 * fh;
+      d = FH_K * 11.0025 * sl;
+      return;
+    case 2:
+      poly6_vd(s_row(t.data(), S_PHPD, p.k), p.u, v, d);
+      d *= 2.0 * SINV * r;
+      return;
+    case 3: {
+      const double y = fma(r1, RINV, -156.0);
+      poly_vd(s_row(t.data(), S_PHPDH, (int)y), eam::fract(y), v, d);
+      d *= RINV;
+      return;
+    }
+    default:
+      poly_vd(s_row(t.data(), S_PHH, p.k), p.u, v, d);
+      d *= 2.0 * SINV * r;
+  }
+}
+
 // FP64 tables in r (exported, a2c_eam_tables64): on each 0.05 A interval the polynomial (degree 8 for the
 // exponential functions, 11 for the Pd polynomials) interpolating the
 // long-double closed form at the Chebyshev points, in Newton form, expanded
@@ -1520,4 +1594,27 @@ extern "C" int a2c_eam_tables64(double* out, int32_t cap) {
   const int n = (int)t.size();
   if (out && cap >= n) std::memcpy(out, t.data(), sizeof(double) * n);
   return n;
+}
+
+// Host-only: an EAM function as the pair-once passes evaluate it (a2c_fe.h).
+extern "C" int a2c_eam_pass(int32_t precision, int32_t fn, int32_t n, const double* r, double* r_at, double* v,
+                            double* d) {
+  if ((precision != A2C_PREC_FP64 && precision != A2C_PREC_MIXED) || fn < 0 || fn > 4 || n < 0) return A2C_EINVAL;
+  if (n > 0 && (!r || !r_at || !v || !d)) return A2C_EINVAL;
+  std::vector<double> t64;
+  std::vector<float4> t32;
+  if (precision == A2C_PREC_FP64) a2c::host_tables64_s(t64);
+  else a2c::host_tables_s(t32);
+  for (int i = 0; i < n; ++i) {
+    if (!(r[i] >= 1.0 && r[i] < 5.999)) return A2C_EINVAL;
+    if (precision == A2C_PREC_FP64) {
+      r_at[i] = r[i];
+      a2c::pass_eval64(t64, fn, r[i], v[i], d[i]);
+    } else {
+      const float s = (float)(r[i] * r[i]);
+      r_at[i] = std::sqrt((double)s);
+      a2c::pass_eval32(t32, fn, s, v[i], d[i]);
+    }
+  }
+  return A2C_OK;
 }
