@@ -344,37 +344,45 @@ struct Closed {
   }
 };
 
-// The owner passes read the EAM functions from polynomial tables on a uniform
-// grid in s = |r|^2 (a node's coordinate is one addition, and dE/ds = (dE/dr) /
-// (2 |r|) is what the gradient needs: no square root per node).  h = 0.5025 / 12
-// puts the switch radii 5.0 and 5.05 A on grid nodes (25 and 25.5025 A^2; 5.35 A
-// joins two forms of the same function); the rows reach past 36 A^2.  Each row is
-// a polynomial in u in [0, 1) of six doubles: f_Pd and its slope interpolated at
-// the Chebyshev points, the pair functions as the integral of the interpolant of
-// their slope, so that value and slope belong together.  Slopes are within
-// 1e-12 of the closed forms at every distance that occurs.  That takes degree 5
-// for the slope of phi_Pd, whose part 2 0.251546 f_Pd falls as e^{-51.6 (r - 5)}
-// between 5.0 and 5.05 A: its two highest coefficients, at most 1e-4 of the
-// slope, share the sixth double as FP32 (rounding 1e-12).  Four functions on
-// this grid fill the 160 KB of LDS (one workgroup per CU); every row gathered
-// costs the CU's LDS ~30 clocks per wave.  f_H =
-// 11.0025 exp(-1.30927 |r|) is computed instead (exp2 by a 256-entry table and a
-// degree-4 polynomial): ~25 FP64 instructions on four SIMDs cost no more than a
-// row, and the two pipes work side by side.
-constexpr double SH = 0.5025 / 12.0, S0 = 25.5025 - 587 * SH, SINV = 1.0 / SH, SB = -S0 / SH;
+// The owner passes read the EAM functions from polynomial tables.  The Pd functions
+// stand on a uniform grid in s = |r|^2 (a node's coordinate is one addition, and
+// dE/ds = (dE/dr) / (2 |r|) is what the gradient needs: no square root per
+// node); h = 0.5025 / 13 puts their switch radii 5.0 and 5.05 A on grid nodes (25
+// and 25.5025 A^2), and the rows reach past 36 A^2.  phi_PdH and phi_HH have rows
+// in r, 1/40 A apart: exponentials are steepest at short distances, where steps
+// in s are the longest in r; their other switch radius 5.35 A is a node of that
+// grid; and a node of an H pair has r at hand from f_H.  A row is a polynomial in
+// u in [0, 1): f_Pd (degree 7, density pass) and its slope (degree 7) interpolated
+// at the Chebyshev points, the pair functions (phi_Pd degree 8, phi_PdH and phi_HH
+// 7) as the integral of the interpolant of their slope, so that value and slope
+// belong together.  The degrees are the lowest whose interpolation errors stay
+// below the FP64 roundings of the closed forms: part of the Pd functions falls as
+// e^{-51.6 (r - 5)} beyond 5.0 A, where degree 5 left 5e-12 of slopes of 0.08, and
+// phi_HH in s 2e-11 at 2 A and 1.7e-9 across 5.35 A; now below 1e-15 and 1e-14
+// (tests/test_pass_tables.py holds every function).  Row pitches are 16-byte
+// multiples that spread a wave's rows over 16 bank groups (8 doubles: 4); the
+// tables fill 158 of the 160 KB of LDS (one workgroup per CU).  f_H = 11.0025
+// exp(-1.30927 |r|) is computed instead (exp2 by a 256-entry table and a degree-4
+// polynomial): ~25 FP64 instructions on four SIMDs cost no more than a row, and the
+// two pipes work side by side.
+// A node's coordinate is x = SINV s + SB; the rows are built on the grid that these
+// two doubles define (rounded apart, the grid would be 4e-15 off: 5e-14 of a slope
+// at 1 A).
+constexpr double SINV = 13.0 / 0.5025, SB = 635 - 25.5025 * SINV, SH = 1.0 / SINV, S0 = -SB / SINV;
 constexpr double SLO = 1.0, SHI = 36.0;  // nodes the tables serve: [1, 6) A
-constexpr int SNT = 839, SP = 6;         // rows, doubles per row
-static_assert(587 * SH < 24.5815 && S0 < 1.0 && S0 + (SNT - 1) * SH > 36.0, "the grid covers [1, 36] A^2");
-enum { S_FPD = 0, S_DFPD = 1, S_PHPD = 2, S_PHPDH = 3, S_PHH = 4, NSTAB = 5 };
-// phi_PdH has its rows in r instead, RH apart from R0 on: e^{-4.8 r} is steepest
-// at the Pd-H distances, where steps in s are the longest in r (slope 1e-10 off
-// at 1.6 A), and a Pd-H node has r at hand from f_H.
-constexpr double RH = 1.0 / 160.0, RINV = 160.0, R0 = 156.0 / 160.0;
-static_assert(R0 + (SNT - 1) * RH > 6.0, "the grid covers [1, 6] A");
-constexpr int S_ROWS = SNT * SP;                 // doubles per function
-constexpr int EXPN = 256;                        // 2^(i / 256)
-constexpr int S_EXP = NSTAB * S_ROWS, S_SIZE = S_EXP + EXPN;
-enum { G_DFPD = 0, G_PHPD = 1, G_PHPDH = 2, G_PHH = 3, NGTAB = 4 };  // the gradient pass's order in LDS
+constexpr int SNT = 908;                 // rows in s
+static_assert(S0 < 1.0 && S0 + (SNT - 1) * SH > 36.0, "the grid covers [1, 36] A^2");
+constexpr double RH = 1.0 / 40.0, RINV = 40.0, RB = -39.0;
+constexpr int RNT = 202;                 // rows in r, the first at 39/40 A
+static_assert((-RB + RNT - 0.5) * RH > 6.0, "the grid covers [1, 6] A");
+constexpr int FD = 7, FP = 10;           // f_Pd rows: degree, pitch
+constexpr int GD = 7, PHD = 8, GP = 18;  // f_Pd' (c0..c7) and phi_Pd (from 8) rows: degrees, common pitch
+constexpr int RD = 7, RP = 18;           // phi_PdH and phi_HH (from 8) rows
+constexpr int EXPN = 256;                // 2^(i / 256)
+// offsets in doubles; each pass stages a contiguous part
+constexpr int S_FPD = 0, S_PD = S_FPD + SNT * FP, S_PH = S_PD + SNT * GP, S_EXP = S_PH + RNT * RP;
+constexpr int S_SIZE = S_EXP + EXPN;
+static_assert(8 * (S_SIZE - S_PD) <= 160 << 10, "the gradient pass's tables fit the LDS");
 
 struct SPos {
   int k;
@@ -382,41 +390,47 @@ struct SPos {
 };
 A2C_HD SPos s_pos(double x) { return {(int)x, eam::fract(x)}; }
 A2C_HD double s_of(double x) { return fma(x, SH, S0); }
-A2C_HD const double* s_row(const double* tab, int f, int k) { return tab + f * S_ROWS + eam::mul24(k, SP); }
+template <int P>
+A2C_HD const double* row_at(const double* tab, int k) { return tab + eam::mul24(k, P); }
+// D + 1 coefficients of a row (16-byte aligned), as 16-byte reads
 template <int D>
-A2C_HD double poly(const double* c, double u) {
-  double v = c[D];
+struct Coef {
+  double c[D + 1];
+  A2C_HD explicit Coef(const double* p) {
 #pragma unroll
-  for (int j = D - 1; j >= 0; --j) v = fma(v, u, c[j]);
+    for (int j = 0; j < D; j += 2) {
+      const double2 v = *reinterpret_cast<const double2*>(p + j);
+      c[j] = v.x;
+      c[j + 1] = v.y;
+    }
+    if (D % 2 == 0) c[D] = p[D];
+  }
+};
+template <int D>
+A2C_HD double poly(const double* row, double u) {
+  const Coef<D> q(row);
+  double v = q.c[D];
+#pragma unroll
+  for (int j = D - 1; j >= 0; --j) v = fma(v, u, q.c[j]);
   return v;
 }
 // value and d/du
-A2C_HD void poly_vd(const double* c, double u, double& v, double& d) {
-  v = fma(c[5], u, c[4]);
-  d = fma(c[5], u, v);
+template <int D>
+A2C_HD void poly_vd(const double* row, double u, double& v, double& d) {
+  const Coef<D> q(row);
+  v = fma(q.c[D], u, q.c[D - 1]);
+  d = fma(q.c[D], u, v);
 #pragma unroll
-  for (int j = 3; j >= 1; --j) {
-    v = fma(v, u, c[j]);
+  for (int j = D - 2; j >= 1; --j) {
+    v = fma(v, u, q.c[j]);
     d = fma(d, u, v);
   }
-  v = fma(v, u, c[0]);
+  v = fma(v, u, q.c[0]);
 }
-// the same for a degree-6 row whose last two coefficients share a double (phi_Pd)
-A2C_HD void poly6_vd(const double* c, double u, double& v, double& d) {
-  const double2 c45 = *reinterpret_cast<const double2*>(c + 4);  // one 16-byte read
-  float f2[2];
-  __builtin_memcpy(f2, &c45.y, 8);
-  const double hy = f2[1];
-  v = fma(hy, u, (double)f2[0]);
-  d = fma(hy, u, v);
-  v = fma(v, u, c45.x);
-  d = fma(d, u, v);
-#pragma unroll
-  for (int j = 3; j >= 1; --j) {
-    v = fma(v, u, c[j]);
-    d = fma(d, u, v);
-  }
-  v = fma(v, u, c[0]);
+// phi_PdH (tab: its rows) or phi_HH (8 beyond) at r, and d/du
+A2C_HD void phi_r(const double* tab, double r, double& v, double& d) {
+  const double y = fma(r, RINV, RB);
+  poly_vd<RD>(row_at<RP>(tab, (int)y), eam::fract(y), v, d);
 }
 A2C_HD long long double_bits(double x) {
   long long b;
@@ -501,7 +515,7 @@ template <bool WANT_PD, bool WANT_H, bool TAIL>
 __device__ __forceinline__ void node_dens(const double* tab, const double* exptab, double x, double& fpd, double& fh) {
   if (WANT_PD) {
     const SPos p = s_pos(x);
-    fpd = poly<5>(s_row(tab, 0, p.k), p.u);
+    fpd = poly<FD>(row_at<FP>(tab, p.k), p.u);
   }
   if (WANT_H) {
     double r, ri, sl;
@@ -662,14 +676,17 @@ __device__ __forceinline__ void dens_list(const double* tab, const double* expta
     });
 }
 
-// Bound by the LDS and the vector ALUs (40^3 cells: 60% and 75% busy): 654 us
-// with the tables in |r|, 276 us; Gauss-Hermite rule 1386 and 604 us.
+// Bound by the LDS (a row of 8 doubles) and the vector ALUs.  40^3 cells, events of
+// a2c_fe_time_eval: 320 us, Gauss-Hermite rule 708 (278 and 621 with rows of
+// degree 5, whose values were 1e-12 off at 1.1 A and 1e-13 beyond 5.0 A; 575 us
+// with rows 8 doubles apart).
 template <int RULE, int TBO, bool BY_SITE>
 __global__ __launch_bounds__(TBO) __attribute__((amdgpu_waves_per_eu(4))) void k_dens_own64(
     const LatDev* __restrict__ lats, const int32_t* __restrict__ ob2l, int nblk, const double* __restrict__ gtab) {
-  __shared__ __align__(16) double tab[S_ROWS + EXPN];  // f_Pd, 2^(i/256)
-  stage16(tab, gtab + S_FPD * S_ROWS, S_ROWS / 2);
-  stage16(tab + S_ROWS, gtab + S_EXP, EXPN / 2);
+  constexpr int ROWS = SNT * FP;
+  __shared__ __align__(16) double tab[ROWS + EXPN];  // f_Pd, 2^(i/256)
+  stage16(tab, gtab + S_FPD, ROWS / 2);
+  stage16(tab + ROWS, gtab + S_EXP, EXPN / 2);
   __syncthreads();
   const int w = xcd_block() * (TBO / TB) + __builtin_amdgcn_readfirstlane(threadIdx.x / TB);
   if (w >= nblk) return;
@@ -684,11 +701,11 @@ __global__ __launch_bounds__(TBO) __attribute__((amdgpu_waves_per_eu(4))) void k
   const Site a = own_site<BY_SITE>(S, ln, wme);
   double rho = 0.0;
   if (ln.pd) {
-    dens_list<RULE, BY_SITE, false, false>(tab, tab + S_ROWS, S, ln, a, img, 1.0, rho);
-    dens_list<RULE, BY_SITE, true, false>(tab, tab + S_ROWS, S, ln, a, img, 1.0, rho);
+    dens_list<RULE, BY_SITE, false, false>(tab, tab + ROWS, S, ln, a, img, 1.0, rho);
+    dens_list<RULE, BY_SITE, true, false>(tab, tab + ROWS, S, ln, a, img, 1.0, rho);
   } else {
-    dens_list<RULE, BY_SITE, false, true>(tab, tab + S_ROWS, S, ln, a, img, wme, rho);
-    dens_list<RULE, BY_SITE, true, true>(tab, tab + S_ROWS, S, ln, a, img, wme, rho);
+    dens_list<RULE, BY_SITE, false, true>(tab, tab + ROWS, S, ln, a, img, wme, rho);
+    dens_list<RULE, BY_SITE, true, true>(tab, tab + ROWS, S, ln, a, img, wme, rho);
   }
   rho = site_sum(rho, K);
   if (ln.ph == 0) gmem(S.epair)[s] = rho;  // free until the gradient pass
@@ -726,25 +743,26 @@ __global__ __launch_bounds__(TB) void k_dens_recv64(const LatDev* __restrict__ l
 
 // One node inside the tables: the pair energy phi and cu = SH dE/ds, E = F'_i f_j
 // + F'_j f_i + phi.  FP multiplies f_Pd', FH f_H' / |r| (it carries FH_D).
+constexpr int G_PH = S_PH - S_PD, G_EXP = S_EXP - S_PD;  // of the staged part
 constexpr double FH_D = 0.5 * SH * FH_K * 11.0025;
 template <int KIND, bool TAIL>
-__device__ __forceinline__ void node_coef(const double* tab, const double* exptab, double x, double FP, double FH,
+__device__ __forceinline__ void node_coef(const double* tab, const double* exptab, double x, double FP_, double FH,
                                           double& phi, double& cu) {
-  const SPos p = s_pos(x);
-  if (KIND == 0) poly6_vd(s_row(tab, G_PHPD, p.k), p.u, phi, cu);
-  if (KIND == 3) poly_vd(s_row(tab, G_PHH, p.k), p.u, phi, cu);
-  if (KIND == 0) cu = fma(FP, poly<5>(s_row(tab, G_DFPD, p.k), p.u), cu);
-  if (KIND != 0) {
-    double r, ri, fh;
+  const double* row = nullptr;
+  SPos p{};
+  if (KIND != 3) {
+    p = s_pos(x);
+    row = row_at<GP>(tab, p.k);
+  }
+  if (KIND == 0) {
+    poly_vd<PHD>(row + 8, p.u, phi, cu);
+    cu = fma(FP_, poly<GD>(row, p.u), cu);
+  } else {
+    double r, ri, fh, d;
     (void)fH_s<TAIL>(exptab, s_of(x), r, ri, fh);
-    if (KIND == 3) {
-      cu = fma(FH, fh * ri, cu);
-    } else {  // phi_PdH from its rows in r
-      const double y = fma(r, RINV, -156.0);
-      double d;
-      poly_vd(s_row(tab, G_PHPDH, (int)y), eam::fract(y), phi, d);
-      cu = fma(fma(FH, fh, (0.5 * SH * RINV) * d), ri, FP * poly<5>(s_row(tab, G_DFPD, p.k), p.u));
-    }
+    phi_r(tab + G_PH + (KIND == 3 ? 8 : 0), r, phi, d);
+    cu = fma(FH, fh, (0.5 * SH * RINV) * d);
+    cu = KIND == 3 ? cu * ri : fma(cu, ri, FP_ * poly<GD>(row, p.u));
   }
 }
 
@@ -951,18 +969,18 @@ __device__ __forceinline__ void grad_list(const double* tab, const double* expta
     });
 }
 
-// Bound by the LDS and the vector ALUs together (each busy 57% of the time at 2
-// waves per SIMD; 163 KB of tables leave one workgroup per CU, and 1024 lanes, 4
-// waves per SIMD, spill: 645 against 625 us).  40^3 cells: 1384 us before (degree
-// 8 / 11 tables in |r|, f_Pd' in closed form, two Newton steps per node, 153
-// instructions per node), 625 us; Gauss-Hermite rule 2920 and 1200 us.  f_H' from a
-// table, too, took 691 us.  Gradient error against 80-bit arithmetic (3^3 and 4^3
-// cells): 4e-12 to 1e-11 before, 3e-13 to 8e-13.
+// Bound by the LDS, with the vector ALUs close behind, at 2 waves per SIMD (the
+// tables leave one workgroup per CU; 1024 lanes, 4 waves per SIMD, spill).  40^3
+// cells, events of a2c_fe_time_eval: 670 us, Gauss-Hermite rule 1368 (562 and 1112
+// with rows of degree 5, phi_HH in s and phi_Pd's last coefficients as floats;
+// 1017 us with rows 17 doubles apart, read as 8-byte words).  Gradient error against
+// 80-bit arithmetic (3^3 and 4^3 cells): 1e-14 to 3e-14; 3e-13 to 8e-13 with those
+// rows, 4e-12 to 1e-11 with closed-form Pd slopes.
 template <int RULE, int TBO>
 __global__ __launch_bounds__(TBO) __attribute__((amdgpu_waves_per_eu(TBO / 256))) void k_grad_own64(
     const LatDev* __restrict__ lats, const int32_t* __restrict__ ob2l, int nblk, const double* __restrict__ gtab) {
-  __shared__ __align__(16) double tab[NGTAB * S_ROWS + EXPN];
-  stage16(tab, gtab + S_DFPD * S_ROWS, (NGTAB * S_ROWS + EXPN) / 2);  // the exp2 table follows the functions
+  __shared__ __align__(16) double tab[G_EXP + EXPN];
+  stage16(tab, gtab + S_PD, (G_EXP + EXPN) / 2);
   __syncthreads();
   const int w = xcd_block() * (TBO / TB) + __builtin_amdgcn_readfirstlane(threadIdx.x / TB);
   if (w >= nblk) return;
@@ -971,7 +989,7 @@ __global__ __launch_bounds__(TBO) __attribute__((amdgpu_waves_per_eu(TBO / 256))
   const int K = S.kl64;
   const OwnerLane ln(S, w - S.owg0_64, K);
   if (ln.row >= ln.rows) return;  // whole lane groups
-  const double* exptab = tab + NGTAB * S_ROWS;
+  const double* exptab = tab + G_EXP;
   const Image img = image_of(S);
   const int s = ln.pd ? ln.row : S.npd + ln.row;
   const Site a = load_row(gmem((const double2*)S.qxy), gmem((const double2*)S.qzs), s);
@@ -1049,14 +1067,45 @@ __global__ __launch_bounds__(TB) void k_grad_recv64(const LatDev* __restrict__ l
 // ================================================================ chemical potential
 // f_H and phi (phi_PdH, or phi_HH for an H neighbor) summed over a pair's nodes,
 // with the rule's weights; false, and zeros, if a node lies outside the tables.
-enum { C_PHPDH = 0, C_PHH = 1, NCTAB = 2 };  // this pass's order in LDS
-template <bool NB_H>
+constexpr int C_EXP = S_EXP - S_PH;  // of the staged part
+template <bool NB_H, bool TAIL>
 __device__ __forceinline__ void node_fh_phi(const double* tab, const double* exptab, double x, double w, double& sf,
                                             double& sp) {
   double r, ri, sl;
-  sf = fma(w, fH_s<true>(exptab, s_of(x), r, ri, sl), sf);
-  const double y = NB_H ? x : fma(r, RINV, -156.0);
-  sp = fma(w, poly<5>(s_row(tab, NB_H ? C_PHH : C_PHPDH, (int)y), eam::fract(y)), sp);
+  sf = fma(w, fH_s<TAIL>(exptab, s_of(x), r, ri, sl), sf);
+  const double y = fma(r, RINV, RB);
+  sp = fma(w, poly<RD>(row_at<RP>(tab + (NB_H ? 8 : 0), (int)y), eam::fract(y)), sp);
+}
+template <bool NB_H, bool TAIL>
+__device__ __forceinline__ void fh_phi_sums27(const double* tab, const double* exptab, const Nodes27& q, double& sf,
+                                              double& sp) {
+#pragma unroll 1
+  for (int k = 0; k < 9; ++k) {
+    const int a2 = k / 3 - 1, a1 = k % 3 - 1;
+    const double xb = q.x0 + q.n1 * (double)(a2 * a2 + a1 * a1) + ((double)a2 * q.t[2] + (double)a1 * q.t[1]);
+    const double w = (a2 ? 1.0 : 4.0) * (a1 ? 1.0 : 4.0);
+#pragma unroll
+    for (int a0 = -1; a0 <= 1; ++a0)
+      node_fh_phi<NB_H, TAIL>(tab, exptab, a0 ? xb + q.n1 + a0 * q.t[0] : xb, a0 ? w : 4.0 * w, sf, sp);
+  }
+  sf *= 11.0025 / 216.0;
+  sp *= 1.0 / 216.0;
+}
+template <bool NB_H, bool TAIL>
+__device__ __forceinline__ void fh_phi_sums12(const double* tab, const double* exptab, const Nodes12& q,
+                                              const double d[3], double& sf, double& sp) {
+  double d0 = d[0], d1 = d[1], d2 = d[2];
+#pragma unroll 1
+  for (int c = 0; c < 3; ++c) {
+    const double ti = q.gi * d0, tj = q.gj * d0;
+    const double x[4] = {q.xi + ti, q.xi - ti, q.xj - tj, q.xj + tj};
+#pragma unroll
+    for (int k = 0; k < 4; ++k) node_fh_phi<NB_H, TAIL>(tab, exptab, x[k], 1.0, sf, sp);
+    d0 = d1;
+    d1 = d2;
+  }
+  sf *= 11.0025 * QW;
+  sp *= QW;
 }
 template <int RULE, bool NB_H>
 __device__ __forceinline__ bool pair_fh_phi(const double* tab, const double* exptab, const double d[3], double si,
@@ -1065,32 +1114,13 @@ __device__ __forceinline__ bool pair_fh_phi(const double* tab, const double* exp
   if (RULE == GH3) {
     const Nodes27 q(d, sqrt(fma(si, si, sj * sj)));
     if (!inside(q.lo, q.hi)) return false;
-#pragma unroll 1
-    for (int k = 0; k < 9; ++k) {
-      const int a2 = k / 3 - 1, a1 = k % 3 - 1;
-      const double xb = q.x0 + q.n1 * (double)(a2 * a2 + a1 * a1) + ((double)a2 * q.t[2] + (double)a1 * q.t[1]);
-      const double w = (a2 ? 1.0 : 4.0) * (a1 ? 1.0 : 4.0);
-#pragma unroll
-      for (int a0 = -1; a0 <= 1; ++a0)
-        node_fh_phi<NB_H>(tab, exptab, a0 ? xb + q.n1 + a0 * q.t[0] : xb, a0 ? w : 4.0 * w, sf, sp);
-    }
-    sf *= 11.0025 / 216.0;
-    sp *= 1.0 / 216.0;
+    if (on_tail(q.hi)) fh_phi_sums27<NB_H, true>(tab, exptab, q, sf, sp);
+    else fh_phi_sums27<NB_H, false>(tab, exptab, q, sf, sp);
   } else {
     const Nodes12 q(d, SQ6 * si, SQ6 * sj);
     if (!inside(q.lo, q.hi)) return false;
-    double d0 = d[0], d1 = d[1], d2 = d[2];
-#pragma unroll 1
-    for (int c = 0; c < 3; ++c) {
-      const double ti = q.gi * d0, tj = q.gj * d0;
-      const double x[4] = {q.xi + ti, q.xi - ti, q.xj - tj, q.xj + tj};
-#pragma unroll
-      for (int k = 0; k < 4; ++k) node_fh_phi<NB_H>(tab, exptab, x[k], 1.0, sf, sp);
-      d0 = d1;
-      d1 = d2;
-    }
-    sf *= 11.0025 * QW;
-    sp *= QW;
+    if (on_tail(q.hi)) fh_phi_sums12<NB_H, true>(tab, exptab, q, d, sf, sp);
+    else fh_phi_sums12<NB_H, false>(tab, exptab, q, d, sf, sp);
   }
   return true;
 }
@@ -1162,15 +1192,16 @@ __device__ __forceinline__ void chem_list(const double* tab, const double* expta
 
 // Chemical potential of the H sites (occupancy.hip has the formula), K lanes per
 // row over the full lists, from rho and F' in row order.  24^3 cells: one lane per
-// site and closed forms 353 us, this 117 us (4 waves per SIMD; LDS and FP64 units both busy);
-// error against 80-bit arithmetic 1e-12 before, 3e-15 now.
+// site and closed forms 353 us, this 118 us (4 waves per SIMD; LDS and FP64 units both
+// busy); error against 80-bit arithmetic 1.3e-12 to 2.3e-12 before, 2.3e-15 to 4.3e-15
+// now.
 template <int RULE, int TBO>
-__global__ __launch_bounds__(TBO) void k_chem64(const LatDev* __restrict__ lat, int units, int K,
+__global__ __launch_bounds__(TBO) __attribute__((amdgpu_waves_per_eu(TBO / 256, TBO / 256))) void k_chem64(const LatDev* __restrict__ lat, int units, int K,
                                                 const double* __restrict__ gtab, ChemArgs c) {
-  __shared__ __align__(16) double tab[NCTAB * S_ROWS + EXPN];
-  stage16(tab, gtab + S_PHPDH * S_ROWS, (NCTAB * S_ROWS + EXPN) / 2);  // phi_PdH, phi_HH, 2^(i/256)
+  __shared__ __align__(16) double tab[C_EXP + EXPN];
+  stage16(tab, gtab + S_PH, (C_EXP + EXPN) / 2);  // phi_PdH, phi_HH, 2^(i/256)
   __syncthreads();
-  const double* exptab = tab + NCTAB * S_ROWS;
+  const double* exptab = tab + C_EXP;
   const int u = xcd_block() * (TBO / TB) + __builtin_amdgcn_readfirstlane(threadIdx.x / TB);
   if (u >= units) return;
   const LatDev& S = *lat;
@@ -1328,62 +1359,57 @@ void host_tables64_s(std::vector<double>& t) {
   static const std::vector<double> built = [] {
     using LD = long double;
     std::vector<double> out((size_t)S_SIZE, 0.0);
-    const LD PI = 3.14159265358979323846264338327950288L, h = 0.5025L / 12, s0 = 25.5025L - 587 * h;
+    const LD PI = 3.14159265358979323846264338327950288L, h = 1 / (LD)SINV, s0 = -(LD)SB / SINV;
     auto node = [&](int i, int n) { return 0.5L - 0.5L * cosl((2 * i + 1) * PI / (2.0L * n)); };
+    constexpr int MAXC = 12;
     // polynomial through (u[i], y[i]), i < n, as monomials
     auto through = [](const LD* u, const LD* y, int n, LD* m) {
-      LD c[SP];
+      LD c[MAXC];
       for (int i = 0; i < n; ++i) c[i] = y[i];
       for (int j = 1; j < n; ++j)
         for (int i = n - 1; i >= j; --i) c[i] = (c[i] - c[i - 1]) / (u[i] - u[i - j]);
-      for (int q = 0; q < SP; ++q) m[q] = 0;
+      for (int q = 0; q < MAXC; ++q) m[q] = 0;
       for (int i = n - 1; i >= 0; --i) {
-        for (int q = SP - 1; q > 0; --q) m[q] = m[q - 1] - u[i] * m[q];
+        for (int q = MAXC - 1; q > 0; --q) m[q] = m[q - 1] - u[i] * m[q];
         m[0] = c[i] - u[i] * m[0];
       }
     };
     enum { VALUE, SLOPE, BOTH };
-    auto fill = [&](int f, int fit, auto g) {  // g: value and slope in r
-      for (int k = 0; k < SNT; ++k) {
+    // rows of degree deg at out[base + k pitch]; g: value and slope in r
+    auto fill = [&](int base, int pitch, int rows, bool in_r, int deg, int fit, auto g) {
+      for (int k = 0; k < rows; ++k) {
         auto at = [&](LD u) {
-          const LD r = f == S_PHPDH ? (156 + k + u) / 160.0L : sqrtl(s0 + (k + u) * h);
+          const LD r = in_r ? (k + u - RB) / RINV : sqrtl(s0 + (k + u) * h);
           const eam::VDT<LD> v = g(r);
-          return eam::VDT<LD>{v.v, v.d * (f == S_PHPDH ? 1 / 160.0L : h / (2 * r))};  // d/du
+          return eam::VDT<LD>{v.v, v.d * (in_r ? 1 / (LD)RINV : h / (2 * r))};  // d/du
         };
-        const bool split = f == S_PHPD;  // degree 6, the last two coefficients as floats
-        const int n = fit == BOTH && !split ? SP - 1 : SP;
-        LD u[SP], y[SP], m[SP + 1];
+        const int n = fit == BOTH ? deg : deg + 1;
+        LD u[MAXC], y[MAXC], m[MAXC];
         for (int i = 0; i < n; ++i) {
           u[i] = node(i, n);
           y[i] = fit == VALUE ? at(u[i]).v : at(u[i]).d;
         }
         through(u, y, n, m);
         if (fit == BOTH) {  // the slope's integral, with the value's mean over the Chebyshev points
-          for (int q = SP; q > 0; --q) m[q] = m[q - 1] / q;  // the slope's degree is n - 1
-          if (!split) m[SP] = 0;
+          for (int q = deg; q > 0; --q) m[q] = m[q - 1] / q;
           m[0] = 0;
           LD c = 0;
-          for (int i = 0; i < SP; ++i) {
-            const LD w = node(i, SP);
+          for (int i = 0; i < 8; ++i) {
+            const LD w = node(i, 8);
             LD v = 0;
-            for (int q = SP; q >= 0; --q) v = v * w + m[q];
+            for (int q = deg; q >= 0; --q) v = v * w + m[q];
             c += at(w).v - v;
           }
-          m[0] = c / SP;
+          m[0] = c / 8;
         }
-        double* row = &out[(size_t)f * S_ROWS + (size_t)k * SP];
-        for (int q = 0; q < SP; ++q) row[q] = (double)m[q];
-        if (split) {
-          const float hi[2] = {(float)m[5], (float)m[6]};
-          std::memcpy(row + 5, hi, sizeof hi);
-        }
+        for (int q = 0; q <= deg; ++q) out[(size_t)base + (size_t)k * pitch + q] = (double)m[q];
       }
     };
-    fill(S_FPD, VALUE, [](LD r) { return eam::f_Pd_vd<LD>(r); });
-    fill(S_DFPD, SLOPE, [](LD r) { return eam::f_Pd_vd<LD>(r); });
-    fill(S_PHPD, BOTH, [](LD r) { return eam::phi_Pd_vd<LD>(r, eam::f_Pd_vd<LD>(r)); });
-    fill(S_PHPDH, BOTH, [](LD r) { return eam::phi_morse_vd<0, LD>(r); });
-    fill(S_PHH, BOTH, [](LD r) { return eam::phi_morse_vd<1, LD>(r); });
+    fill(S_FPD, FP, SNT, false, FD, VALUE, [](LD r) { return eam::f_Pd_vd<LD>(r); });
+    fill(S_PD, GP, SNT, false, GD, SLOPE, [](LD r) { return eam::f_Pd_vd<LD>(r); });
+    fill(S_PD + 8, GP, SNT, false, PHD, BOTH, [](LD r) { return eam::phi_Pd_vd<LD>(r, eam::f_Pd_vd<LD>(r)); });
+    fill(S_PH, RP, RNT, true, RD, BOTH, [](LD r) { return eam::phi_morse_vd<0, LD>(r); });
+    fill(S_PH + 8, RP, RNT, true, RD, BOTH, [](LD r) { return eam::phi_morse_vd<1, LD>(r); });
     for (int i = 0; i < EXPN; ++i) out[S_EXP + i] = (double)exp2l((LD)i / EXPN);
     return out;
   }();
@@ -1397,28 +1423,21 @@ void pass_eval64(const std::vector<double>& t, int fn, double r, double& v, doub
   const SPos p = s_pos(x);
   double r1, ri, sl;
   const double fh = fH_s<true>(exptab, s, r1, ri, sl);
-  switch (fn) {
-    case 0:
-      v = poly<5>(s_row(t.data(), S_FPD, p.k), p.u);
-      d = 2.0 * SINV * r * poly<5>(s_row(t.data(), S_DFPD, p.k), p.u);
-      return;
-    case 1:
-      v = 11.0025 * fh;
-      d = FH_K * 11.0025 * sl;
-      return;
-    case 2:
-      poly6_vd(s_row(t.data(), S_PHPD, p.k), p.u, v, d);
-      d *= 2.0 * SINV * r;
-      return;
-    case 3: {
-      const double y = fma(r1, RINV, -156.0);
-      poly_vd(s_row(t.data(), S_PHPDH, (int)y), eam::fract(y), v, d);
-      d *= RINV;
-      return;
+  if (fn == 1) {
+    v = 11.0025 * fh;
+    d = FH_K * 11.0025 * sl;
+  } else if (fn > 2) {
+    phi_r(&t[S_PH + (fn == 3 ? 0 : 8)], r1, v, d);
+    d *= RINV;
+  } else {
+    const double* row = row_at<GP>(&t[S_PD], p.k);
+    if (fn == 0) {
+      v = poly<FD>(row_at<FP>(&t[S_FPD], p.k), p.u);
+      d = poly<GD>(row, p.u);
+    } else {
+      poly_vd<PHD>(row + 8, p.u, v, d);
     }
-    default:
-      poly_vd(s_row(t.data(), S_PHH, p.k), p.u, v, d);
-      d *= 2.0 * SINV * r;
+    d *= 2.0 * SINV * r;
   }
 }
 
