@@ -385,29 +385,48 @@ __global__ __launch_bounds__(TB) void k_grad32(const LatDev* __restrict__ lats, 
 // received slot; a gather kernel adds the received shares in FP64.  Each
 // buffer entry is written by exactly one lane, so results are deterministic.
 
-// The owner passes read the EAM functions from cubic tables on a uniform
-// grid in s = |r|^2: a node's s is D2 + a^2 +- 2 a d_c (linear in what
-// differs between the nodes of a pair), so the table coordinate of a node is
-// one addition, and dE/ds = (dE/dr) / (2 |r|) is the factor every gradient term needs --
-// no square root and no division per node.  h = 0.5025 / 14 puts the switch
-// radii 5.0 and 5.05 A on grid nodes (25 and 25.5025 A^2; 5.35 A joins two
-// forms of the same function); SNT intervals from S0 reach past 36 A^2.
+// The owner passes read the EAM functions from cubic tables.  The Pd functions
+// stand on a uniform grid in s = |r|^2: a node's s is D2 + a^2 +- 2 a d_c (linear
+// in what differs between the nodes of a pair), so the table coordinate of a node
+// is one addition, and dE/ds = (dE/dr) / (2 |r|) is the factor every gradient term
+// needs -- no square root and no division per node.  h = 0.5025 / 14 puts their
+// switch radii 5.0 and 5.05 A on grid nodes (25 and 25.5025 A^2); SNT intervals
+// from S0 reach past 36 A^2.  phi_PdH and phi_HH have rows in r, 1/160 A apart from
+// 156/160 A (their switch radius 5.35 A is a grid node): exponentials are steepest
+// at short distances, where steps in s are the longest in r, and a node of an H
+// pair has r at hand from f_H.
 // Rows: values (S_FPD, the density pass) and slopes (S_DFPD) interpolate at
-// the Chebyshev points; the pair functions (S_PH*) integrate the quadratic
-// interpolating their slope, so value and slope come from one row.
+// the Chebyshev points; the pair functions (S_PHPD, R_PH*) integrate the quadratic
+// interpolating their slope, so value and slope come from one row.  Below 1.8 A
+// the quadratic in s is coarser for phi_Pd than the Hermite tables in r: Pd-Pd
+// pairs with a node there are evaluated node by node from those.
 // f_H = 11.0025 exp(-1.30927 |r|) is evaluated directly: |r| and the
 // exponential cost fewer clocks (8 for each transcendental) than one more
 // 16-byte row gathered from LDS (~12 clocks of the whole CU's LDS, which the
 // two other rows of a Pd-H node already keep busy).
-// Error against FP64 at 40^3 cells, tables in |r| (h = 0.01 A) and these: gradient
-// 6.8e-6 and 4.7e-7, objective 6.8e-9 and 7.8e-9 (12-point rule).
-constexpr double SH64 = 0.5025 / 14.0, S064 = 25.5025 - 683 * SH64;
-constexpr float SH = (float)SH64, S0 = (float)S064, SINV = (float)(1.0 / SH64), SB = (float)(-S064 / SH64);
+// Every function's error is held to that of the Hermite tables in r
+// (tests/test_pass_tables.py).
+// A node's coordinate is x = SINV s + SB, and f_H's s = SH x + S0; the rows are built on
+// the grid that the first two floats define.  The four are floats near 14 / 0.5025
+// and 683 - 25.5025 SINV that invert each other to 4e-10 (rounded apart: 1e-7 of
+// every s, a bias of all values); the radii are 2e-5 of a row off their nodes.
+constexpr float SINV = 27.860683f, SB = -27.517103f, SH = 0.035892874f, S0 = 0.9876679f;
+constexpr double SH64 = 1.0 / (double)SINV, S064 = -(double)SB / (double)SINV;
+static_assert((double)SH - SH64 < 1e-9 * SH64 && SH64 - (double)SH < 1e-9 * SH64 &&
+                  (double)S0 + (double)SB * SH < 1e-9 && (double)S0 + (double)SB * SH > -1e-9,
+              "SH and S0 invert SINV and SB");
 constexpr float SLO = 1.0f, SHI = 36.0f;  // nodes the tables serve: [1, 6) A
+constexpr float SLO_PHPD = 1.8f * 1.8f;   // and phi_Pd's rows in s
+template <int KIND>
+constexpr float s_lo() { return KIND == 0 ? SLO_PHPD : SLO; }
 constexpr int SNT = 977;
-enum { S_FPD = 0, S_DFPD = 1, S_PHPD = 2, S_PHPDH = 3, S_PHH = 4, NSTAB = 5 };  // S_DFPD.. are G_FPD.. of the gradient pass
+constexpr float RINV = 160.0f, RB = -156.0f;
+constexpr int RNT = 806;
 constexpr int S_BASE = NTAB * NT;  // first row of these tables after those in r
-static_assert(683 * SH64 < 24.515 && S064 < 1.0 && S064 + (SNT - 1) * SH64 > 36.0, "the grid covers [1, 36] A^2");
+enum { S_FPD = 0, S_DFPD = SNT, S_PHPD = 2 * SNT, R_PHPDH = 3 * SNT, R_PHH = R_PHPDH + RNT, S_ROWS = R_PHH + RNT };
+enum { P_DFPD = 0, P_PHPD = SNT, P_PHPDH = 2 * SNT, P_PHH = P_PHPDH + RNT, P_ROWS = P_PHH + RNT };  // staged by the gradient pass
+static_assert(S064 < 1.0 && S064 + (SNT - 1) * SH64 > 36.0, "the grid covers [1, 36] A^2");
+static_assert((RNT - 1 - (double)RB) / (double)RINV > 6.0, "the grid covers [1, 6] A");
 
 // Table coordinates and displacement squares of one pair.  12-point rule: the
 // nodes of site i have s = bi +- 2 ai d_c, of site j bj -+ 2 aj d_c.
@@ -445,7 +464,8 @@ struct Nodes27 {
     n1 = s3 * SINV;
   }
 };
-__device__ __forceinline__ bool inside(float lo, float hi) { return lo >= SLO && hi < SHI; }
+template <int KIND>
+__device__ __forceinline__ bool inside(float lo, float hi) { return lo >= s_lo<KIND>() && hi < SHI; }
 
 // The nodes of a pair one at a time, for the pairs with a node outside.
 // x(k): table coordinate of node k; w, off: its weight and displacement.
@@ -478,12 +498,12 @@ struct Edge {
   }
 };
 
-// f_H / 11.0025 at s, and 1/|r|: 2^(K r), K = -1.30927 log2(e) split into
+// f_H / 11.0025 at s, |r| and 1/|r|: 2^(K r), K = -1.30927 log2(e) split into
 // FP32 hi and lo parts, with the rounding of K r carried into a first-order
 // correction (within about an ulp of FP32).  Callers scale their sums.
-A2C_HD float fH_s(float s, float& rinv) {
+A2C_HD float fH_s(float s, float& r, float& rinv) {
   rinv = rsq(s);
-  const float r = s * rinv;
+  r = s * rinv;
   const float e = FH_KHI * r;
   const float el = fmaf(FH_KLO, r, fmaf(FH_KHI, r, -e));
   return eam::exp2_est(e) * fmaf(el, LN2F, 1.0f);
@@ -498,7 +518,7 @@ A2C_HD SPos s_pos(float x) { return {(int)x, eam::fract(x)}; }
 // node outside is evaluated node by node: the exponential tails from 6 A on,
 // NaN below 1 A -- no physical configuration comes that close, and the
 // non-finite objective makes the caller fall back to the FP64 path).
-__device__ __forceinline__ float s_of(float x) { return fmaf(x, SH, S0); }
+A2C_HD float s_of(float x) { return fmaf(x, SH, S0); }
 __device__ __forceinline__ bool s_in(float s) { return s >= SLO && s < SHI; }
 __device__ __forceinline__ float s_tail(int w, float s) { return tail(w, s * rsq(s)); }
 
@@ -516,8 +536,8 @@ __device__ __forceinline__ void node_dens(const float4* tab, float x, float& fpd
     }
   }
   if (WANT_H) {
-    float ri;
-    fh = in || s >= SHI ? fH_s(s, ri) : __builtin_nanf("");
+    float r, ri;
+    fh = in || s >= SHI ? fH_s(s, r, ri) : __builtin_nanf("");
   }
 }
 
@@ -578,11 +598,11 @@ __device__ __forceinline__ void pair_dens(const float4* tab, const float d[3], f
   bool in;
   if (RULE == GH3) {
     const Nodes27 q(d, sqrtf(as * as + bs * bs));
-    in = inside(q.lo, q.hi);
+    in = inside<3>(q.lo, q.hi);
     if (in) pair_density2_gh<NB_H, ME_H, true>(tab, q, mine, theirs);
   } else {
     const Nodes12 q(d, SQ6F * as, SQ6F * bs);
-    in = inside(q.lo, q.hi);
+    in = inside<3>(q.lo, q.hi);
     if (in) pair_density2<NB_H, ME_H, true>(tab, q, d, mine, theirs);
   }
   if (!in) {  // node by node, rolled (rare: a call would cost every pair the registers it keeps across it)
@@ -634,7 +654,7 @@ __device__ __forceinline__ void dens_list(const float4* tab, const LatDev& S, co
 // cells: 70% and 88% of the time busy).  6 waves per SIMD: 80 VGPRs hold both
 // rules' node blocks without spills.  40^3 cells, 12-point / Gauss-Hermite rule:
 // 214 / 340 us with tables in |r|, sites in lattice order and the loads of a
-// pair in its own turn, 147 / 255 us as it is.
+// pair in its own turn, 146 / 260 us as it is (events of a2c_fe_time_eval).
 template <int RULE, bool BY_SITE>
 __global__ __launch_bounds__(TB) __attribute__((amdgpu_waves_per_eu(6))) void k_dens_own(
     const LatDev* __restrict__ lats, const int32_t* __restrict__ ob2l, const float4* __restrict__ gtab) {
@@ -642,7 +662,7 @@ __global__ __launch_bounds__(TB) __attribute__((amdgpu_waves_per_eu(6))) void k_
   const int w = xcd_block();
   const LatDev& S = lats[ob2l[w]];
   if (S.rule != RULE) return;  // whole workgroup: the other rule's instance serves this lattice
-  stage16(tab, gtab + S_BASE + S_FPD * SNT, SNT);
+  stage16(tab, gtab + S_BASE + S_FPD, SNT);
   __syncthreads();
   const int K = S.kl32;
   const OwnerLane ln(S, w - S.owg0_32, K);
@@ -699,24 +719,41 @@ struct PairSums2 {
 // One node: the pair energy phi and cu = SH dE/ds, E = F'_i f_j + F'_j f_i + phi
 // (f_k: the density function of site k's species; KIND as in point_coef).
 // FP multiplies f_Pd', FH f_H' / |r| (it carries FH_D).  tab: LDS rows of the
-// gradient pass (G_*).
+// gradient pass (P_*), gtab: the tables in r.
 constexpr float FH_D = (float)(0.5 * SH64 * FH_K * 11.0025);
+// phi_PdH or phi_HH (tab: its rows) at r, and d/du
+A2C_HD void phi_r(const float4* tab, float r, float& v, float& d) {
+  const float y = fmaf(r, RINV, RB);
+  cubic_vd(tab[(int)y], eam::fract(y), v, d);
+}
+// phi_Pd from the Hermite rows in r (tab: all of its rows), and d/du
+A2C_HD void phi_Pd_r(const float4* tab, float r, float& v, float& d) {
+  const float y = fmaxf(fmaf(r, INVH, -R0 * INVH), 0.0f);
+  cubic_vd(tab[(int)y], eam::fract(y), v, d);
+}
 template <int KIND, bool IN>
-__device__ __forceinline__ void node_coef(const float4* tab, float x, float FP, float FH, float& phi, float& cu) {
-  constexpr int WP = KIND == 0 ? G_PHPD : (KIND == 3 ? G_PHH : G_PHPDH);
+__device__ __forceinline__ void node_coef(const float4* tab, const float4* __restrict__ gtab, float x, float FP,
+                                          float FH, float& phi, float& cu) {
   constexpr int TP = KIND == 0 ? T_PHPD : (KIND == 3 ? T_PHH : T_PHPDH);
   const float s = s_of(x);
   if (IN || s_in(s)) {
     const SPos p = s_pos(x);
-    float dphi;
-    cubic_vd(tab[WP * SNT + p.k], p.u, phi, dphi);
-    cu = dphi;
-    if (KIND != 3) cu = fmaf(FP, quad(tab[G_FPD * SNT + p.k], p.u), cu);
-    if (KIND != 0) {
-      float ri;
-      const float fh = fH_s(s, ri);
-      cu = fmaf(FH, fh * ri, cu);
+    float d;
+    if (KIND == 0) {
+      if (IN || s >= SLO_PHPD) {
+        cubic_vd(tab[P_PHPD + p.k], p.u, phi, cu);
+      } else {
+        const float ri = rsq(s);
+        phi_Pd_r(gtab + T_PHPD * NT, s * ri, phi, d);
+        cu = (0.5f * SH * INVH) * d * ri;
+      }
+    } else {
+      float r, ri;
+      const float fh = fH_s(s, r, ri);
+      phi_r(tab + (KIND == 3 ? P_PHH : P_PHPDH), r, phi, d);
+      cu = fmaf(FH, fh, (0.5f * SH * RINV) * d) * ri;
     }
+    if (KIND != 3) cu = fmaf(FP, cubic(tab[P_DFPD + p.k], p.u), cu);
   } else {
     const float ri = rsq(s);
     phi = s_tail(TP, s);
@@ -724,8 +761,8 @@ __device__ __forceinline__ void node_coef(const float4* tab, float x, float FP, 
     if (KIND != 3) c = fmaf(FP, TAIL[T_FPD][1] * s_tail(T_FPD, s), c);
     cu = 0.5f * SH * c * ri;
     if (KIND != 0) {
-      float r2;
-      cu = fmaf(FH, s >= SHI ? fH_s(s, r2) * ri : __builtin_nanf(""), cu);
+      float r1, r2;
+      cu = fmaf(FH, s >= SHI ? fH_s(s, r1, r2) * ri : __builtin_nanf(""), cu);
     }
   }
 }
@@ -739,7 +776,7 @@ __device__ __forceinline__ void node_coef(const float4* tab, float x, float FP, 
 // d0 and h2: unrolled, the table rows of all nodes are in flight and their
 // registers leave 4 waves per SIMD.
 template <int KIND, bool IN>
-__device__ __forceinline__ PairSums2 pair_grad2(const float4* tab, const Nodes12& n, const float d[3], float ai,
+__device__ __forceinline__ PairSums2 pair_grad2(const float4* tab, const float4* gtab, const Nodes12& n, const float d[3], float ai,
                                                 float aj, float FP, float FH) {
   float pe = 0.0f, su = 0.0f, d0 = d[0], d1 = d[1], d2 = d[2], h0 = 0.0f, h1 = 0.0f, h2 = 0.0f;
   float a = ai, xb = n.xi, g = n.gi;
@@ -751,8 +788,8 @@ __device__ __forceinline__ PairSums2 pair_grad2(const float4* tab, const Nodes12
     for (int c = 0; c < 3; ++c) {
       const float t = g * d0;
       float phi0, phi1, u0, u1;
-      node_coef<KIND, IN>(tab, xb + t, FP, FH, phi0, u0);
-      node_coef<KIND, IN>(tab, xb - t, FP, FH, phi1, u1);
+      node_coef<KIND, IN>(tab, gtab, xb + t, FP, FH, phi0, u0);
+      node_coef<KIND, IN>(tab, gtab, xb - t, FP, FH, phi1, u1);
       pe += phi0 + phi1;
       const float T = u0 - u1;
       ue += u0 + u1;
@@ -784,7 +821,7 @@ __device__ __forceinline__ PairSums2 pair_grad2(const float4* tab, const Nodes12
 //   q-gradient  sum u r = d U + sqrt(3) s Va,
 //   Sz = sum u (r . z) = sqrt(3) d . Va + 3 s Wn,  d/dsigma_k = Sz sigma_k / s.
 template <int KIND, bool IN>
-__device__ __forceinline__ PairSums2 pair_grad2_gh(const float4* tab, const Nodes27& q, const float d[3], float sd,
+__device__ __forceinline__ PairSums2 pair_grad2_gh(const float4* tab, const float4* gtab, const Nodes27& q, const float d[3], float sd,
                                                    float si, float sj, float FP, float FH) {
   float pe = 0.0f, U = 0.0f, V0 = 0.0f, V1 = 0.0f, V2 = 0.0f, Wn = 0.0f;
 #pragma unroll 1  // one z plane (9 nodes, unrolled) per trip, as in pair_density2_gh
@@ -798,7 +835,7 @@ __device__ __forceinline__ PairSums2 pair_grad2_gh(const float4* tab, const Node
         const int n = a0 * a0 + a1 * a1;
         const float w = ghwf(a0) * ghwf(a1);
         float phi, cc;
-        node_coef<KIND, IN>(tab, base + q.n1 * (float)n + (a0 * q.t[0] + a1 * q.t[1]), FP, FH, phi, cc);
+        node_coef<KIND, IN>(tab, gtab, base + q.n1 * (float)n + (a0 * q.t[0] + a1 * q.t[1]), FP, FH, phi, cc);
         p9 += w * phi;
         const float u = w * cc;
         u9 += u;
@@ -828,7 +865,7 @@ __device__ __forceinline__ PairSums2 pair_grad2_gh(const float4* tab, const Node
 }
 
 template <int RULE, int KIND>
-__device__ __forceinline__ PairSums2 pair_grad(const float4* tab, const float d[3], float as, float bs, float Fi,
+__device__ __forceinline__ PairSums2 pair_grad(const float4* tab, const float4* gtab, const float d[3], float as, float bs, float Fi,
                                                float Fj) {
   const float FP = KIND == 0 ? Fi + Fj : (KIND == 1 ? Fj : Fi);           // F' of the H site multiplies f_Pd'
   const float FH = FH_D * (KIND == 3 ? Fi + Fj : (KIND == 1 ? Fi : Fj));  // F' of the Pd site f_H'
@@ -837,13 +874,13 @@ __device__ __forceinline__ PairSums2 pair_grad(const float4* tab, const float d[
   if (RULE == GH3) {
     const float sd = sqrtf(as * as + bs * bs);
     const Nodes27 n(d, sd);
-    in = inside(n.lo, n.hi);
-    if (in) p = pair_grad2_gh<KIND, true>(tab, n, d, sd, as, bs, FP, FH);
+    in = inside<KIND>(n.lo, n.hi);
+    if (in) p = pair_grad2_gh<KIND, true>(tab, gtab, n, d, sd, as, bs, FP, FH);
   } else {
     const float ai = SQ6F * as, aj = SQ6F * bs;
     const Nodes12 n(d, ai, aj);
-    in = inside(n.lo, n.hi);
-    if (in) p = pair_grad2<KIND, true>(tab, n, d, ai, aj, FP, FH);
+    in = inside<KIND>(n.lo, n.hi);
+    if (in) p = pair_grad2<KIND, true>(tab, gtab, n, d, ai, aj, FP, FH);
   }
   if (!in) {  // node by node, rolled, as in pair_dens
     Edge<RULE> q(d, as, bs);
@@ -852,7 +889,7 @@ __device__ __forceinline__ PairSums2 pair_grad(const float4* tab, const float d[
 #pragma unroll 1
     for (int k = 0; k < Edge<RULE>::N; ++k) {
       float phi, u;
-      node_coef<KIND, false>(tab, q.x(k), FP, FH, phi, u);
+      node_coef<KIND, false>(tab, gtab, q.x(k), FP, FH, phi, u);
       p.pe = fmaf(q.w, phi, p.pe);
       u *= 2.0f * SINV * q.w;
       float ro = 0.0f;  // r . off
@@ -879,7 +916,7 @@ struct Own {
   double e = 0.0, g0 = 0.0, g1 = 0.0, g2 = 0.0, gs = 0.0;
 };
 template <int RULE, int KIND>
-__device__ __forceinline__ void grad_list(const float4* tab, const LatDev& S, const OwnerLane& ln, const Site& a,
+__device__ __forceinline__ void grad_list(const float4* tab, const float4* gtab, const LatDev& S, const OwnerLane& ln, const Site& a,
                                           float Fi, const Image& img, double wme, Own& o) {
   constexpr bool ME_H = KIND >= 2, NB_H = KIND & 1;
   const Ell& L = ME_H ? (NB_H ? S.hh : S.hpd) : (NB_H ? S.pdh : S.pdpd);
@@ -897,7 +934,7 @@ __device__ __forceinline__ void grad_list(const float4* tab, const LatDev& S, co
         return p;
       },
       [&](const Pair32& q, float Fj, double wj, int jl, int rv) {
-        const PairSums2 p = pair_grad<RULE, KIND>(tab, q.d, as, q.bs, Fi, Fj);
+        const PairSums2 p = pair_grad<RULE, KIND>(tab, gtab, q.d, as, q.bs, Fi, Fj);
         o.e += wj * p.pe;
         o.g0 += wj * p.g[0];
         o.g1 += wj * p.g[1];
@@ -914,14 +951,14 @@ __device__ __forceinline__ void grad_list(const float4* tab, const LatDev& S, co
 
 // Bound by what a pair moves: 8 B of list, ~50 B gathered through L1 and 16 B of
 // share written (0.33 GB at 40^3 cells) keep the kernel at 246 us with its
-// nodes taken out; with them 261 us (12-point rule; 364 us before the tables
-// in |r|^2, the row order and the pipelined loads) and 508 us (Gauss-Hermite;
-// 651 us).
+// nodes taken out; with them 263 us (12-point rule; 364 us before the tables,
+// the row order and the pipelined loads) and 493 us (Gauss-Hermite; 651 us), events of
+// a2c_fe_time_eval.
 template <int RULE, int TBO>
 __global__ __launch_bounds__(TBO) __attribute__((amdgpu_waves_per_eu(TBO / 128))) void k_grad_own(
     const LatDev* __restrict__ lats, const int32_t* __restrict__ ob2l, int nblk, const float4* __restrict__ gtab) {
-  __shared__ float4 tab[NGTAB * SNT];
-  stage16(tab, gtab + S_BASE + S_DFPD * SNT, NGTAB * SNT);
+  __shared__ float4 tab[P_ROWS];
+  stage16(tab, gtab + S_BASE + S_DFPD, P_ROWS);
   __syncthreads();
   const int w = xcd_block() * (TBO / TB) + __builtin_amdgcn_readfirstlane(threadIdx.x / TB);
   if (w >= nblk) return;
@@ -936,12 +973,12 @@ __global__ __launch_bounds__(TBO) __attribute__((amdgpu_waves_per_eu(TBO / 128))
   const float Fi = gmem((const float2*)S.aux)[s].x;
   Own o;
   if (ln.pd) {
-    grad_list<RULE, 0>(tab, S, ln, a, Fi, img, 1.0, o);
-    grad_list<RULE, 1>(tab, S, ln, a, Fi, img, 1.0, o);
+    grad_list<RULE, 0>(tab, gtab, S, ln, a, Fi, img, 1.0, o);
+    grad_list<RULE, 1>(tab, gtab, S, ln, a, Fi, img, 1.0, o);
   } else {
     const double wme = gmem((const double*)S.xrow)[ln.row];
-    grad_list<RULE, 2>(tab, S, ln, a, Fi, img, wme, o);
-    grad_list<RULE, 3>(tab, S, ln, a, Fi, img, wme, o);
+    grad_list<RULE, 2>(tab, gtab, S, ln, a, Fi, img, wme, o);
+    grad_list<RULE, 3>(tab, gtab, S, ln, a, Fi, img, wme, o);
   }
   o.e = site_sum(o.e, K);
   o.g0 = site_sum(o.g0, K);
@@ -1040,18 +1077,20 @@ Row through(const long double* u, const long double* y, int n) {
   return m;
 }
 enum { FIT_VALUE, FIT_SLOPE, FIT_BOTH };
+// rows of the tables in s, or in r; g gives a function's value and slope in |r|
 template <class Fn>
-void fill_table_s(float4* out, int fit, Fn g) {
-  const long double PI = 3.14159265358979323846264338327950288L, h = 0.5025L / 14, s0 = 25.5025L - 683 * h;
+void fill_rows(float4* out, int rows, bool in_r, int fit, Fn g) {
+  using LD = long double;
+  const LD PI = 3.14159265358979323846264338327950288L;
   auto node = [&](int i, int n) { return 0.5L - 0.5L * cosl((2 * i + 1) * PI / (2.0L * n)); };
-  for (int k = 0; k < SNT; ++k) {
-    auto at = [&](long double u) {
-      const long double r = sqrtl(s0 + (k + u) * h);
-      const eam::VDT<long double> v = g(r);
-      return eam::VDT<long double>{v.v, v.d * h / (2 * r)};
+  for (int k = 0; k < rows; ++k) {
+    auto at = [&](LD u) {
+      const LD x = k + u, r = in_r ? (x - (LD)RB) / (LD)RINV : sqrtl((x - (LD)SB) / (LD)SINV);
+      const eam::VDT<LD> v = g(r);
+      return eam::VDT<LD>{v.v, v.d / (in_r ? (LD)RINV : 2 * r * (LD)SINV)};  // d/du
     };
-    const int n = fit == FIT_VALUE ? 4 : 3;
-    long double u[4], y[4];
+    const int n = fit == FIT_BOTH ? 3 : 4;
+    LD u[4], y[4];
     for (int i = 0; i < n; ++i) {
       u[i] = node(i, n);
       y[i] = fit == FIT_VALUE ? at(u[i]).v : at(u[i]).d;
@@ -1060,7 +1099,7 @@ void fill_table_s(float4* out, int fit, Fn g) {
     if (fit == FIT_BOTH) {  // the slope's integral, with the value's mean over four points
       m = Row{{0, m.c[0], m.c[1] / 2, m.c[2] / 3}};
       for (int i = 0; i < 4; ++i) {
-        const long double w = node(i, 4);
+        const LD w = node(i, 4);
         y[i] = at(w).v - w * (m.c[1] + w * (m.c[2] + w * m.c[3]));
       }
       m.c[0] = (y[0] + y[1] + y[2] + y[3]) / 4;
@@ -1074,12 +1113,12 @@ void fill_table_s(float4* out, int fit, Fn g) {
 void host_tables_s(std::vector<float4>& t) {
   static const std::vector<float4> built = [] {  // once per process
     using LD = long double;
-    std::vector<float4> u((size_t)NSTAB * SNT);
-    fill_table_s(&u[S_FPD * SNT], FIT_VALUE, [](LD r) { return eam::f_Pd_vd<LD>(r); });
-    fill_table_s(&u[S_DFPD * SNT], FIT_SLOPE, [](LD r) { return eam::f_Pd_vd<LD>(r); });
-    fill_table_s(&u[S_PHPD * SNT], FIT_BOTH, [](LD r) { return eam::phi_Pd_vd<LD>(r, eam::f_Pd_vd<LD>(r)); });
-    fill_table_s(&u[S_PHPDH * SNT], FIT_BOTH, [](LD r) { return eam::phi_morse_vd<0, LD>(r); });
-    fill_table_s(&u[S_PHH * SNT], FIT_BOTH, [](LD r) { return eam::phi_morse_vd<1, LD>(r); });
+    std::vector<float4> u((size_t)S_ROWS);
+    fill_rows(&u[S_FPD], SNT, false, FIT_VALUE, [](LD r) { return eam::f_Pd_vd<LD>(r); });
+    fill_rows(&u[S_DFPD], SNT, false, FIT_SLOPE, [](LD r) { return eam::f_Pd_vd<LD>(r); });
+    fill_rows(&u[S_PHPD], SNT, false, FIT_BOTH, [](LD r) { return eam::phi_Pd_vd<LD>(r, eam::f_Pd_vd<LD>(r)); });
+    fill_rows(&u[R_PHPDH], RNT, true, FIT_BOTH, [](LD r) { return eam::phi_morse_vd<0, LD>(r); });
+    fill_rows(&u[R_PHH], RNT, true, FIT_BOTH, [](LD r) { return eam::phi_morse_vd<1, LD>(r); });
     return u;
   }();
   t.insert(t.end(), built.begin(), built.end());
@@ -1099,26 +1138,39 @@ void host_tables(std::vector<float4>& t) {
   t = built;
 }
 
-// One EAM function (order of a2c_eam_tables) at r in [1, 6) as the pair-once passes
-// take it from the tables t: value, and slope in r.
-void pass_eval32(const std::vector<float4>& t, int fn, float s, double& v, double& d) {
-  const SPos p = s_pos(fmaf(s, SINV, SB));
-  const double r = std::sqrt((double)s);
-  float vf = 0.0f, df = 0.0f, ri;
+// One EAM function (order of a2c_eam_tables) near r in [1, 6) A as the pair-once
+// passes take it from the tables t (those in r, then these), value and slope in r,
+// at the radius returned: what the FP32 table coordinate of r stands for.
+double pass_eval32(const std::vector<float4>& t, int fn, double r0, double& v, double& d) {
+  const float x = fmaf((float)(r0 * r0), SINV, SB);
+  const double r_at = std::sqrt(((double)x - (double)SB) / (double)SINV);
+  const SPos p = s_pos(x);
+  const float4* u = &t[S_BASE];
+  const float s = s_of(x);
+  const double ds = 2.0 * SINV * r_at;  // of d/du in s
+  float vf = 0.0f, df = 0.0f, r, ri;
+  const float fh = fH_s(s, r, ri);
   if (fn == T_FH) {
-    vf = fH_s(s, ri);
-    v = (double)FH_C * vf;
-    d = FH_K * FH_C * vf;
-    return;
+    v = (double)FH_C * fh;
+    d = FH_K * FH_C * fh;
+    return r_at;
   }
   if (fn == T_FPD) {
-    vf = cubic(t[S_FPD * SNT + p.k], p.u);
-    df = quad(t[S_DFPD * SNT + p.k], p.u);
+    vf = cubic(u[S_FPD + p.k], p.u);
+    df = cubic(u[S_DFPD + p.k], p.u);
+    d = ds * df;
+  } else if (fn == T_PHPD && s < SLO_PHPD) {
+    phi_Pd_r(&t[T_PHPD * NT], r, vf, df);
+    d = (double)INVH * df;
+  } else if (fn == T_PHPD) {
+    cubic_vd(u[S_PHPD + p.k], p.u, vf, df);
+    d = ds * df;
   } else {
-    cubic_vd(t[(fn == T_PHPD ? S_PHPD : fn == T_PHPDH ? S_PHPDH : S_PHH) * SNT + p.k], p.u, vf, df);
+    phi_r(u + (fn == T_PHPDH ? R_PHPDH : R_PHH), r, vf, df);
+    d = (double)RINV * df;
   }
   v = vf;
-  d = 2.0 * SINV * r * df;
+  return r_at;
 }
 
 int build_tables(a2c_fe_ctx* c) {

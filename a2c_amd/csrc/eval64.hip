@@ -1623,16 +1623,14 @@ extern "C" int a2c_eam_pass(int32_t precision, int32_t fn, int32_t n, const doub
   std::vector<double> t64;
   std::vector<float4> t32;
   if (precision == A2C_PREC_FP64) a2c::host_tables64_s(t64);
-  else a2c::host_tables_s(t32);
+  else a2c::host_tables(t32), a2c::host_tables_s(t32);
   for (int i = 0; i < n; ++i) {
     if (!(r[i] >= 1.0 && r[i] < 5.999)) return A2C_EINVAL;
     if (precision == A2C_PREC_FP64) {
       r_at[i] = r[i];
       a2c::pass_eval64(t64, fn, r[i], v[i], d[i]);
     } else {
-      const float s = (float)(r[i] * r[i]);
-      r_at[i] = std::sqrt((double)s);
-      a2c::pass_eval32(t32, fn, s, v[i], d[i]);
+      r_at[i] = a2c::pass_eval32(t32, fn, r[i], v[i], d[i]);
     }
   }
   return A2C_OK;

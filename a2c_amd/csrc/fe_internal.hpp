@@ -676,7 +676,7 @@ constexpr int T64_PART1 = T64_NF * T64_N * T64_P;                // doubles
 constexpr int T64_SIZE = T64_PART1 + T64Q_NF * T64_N * T64Q_P;  // doubles
 void host_tables64(std::vector<double>& t);
 void pass_eval64(const std::vector<double>& t, int fn, double r, double& v, double& d);
-void pass_eval32(const std::vector<float4>& t, int fn, float s, double& v, double& d);
+double pass_eval32(const std::vector<float4>& t, int fn, double r, double& v, double& d);  // returns the radius
 void host_tables64_s(std::vector<double>& t);  // those of the FP64 owner passes, in |r|^2 (eval64.hip)
 // The FP32 and FP64 EAM tables on one device, uploaded at the first call for
 // that device and shared by every context and batch of the process until it

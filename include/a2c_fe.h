@@ -333,8 +333,8 @@ int a2c_eam_tables64(double* out, int32_t cap);
 /* Host-only (no GPU): an EAM function (fn 0..4, in the order of a2c_eam_tables)
  * at n radii in [1, 5.999) A as the pair-once passes of a precision
  * (A2C_PREC_FP64, A2C_PREC_MIXED) evaluate it from their tables: value[i] and
- * slope[i] (d/dr) at r_at[i], which is r[i] in FP64 and the root of r[i]^2 rounded
- * to FP32 in the mixed passes.  Measures those tables against the closed forms.
+ * slope[i] (d/dr) at r_at[i], which is r[i] in FP64 and, in the mixed passes, the
+ * radius that the FP32 table coordinate of r[i] stands for.  Measures those tables against the closed forms.
  * A2C_EINVAL for other arguments. */
 int a2c_eam_pass(int32_t precision, int32_t fn, int32_t n, const double* r, double* r_at, double* value,
                  double* slope);

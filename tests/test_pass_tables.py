@@ -55,7 +55,7 @@ def plain(fn, r, precision):
     return horner(tab[k], (r - 1.0) / 0.05 - k, 0.05)
 
 
-CASES = [("fp64", f) for f in range(5)] + [("mixed", F_H)]
+CASES = [(p, f) for p in ("fp64", "mixed") for f in range(5)]
 
 
 @pytest.mark.parametrize("precision,fn", CASES)
