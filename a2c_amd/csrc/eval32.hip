@@ -520,7 +520,9 @@ A2C_HD SPos s_pos(float x) { return {(int)x, eam::fract(x)}; }
 // non-finite objective makes the caller fall back to the FP64 path).
 A2C_HD float s_of(float x) { return fmaf(x, SH, S0); }
 __device__ __forceinline__ bool s_in(float s) { return s >= SLO && s < SHI; }
-__device__ __forceinline__ float s_tail(int w, float s) { return tail(w, s * rsq(s)); }
+__device__ __forceinline__ float s_tail(int w, float s) {  // by s: at 36 the rounded radius may fall short of 6
+  return s >= SHI ? TAIL[w][0] * __expf(TAIL[w][1] * (s * rsq(s) - TAIL[w][2])) : __builtin_nanf("");
+}
 
 // Densities at one node: f_Pd (tab: its value rows) and f_H / 11.0025, as wanted.
 template <bool WANT_PD, bool WANT_H, bool IN>
