@@ -197,8 +197,9 @@ int a2c_fe_set_occupancy(a2c_fe_ctx* c, const double* x) {
 int a2c_fe_build_neighbors(a2c_fe_ctx* c, const double* X, a2c_nbr_stats* stats) {
   if (int rc = check_ctx(c)) return rc;
   if (!X && c->N > 0) return set_err(c, A2C_EINVAL, "X is null");
-  // once per build: straight from the caller's array (ordered on the stream;
-  // the build synchronises before it returns), no pinned staging
+  // once per build: straight from the caller's array, no pinned staging.  The
+  // build waits for the list widths, behind this copy and the count pass; its last
+  // passes may still run when it returns
   if (c->N > 0) A2C_HIP(c, hipMemcpyAsync(c->dX, X, 32 * (size_t)c->N, hipMemcpyHostToDevice, c->stream));
   c->lat_dirty = true;
   if (int rc = nbr_build(c)) return rc;

@@ -8,8 +8,11 @@
 // 0.75a^2 < d2 < 1.25a^2, else (minimizer.cpp:935-947); HH1 = H neighbors with
 // d2 < 0.75a^2 (:999-1004).
 //
-// Passes, all on the device (one host synchronisation, for the list widths after
-// the count pass; the caller's positions have been read by then):
+// Passes, all on the device.  The host waits once, for the list widths after the
+// count pass (the caller's positions have been read by then), and on a specimen
+// with a non-periodic axis once before, for the bounding box; the passes behind the
+// widths are still queued when the build returns, and whoever reads the lists from
+// the host waits for the stream first:
 //   k_bin     cell of each site and the cell histogram
 //   k_scan    exclusive scan of the histogram (one workgroup)
 //   k_place   positions as floats in cell order, with the site index, so a

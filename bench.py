@@ -487,6 +487,7 @@ def measure(A, args, X, x, box, npd, nh, quad, steps, warmup, calib=False, paths
     fe.set_occupancy(x)
     t0 = time.perf_counter()
     st = fe.findNeighbors(X)
+    fe.sync()  # the build's last passes run on after it returns
     nbr_ms = (time.perf_counter() - t0) * 1e3
     U = (st["total"][0] / 2.0, float(st["total"][1]), st["total"][3] / 2.0)  # unordered PdPd, PdH, HH
     K = POINTS[quad]
