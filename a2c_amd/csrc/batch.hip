@@ -16,7 +16,8 @@
 // line search with approximate Wolfe acceptance in FP64, steepest-descent
 // restart on failure, TAO's gatol/grtol/gttol tests, and the mixed -> FP64
 // switch.  In a batch every step is one launch over all slots that need it
-// (segmented kernels; the recursion of a small slot in one workgroup), and
+// (segmented kernels; the recursion in its vector-free form, three passes, for up
+// to VF_PAIRS pairs, else pass by pass, a small slot's in one workgroup), and
 // each scalar decision is taken per slot on the host after one
 // synchronisation per round.  Slots can be added and started between
 // iterations (continuous batching).
@@ -457,9 +458,10 @@ __global__ __launch_bounds__(TB) void k_seg_bound(const SegBound* __restrict__ o
   }
 }
 
-// Two-loop recursion of one small slot in one workgroup.  The segmented form
-// costs ~4 launches per stored pair; a slot of a few thousand sites is
-// launch-bound, so one workgroup per slot runs the whole recursion (every dot
+// Two-loop recursion of one small slot with more than VF_PAIRS pairs (fewer take
+// the vector-free form) in one workgroup.  The segmented form costs ~4 launches
+// per stored pair; a slot of a few thousand sites is launch-bound, so one
+// workgroup per slot runs the whole recursion (every dot
 // a fixed-order block sum), then d = -H g with the active part of the sigma
 // bound zeroed, and writes g . d.  Pass t applies the update of step t and
 // forms the dot the next step needs, so the recursion takes 2 np + 1 passes.
@@ -1927,7 +1929,9 @@ size_t a2c_batch_footprint(int32_t n_pd, int32_t n_h, int32_t lmvm_m) {
   // lists ~100 int32 per site, the owned/received halves of two pair lists
   // per site (~28 wide: 2 int32 per owned slot, a 32-byte share per received
   // slot), optimizer (7 + 2m) x 4N doubles; plus a quarter for the device
-  // cache's size classes (a block is rounded up by at most a quarter)
+  // cache's size classes (a block is rounded up by at most a quarter) and for
+  // the row-order copies (~70 bytes per site) and the received halves' spare slot (64).
+  // An FCC lattice of 262,144 sites takes 0.83 of it, its optimizer included.
   const size_t raw =
       N * (4 * 32 + 40 + 100 * 4 + 2 * 28 * (2 * 4 + 32) + (7 + 2 * (size_t)std::max(lmvm_m, 1)) * 32) +
       ((size_t)1 << 20);

@@ -863,31 +863,31 @@ __device__ __forceinline__ PairSums pair_sums27(const double* tab, const double*
 // One pair in closed form, node by node.
 template <int RULE, int KIND>
 __device__ __forceinline__ PairSums closed_sums(const double d[3], double si, double sj, double Fi, double Fj) {
-      const Closed<RULE> q(d, si, sj);
-      PairSums p{};
-      double sz = 0.0;
-  #pragma unroll 1
-      for (int k = 0; k < Closed<RULE>::N; ++k) {
-        double z[3], w, phi, c;
-        const double r = q.node(k, z, w);
-        pair_point<A2C_DERIV_ANALYTIC, KIND>(r, Fi, Fj, 0.0, phi, c);
-        p.pe += w * phi;
-        const double u = w * c / r;
-        double ro = 0.0;  // r . z
-  #pragma unroll
-        for (int x = 0; x < 3; ++x) {
-          const double rx = d[x] + z[x];
-          p.g[x] += u * rx;
-          ro += rx * z[x];
-        }
-        if (RULE == GH3) sz += u * ro;
-        else if (k < 6) p.gsi += u * ro / q.ai;
-        else p.gsj += u * ro / q.aj;
-      }
-      if (RULE == GH3) {  // z = s (node): d/dsigma_k = (sum u r . node) sigma_k / s
-        p.gsi = sz * si / (q.sd * q.sd);
-        p.gsj = sz * sj / (q.sd * q.sd);
-      }
+  const Closed<RULE> q(d, si, sj);
+  PairSums p{};
+  double sz = 0.0;
+#pragma unroll 1
+  for (int k = 0; k < Closed<RULE>::N; ++k) {
+    double z[3], w, phi, c;
+    const double r = q.node(k, z, w);
+    pair_point<A2C_DERIV_ANALYTIC, KIND>(r, Fi, Fj, 0.0, phi, c);
+    p.pe += w * phi;
+    const double u = w * c / r;
+    double ro = 0.0;  // r . z
+#pragma unroll
+    for (int x = 0; x < 3; ++x) {
+      const double rx = d[x] + z[x];
+      p.g[x] += u * rx;
+      ro += rx * z[x];
+    }
+    if (RULE == GH3) sz += u * ro;
+    else if (k < 6) p.gsi += u * ro / q.ai;
+    else p.gsj += u * ro / q.aj;
+  }
+  if (RULE == GH3) {  // z = s (node): d/dsigma_k = (sum u r . node) sigma_k / s
+    p.gsi = sz * si / (q.sd * q.sd);
+    p.gsj = sz * sj / (q.sd * q.sd);
+  }
   return p;
 }
 // false, and zeros, if a node lies outside the tables

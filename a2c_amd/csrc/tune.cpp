@@ -25,15 +25,19 @@ a2c_tune_table default_table() {
   // The FP64 gradient pass runs 512 lanes per CU at a time (its tables fill the
   // LDS), 131,072 on 256 CUs, and a lattice takes ceil(sites K / 131072) rounds of
   // length ~ 1/K: alone it finishes soonest at the K whose last round is
-  // fullest, so the classes end at multiples of 1/8 of that capacity.  FP64, 12-point
-  // rule, K = 1/2/4/8, us per evaluation: 13,824 sites 195/129/100/90, 32,768
-  // sites 205/143/123/136, 64,000 sites 211/174/181/215, 85,184 sites 277/283/252/
-  // 301, 110,592 sites 292/290/316/346, 140,608 sites 486/410/391/441, 175,616
-  // sites 499/424/465/531, 373,248 sites 820/860/942/1113.  The mixed passes hold
-  // twice the lanes in smaller workgroups and want K = 8 up to 16,384 sites (13,824
-  // sites 128/87/68/63), 2 on the largest (373,248 sites 410/407/433/509), and
-  // 4 between, where 8 gains little alone (27,000 sites 135/95/83/80) and costs
-  // 15% in a batch's full launches.
+  // fullest, so up to 1.5 times that capacity the classes end at multiples of 1/8 of
+  // it.  Beyond, the last of many rounds weighs less than what more lanes per row
+  // cost, and K = 1 was fastest at every size measured.  FP64, 12-point rule, K =
+  // 1/2/4/8, us per evaluation: 13,824 sites 215/140/106/96, 32,768 sites
+  // 228/155/136/149, 64,000 sites 230/198/206/237, 85,184 sites 321/333/289/338,
+  // 110,592 sites 335/341/367/391, 140,608 sites 568/478/452/500, 175,616 sites
+  // 581/496/538/601, 216,000 sites 611/641/634/757, 373,248 sites 922/979/1075/1248.
+  // A lattice's K is the same in a batch's full launches, where only the cost per
+  // lane counts: K = 4 for 1 adds 10% there in FP64.  The mixed passes hold twice the
+  // lanes in smaller workgroups and want K = 8 up to 16,384 sites (13,824 sites
+  // 132/88/68/62), 2 on the largest (373,248 sites 428/408/437/511), and 4 between,
+  // where 8 gains little alone (27,000 sites 139/96/83/81) and costs 15% in a batch's
+  // full launches.
   static const int32_t max_sites[] = {16384, 32768, 65536, 98304, 131072, 163840, 196608, INT_MAX};
   static const int32_t lanes_mixed[] = {8, 4, 4, 4, 4, 4, 4, 2};
   static const int32_t lanes_fp64[] = {8, 4, 2, 4, 1, 4, 2, 1};

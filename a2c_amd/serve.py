@@ -73,8 +73,12 @@ def materialize(req):
     return X, x, box, npd, nh
 
 
-# Cost of one LMVM iteration of a lattice (mixed precision, in a batch): a
-# fixed part (~50 launches and 3 host round trips) and a per-site part.
+# What the policies charge an LMVM iteration of a lattice: a fixed part (launches
+# and host round trips) and a per-site part, in the seconds of a slow iteration of
+# several trials with slower kernels.  One of a trial takes 1.05e-4 s + 1.34e-9 s per
+# site (mixed, lattices of 1,728 to 884,736 sites, alone and in batches); the
+# policies depend on the parts' ratio and on the sizes that a tick of TICK_MIN_S
+# carries, which were chosen with these values.
 ITER_FIXED_S = 4e-4
 ITER_SITE_S = 9e-9
 
