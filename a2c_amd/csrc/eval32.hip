@@ -723,9 +723,13 @@ struct PairSums2 {
 // FP multiplies f_Pd', FH f_H' / |r| (it carries FH_D).  tab: LDS rows of the
 // gradient pass (P_*), gtab: the tables in r.
 constexpr float FH_D = (float)(0.5 * SH64 * FH_K * 11.0025);
-// phi_PdH or phi_HH (tab: its rows) at r, and d/du
-A2C_HD void phi_r(const float4* tab, float r, float& v, float& d) {
-  const float y = fmaf(r, RINV, RB);
+// phi_PdH or phi_HH (tab: its rows) at |r|^2 = s, r = sqrt(s) and ri = 1 / r rounded, and
+// d/du.  The coordinate carries what r lost to rounding (0.5 ri (s - r^2)): the
+// objective's noise, which ends the mixed phase of a relaxation, follows it.  40^3
+// cells: +6 us, Gauss-Hermite +29; 64 lattices relaxed together 3,318 FP64 evaluations
+// without it, 2,895 with it, 61.8 and 67.1 relaxations/s.
+A2C_HD void phi_r(const float4* tab, float s, float r, float ri, float& v, float& d) {
+  const float y = fmaf(r, RINV, fmaf((0.5f * RINV) * ri, fmaf(-r, r, s), RB));
   cubic_vd(tab[(int)y], eam::fract(y), v, d);
 }
 // phi_Pd from the Hermite rows in r (tab: all of its rows), and d/du
@@ -752,7 +756,7 @@ __device__ __forceinline__ void node_coef(const float4* tab, const float4* __res
     } else {
       float r, ri;
       const float fh = fH_s(s, r, ri);
-      phi_r(tab + (KIND == 3 ? P_PHH : P_PHPDH), r, phi, d);
+      phi_r(tab + (KIND == 3 ? P_PHH : P_PHPDH), s, r, ri, phi, d);
       cu = fmaf(FH, fh, (0.5f * SH * RINV) * d) * ri;
     }
     if (KIND != 3) cu = fmaf(FP, cubic(tab[P_DFPD + p.k], p.u), cu);
@@ -953,8 +957,8 @@ __device__ __forceinline__ void grad_list(const float4* tab, const float4* gtab,
 
 // Bound by what a pair moves: 8 B of list, ~50 B gathered through L1 and 16 B of
 // share written (0.33 GB at 40^3 cells) keep the kernel at 246 us with its
-// nodes taken out; with them 263 us (12-point rule; 364 us before the tables,
-// the row order and the pipelined loads) and 493 us (Gauss-Hermite; 651 us), events of
+// nodes taken out; with them 275 us (12-point rule; 364 us before the tables,
+// the row order and the pipelined loads) and 535 us (Gauss-Hermite; 651 us), events of
 // a2c_fe_time_eval.
 template <int RULE, int TBO>
 __global__ __launch_bounds__(TBO) __attribute__((amdgpu_waves_per_eu(TBO / 128))) void k_grad_own(
@@ -1168,7 +1172,7 @@ double pass_eval32(const std::vector<float4>& t, int fn, double r0, double& v, d
     cubic_vd(u[S_PHPD + p.k], p.u, vf, df);
     d = ds * df;
   } else {
-    phi_r(u + (fn == T_PHPDH ? R_PHPDH : R_PHH), r, vf, df);
+    phi_r(u + (fn == T_PHPDH ? R_PHPDH : R_PHH), s, r, ri, vf, df);
     d = (double)RINV * df;
   }
   v = vf;

@@ -84,3 +84,18 @@ def test_pass_tables(precision, fn):
             bad.append((lo, hi, "value %.1e of %.1e" % (ev[np.argmax(ev / bv)], bv[np.argmax(ev / bv)]),
                         "slope %.1e of %.1e" % (ed[np.argmax(ed / bd)], bd[np.argmax(ed / bd)])))
     assert not bad, "\n".join(map(str, bad))
+
+
+@pytest.mark.parametrize("fn", [PHI_PDH, PHI_HH])
+@pytest.mark.parametrize("lo,hi", [(1.7, 2.2), (2.2, 2.6), (3.2, 3.6), (4.2, 4.6)])
+def test_mixed_coordinate_noise(fn, lo, hi):
+    """What a pair function's value in the mixed passes loses to its argument: the
+    rms error over the slope is at most half an FP32 unit of r (two roundings of rms
+    0.29 units beside the table coordinate's), plus one of the value.  Noise of the
+    objective ends the mixed phase of a relaxation; a rounded radius alone leaves
+    0.8 units."""
+    r = np.random.default_rng(fn).uniform(lo, hi, 20000)
+    at, v, _ = A.eam_pass(fn, r, "mixed")
+    e, slope = O.eam(ORACLE[fn], at), np.mean(np.abs(O.eam_d(ORACLE[fn], at)))
+    rms = np.sqrt(np.mean((v - e) ** 2)) / slope
+    assert rms <= 2.0 ** -24 * (0.5 * np.mean(r) + np.mean(np.abs(e)) / slope)
