@@ -59,7 +59,7 @@ constexpr int NLANES = 5;
 // time may add: for a lattice that alone fills fewer SIMDs than the device
 // has, and for one that fills them (where near-equal throughputs differ
 // alone: at 24^3 cells mixed, K = 2 and 4 are within 5% per site in a full
-// launch, and 158 and 154 us alone).
+// launch, and 171 and 169 us alone).
 constexpr double LATENCY_COST = 1.25, THROUGHPUT_SLACK = 1.05;
 const int LANES[NLANES] = {1, 2, 4, 8, 16};
 bool valid_lanes(int k) { return k == 1 || k == 2 || k == 4 || k == 8 || k == 16; }
